@@ -317,6 +317,24 @@ def test_masked_attention_parity_half(hexmi, oracle, case, dtype, with_mask):
     assert (got32 - want).abs().max() <= (5e-3 if dtype == torch.float16 else 3e-2)
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("case", [(2, 5, 1, 64), (1, 33, 3, 128), (3, 129, 63, 64), (2, 130, 65, 128), (2, 64, 127, 80),
+                                  (3, 128, 130, 128), (1, 300, 1023, 96), (2, 257, 2051, 128)])
+def test_masked_attention_mask_rows_of_any_length_and_alignment(hexmi, oracle, case, dtype):
+    # mask rows of an odd number of keys on the matrix-core kernel, the mask itself one element off its allocation;
+    # the tolerances are those of test_masked_attention_parity_half (the same sums, the same roundings)
+    B, Sq, Skv, D = case
+    g = _gen(27)
+    q = torch.randn(B, Sq, D, generator=g).to(dtype)
+    k, v = torch.randn(B, Skv, D, generator=g).to(dtype), torch.randn(B, Skv, D, generator=g).to(dtype)
+    mask = _mask(B, Sq, Skv, dtype, 28)
+    shifted = torch.empty(mask.numel() + 1, dtype=dtype, device="cuda")[1:].view(B, Sq, Skv)
+    shifted.copy_(mask)
+    got = hexmi.attention(q.cuda(), k.cuda(), v.cuda(), shifted, out_dtype=torch.float32).cpu()
+    want = _oracle_masked(oracle, q, k, v, mask, 1.0 / math.sqrt(D))
+    assert (got - want).abs().max() <= (5e-3 if dtype == torch.float16 else 3e-2)
+
+
 @pytest.mark.parametrize("case", [(2, 50, 70, 32), (1, 64, 64, 128), (1, 33, 129, 64),
                                   # Skv % 4 == 0 with head size 64 / 128: the fp32 matrix-core kernel with a mask
                                   (2, 200, 72, 64), (1, 130, 516, 128), (3, 129, 1028, 64),
