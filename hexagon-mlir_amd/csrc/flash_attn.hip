@@ -764,15 +764,20 @@ int launch_rowwise(const void* Q, const void* K, const void* V, const void* mask
   return launch_status();
 }
 
+// the matrix-core kernels address a head's keys with 32-bit byte offsets
+// and take the row maximum of the raw scores before scaling them, which is the maximum of the scaled scores only
+// for a positive scale: zero and negative scales go to the row-wise kernel, which scales first
+inline bool matrix_core_operands(const void* Q, const void* K, const void* V, const void* O, int64_t head_bytes,
+                                 float scale_log2e) {
+  return aligned_to(Q, 16) && aligned_to(K, 16) && aligned_to(V, 16) && aligned_to(O, 16) && head_bytes < 0x7fffffff &&
+         scale_log2e > 0.0f;
+}
+
 // mask == nullptr and Skv == S: the tuned kernels; otherwise the general ones.
 template <typename T, typename OutT>
 int dispatch_half(const void* Q, const void* K, const void* V, const void* mask, void* O, int64_t ZH, int64_t S,
                   int64_t Skv, int64_t D, float scale_log2e, bool causal, hipStream_t st) {
-  // the matrix-core kernels address a head's keys with 32-bit byte offsets
-  // and take the row maximum of the raw scores before scaling them, which is the maximum of the scaled scores only
-  // for a positive scale: zero and negative scales go to the row-wise kernel, which scales first
-  const bool ok = aligned_to(Q, 16) && aligned_to(K, 16) && aligned_to(V, 16) && aligned_to(O, 16) &&
-                  Skv * D * (int64_t)sizeof(T) < 0x7fffffff && scale_log2e > 0.0f;
+  const bool ok = matrix_core_operands(Q, K, V, O, Skv * D * (int64_t)sizeof(T), scale_log2e);
   const bool plain = !mask && Skv == S;
   if (ok && plain && D == 128) return launch_mfma<T, OutT, 128>(Q, K, V, O, ZH, S, scale_log2e, causal, st);
   if (ok && plain && D == 64) return launch_mfma<T, OutT, 64>(Q, K, V, O, ZH, S, scale_log2e, causal, st);
@@ -802,8 +807,19 @@ int dispatch_half(const void* Q, const void* K, const void* V, const void* mask,
 }
 
 int attention_any(const void* Q, const void* K, const void* V, const void* mask, void* O, int64_t ZH, int64_t S,
-                  int64_t Skv, int64_t D, float sm_scale, bool cz, int in_dtype, int out_dtype, hipStream_t st) {
+                  int64_t Skv, int64_t D, float sm_scale, bool cz, int in_dtype, int out_dtype, void* workspace,
+                  int64_t workspace_bytes, hipStream_t st) {
   const float c = sm_scale * 1.44269504088896340736f;
+  const bool half = (in_dtype == HEXMI_F16 || in_dtype == HEXMI_BF16) && (out_dtype == in_dtype || out_dtype == HEXMI_F32);
+  const bool mask_ok = mask == nullptr || ZH * S * Skv >= 8;            // flash_keys reads masks in pieces of eight
+  if (half && mask_ok && matrix_core_operands(Q, K, V, O, Skv * D * 2, c)) {
+    const FlashKeysPlan plan = plan_flash_keys(ZH, S, Skv, D, cz, mask != nullptr, workspace != nullptr);
+    if (plan.splits > 0) {
+      if (plan.splits > 1 && (workspace_bytes < flash_keys_workspace(plan, ZH, S, D) || !aligned_to(workspace, 16)))
+        return HEXMI_EINVAL;
+      return flash_keys(Q, K, V, mask, O, ZH, S, Skv, D, c, cz, in_dtype, out_dtype, plan, static_cast<float*>(workspace), st);
+    }
+  }
   if (in_dtype == HEXMI_F16 && out_dtype == HEXMI_F16) return dispatch_half<f16, f16>(Q, K, V, mask, O, ZH, S, Skv, D, c, cz, st);
   if (in_dtype == HEXMI_F16 && out_dtype == HEXMI_F32) return dispatch_half<f16, float>(Q, K, V, mask, O, ZH, S, Skv, D, c, cz, st);
   if (in_dtype == HEXMI_BF16 && out_dtype == HEXMI_BF16) return dispatch_half<bf16, bf16>(Q, K, V, mask, O, ZH, S, Skv, D, c, cz, st);
@@ -831,19 +847,35 @@ extern "C" int hexmi_flash_attn_fwd(const void* Q, const void* K, const void* V,
   if (!Q || !K || !V || !O) return HEXMI_EINVAL;
   if (S > 0x7fffffff / 2 || Z * H > 0x7fffffff) return HEXMI_ENOTSUP;
   begin_call();
-  return attention_any(Q, K, V, nullptr, O, Z * H, S, S, D, sm_scale, causal != 0, in_dtype, out_dtype,
+  return attention_any(Q, K, V, nullptr, O, Z * H, S, S, D, sm_scale, causal != 0, in_dtype, out_dtype, nullptr, 0,
                        as_stream(stream));
 }
 
 extern "C" int hexmi_attention(const void* Q, const void* K, const void* V, const void* mask, void* O, int64_t batch,
                                int64_t seq_q, int64_t seq_kv, int64_t head_dim, float sm_scale, int in_dtype,
                                int out_dtype, hexmi_stream_t stream) {
+  return hexmi_attention_ws(Q, K, V, mask, O, batch, seq_q, seq_kv, head_dim, sm_scale, in_dtype, out_dtype, nullptr, 0,
+                            stream);
+}
+
+extern "C" int64_t hexmi_attention_workspace(int64_t batch, int64_t seq_q, int64_t seq_kv, int64_t head_dim,
+                                             int has_mask, int in_dtype) {
+  if (batch <= 0 || seq_q <= 0 || seq_kv <= 0 || head_dim <= 0) return 0;
+  if (seq_q > 0x7fffffff / 2 || seq_kv > 0x7fffffff / 2 || batch > 0x7fffffff) return 0;
+  if (in_dtype != HEXMI_F16 && in_dtype != HEXMI_BF16) return 0;
+  return flash_keys_workspace(plan_flash_keys(batch, seq_q, seq_kv, head_dim, false, has_mask != 0, true), batch, seq_q,
+                              head_dim);
+}
+
+extern "C" int hexmi_attention_ws(const void* Q, const void* K, const void* V, const void* mask, void* O, int64_t batch,
+                                  int64_t seq_q, int64_t seq_kv, int64_t head_dim, float sm_scale, int in_dtype,
+                                  int out_dtype, void* workspace, int64_t workspace_bytes, hexmi_stream_t stream) {
   if (batch < 0 || seq_q < 0 || seq_kv < 0 || head_dim < 0) return HEXMI_EINVAL;
   if (batch == 0 || seq_q == 0 || head_dim == 0) return HEXMI_OK;
   if (seq_kv == 0) return HEXMI_EINVAL;                    // a softmax over no keys is undefined
   if (!Q || !K || !V || !O) return HEXMI_EINVAL;
   if (seq_q > 0x7fffffff / 2 || seq_kv > 0x7fffffff / 2 || batch > 0x7fffffff) return HEXMI_ENOTSUP;
   begin_call();
-  return attention_any(Q, K, V, mask, O, batch, seq_q, seq_kv, head_dim, sm_scale, false, in_dtype, out_dtype,
-                       as_stream(stream));
+  return attention_any(Q, K, V, mask, O, batch, seq_q, seq_kv, head_dim, sm_scale, false, in_dtype, out_dtype, workspace,
+                       workspace_bytes, as_stream(stream));
 }

@@ -338,6 +338,26 @@ int hexmi_attention(const void *Q, const void *K, const void *V,
                     int64_t seq_kv, int64_t head_dim, float sm_scale,
                     int in_dtype, int out_dtype, hexmi_stream_t stream);
 
+/* hexmi_attention with a caller-owned scratch buffer, for problems of too few
+ * queries to fill the chip (a decode step over a long context): the keys are
+ * then cut into chunks that workgroups of their own take, and their fp32 sums
+ * and (max, sum) pairs are merged by a second launch with the recurrence of the
+ * kernel itself (the reference merges its key blocks the same way,
+ * test/python/triton/test_flash_attention.py:61-87).
+ * hexmi_attention_workspace returns the bytes that takes for these sizes on the
+ * current device, 0 when the one-launch kernels run anyway (self-attention
+ * without a mask always does). workspace may be NULL (one
+ * launch whatever the sizes); one that is smaller than the query's answer or not
+ * 16-byte aligned is HEXMI_EINVAL. It needs no initialisation and holds no state
+ * between calls; two calls that overlap in time need a workspace each. */
+int64_t hexmi_attention_workspace(int64_t batch, int64_t seq_q, int64_t seq_kv,
+                                  int64_t head_dim, int has_mask, int in_dtype);
+int hexmi_attention_ws(const void *Q, const void *K, const void *V,
+                       const void *mask, void *O, int64_t batch, int64_t seq_q,
+                       int64_t seq_kv, int64_t head_dim, float sm_scale,
+                       int in_dtype, int out_dtype, void *workspace,
+                       int64_t workspace_bytes, hexmi_stream_t stream);
+
 /* Element-wise operators, sum reduction, rotary embedding ------------------ */
 
 /* y[i] = f(x[i]), fp32 arithmetic, result rounded to `dtype`.

@@ -476,3 +476,70 @@ def test_causal_attention_block_counts_off_the_power_of_two(hexmi, case):
     assert not torch.isnan(got).any()
     want = torch.nn.functional.scaled_dot_product_attention(q.float(), k.float(), v.float(), is_causal=True, scale=scale)
     assert (got - want).abs().max() <= 5e-3
+
+
+# units of 64 queries whose keys four groups of waves share (flash_attn_keys.hip): one step of 128 keys and its edges,
+# groups left without a tile, ragged row tiles; and few enough queries that the key range is cut over workgroups
+KEY_GROUP_CASES = [(1, 1, 65, 64), (2, 33, 96, 128), (3, 64, 97, 64), (1, 65, 127, 128), (8, 31, 128, 64), (2, 32, 129, 128),
+                   (2, 96, 160, 64), (1, 200, 257, 128), (16, 127, 385, 64), (8, 1, 4096, 128), (3, 2, 8191, 64), (24, 70, 1000, 128)]
+
+
+@pytest.mark.parametrize("with_mask", [True, False])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("case", KEY_GROUP_CASES)
+def test_attention_keys_shared_by_wave_groups(hexmi, case, dtype, with_mask):
+    # against the same sums in fp32; fp32 output, so what differs is the rounding of the probabilities to the 16-bit
+    # type (relative 2^-11 / 2^-8 each, averaged over V of unit variance): the bounds of the parity tests above
+    B, Sq, Skv, D = case
+    g = _gen(61)
+    q = torch.randn(B, Sq, D, generator=g).to(dtype)
+    k, v = torch.randn(B, Skv, D, generator=g).to(dtype), torch.randn(B, Skv, D, generator=g).to(dtype)
+    mask = _mask(B, Sq, Skv, dtype, 62) if with_mask else None
+    scores = q.float() @ k.float().transpose(1, 2) / math.sqrt(D)
+    if mask is not None:
+        scores = scores + mask.float()
+    want = torch.softmax(scores, dim=-1) @ v.float()
+    got = hexmi.attention(q.cuda(), k.cuda(), v.cuda(), None if mask is None else mask.cuda(), out_dtype=torch.float32).cpu()
+    assert (got - want).abs().max() <= (5e-3 if dtype == torch.float16 else 3e-2)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("case", [(1, 1, 65, 64), (1, 3, 127, 128), (2, 4, 128, 64), (1, 8, 129, 128), (1, 24, 300, 64),
+                                  (1, 16, 257, 128), (2, 12, 1000, 64), (1, 2, 2049, 128), (1, 1, 4100, 64)])
+def test_causal_attention_keys_shared_by_wave_groups(hexmi, case, dtype):
+    Z, H, S, D = case
+    q, k, v = _qkv(Z, H, S, D, dtype, seed=63)
+    scores = (q.float() @ k.float().transpose(2, 3) / math.sqrt(D)).masked_fill(torch.ones(S, S).triu(1).bool(), float("-inf"))
+    want = torch.softmax(scores, dim=-1) @ v.float()
+    got = hexmi.flash_attention(q.cuda(), k.cuda(), v.cuda(), None, True, out_dtype=torch.float32).cpu()
+    assert (got - want).abs().max() <= (5e-3 if dtype == torch.float16 else 3e-2)
+
+
+def test_attention_workspace(hexmi):
+    # the size asked for is enough and needed; without one the same problem runs in one launch, to the same rounding;
+    # rows with every key masked out stay NaN through the merge
+    from hexmi import _lib
+    lib = _lib.lib()
+    B, Sq, Skv, D = 4, 1, 4096, 128
+    g = _gen(64)
+    q, k, v = (torch.randn(B, n, D, generator=g).half().cuda() for n in (Sq, Skv, Skv))
+    mask = torch.zeros(B, Sq, Skv, dtype=torch.float16, device="cuda")
+    mask[:, :, :2000] = float("-inf")
+    mask[2] = float("-inf")
+    need = lib.hexmi_attention_workspace(B, Sq, Skv, D, 1, _lib.F16)
+    assert need > 0 and lib.hexmi_attention_workspace(4096, 2048, 2048, 128, 1, _lib.F16) == 0
+    assert lib.hexmi_attention_workspace(B, Sq, Skv, D, 1, _lib.F32) == 0
+    ws = torch.empty(need, dtype=torch.uint8, device="cuda")
+    outs = [torch.zeros(B, Sq, D, dtype=torch.float16, device="cuda") for _ in range(2)]
+
+    def call(out, workspace, size):
+        return lib.hexmi_attention_ws(q.data_ptr(), k.data_ptr(), v.data_ptr(), mask.data_ptr(), out.data_ptr(), B, Sq, Skv,
+                                      D, D ** -0.5, _lib.F16, _lib.F16, workspace, size, None)
+    torch.cuda.synchronize()
+    assert call(outs[0], ws.data_ptr(), need - 1) == _lib.EINVAL
+    assert call(outs[0], ws.data_ptr(), need) == _lib.OK
+    assert call(outs[1], None, 0) == _lib.OK
+    torch.cuda.synchronize()
+    assert torch.isnan(outs[0][2]).all() and torch.isnan(outs[1][2]).all()
+    keep = [0, 1, 3]
+    assert (outs[0][keep].float() - outs[1][keep].float()).abs().max() <= 1e-3
