@@ -94,6 +94,23 @@ def test_gemm_few_rows_against_transposed_weights(hexmi, oracle, dtype, M, N, K)
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("M,N,K", [
+    (9, 50257, 96), (16, 33001, 1120),              # 16 rows: 32 channels a workgroup
+    (17, 5121, 544), (32, 11001, 4128),             # 32 rows: 32 and 64 channels, the larger weights read non-temporally
+    (33, 5121, 2080), (64, 11007, 2048), (40, 8200, 32), (64, 77, 480)])     # 64 rows; fewer rounds of K than waves
+def test_gemm_few_rows_wide_workgroups(hexmi, dtype, M, N, K):
+    a, b = _inputs(M, N, K, dtype, True, seed=M + K)
+    want, mag = a.double() @ b.double().t(), a.double().abs() @ b.double().t().abs()
+    got = hexmi.matmul(a.cuda(), b.cuda(), out_dtype=torch.float32, trans_b=True).cpu()
+    # fp32 products summed in parts: K roundings of at most 2^-24 of the magnitude, far fewer in effect
+    assert ((got.double() - want).abs() <= 1e-5 * mag + 1e-30).all()
+    g = _gen(K)
+    bias, resid = torch.randn(N, generator=g).to(dtype), torch.randn(M, N, generator=g).to(dtype)
+    fused = hexmi.matmul(a.cuda(), b.cuda(), trans_b=True, bias=bias.cuda(), residual=resid.cuda()).cpu()
+    assert close16(fused, (want + bias.double() + resid.double()).to(dtype), max_ulp=1, atol=2e-5 * float(mag.max()))
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("M", [1, 2, 3, 4])
 @pytest.mark.parametrize("N,K", [(64, 8), (104, 64), (4096, 2048), (1000, 2056), (256, 4096), (136, 11008)])
 def test_gemm_few_rows_against_row_major_weights(hexmi, oracle, dtype, M, N, K):
