@@ -1479,6 +1479,13 @@ int launch_f32(bool trans_b, const void* A, const void* B, void* C, int64_t M, i
   return launch_status();
 }
 
+// 128 x 128 tiles: four LDS stages (128 KiB, one workgroup per CU) hide the copies of a tile's short slabs, two (64 KiB)
+// let two workgroups share a CU, one's first copies and last stores under the other's MFMAs and no round of its own for
+// what the first round leaves over. With a tile or less per CU four are ahead (us, four / two: 172 tiles of K = 4096
+// 37.6 / 53.4, 256 of 2048 20.3 / 26.4, 96 of 768 11.1 / 13.2), with more two (288 tiles of K = 768 with bias 19.8 / 14.7, 384
+// of 768 20.5 / 15.4, 344 of 4096 67.5 / 61.3, 480 of 3072 50.4 / 46.0, 1024 of 4096 132 / 126, 1536 of 768 65.5 / 47.7).
+inline bool two_per_cu(int64_t tiles) { return tiles > hexmi_num_cus(); }
+
 // out_elems: 16-bit results leave the paired-slab kernel one element per lane (the caller has checked that this
 // kernel takes the product: K % 64 == 0, short rows, no bias or residual).
 template <typename T, typename OutT, int WM, int WN, bool TRANS_B, int NWN = 2>
@@ -1489,28 +1496,25 @@ int launch_tiled(const T* A, const T* B, OutT* C, int64_t M, int64_t N, int64_t 
   // K % 64 == 0: the paired-slab kernel; its per-lane copy offsets (up to 256 rows, or 64 rows of K) must stay
   // below 2^31 bytes
   if (NWN == 2 && K % BK2 == 0 && lda < (1 << 21) && ldb < (1 << 21)) {
-    constexpr int NS = WM <= 2 ? 4 : 2;            // small tiles: four stages (their slabs are short)
+    const dim3 grid(tiles_m * tiles_n);
+#define HEXMI_K64(TAIL, NS, EPI)                                                                                        \
+  hipLaunchKernelGGL((gemm_kernel_k64<T, OutT, WM, WN, TRANS_B, TAIL, false, NS, EPI>), grid, dim3(256), 0, s, A, B, C, \
+                     (int)M, (int)N, (int)K, lda, ldb, ldc, tiles_m, tiles_n, nullptr, EPI ? bias : nullptr,             \
+                     EPI ? resid : nullptr, EPI ? ldr : 0, EPI ? 0 : out_elems)
+#define HEXMI_K64_TAIL(NS, EPI) \
+  do { if ((K / BK2) % NS == 0) HEXMI_K64(false, NS, EPI); else HEXMI_K64(true, NS, EPI); } while (0)
     if constexpr (WM == 2 && WN == 2) {
+      const bool two = two_per_cu((int64_t)tiles_m * tiles_n);
       if (bias || resid) {                          // the instantiations that carry the epilogue operands
-        if ((K / BK2) % NS == 0)
-          hipLaunchKernelGGL((gemm_kernel_k64<T, OutT, WM, WN, TRANS_B, false, false, NS, true>),
-                             dim3(tiles_m * tiles_n), dim3(256), 0, s, A, B, C, (int)M, (int)N, (int)K, lda, ldb, ldc,
-                             tiles_m, tiles_n, nullptr, bias, resid, ldr);
-        else
-          hipLaunchKernelGGL((gemm_kernel_k64<T, OutT, WM, WN, TRANS_B, true, false, NS, true>),
-                             dim3(tiles_m * tiles_n), dim3(256), 0, s, A, B, C, (int)M, (int)N, (int)K, lda, ldb, ldc,
-                             tiles_m, tiles_n, nullptr, bias, resid, ldr);
-        return launch_status();
+        if (two) HEXMI_K64_TAIL(2, true); else HEXMI_K64_TAIL(4, true);
+      } else {
+        if (two) HEXMI_K64_TAIL(2, false); else HEXMI_K64_TAIL(4, false);
       }
+    } else {
+      HEXMI_K64_TAIL((WM <= 2 ? 4 : 2), false);
     }
-    if ((K / BK2) % NS == 0)
-      hipLaunchKernelGGL((gemm_kernel_k64<T, OutT, WM, WN, TRANS_B, false, false, NS>), dim3(tiles_m * tiles_n),
-                         dim3(256), 0, s, A, B, C, (int)M, (int)N, (int)K, lda, ldb, ldc, tiles_m, tiles_n, nullptr,
-                         nullptr, nullptr, 0, out_elems);
-    else
-      hipLaunchKernelGGL((gemm_kernel_k64<T, OutT, WM, WN, TRANS_B, true, false, NS>), dim3(tiles_m * tiles_n),
-                         dim3(256), 0, s, A, B, C, (int)M, (int)N, (int)K, lda, ldb, ldc, tiles_m, tiles_n, nullptr,
-                         nullptr, nullptr, 0, out_elems);
+#undef HEXMI_K64_TAIL
+#undef HEXMI_K64
     return launch_status();
   }
   if (out_elems) return HEXMI_ENOTSUP;             // only the paired-slab kernel has that epilogue
@@ -1531,9 +1535,9 @@ int launch_tiled(const T* A, const T* B, OutT* C, int64_t M, int64_t N, int64_t 
   return launch_status();
 }
 
-// 256 x 256 or 128 x 128 tiles. Either kind runs one workgroup per CU at a time, so a launch is whole rounds over
-// the CUs and the last round may be nearly empty. With every round full the large tiles run about 1.3 times the
-// rate of the small ones (fp16 K = 4096: 1.4 against 1.08 PFLOP/s; int8 weights: 1.2 against 0.93), and a round
+// 256 x 256 or 128 x 128 tiles. A launch is whole rounds over the CUs and the last round may be nearly empty. With every
+// round full the large tiles run about 1.2 to 1.3 times the rate of the small ones, two of which share a CU there
+// (fp16 K = 4096: 1.34 against 1.09 PFLOP/s; three rounds at K = 1024: 1.10 against 0.94), and a round
 // that is not full runs its tiles somewhat faster: the large tiles are taken when 1.48 times the fill of their
 // rounds is at least the fill of the small tiles' rounds. (fp16, K = 4096, 256 CUs: 128 large tiles 825 TFLOP/s
 // against 1074 with small ones, 289 tiles 920 against 1019, 192 tiles 1152 against 1077, 324 tiles 1020 against 965;
@@ -1642,15 +1646,17 @@ int launch_w8a16(const f16* A, const int8_t* W, const f16* scales, f16* C, int64
   constexpr int BM = 2 * WM * 32, BN = 2 * WN * 32;
   const int tiles_m = (int)((M + BM - 1) / BM), tiles_n = (int)((N + BN - 1) / BN);
   if (K % BK2 == 0 && K < (1 << 21)) {
-    constexpr int NS = WM <= 2 ? 4 : 2;
-    if ((K / BK2) % NS == 0)
-      hipLaunchKernelGGL((gemm_kernel_k64<f16, f16, WM, WN, true, false, true, NS>), dim3(tiles_m * tiles_n),
-                         dim3(256), 0, s, A, static_cast<const void*>(W), C, (int)M, (int)N, (int)K, K, K, N, tiles_m,
-                         tiles_n, scales);
-    else
-      hipLaunchKernelGGL((gemm_kernel_k64<f16, f16, WM, WN, true, true, true, NS>), dim3(tiles_m * tiles_n),
-                         dim3(256), 0, s, A, static_cast<const void*>(W), C, (int)M, (int)N, (int)K, K, K, N, tiles_m,
-                         tiles_n, scales);
+#define HEXMI_K64(TAIL, NS)                                                                                          \
+  hipLaunchKernelGGL((gemm_kernel_k64<f16, f16, WM, WN, true, TAIL, true, NS>), dim3(tiles_m * tiles_n), dim3(256), 0, s, A, \
+                     static_cast<const void*>(W), C, (int)M, (int)N, (int)K, K, K, N, tiles_m, tiles_n, scales)
+#define HEXMI_K64_TAIL(NS) do { if ((K / BK2) % NS == 0) HEXMI_K64(false, NS); else HEXMI_K64(true, NS); } while (0)
+    if constexpr (WM <= 2) {
+      if (two_per_cu((int64_t)tiles_m * tiles_n)) HEXMI_K64_TAIL(2); else HEXMI_K64_TAIL(4);
+    } else {
+      HEXMI_K64_TAIL(2);
+    }
+#undef HEXMI_K64_TAIL
+#undef HEXMI_K64
     return launch_status();
   }
   if ((K / BK) % 4 == 0)

@@ -130,6 +130,27 @@ def test_gemm_few_rows_against_row_major_weights(hexmi, oracle, dtype, M, N, K):
     assert close16(fused, ref, max_ulp=1, atol=2e-5 * float(mag.max()))
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("trans_b", [False, True])
+@pytest.mark.parametrize("K", [64, 128, 192, 448])
+def test_gemm_two_small_tiles_per_cu(hexmi, dtype, trans_b, K):
+    # 16 x 17 tiles of 128 x 128, more than there are CUs: one slab, whole and guarded last passes; rows of the output on
+    # and (B as [N,K]) off the boundaries; the epilogue operands; fp32 results
+    M = 2040
+    for N in ((2104, 2101) if trans_b else (2104,)):
+        a, b = _inputs(M, N, K, dtype, trans_b, seed=K + N)
+        ad, bd = a.cuda(), b.cuda()
+        bt = b.double().t() if trans_b else b.double()
+        want, mag = a.double() @ bt, float((a.double().abs() @ bt.abs()).max())
+        got32 = hexmi.matmul(ad, bd, out_dtype=torch.float32, trans_b=trans_b).cpu()
+        assert ((got32.double() - want).abs().max()) <= 1e-5 * mag
+        assert close16(hexmi.matmul(ad, bd, trans_b=trans_b).cpu(), want.to(dtype), max_ulp=1, atol=1e-5 * mag)
+        g = _gen(K)
+        bias, resid = torch.randn(N, generator=g).to(dtype), torch.randn(M, N, generator=g).to(dtype)
+        fused = hexmi.matmul(ad, bd, trans_b=trans_b, bias=bias.cuda(), residual=resid.cuda()).cpu()
+        assert close16(fused, (want + bias.double() + resid.double()).to(dtype), max_ulp=1, atol=2e-5 * mag)
+
+
 def test_gemm_closed_forms(hexmi):
     g = _gen(1)
     a = torch.randn(256, 128, generator=g).half()
