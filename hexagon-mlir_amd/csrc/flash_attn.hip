@@ -811,6 +811,8 @@ int attention_any(const void* Q, const void* K, const void* V, const void* mask,
                   int64_t workspace_bytes, hipStream_t st) {
   const float c = sm_scale * 1.44269504088896340736f;
   const bool half = (in_dtype == HEXMI_F16 || in_dtype == HEXMI_BF16) && (out_dtype == in_dtype || out_dtype == HEXMI_F32);
+  if (half && flash_decode_takes(ZH, S, Skv, D) && matrix_core_operands(Q, K, V, O, Skv * D * 2, c))
+    return flash_decode(Q, K, V, mask, O, ZH, Skv, D, c, in_dtype, out_dtype, st);
   const bool mask_ok = mask == nullptr || ZH * S * Skv >= 8;            // flash_keys reads masks in pieces of eight
   if (half && mask_ok && matrix_core_operands(Q, K, V, O, Skv * D * 2, c)) {
     const FlashKeysPlan plan = plan_flash_keys(ZH, S, Skv, D, cz, mask != nullptr, workspace != nullptr);

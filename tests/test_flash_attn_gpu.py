@@ -515,6 +515,42 @@ def test_causal_attention_keys_shared_by_wave_groups(hexmi, case, dtype):
     assert (got - want).abs().max() <= (5e-3 if dtype == torch.float16 else 3e-2)
 
 
+# one query of each of many heads (flash_decode.hip): the shortest key range, tiles of 32 (heads of 128) and 64 keys and
+# their edges, waves left without a tile, a second tile of some waves
+DECODE_CASES = [(130, 65, 64), (129, 66, 128), (131, 95, 128), (130, 128, 64), (129, 255, 128), (300, 257, 128),
+                (130, 511, 64), (129, 2051, 128), (513, 577, 64)]
+
+
+@pytest.mark.parametrize("with_mask", [True, False])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("case", DECODE_CASES)
+def test_attention_one_query_of_many_heads(hexmi, case, dtype, with_mask):
+    # everything is summed in fp32 and the output is fp32: a score is off by about D * 2^-24 * |score| < 5e-5, so is a
+    # probability by that share, and the result by no more of |V| < 6 (the errors average): 1e-4. Mask rows start one
+    # element off the allocation; a head with every key masked out gives NaN
+    B, Skv, D = case
+    g = _gen(65)
+    q = torch.randn(B, 1, D, generator=g).to(dtype)
+    k, v = torch.randn(B, Skv, D, generator=g).to(dtype), torch.randn(B, Skv, D, generator=g).to(dtype)
+    scores = (q.float() @ k.float().transpose(1, 2)) / math.sqrt(D)
+    shifted = None
+    if with_mask:
+        mask = _mask(B, 1, Skv, dtype, 66)
+        mask[1, :, :Skv - 1] = float("-inf")
+        mask[1, :, Skv - 1] = 0.0
+        mask[2, :, Skv // 2:] = float("-inf")
+        mask[B - 1] = float("-inf")
+        scores = scores + mask.float()
+        shifted = torch.empty(mask.numel() + 1, dtype=dtype, device="cuda")[1:].view(B, 1, Skv)
+        shifted.copy_(mask)
+    want = torch.softmax(scores, dim=-1) @ v.float()
+    got = hexmi.attention(q.cuda(), k.cuda(), v.cuda(), shifted, out_dtype=torch.float32).cpu()
+    if with_mask:
+        assert torch.isnan(got[B - 1]).all()
+        got, want = got[:B - 1], want[:B - 1]
+    assert (got - want).abs().max() <= 1e-4
+
+
 def test_attention_workspace(hexmi):
     # the size asked for is enough and needed; without one the same problem runs in one launch, to the same rounding;
     # rows with every key masked out stay NaN through the merge
