@@ -60,7 +60,7 @@ struct MaskTileLoader {
 };
 
 // GENERAL: the number of keys (Skv) may differ from the number of queries (S) and an additive mask
-// [ZH, S, Skv] (same dtype as Q; may be null) is added to the scaled scores before the softmax, as
+// [ZH, S, Skv] (MASKED, same dtype as Q) is added to the scaled scores before the softmax, as
 // tm_tensor.attention does (qcom_hexagon_backend/lib/Transforms/LowerTmTensor.cpp:157-160).
 // NW waves per workgroup (4 or 8), 32 query rows each: every K / V tile copied into LDS serves NW*32 query rows.
 // Eight waves halve the L2 -> LDS copy traffic (each query block streams the whole K and V of its head), worth
@@ -76,16 +76,22 @@ struct MaskTileLoader {
 // scores are the sum over both halves' K tiles, the output two sets of accumulators, the second half's tiles padded
 // like a narrow head's; twice the LDS and about 100 registers more, so one workgroup per CU.
 template <typename T, typename OutT, int D, bool CAUSAL, bool GENERAL = false, int NW = 4, bool MASK_LDS = false,
-          bool PADDED = false, bool WIDE = false>
+          bool PADDED = false, bool WIDE = false, bool MASKED = false>
 __global__ __launch_bounds__(NW * 64, NW == 4 && !WIDE ? (D == 64 && !GENERAL ? 3 : 2) : 1)
 void flash_fwd_kernel(const T* __restrict__ Q, const T* __restrict__ K, const T* __restrict__ V,
                       OutT* __restrict__ O, int ZH, int S, float scale_log2e, const T* __restrict__ Mk = nullptr,
-                      int Skv_arg = 0, float mask_factor = 0.0f, int group_heads = 0, int head_dim = D) {
+                      int Skv_arg = 0, float sm_scale = 0.0f, int group_heads = 0, int head_dim = D) {
   static_assert(!(CAUSAL && GENERAL), "the causal kernel has as many keys as queries and no mask");
   static_assert(!WIDE || (PADDED && D == 128 && NW == 4 && !GENERAL), "two halves of 128 columns, four waves, no mask");
   const int dh = PADDED ? head_dim : D;                 // elements between rows in memory
-  static_assert(!MASK_LDS || (GENERAL && NW == 8), "staged mask tiles: general kernel, 8 waves");
+  static_assert(!MASKED || GENERAL, "masks: general kernel");
+  static_assert(!MASK_LDS || (MASKED && NW == 8), "staged mask tiles: 8 waves");
   const int Skv = GENERAL ? Skv_arg : S;
+  // With a mask, scores and maxima are in natural units (sm_scale * q k + mask) and a difference to the maximum is taken
+  // before it is multiplied by log2 e, so that rows whose keys all carry one large finite value come out right (see
+  // kUnit in flash_attn_keys.hip; one instruction more per score, 1 to 3 %); without one, a raw score is scaled into log2
+  // units as its exponent is taken.
+  constexpr float kUnit = MASKED ? kLog2e : 1.0f, kLag = kRescaleLag / kUnit;
   typedef typename MfmaT<T>::Frag Frag;
   constexpr int DS = D / 16;                        // 16-wide steps over the head dimension
   constexpr int DT = D / 32;                        // 32-wide output tiles over the head dimension
@@ -263,11 +269,11 @@ void flash_fwd_kernel(const T* __restrict__ Q, const T* __restrict__ K, const T*
       for (int r = 0; r < 16; ++r) mx1 = fmaxf(mx1, s[1][r]);
       mx = fmaxf(mx, mx1);
       mx = fmaxf(mx, other_half(mx));
-      const float m_blk = mx * scale_log2e;
-      const bool grow = m_blk > m_i + kRescaleLag;
+      const float m_blk = MASKED ? mx : mx * scale_log2e;
+      const bool grow = m_blk > m_i + kLag;
       if (__builtin_amdgcn_ballot_w64(grow) != 0) {
         const float m_new = grow ? m_blk : m_i;
-        const float alpha = grow ? __builtin_amdgcn_exp2f(m_i - m_new) : 1.0f;
+        const float alpha = grow ? __builtin_amdgcn_exp2f((m_i - m_new) * kUnit) : 1.0f;
         l_i *= alpha;
         m_i = m_new;
 #pragma unroll
@@ -287,7 +293,7 @@ void flash_fwd_kernel(const T* __restrict__ Q, const T* __restrict__ K, const T*
     auto exp_tile = [&](const f32x16& s, Frag* pf) __attribute__((always_inline)) {
       float p[16];
 #pragma unroll
-      for (int r = 0; r < 16; ++r) p[r] = __builtin_amdgcn_exp2f(fmaf(s[r], scale_log2e, neg_m));
+      for (int r = 0; r < 16; ++r) p[r] = __builtin_amdgcn_exp2f(MASKED ? (s[r] + neg_m) * kUnit : fmaf(s[r], scale_log2e, neg_m));
       pf[0] = MfmaT<T>::pack(&p[0]);
       pf[1] = MfmaT<T>::pack(&p[8]);
       // the running sum takes the probabilities as rounded for the matrix cores (what P V actually multiplies),
@@ -331,11 +337,9 @@ void flash_fwd_kernel(const T* __restrict__ Q, const T* __restrict__ K, const T*
         for (int dt = 0; dt < (WIDE ? DT : 1); ++dt) o_accb[dt] = MfmaT<T>::run(vf.f[hf][dt], pf[hf], o_accb[dt]);
     };
 
-    // mask row of this lane's query (GENERAL with a mask only)
+    // mask row of this lane's query
     const T* mask_row = nullptr;
-    if constexpr (GENERAL && !MASK_LDS) {
-      if (Mk) mask_row = Mk + ((int64_t)zh * S + (qrow < S ? qrow : S - 1)) * Skv;
-    }
+    if constexpr (MASKED && !MASK_LDS) mask_row = Mk + ((int64_t)zh * S + (qrow < S ? qrow : S - 1)) * Skv;
 
     // One key block. The global -> LDS copies of the next block (next >= 0, into the other stage) are issued a
     // few at a time between the score MFMAs: issued in one burst after the barrier, the 32 KiB of a block keep the
@@ -353,23 +357,21 @@ void flash_fwd_kernel(const T* __restrict__ Q, const T* __restrict__ K, const T*
       // needs the alignment of an element (one 8-byte load either way), so mask rows of any length are read here.
       typedef T MaskRun __attribute__((ext_vector_type(4)));
       MaskRun mk[2][4];
-      if constexpr (GENERAL && !MASK_LDS) {
-        if (mask_row) {
-          if (n0 + kBlockN <= Skv) {
+      if constexpr (MASKED && !MASK_LDS) {
+        if (n0 + kBlockN <= Skv) {
 #pragma unroll
-            for (int jt = 0; jt < 2; ++jt)
+          for (int jt = 0; jt < 2; ++jt)
 #pragma unroll
-              for (int g4 = 0; g4 < 4; ++g4)
-                __builtin_memcpy(&mk[jt][g4], mask_row + n0 + jt * 32 + 8 * g4 + 4 * half, sizeof(MaskRun));
-          } else {                                           // the row ends in this block: by elements, none past it
+            for (int g4 = 0; g4 < 4; ++g4)
+              __builtin_memcpy(&mk[jt][g4], mask_row + n0 + jt * 32 + 8 * g4 + 4 * half, sizeof(MaskRun));
+        } else {                                             // the row ends in this block: by elements, none past it
 #pragma unroll
-            for (int jt = 0; jt < 2; ++jt)
+          for (int jt = 0; jt < 2; ++jt)
 #pragma unroll
-              for (int e = 0; e < 16; ++e) {
-                const int key = n0 + jt * 32 + 8 * (e / 4) + 4 * half + e % 4;
-                mk[jt][e / 4][e % 4] = mask_row[key < Skv ? key : Skv - 1];
-              }
-          }
+            for (int e = 0; e < 16; ++e) {
+              const int key = n0 + jt * 32 + 8 * (e / 4) + 4 * half + e % 4;
+              mk[jt][e / 4][e % 4] = mask_row[key < Skv ? key : Skv - 1];
+            }
         }
       }
       // ---- scores: s[jt][r] = Q[qrow] . K[n0 + jt*32 + 8*(r/4) + 4*half + r%4]. The MFMA chains of the two 32-key
@@ -447,14 +449,11 @@ void flash_fwd_kernel(const T* __restrict__ Q, const T* __restrict__ K, const T*
           for (int g4 = 0; g4 < 4; ++g4)
             mk[jt][g4] = *reinterpret_cast<const MaskRun*>(m_row + ((jt * 4 + g4) ^ ((row >> 1) & 7)) * 8);
       }
-      if constexpr (GENERAL) {
-        if (MASK_LDS || mask_row) {
-          // softmax(scale*s + mask) = softmax(scale * (s + mask/scale)): fold the mask into the raw scores
+      if constexpr (MASKED) {
 #pragma unroll
-          for (int jt = 0; jt < 2; ++jt)
+        for (int jt = 0; jt < 2; ++jt)
 #pragma unroll
-            for (int r = 0; r < 16; ++r) s[jt][r] = fmaf(to_f32<T>(mk[jt][r / 4][r % 4]), mask_factor, s[jt][r]);
-        }
+          for (int r = 0; r < 16; ++r) s[jt][r] = fmaf(s[jt][r], sm_scale, to_f32<T>(mk[jt][r / 4][r % 4]));
       }
       const bool need_mask = (CAUSAL && n0 + kBlockN - 1 > q0) || (n0 + kBlockN > Skv);
       block_max(n0, need_mask, s);
@@ -708,40 +707,26 @@ int launch_mfma(const void* Q, const void* K, const void* V, void* O, int64_t ZH
 template <typename T, typename OutT, int D>
 int launch_mfma_general(const void* Q, const void* K, const void* V, const void* mask, void* O, int64_t ZH, int64_t S,
                         int64_t Skv, float scale_log2e, hipStream_t st, int head_dim = D) {
-  const float mask_factor = 1.44269504088896340736f / scale_log2e;     // mask / sm_scale
-  if (head_dim < D) {
-    const int64_t units = (S + 127) / 128 * ZH;
-    if (units > 0x7fffffff) return HEXMI_ENOTSUP;
-    const int64_t blocks = resident_grid(units, 2);
-    if (blocks <= 0) return HEXMI_ELAUNCH;
-    hipLaunchKernelGGL((flash_fwd_kernel<T, OutT, D, false, true, 4, false, true>), dim3((unsigned)blocks), dim3(256), 0, st,
-                       static_cast<const T*>(Q), static_cast<const T*>(K), static_cast<const T*>(V),
-                       static_cast<OutT*>(O), (int)ZH, (int)S, scale_log2e, static_cast<const T*>(mask), (int)Skv,
-                       mask_factor, 0, head_dim);
-    return launch_status();
-  }
   // a mask whose rows are whole 16-byte chunks is staged through LDS by 256-row workgroups (one per CU); the
   // copies address a workgroup's 256 mask rows with 32-bit byte offsets
-  if (mask != nullptr && Skv % 8 == 0 && aligned_to(mask, 16) && S > 128 && Skv <= (1 << 21)) {
-    const int64_t units8 = (S + 255) / 256 * ZH;
-    if (units8 > 0x7fffffff) return HEXMI_ENOTSUP;
-    const int64_t blocks8 = resident_grid(units8, 1);
-    if (blocks8 <= 0) return HEXMI_ELAUNCH;
-    hipLaunchKernelGGL((flash_fwd_kernel<T, OutT, D, false, true, 8, true>), dim3((unsigned)blocks8), dim3(512), 0,
-                       st, static_cast<const T*>(Q), static_cast<const T*>(K), static_cast<const T*>(V),
-                       static_cast<OutT*>(O), (int)ZH, (int)S, scale_log2e, static_cast<const T*>(mask), (int)Skv,
-                       mask_factor);
-    return launch_status();
-  }
-  const int64_t nqb = (S + 127) / 128;
-  const int64_t units = nqb * ZH;
+  const bool staged = mask != nullptr && head_dim == D && Skv % 8 == 0 && aligned_to(mask, 16) && S > 128 && Skv <= (1 << 21);
+  const int rows = staged ? 256 : 128;
+  const int64_t units = (S + rows - 1) / rows * ZH;
   if (units > 0x7fffffff) return HEXMI_ENOTSUP;
-  const int64_t blocks = resident_grid(units, 2);
+  const int64_t blocks = resident_grid(units, staged ? 1 : 2);
   if (blocks <= 0) return HEXMI_ELAUNCH;
-  hipLaunchKernelGGL((flash_fwd_kernel<T, OutT, D, false, true>), dim3((unsigned)blocks), dim3(256), 0, st,
-                     static_cast<const T*>(Q), static_cast<const T*>(K), static_cast<const T*>(V),
-                     static_cast<OutT*>(O), (int)ZH, (int)S, scale_log2e, static_cast<const T*>(mask), (int)Skv,
-                     mask_factor);
+  const float sm_scale = scale_log2e / kLog2e;
+#define HEXMI_GENERAL(NW, LDS, PAD, MASK)                                                                                 \
+  hipLaunchKernelGGL((flash_fwd_kernel<T, OutT, D, false, true, NW, LDS, PAD, false, MASK>), dim3((unsigned)blocks),       \
+                     dim3(NW * 64), 0, st, static_cast<const T*>(Q), static_cast<const T*>(K), static_cast<const T*>(V),  \
+                     static_cast<OutT*>(O), (int)ZH, (int)S, scale_log2e, static_cast<const T*>(mask), (int)Skv, sm_scale, \
+                     0, head_dim)
+  if (staged) HEXMI_GENERAL(8, true, false, true);
+  else if (head_dim < D && mask != nullptr) HEXMI_GENERAL(4, false, true, true);
+  else if (head_dim < D) HEXMI_GENERAL(4, false, true, false);
+  else if (mask != nullptr) HEXMI_GENERAL(4, false, false, true);
+  else HEXMI_GENERAL(4, false, false, false);
+#undef HEXMI_GENERAL
   return launch_status();
 }
 
@@ -809,17 +794,17 @@ int dispatch_half(const void* Q, const void* K, const void* V, const void* mask,
 int attention_any(const void* Q, const void* K, const void* V, const void* mask, void* O, int64_t ZH, int64_t S,
                   int64_t Skv, int64_t D, float sm_scale, bool cz, int in_dtype, int out_dtype, void* workspace,
                   int64_t workspace_bytes, hipStream_t st) {
-  const float c = sm_scale * 1.44269504088896340736f;
+  const float c = sm_scale * kLog2e;
   const bool half = (in_dtype == HEXMI_F16 || in_dtype == HEXMI_BF16) && (out_dtype == in_dtype || out_dtype == HEXMI_F32);
   if (half && flash_decode_takes(ZH, S, Skv, D) && matrix_core_operands(Q, K, V, O, Skv * D * 2, c))
-    return flash_decode(Q, K, V, mask, O, ZH, Skv, D, c, in_dtype, out_dtype, st);
+    return flash_decode(Q, K, V, mask, O, ZH, Skv, D, sm_scale, in_dtype, out_dtype, st);
   const bool mask_ok = mask == nullptr || ZH * S * Skv >= 8;            // flash_keys reads masks in pieces of eight
   if (half && mask_ok && matrix_core_operands(Q, K, V, O, Skv * D * 2, c)) {
     const FlashKeysPlan plan = plan_flash_keys(ZH, S, Skv, D, cz, mask != nullptr, workspace != nullptr);
     if (plan.splits > 0) {
       if (plan.splits > 1 && (workspace_bytes < flash_keys_workspace(plan, ZH, S, D) || !aligned_to(workspace, 16)))
         return HEXMI_EINVAL;
-      return flash_keys(Q, K, V, mask, O, ZH, S, Skv, D, c, cz, in_dtype, out_dtype, plan, static_cast<float*>(workspace), st);
+      return flash_keys(Q, K, V, mask, O, ZH, S, Skv, D, sm_scale, cz, in_dtype, out_dtype, plan, static_cast<float*>(workspace), st);
     }
   }
   if (in_dtype == HEXMI_F16 && out_dtype == HEXMI_F16) return dispatch_half<f16, f16>(Q, K, V, mask, O, ZH, S, Skv, D, c, cz, st);

@@ -60,10 +60,16 @@ struct GroupTileLoader {
 template <typename T, typename OutT, int D, bool CAUSAL, bool MASKED, bool PADDED>
 __global__ __launch_bounds__(512, D == 64 && !MASKED ? 4 : 2)
 void flash_keys_kernel(const T* __restrict__ Q, const T* __restrict__ K, const T* __restrict__ V, OutT* __restrict__ O,
-                       int ZH, int S, int Skv, float scale_log2e, const T* __restrict__ Mk, float mask_factor,
-                       float* __restrict__ part, int chunk, int splits, int head_dim) {
+                       int ZH, int S, int Skv, float scale, const T* __restrict__ Mk, float* __restrict__ part,
+                       int chunk, int splits, int head_dim) {
   const int dh = PADDED ? head_dim : D;                 // elements between rows in memory
   static_assert(!(CAUSAL && MASKED), "the causal kernel has no mask");
+  // Without a mask `scale` carries log2 e and a score is scaled as its exponent is taken: one instruction. With one the
+  // score is scaled and the mask added to it in natural units, and the difference to the maximum is taken before it
+  // is multiplied by log2 e. That way a row whose keys all carry the same large finite value gives the average of V as any
+  // other constant does: the value divided by the scale and added to the raw score overflowed from -3e37 on (bf16, heads
+  // of 128), and a maximum that was multiplied and rounded was off by more than an exponent holds from about -2e9 on.
+  constexpr float kUnit = MASKED ? kLog2e : 1.0f, kLag = kRescaleLag / kUnit;
   typedef typename MfmaT<T>::Frag Frag;
   constexpr int DS = D / 16, DT = D / 32, CPR = D / 8;
   constexpr int kTile = kTileKeys * D;
@@ -244,7 +250,7 @@ void flash_keys_kernel(const T* __restrict__ Q, const T* __restrict__ K, const T
       for (int g4 = 0; g4 < 4; ++g4)
         mk[g4] = *reinterpret_cast<const MaskRun*>(m_wave + (row * 4 + (g4 ^ (row / 4 % 4))) * 8 + half * 4);
 #pragma unroll
-      for (int r = 0; r < 16; ++r) s[r] = fmaf(to_f32<T>(mk[r / 4][r % 4]), mask_factor, s[r]);
+      for (int r = 0; r < 16; ++r) s[r] = fmaf(s[r], scale, to_f32<T>(mk[r / 4][r % 4]));
     }
     if ((CAUSAL && n0 + kTileKeys - 1 > q0) || n0 + kTileKeys > Skv) {
 #pragma unroll
@@ -257,11 +263,11 @@ void flash_keys_kernel(const T* __restrict__ Q, const T* __restrict__ K, const T
 #pragma unroll
     for (int r = 0; r < 16; ++r) mx = fmaxf(mx, s[r]);
     mx = fmaxf(mx, other_half(mx));
-    const float m_blk = mx * scale_log2e;
-    const bool grow = m_blk > m_i + kRescaleLag;
+    const float m_blk = MASKED ? mx : mx * scale;
+    const bool grow = m_blk > m_i + kLag;
     if (__builtin_amdgcn_ballot_w64(grow) != 0) {
       const float m_new = grow ? m_blk : m_i;
-      const float alpha = grow ? __builtin_amdgcn_exp2f(m_i - m_new) : 1.0f;
+      const float alpha = grow ? __builtin_amdgcn_exp2f((m_i - m_new) * kUnit) : 1.0f;
       l_i *= alpha;
       m_i = m_new;
 #pragma unroll
@@ -272,7 +278,7 @@ void flash_keys_kernel(const T* __restrict__ Q, const T* __restrict__ K, const T
     }
     float p[16];
 #pragma unroll
-    for (int r = 0; r < 16; ++r) p[r] = __builtin_amdgcn_exp2f(fmaf(s[r], scale_log2e, neg_m));
+    for (int r = 0; r < 16; ++r) p[r] = __builtin_amdgcn_exp2f(MASKED ? (s[r] + neg_m) * kUnit : fmaf(s[r], scale, neg_m));
     const Frag pf[2] = {MfmaT<T>::pack(&p[0]), MfmaT<T>::pack(&p[8])};
     l_i = MfmaT<T>::sum8(pf[1], MfmaT<T>::sum8(pf[0], l_i));
 #pragma unroll
@@ -317,10 +323,10 @@ void flash_keys_kernel(const T* __restrict__ Q, const T* __restrict__ K, const T
 #pragma unroll
   for (int g = 0; g < kGroups; ++g) {
     const f32x2 v = *ml_of(g);
-    l = fmaf(v[1], __builtin_amdgcn_exp2f(v[0] + base), l);
+    l = fmaf(v[1], __builtin_amdgcn_exp2f((v[0] + base) * kUnit), l);
   }
   l += other_half(l);
-  const float w = __builtin_amdgcn_exp2f(m_i + base);
+  const float w = __builtin_amdgcn_exp2f((m_i + base) * kUnit);
   f32x4* pieces[kGroups] = {reinterpret_cast<f32x4*>(k_lds0), reinterpret_cast<f32x4*>(k_lds1),
                             reinterpret_cast<f32x4*>(v_lds0), reinterpret_cast<f32x4*>(v_lds1)};
 #pragma unroll
@@ -366,13 +372,14 @@ void flash_keys_kernel(const T* __restrict__ Q, const T* __restrict__ K, const T
     *reinterpret_cast<f32x2*>(part + (int64_t)splits * rows * D + ((int64_t)split * rows + row) * 2) = f32x2{m, l};
 }
 
-// The chunks of a row added up: O = sum_s 2^(m_s - m) o_s / sum_s 2^(m_s - m) l_s with m the largest m_s. A thread
+// The chunks of a row added up: O = sum_s 2^(u (m_s - m)) o_s / sum_s 2^(u (m_s - m)) l_s with m the largest m_s and u the
+// log2 units of an m_s (kUnit of the kernel that wrote them). A thread
 // takes four columns; rows of units that were one chunk are already in O. Bound by reading the sums, which have just
 // been written and come from L2 / Infinity Cache.
 template <typename OutT, int D, bool CAUSAL>
 __global__ __launch_bounds__(256)
 void flash_merge_kernel(const float* __restrict__ part, OutT* __restrict__ O, int64_t rows, int S, int chunk, int splits,
-                        int head_dim) {
+                        int head_dim, float unit) {
   constexpr int TPR = D / 4;                               // threads per row
   const int64_t row = (int64_t)blockIdx.x * (256 / TPR) + threadIdx.x / TPR;
   if (row >= rows) return;
@@ -394,7 +401,7 @@ void flash_merge_kernel(const float* __restrict__ part, OutT* __restrict__ O, in
   for (int s = 0; s < n; ++s) {
     const f32x2 v = *reinterpret_cast<const f32x2*>(ml + ((int64_t)s * rows + row) * 2);
     const f32x4 x = *reinterpret_cast<const f32x4*>(part + ((int64_t)s * rows + row) * D + d);
-    const float w = __builtin_amdgcn_exp2f(v[0] + base);
+    const float w = __builtin_amdgcn_exp2f((v[0] + base) * unit);
     l = fmaf(v[1], w, l);
 #pragma unroll
     for (int e = 0; e < 4; ++e) o[e] = fmaf(x[e], w, o[e]);
@@ -405,16 +412,16 @@ void flash_merge_kernel(const float* __restrict__ part, OutT* __restrict__ O, in
 
 template <typename T, typename OutT, int D>
 int launch_keys(const void* Q, const void* K, const void* V, const void* mask, void* O, int64_t ZH, int64_t S,
-                int64_t Skv, int head_dim, float scale_log2e, bool causal, const FlashKeysPlan& plan, float* part, hipStream_t st) {
+                int64_t Skv, int head_dim, float sm_scale, bool causal, const FlashKeysPlan& plan, float* part, hipStream_t st) {
   const int64_t blocks = (S + kRows - 1) / kRows * ZH * plan.splits, rows = ZH * S;
   const int64_t merge_blocks = (rows + 1024 / D - 1) / (1024 / D);
   if (blocks > 0x7fffffff || merge_blocks > 0x7fffffff) return HEXMI_ENOTSUP;
-  const float mask_factor = 1.44269504088896340736f / scale_log2e;     // mask / sm_scale
+  const float unit = mask != nullptr ? kLog2e : 1.0f, scale = mask != nullptr ? sm_scale : sm_scale * kLog2e;
 #define HEXMI_KEYS(C, M, P)                                                                                           \
   hipLaunchKernelGGL((flash_keys_kernel<T, OutT, D, C, M, P>), dim3((unsigned)blocks), dim3(512), 0, st,              \
                      static_cast<const T*>(Q), static_cast<const T*>(K), static_cast<const T*>(V),                    \
-                     static_cast<OutT*>(O), (int)ZH, (int)S, (int)Skv, scale_log2e, static_cast<const T*>(mask),      \
-                     mask_factor, part, plan.chunk, plan.splits, head_dim)
+                     static_cast<OutT*>(O), (int)ZH, (int)S, (int)Skv, scale, static_cast<const T*>(mask), part,      \
+                     plan.chunk, plan.splits, head_dim)
   if (head_dim < D) {
     if (causal) HEXMI_KEYS(true, false, true);
     else if (mask != nullptr) HEXMI_KEYS(false, true, true);
@@ -428,10 +435,10 @@ int launch_keys(const void* Q, const void* K, const void* V, const void* mask, v
   if (plan.splits > 1) {
     if (causal)
       hipLaunchKernelGGL((flash_merge_kernel<OutT, D, true>), dim3((unsigned)merge_blocks), dim3(256), 0, st, part,
-                         static_cast<OutT*>(O), rows, (int)S, plan.chunk, plan.splits, head_dim);
+                         static_cast<OutT*>(O), rows, (int)S, plan.chunk, plan.splits, head_dim, unit);
     else
       hipLaunchKernelGGL((flash_merge_kernel<OutT, D, false>), dim3((unsigned)merge_blocks), dim3(256), 0, st, part,
-                         static_cast<OutT*>(O), rows, (int)S, plan.chunk, plan.splits, head_dim);
+                         static_cast<OutT*>(O), rows, (int)S, plan.chunk, plan.splits, head_dim, unit);
   }
   return launch_status();
 }
@@ -490,11 +497,11 @@ int64_t flash_keys_workspace(const FlashKeysPlan& p, int64_t ZH, int64_t S, int6
 }
 
 int flash_keys(const void* Q, const void* K, const void* V, const void* mask, void* O, int64_t ZH, int64_t S,
-               int64_t Skv, int64_t D, float scale_log2e, bool causal, int in_dtype, int out_dtype,
+               int64_t Skv, int64_t D, float sm_scale, bool causal, int in_dtype, int out_dtype,
                const FlashKeysPlan& plan, float* part, hipStream_t st) {
 #define HEXMI_KEYS_D(T, OutT)                                                                                          \
-  return D > 64 ? launch_keys<T, OutT, 128>(Q, K, V, mask, O, ZH, S, Skv, (int)D, scale_log2e, causal, plan, part, st) \
-                : launch_keys<T, OutT, 64>(Q, K, V, mask, O, ZH, S, Skv, (int)D, scale_log2e, causal, plan, part, st)
+  return D > 64 ? launch_keys<T, OutT, 128>(Q, K, V, mask, O, ZH, S, Skv, (int)D, sm_scale, causal, plan, part, st) \
+                : launch_keys<T, OutT, 64>(Q, K, V, mask, O, ZH, S, Skv, (int)D, sm_scale, causal, plan, part, st)
   if (in_dtype == HEXMI_F16 && out_dtype == HEXMI_F16) HEXMI_KEYS_D(f16, f16);
   if (in_dtype == HEXMI_F16 && out_dtype == HEXMI_F32) HEXMI_KEYS_D(f16, float);
   if (in_dtype == HEXMI_BF16 && out_dtype == HEXMI_BF16) HEXMI_KEYS_D(bf16, bf16);

@@ -12,6 +12,7 @@ namespace {
 constexpr int kWideMinS = 2048;  // sequences at least this long may use 8-wave (256-row) workgroups
 constexpr int kBlockN = 64;    // keys per step
 constexpr float kRescaleLag = 8.0f;   // how far (log2) the softmax reference maximum may trail the true one
+constexpr float kLog2e = 1.44269504088896340736f;
 
 template <typename T> struct MfmaT;
 template <> struct MfmaT<f16> {

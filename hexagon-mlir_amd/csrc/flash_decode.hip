@@ -7,7 +7,8 @@
 // D / 8 lanes, so a wave's load takes 64 * 8 / D rows; a wave asks for kU such loads of K and of V (16 KiB) before it
 // uses the first, and two workgroups fit a compute unit. Lane group g of a wave takes kU consecutive keys of the wave's
 // tile, whose mask values are then one 16-byte piece. Scores, probabilities and sums stay in fp32; every lane group has
-// its own running (max, sum), and they meet once at the end.
+// its own running (max, sum), and they meet once at the end. With a mask scores and maxima are in natural units (the reason
+// is at kUnit in flash_attn_keys.hip), without one in log2 units.
 // 512 heads x 2048 keys of 128 with a mask (537 MB): 99 us on the 128-query kernel, 79 here (6.8 TB/s); 256 x 8192 of 64
 // with a mask 199 -> 80, 512 x 128 of 64 7.4 -> 4.5.
 #include "flash_attn_tiles.h"
@@ -30,7 +31,8 @@ __device__ __forceinline__ float row_sum(float v) {    // over the D / 8 lanes t
 template <typename T, typename OutT, int D, bool MASKED>
 __global__ __launch_bounds__(kWaves * kWave, 4)
 void flash_decode_kernel(const T* __restrict__ Q, const T* __restrict__ K, const T* __restrict__ V,
-                         const T* __restrict__ Mk, OutT* __restrict__ O, int Skv, float scale_log2e) {
+                         const T* __restrict__ Mk, OutT* __restrict__ O, int Skv, float scale) {
+  constexpr float kUnit = MASKED ? kLog2e : 1.0f;       // log2 units of a score's unit
   constexpr int LPR = D / 8, GROUPS = kWave / LPR, TILE = GROUPS * kU;
   typedef T Piece __attribute__((ext_vector_type(8)));
   __shared__ float o_lds[kWaves][D];
@@ -82,8 +84,8 @@ void flash_decode_kernel(const T* __restrict__ Q, const T* __restrict__ K, const
       float dot = 0.0f;
 #pragma unroll
       for (int e = 0; e < 8; ++e) dot = fmaf(to_f32<T>(k[e]), q[e], dot);
-      s[u] = row_sum<LPR>(dot) * scale_log2e;
-      if constexpr (MASKED) s[u] = fmaf(to_f32<T>(mk[u]), 1.44269504088896340736f, s[u]);
+      if constexpr (MASKED) s[u] = fmaf(row_sum<LPR>(dot), scale, to_f32<T>(mk[u]));
+      else s[u] = row_sum<LPR>(dot) * scale;
     }
     if (!whole) {                                      // keys past the end: no weight, and nothing of V
 #pragma unroll
@@ -97,14 +99,14 @@ void flash_decode_kernel(const T* __restrict__ Q, const T* __restrict__ K, const
 #pragma unroll
     for (int u = 0; u < kU; ++u) m_new = fmaxf(m_new, s[u]);
     const float base = m_new == -INFINITY ? 0.0f : m_new;        // every key so far masked out: exp2(-inf) = 0, not NaN
-    const float alpha = __builtin_amdgcn_exp2f(m - base);
+    const float alpha = __builtin_amdgcn_exp2f((m - base) * kUnit);
     m = m_new;
     l *= alpha;
 #pragma unroll
     for (int e = 0; e < 8; ++e) o[e] *= alpha;
 #pragma unroll
     for (int u = 0; u < kU; ++u) {
-      const float p = __builtin_amdgcn_exp2f(s[u] - base);
+      const float p = __builtin_amdgcn_exp2f((s[u] - base) * kUnit);
       const Piece v = __builtin_bit_cast(Piece, vp[u]);
       l += p;
 #pragma unroll
@@ -116,7 +118,7 @@ void flash_decode_kernel(const T* __restrict__ Q, const T* __restrict__ K, const
 #pragma unroll
   for (int x = LPR; x < kWave; x *= 2) m_all = fmaxf(m_all, __shfl_xor(m_all, x));
   const float base = m_all == -INFINITY ? 0.0f : m_all;
-  const float w = __builtin_amdgcn_exp2f(m - base);
+  const float w = __builtin_amdgcn_exp2f((m - base) * kUnit);
   l *= w;
 #pragma unroll
   for (int e = 0; e < 8; ++e) o[e] *= w;
@@ -143,7 +145,7 @@ void flash_decode_kernel(const T* __restrict__ Q, const T* __restrict__ K, const
   const float top_base = top == -INFINITY ? 0.0f : top;          // every key of the row masked out: 0 / 0, NaN
 #pragma unroll
   for (int i = 0; i < kWaves; ++i) {
-    const float f = __builtin_amdgcn_exp2f(m_lds[i] - top_base);
+    const float f = __builtin_amdgcn_exp2f((m_lds[i] - top_base) * kUnit);
     sum = fmaf(l_lds[i], f, sum);
     out = fmaf(o_lds[i][d], f, out);
   }
@@ -152,11 +154,11 @@ void flash_decode_kernel(const T* __restrict__ Q, const T* __restrict__ K, const
 
 template <typename T, typename OutT, int D>
 int launch_decode(const void* Q, const void* K, const void* V, const void* mask, void* O, int64_t ZH, int64_t Skv,
-                  float scale_log2e, hipStream_t st) {
+                  float sm_scale, hipStream_t st) {
 #define HEXMI_DECODE(M)                                                                                              \
   hipLaunchKernelGGL((flash_decode_kernel<T, OutT, D, M>), dim3((unsigned)ZH), dim3(kWaves * kWave), 0, st,            \
                      static_cast<const T*>(Q), static_cast<const T*>(K), static_cast<const T*>(V),                    \
-                     static_cast<const T*>(mask), static_cast<OutT*>(O), (int)Skv, scale_log2e)
+                     static_cast<const T*>(mask), static_cast<OutT*>(O), (int)Skv, (M) ? sm_scale : sm_scale * kLog2e)
   if (mask != nullptr) HEXMI_DECODE(true);
   else HEXMI_DECODE(false);
 #undef HEXMI_DECODE
@@ -174,10 +176,10 @@ bool flash_decode_takes(int64_t ZH, int64_t S, int64_t Skv, int64_t D) {
 }
 
 int flash_decode(const void* Q, const void* K, const void* V, const void* mask, void* O, int64_t ZH, int64_t Skv,
-                 int64_t D, float scale_log2e, int in_dtype, int out_dtype, hipStream_t st) {
+                 int64_t D, float sm_scale, int in_dtype, int out_dtype, hipStream_t st) {
 #define HEXMI_DECODE_D(T, OutT)                                                                      \
-  return D == 128 ? launch_decode<T, OutT, 128>(Q, K, V, mask, O, ZH, Skv, scale_log2e, st)          \
-                  : launch_decode<T, OutT, 64>(Q, K, V, mask, O, ZH, Skv, scale_log2e, st)
+  return D == 128 ? launch_decode<T, OutT, 128>(Q, K, V, mask, O, ZH, Skv, sm_scale, st)          \
+                  : launch_decode<T, OutT, 64>(Q, K, V, mask, O, ZH, Skv, sm_scale, st)
   if (in_dtype == HEXMI_F16 && out_dtype == HEXMI_F16) HEXMI_DECODE_D(f16, f16);
   if (in_dtype == HEXMI_F16 && out_dtype == HEXMI_F32) HEXMI_DECODE_D(f16, float);
   if (in_dtype == HEXMI_BF16 && out_dtype == HEXMI_BF16) HEXMI_DECODE_D(bf16, bf16);

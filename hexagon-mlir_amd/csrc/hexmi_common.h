@@ -265,12 +265,12 @@ FlashKeysPlan plan_flash_keys(int64_t ZH, int64_t S, int64_t Skv, int64_t D, boo
                               bool may_split);
 int64_t flash_keys_workspace(const FlashKeysPlan& plan, int64_t ZH, int64_t S, int64_t D);
 int flash_keys(const void* Q, const void* K, const void* V, const void* mask, void* O, int64_t ZH, int64_t S,
-               int64_t Skv, int64_t D, float scale_log2e, bool causal, int in_dtype, int out_dtype,
+               int64_t Skv, int64_t D, float sm_scale, bool causal, int in_dtype, int out_dtype,
                const FlashKeysPlan& plan, float* part, hipStream_t st);
 
 // 16-bit attention of one query per head over many heads (flash_decode.hip): whether it takes a problem, and the launch.
 bool flash_decode_takes(int64_t ZH, int64_t S, int64_t Skv, int64_t D);
 int flash_decode(const void* Q, const void* K, const void* V, const void* mask, void* O, int64_t ZH, int64_t Skv,
-                 int64_t D, float scale_log2e, int in_dtype, int out_dtype, hipStream_t st);
+                 int64_t D, float sm_scale, int in_dtype, int out_dtype, hipStream_t st);
 
 }  // namespace hexmi

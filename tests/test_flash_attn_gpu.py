@@ -579,3 +579,37 @@ def test_attention_workspace(hexmi):
     assert torch.isnan(outs[0][2]).all() and torch.isnan(outs[1][2]).all()
     keep = [0, 1, 3]
     assert (outs[0][keep].float() - outs[1][keep].float()).abs().max() <= 1e-3
+
+
+# one case for each kernel that takes a mask, at key counts with and without whole runs of four: the key-group kernel (one
+# workgroup's keys, padded heads, keys cut into chunks), the decode kernel, and, from 360 units of 64 queries on, the
+# 128-query kernel (mask staged through LDS, read in runs, padded heads)
+FINITE_MASK_CASES = [(2, 40, 256, 128), (2, 40, 255, 128), (3, 70, 60, 64), (2, 33, 130, 80), (4, 3, 4096, 128), (4, 3, 4095, 64),
+                     (130, 1, 300, 128), (130, 1, 301, 64), (90, 200, 72, 128), (90, 200, 72, 64), (90, 200, 76, 128),
+                     (90, 200, 76, 80), (90, 200, 75, 128), (90, 200, 75, 64)]
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("case", FINITE_MASK_CASES)
+def test_masked_attention_rows_of_one_large_finite_value(hexmi, case, dtype):
+    # a row whose keys all carry the same value: the value drowns the scores in fp32 and the result is the average of V
+    # (torch's own fp32 softmax gives it), whatever the value; beside ordinary keys such a value is no weight at all.
+    # fp16's lowest leaves the scores a spacing of 2^-8, which a probability may be off by, and the result by that share
+    # of an average of |V| (below 1): 1e-2 covers it with the 16-bit rounding of the probabilities (5e-3)
+    B, Sq, Skv, D = case
+    g = _gen(71)
+    q = torch.randn(B, Sq, D, generator=g).to(dtype)
+    k, v = torch.randn(B, Skv, D, generator=g).to(dtype), torch.randn(B, Skv, D, generator=g).to(dtype)
+    values = [-65504.0, -3e4] if dtype == torch.float16 else [-1e38, -1e30, -2e9, torch.finfo(dtype).min, 1e30]
+    mask = _mask(B, Sq, Skv, dtype, 72)
+    rows = mask.view(B * Sq, Skv)
+    for i, value in enumerate(values):
+        rows[i] = value                                                  # the whole row
+        rows[-1 - i, Skv // 3:] = value                                  # all but a few keys
+    if dtype == torch.bfloat16:
+        rows[-1 - values.index(1e30), :] = 1e30
+    scores = q.float() @ k.float().transpose(1, 2) / math.sqrt(D) + mask.float()
+    want = torch.softmax(scores, dim=-1) @ v.float()
+    got = hexmi.attention(q.cuda(), k.cuda(), v.cuda(), mask.cuda(), out_dtype=torch.float32).cpu()
+    assert torch.isfinite(got).all()
+    assert (got - want).abs().max() <= (1e-2 if dtype == torch.float16 else 3e-2)
