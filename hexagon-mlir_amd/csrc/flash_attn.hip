@@ -61,7 +61,7 @@ struct MaskTileLoader {
 
 // GENERAL: the number of keys (Skv) may differ from the number of queries (S) and an additive mask
 // [ZH, S, Skv] (MASKED, same dtype as Q) is added to the scaled scores before the softmax, as
-// tm_tensor.attention does (qcom_hexagon_backend/lib/Transforms/LowerTmTensor.cpp:157-160).
+// tm_tensor.attention does (qcom_hexagon_backend/lib/Transforms/LowerTmTensor.cpp:157-160); with a mask Skv % 4 == 0.
 // NW waves per workgroup (4 or 8), 32 query rows each: every K / V tile copied into LDS serves NW*32 query rows.
 // Eight waves halve the L2 -> LDS copy traffic (each query block streams the whole K and V of its head), worth
 // 1-9 % from 2048 keys on; short sequences and small grids prefer the larger number of 128-row workgroups. (Measured on random
@@ -353,26 +353,18 @@ void flash_fwd_kernel(const T* __restrict__ Q, const T* __restrict__ K, const T*
       const bool spread = next >= 0 && (next + 1) * kBlockN <= Skv && !(CAUSAL && n0 > q0 + 31);
       if (next >= 0 && !spread) load_kv(next, k_dst, v_dst, m_dst, kb_dst, vb_dst);
       if (CAUSAL && n0 > q0 + 31) return;
-      // mask values of this lane's 32 scores: four runs of four consecutive keys per 32-key tile. A run's load only
-      // needs the alignment of an element (one 8-byte load either way), so mask rows of any length are read here.
+      // mask values of this lane's 32 scores: four runs of four consecutive keys per 32-key tile
       typedef T MaskRun __attribute__((ext_vector_type(4)));
       MaskRun mk[2][4];
       if constexpr (MASKED && !MASK_LDS) {
-        if (n0 + kBlockN <= Skv) {
 #pragma unroll
-          for (int jt = 0; jt < 2; ++jt)
+        for (int jt = 0; jt < 2; ++jt)
 #pragma unroll
-            for (int g4 = 0; g4 < 4; ++g4)
-              __builtin_memcpy(&mk[jt][g4], mask_row + n0 + jt * 32 + 8 * g4 + 4 * half, sizeof(MaskRun));
-        } else {                                             // the row ends in this block: by elements, none past it
-#pragma unroll
-          for (int jt = 0; jt < 2; ++jt)
-#pragma unroll
-            for (int e = 0; e < 16; ++e) {
-              const int key = n0 + jt * 32 + 8 * (e / 4) + 4 * half + e % 4;
-              mk[jt][e / 4][e % 4] = mask_row[key < Skv ? key : Skv - 1];
-            }
-        }
+          for (int g4 = 0; g4 < 4; ++g4) {
+            int key = n0 + jt * 32 + 8 * g4 + 4 * half;
+            key = key + 4 <= Skv ? key : Skv - 4;            // past the end: any valid run, those scores are dropped
+            mk[jt][g4] = *reinterpret_cast<const MaskRun*>(mask_row + key);
+          }
       }
       // ---- scores: s[jt][r] = Q[qrow] . K[n0 + jt*32 + 8*(r/4) + 4*half + r%4]. The MFMA chains of the two 32-key
       // tiles are interleaved (a chain alone waits for its own previous result) and their K fragments are read
@@ -758,6 +750,9 @@ inline bool matrix_core_operands(const void* Q, const void* K, const void* V, co
          scale_log2e > 0.0f;
 }
 
+// whether the rows of a mask are whole aligned runs of four keys
+inline bool mask_in_runs(const void* mask, int64_t Skv) { return Skv % 4 == 0 && aligned_to(mask, 8); }
+
 // mask == nullptr and Skv == S: the tuned kernels; otherwise the general ones.
 template <typename T, typename OutT>
 int dispatch_half(const void* Q, const void* K, const void* V, const void* mask, void* O, int64_t ZH, int64_t S,
@@ -781,9 +776,8 @@ int dispatch_half(const void* Q, const void* K, const void* V, const void* mask,
     if (causal) return launch_mfma_wide<T, OutT, true>(Q, K, V, O, ZH, S, (int)D, scale_log2e, st);
     return launch_mfma_wide<T, OutT, false>(Q, K, V, O, ZH, S, (int)D, scale_log2e, st);
   }
-  // any key count and any mask alignment (see the mask reads of process()): 509 queries over 2555 keys with a mask,
-  // 32 heads of 128, take 121 us here and 11.4 ms on the row-wise kernel
-  const bool general_ok = ok && !causal;
+  // (a mask is read in runs of four keys; without one any key count goes: cross-attention over 77 keys, say)
+  const bool general_ok = ok && !causal && (!mask || mask_in_runs(mask, Skv));
   if (general_ok && D == 128) return launch_mfma_general<T, OutT, 128>(Q, K, V, mask, O, ZH, S, Skv, scale_log2e, st);
   if (general_ok && D == 64) return launch_mfma_general<T, OutT, 64>(Q, K, V, mask, O, ZH, S, Skv, scale_log2e, st);
   if (general_ok && D % 8 == 0 && D < 64) return launch_mfma_general<T, OutT, 64>(Q, K, V, mask, O, ZH, S, Skv, scale_log2e, st, (int)D);
@@ -798,9 +792,12 @@ int attention_any(const void* Q, const void* K, const void* V, const void* mask,
   const bool half = (in_dtype == HEXMI_F16 || in_dtype == HEXMI_BF16) && (out_dtype == in_dtype || out_dtype == HEXMI_F32);
   if (half && flash_decode_takes(ZH, S, Skv, D) && matrix_core_operands(Q, K, V, O, Skv * D * 2, c))
     return flash_decode(Q, K, V, mask, O, ZH, Skv, D, sm_scale, in_dtype, out_dtype, st);
-  const bool mask_ok = mask == nullptr || ZH * S * Skv >= 8;            // flash_keys reads masks in pieces of eight
-  if (half && mask_ok && matrix_core_operands(Q, K, V, O, Skv * D * 2, c)) {
-    const FlashKeysPlan plan = plan_flash_keys(ZH, S, Skv, D, cz, mask != nullptr, workspace != nullptr);
+  // Masks that are not whole runs of four keys: flash_keys at any size, with the probabilities in full precision (the
+  // row-wise kernel, the only other one that reads such a mask, holds them in fp32: 32 heads x 509 queries x 2555 keys
+  // of 128 take it 11.4 ms). It reads masks in pieces of eight.
+  const bool any_mask = mask != nullptr && !mask_in_runs(mask, Skv);
+  if (half && (!any_mask || ZH * S * Skv >= 8) && matrix_core_operands(Q, K, V, O, Skv * D * 2, c)) {
+    const FlashKeysPlan plan = plan_flash_keys(ZH, S, Skv, D, cz, mask != nullptr, any_mask, workspace != nullptr);
     if (plan.splits > 0) {
       if (plan.splits > 1 && (workspace_bytes < flash_keys_workspace(plan, ZH, S, D) || !aligned_to(workspace, 16)))
         return HEXMI_EINVAL;
@@ -850,8 +847,9 @@ extern "C" int64_t hexmi_attention_workspace(int64_t batch, int64_t seq_q, int64
   if (batch <= 0 || seq_q <= 0 || seq_kv <= 0 || head_dim <= 0) return 0;
   if (seq_q > 0x7fffffff / 2 || seq_kv > 0x7fffffff / 2 || batch > 0x7fffffff) return 0;
   if (in_dtype != HEXMI_F16 && in_dtype != HEXMI_BF16) return 0;
-  return flash_keys_workspace(plan_flash_keys(batch, seq_q, seq_kv, head_dim, false, has_mask != 0, true), batch, seq_q,
-                              head_dim);
+  // (an unaligned mask does not change how a problem's keys are cut, see plan_flash_keys)
+  return flash_keys_workspace(plan_flash_keys(batch, seq_q, seq_kv, head_dim, false, has_mask != 0, false, true), batch,
+                              seq_q, head_dim);
 }
 
 extern "C" int hexmi_attention_ws(const void* Q, const void* K, const void* V, const void* mask, void* O, int64_t batch,

@@ -12,6 +12,8 @@
 //
 // Per wave and 32-key tile the work is that of flash_attn.hip: S^T = K Q^T (a lane holds 16 scores of one query),
 // online softmax in fp32 with a lagging maximum, O^T += V^T P^T with the probabilities taken from the score registers.
+#include <type_traits>
+
 #include "flash_attn_tiles.h"
 
 namespace hexmi {
@@ -57,13 +59,41 @@ struct GroupTileLoader {
   }
 };
 
-template <typename T, typename OutT, int D, bool CAUSAL, bool MASKED, bool PADDED>
+// p[0..7] -= the eight packed values, exactly (they are the roundings of p). One instruction per value in fp16: left to
+// itself the compiler converts every value a second time, to have it alone in a register.
+__device__ __forceinline__ void take_part(const f16x8& part, float* p) {
+  const u32x4 u = __builtin_bit_cast(u32x4, part);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    asm("v_fma_mix_f32 %0, %1, -1.0, %0 op_sel_hi:[1,0,0]" : "+v"(p[2 * i]) : "v"(u[i]));
+    asm("v_fma_mix_f32 %0, %1, -1.0, %0 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "+v"(p[2 * i + 1]) : "v"(u[i]));
+  }
+}
+__device__ __forceinline__ void take_part(const bf16x8& part, float* p) {
+  const u32x4 u = __builtin_bit_cast(u32x4, part);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    p[2 * i] -= __builtin_bit_cast(float, u[i] << 16);
+    p[2 * i + 1] -= __builtin_bit_cast(float, u[i] & 0xffff0000u);
+  }
+}
+
+// FULL: the probabilities go into P V as two or three 16-bit parts, each the rounding of what the parts before it leave, and
+// their sum is taken in fp32. Two parts hold 22 bits (fp16; the exponents are raised by 6 so that the second part of a
+// small probability stays above 2^-24) or 16 (bf16, whose result is rounded to 8), three 24 (bf16 with an fp32 result). For
+// an fp32 result the parts of a tile meet in registers of their own, so that the running sum is rounded once a tile.
+// A part costs its share of MFMAs: 32 heads x 509 queries x 2555 keys of 128 with a mask 40 us in one part, 46 in two.
+template <typename T, typename OutT, int D, bool CAUSAL, bool MASKED, bool PADDED, bool FULL>
 __global__ __launch_bounds__(512, D == 64 && !MASKED ? 4 : 2)
 void flash_keys_kernel(const T* __restrict__ Q, const T* __restrict__ K, const T* __restrict__ V, OutT* __restrict__ O,
                        int ZH, int S, int Skv, float scale, const T* __restrict__ Mk, float* __restrict__ part,
                        int chunk, int splits, int head_dim) {
   const int dh = PADDED ? head_dim : D;                 // elements between rows in memory
   static_assert(!(CAUSAL && MASKED), "the causal kernel has no mask");
+  static_assert(!FULL || MASKED, "full probabilities: masked kernel");
+  constexpr int kParts = !FULL ? 1 : (sizeof(OutT) == 4 && std::is_same<T, bf16>::value ? 3 : 2);
+  constexpr bool kTileSums = FULL && sizeof(OutT) == 4;
+  constexpr float kRaise = FULL && std::is_same<T, f16>::value ? 6.0f : 0.0f;
   // Without a mask `scale` carries log2 e and a score is scaled as its exponent is taken: one instruction. With one the
   // score is scaled and the mask added to it in natural units, and the difference to the maximum is taken before it
   // is multiplied by log2 e. That way a row whose keys all carry the same large finite value gives the average of V as any
@@ -278,13 +308,47 @@ void flash_keys_kernel(const T* __restrict__ Q, const T* __restrict__ K, const T
     }
     float p[16];
 #pragma unroll
-    for (int r = 0; r < 16; ++r) p[r] = __builtin_amdgcn_exp2f(MASKED ? (s[r] + neg_m) * kUnit : fmaf(s[r], scale, neg_m));
-    const Frag pf[2] = {MfmaT<T>::pack(&p[0]), MfmaT<T>::pack(&p[8])};
-    l_i = MfmaT<T>::sum8(pf[1], MfmaT<T>::sum8(pf[0], l_i));
+    for (int r = 0; r < 16; ++r) {
+      if constexpr (FULL) p[r] = __builtin_amdgcn_exp2f(fmaf(s[r] + neg_m, kUnit, kRaise));
+      else p[r] = __builtin_amdgcn_exp2f(MASKED ? (s[r] + neg_m) * kUnit : fmaf(s[r], scale, neg_m));
+    }
+    if constexpr (FULL) {
+      float sum[4];
 #pragma unroll
-    for (int hf = 0; hf < 2; ++hf)
+      for (int r = 0; r < 4; ++r) sum[r] = (p[r] + p[r + 4]) + (p[r + 8] + p[r + 12]);
+      l_i += (sum[0] + sum[1]) + (sum[2] + sum[3]);
+    }
+    Frag pf[kParts][2];
 #pragma unroll
-      for (int dt = 0; dt < DT; ++dt) o_acc[dt] = MfmaT<T>::run(vf[hf][dt], pf[hf], o_acc[dt]);
+    for (int part = 0; part < kParts; ++part) {
+      pf[part][0] = MfmaT<T>::pack(&p[0]);
+      pf[part][1] = MfmaT<T>::pack(&p[8]);
+      if constexpr (!FULL) l_i = MfmaT<T>::sum8(pf[part][1], MfmaT<T>::sum8(pf[part][0], l_i));
+      if (part + 1 < kParts) {
+        take_part(pf[part][0], &p[0]);
+        take_part(pf[part][1], &p[8]);
+      }
+      if constexpr (!kTileSums) {
+#pragma unroll
+        for (int hf = 0; hf < 2; ++hf)
+#pragma unroll
+          for (int dt = 0; dt < DT; ++dt) o_acc[dt] = MfmaT<T>::run(vf[hf][dt], pf[part][hf], o_acc[dt]);
+      }
+    }
+    if constexpr (kTileSums) {
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt) {
+        f32x16 tile;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) tile[r] = 0.0f;
+#pragma unroll
+        for (int part = kParts - 1; part >= 0; --part)
+#pragma unroll
+          for (int hf = 0; hf < 2; ++hf) tile = MfmaT<T>::run(vf[hf][dt], pf[part][hf], tile);
+#pragma unroll
+        for (int r = 0; r < 16; ++r) o_acc[dt][r] += tile[r];
+      }
+    }
   };
 
   // This wave's copies of the next tile are in LDS. The two mask loads behind them stay in flight (loads complete in
@@ -417,19 +481,21 @@ int launch_keys(const void* Q, const void* K, const void* V, const void* mask, v
   const int64_t merge_blocks = (rows + 1024 / D - 1) / (1024 / D);
   if (blocks > 0x7fffffff || merge_blocks > 0x7fffffff) return HEXMI_ENOTSUP;
   const float unit = mask != nullptr ? kLog2e : 1.0f, scale = mask != nullptr ? sm_scale : sm_scale * kLog2e;
-#define HEXMI_KEYS(C, M, P)                                                                                           \
-  hipLaunchKernelGGL((flash_keys_kernel<T, OutT, D, C, M, P>), dim3((unsigned)blocks), dim3(512), 0, st,              \
+#define HEXMI_KEYS(C, M, P, F)                                                                                        \
+  hipLaunchKernelGGL((flash_keys_kernel<T, OutT, D, C, M, P, F>), dim3((unsigned)blocks), dim3(512), 0, st,           \
                      static_cast<const T*>(Q), static_cast<const T*>(K), static_cast<const T*>(V),                    \
                      static_cast<OutT*>(O), (int)ZH, (int)S, (int)Skv, scale, static_cast<const T*>(mask), part,      \
                      plan.chunk, plan.splits, head_dim)
   if (head_dim < D) {
-    if (causal) HEXMI_KEYS(true, false, true);
-    else if (mask != nullptr) HEXMI_KEYS(false, true, true);
-    else HEXMI_KEYS(false, false, true);
+    if (causal) HEXMI_KEYS(true, false, true, false);
+    else if (plan.full) HEXMI_KEYS(false, true, true, true);
+    else if (mask != nullptr) HEXMI_KEYS(false, true, true, false);
+    else HEXMI_KEYS(false, false, true, false);
   } else {
-    if (causal) HEXMI_KEYS(true, false, false);
-    else if (mask != nullptr) HEXMI_KEYS(false, true, false);
-    else HEXMI_KEYS(false, false, false);
+    if (causal) HEXMI_KEYS(true, false, false, false);
+    else if (plan.full) HEXMI_KEYS(false, true, false, true);
+    else if (mask != nullptr) HEXMI_KEYS(false, true, false, false);
+    else HEXMI_KEYS(false, false, false, false);
   }
 #undef HEXMI_KEYS
   if (plan.splits > 1) {
@@ -462,17 +528,20 @@ int launch_keys(const void* Q, const void* K, const void* V, const void* mask, v
 // Chunks only where half the compute units would stay idle: a merge costs its launch (4 us, and 3 of the host's) and
 // the fp32 sums, a step (128 keys) about 1.2 us with heads of 128 and 0.8 with heads of 64 (8 heads x 1 x 8192: 65 us in
 // one chunk, 15 in 16; 32 heads x 200 x 2000 of 64: 20.5 and 17.5 in two).
-FlashKeysPlan plan_flash_keys(int64_t ZH, int64_t S, int64_t Skv, int64_t D, bool causal, bool masked, bool may_split) {
+FlashKeysPlan plan_flash_keys(int64_t ZH, int64_t S, int64_t Skv, int64_t D, bool causal, bool masked, bool any_mask,
+                              bool may_split) {
   FlashKeysPlan p;
   const int64_t cus = hexmi_num_cus(), units = (S + kRows - 1) / kRows * ZH;
-  if (D % 8 != 0 || D > 128 || cus <= 0 || Skv <= 64 || (causal && S >= 4096)) return p;
+  if (D % 8 != 0 || D > 128 || cus <= 0) return p;
+  if (!any_mask && (Skv <= 64 || (causal && S >= 4096))) return p;
   D = D <= 64 ? 64 : 128;                                  // narrower heads on tiles padded with zero columns
   bool take = units <= cus;
   if (causal)
     take = take || (D == 128 ? units <= 2 * cus && S >= 768 : (units <= 2 * cus && S >= 256) || (units <= 4 * cus && S >= 768));
   else if (D == 64)
     take = take || (S <= 64 && (!masked || Skv >= 512)) || (units <= 2 * cus && Skv >= 512);
-  if (!take) return p;
+  if (!take && !any_mask) return p;
+  p.full = any_mask;
   const int64_t steps = (Skv + kStepKeys - 1) / kStepKeys;
   p.chunk = (int)steps;
   p.splits = 1;

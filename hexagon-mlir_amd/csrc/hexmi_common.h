@@ -257,11 +257,13 @@ bool flash_attn_f32_mfma(const float* Q, const float* K, const float* V, const f
 
 // 16-bit flash attention of few (head, query block) units, the keys of a unit divided inside and over workgroups
 // (flash_attn_keys.hip). plan: splits == 0, leave it to the other kernels; > 1, the fp32 sums of that many chunks of
-// the key range go through a workspace.
+// the key range go through a workspace; full, the probabilities keep fp32 precision into the second product. any_mask: a
+// mask that is not whole aligned runs of four keys, which no other kernel of that speed reads (taken at any size, full).
 struct FlashKeysPlan {
   int chunk = 0, splits = 0;
+  bool full = false;
 };
-FlashKeysPlan plan_flash_keys(int64_t ZH, int64_t S, int64_t Skv, int64_t D, bool causal, bool masked,
+FlashKeysPlan plan_flash_keys(int64_t ZH, int64_t S, int64_t Skv, int64_t D, bool causal, bool masked, bool any_mask,
                               bool may_split);
 int64_t flash_keys_workspace(const FlashKeysPlan& plan, int64_t ZH, int64_t S, int64_t D);
 int flash_keys(const void* Q, const void* K, const void* V, const void* mask, void* O, int64_t ZH, int64_t S,

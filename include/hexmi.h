@@ -336,6 +336,11 @@ int hexmi_flash_attn_fwd(const void *Q, const void *K, const void *V, void *O,
  * any 16-bit value on the matrix-core and decode kernels: a row whose keys all
  * carry the lowest one gives the average of V (the fp32 and row-wise kernels
  * hold down to about -1e9 and -2e38).
+ * Scores, sums and maxima are fp32. 16-bit inputs have their probabilities
+ * rounded to in_dtype for P V, as the reference's linalg form has, except
+ * with a mask that is not whole aligned runs of four keys (seq_kv % 4 != 0, or
+ * a base off the 8-byte boundary) and with one query each of many heads, where
+ * they keep fp32 precision.
  * in_dtype / out_dtype as for hexmi_flash_attn_fwd. */
 int hexmi_attention(const void *Q, const void *K, const void *V,
                     const void *mask, void *O, int64_t batch, int64_t seq_q,

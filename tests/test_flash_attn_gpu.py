@@ -321,8 +321,8 @@ def test_masked_attention_parity_half(hexmi, oracle, case, dtype, with_mask):
 @pytest.mark.parametrize("case", [(2, 5, 1, 64), (1, 33, 3, 128), (3, 129, 63, 64), (2, 130, 65, 128), (2, 64, 127, 80),
                                   (3, 128, 130, 128), (1, 300, 1023, 96), (2, 257, 2051, 128)])
 def test_masked_attention_mask_rows_of_any_length_and_alignment(hexmi, oracle, case, dtype):
-    # mask rows of an odd number of keys on the matrix-core kernel, the mask itself one element off its allocation;
-    # the tolerances are those of test_masked_attention_parity_half (the same sums, the same roundings)
+    # mask rows of an odd number of keys on the matrix cores, the mask itself one element off its allocation; the
+    # tolerances are those of test_masked_attention_parity_half (the test below holds these masks to fp32 sums)
     B, Sq, Skv, D = case
     g = _gen(27)
     q = torch.randn(B, Sq, D, generator=g).to(dtype)
@@ -613,3 +613,29 @@ def test_masked_attention_rows_of_one_large_finite_value(hexmi, case, dtype):
     got = hexmi.attention(q.cuda(), k.cuda(), v.cuda(), mask.cuda(), out_dtype=torch.float32).cpu()
     assert torch.isfinite(got).all()
     assert (got - want).abs().max() <= (1e-2 if dtype == torch.float16 else 3e-2)
+
+
+# masks that are not whole aligned runs of four keys: few keys, one step and its edges, key chunks, far more units than
+# compute units, padded heads; the last two have whole runs in a mask that starts one element off its allocation
+ANY_MASK_CASES = [(2, 5, 1, 64), (1, 33, 3, 128), (3, 129, 63, 64), (2, 130, 65, 128), (2, 64, 127, 80), (3, 2, 4095, 128),
+                  (90, 200, 75, 128), (150, 200, 129, 64), (90, 200, 76, 24), (3, 70, 512, 128)]
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("case", ANY_MASK_CASES)
+def test_masked_attention_any_mask_in_fp32(hexmi, case, dtype):
+    # these masks keep fp32 probabilities (in 16-bit parts on the matrix cores). A raw score adds up D <= 128 products
+    # whose partial sums stay below about 60: 128 roundings of 60 * 2^-24 at random signs are 4e-5, scaled by 1/sqrt(D)
+    # 4e-6; the exponent adds its own 2^-23 * |t| < 3e-6. A probability is off by that share, the result by no more of an
+    # average of |V|: 2e-5. (16-bit probabilities alone are off by up to 5e-4 and 4e-3.)
+    B, Sq, Skv, D = case
+    g = _gen(73)
+    q = torch.randn(B, Sq, D, generator=g).to(dtype)
+    k, v = torch.randn(B, Skv, D, generator=g).to(dtype), torch.randn(B, Skv, D, generator=g).to(dtype)
+    mask = _mask(B, Sq, Skv, dtype, 74)
+    shifted = torch.empty(mask.numel() + 1, dtype=dtype, device="cuda")[1:].view(B, Sq, Skv)
+    shifted.copy_(mask)
+    scores = q.double() @ k.double().transpose(1, 2) / math.sqrt(D) + mask.double()
+    want = torch.softmax(scores, dim=-1) @ v.double()
+    got = hexmi.attention(q.cuda(), k.cuda(), v.cuda(), shifted, out_dtype=torch.float32).cpu()
+    assert (got.double() - want).abs().max() <= 2e-5
