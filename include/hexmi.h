@@ -332,7 +332,8 @@ int hexmi_flash_attn_fwd(const void *Q, const void *K, const void *V, void *O,
  * sm_scale = 1/sqrt(head_dim); here the caller passes it. -inf mask entries
  * remove a key; a row whose keys are all removed yields NaN, as the
  * reference's max / sub / exp / div sequence does. A removed key takes part
- * with weight 0, so K and V have to be finite there too. Finite entries may be
+ * with weight 0, so K and V have to be finite there too (and an infinity in V
+ * comes out as infinity or NaN). Finite entries may be
  * any 16-bit value on the matrix-core and decode kernels: a row whose keys all
  * carry the lowest one gives the average of V (the fp32 and row-wise kernels
  * hold down to about -1e9 and -2e38).

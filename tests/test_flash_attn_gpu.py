@@ -639,3 +639,29 @@ def test_masked_attention_any_mask_in_fp32(hexmi, case, dtype):
     want = torch.softmax(scores, dim=-1) @ v.double()
     got = hexmi.attention(q.cuda(), k.cuda(), v.cuda(), shifted, out_dtype=torch.float32).cpu()
     assert (got.double() - want).abs().max() <= 2e-5
+
+
+@pytest.mark.parametrize("with_mask", [True, False])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("case", [(2, 40, 65, 128), (3, 20, 79, 64), (2, 33, 130, 80), (2, 1, 4095, 128), (130, 1, 301, 64),
+                                  (130, 1, 70, 128)])
+def test_attention_infinities_in_the_last_row_of_v(hexmi, case, dtype, with_mask):
+    # odd columns of the last key are +inf or -inf: they come out infinite or NaN (a tile repeats the last row past the end
+    # at weight 0, and probabilities in parts have negative ones), the even columns as without them; and a head's
+    # NaN stays in that head. Bound: the parity tests'
+    B, Sq, Skv, D = case
+    g = _gen(75)
+    q = torch.randn(B, Sq, D, generator=g).to(dtype)
+    k, v = torch.randn(B, Skv, D, generator=g).to(dtype), torch.randn(B, Skv, D, generator=g).to(dtype)
+    v[:, -1, 1::4] = float("inf")
+    v[:, -1, 3::4] = -float("inf")
+    k[1, 0], v[1, 0] = float("nan"), float("nan")
+    mask = torch.randn(B, Sq, Skv, generator=g).to(dtype) if with_mask else None
+    got = hexmi.attention(q.cuda(), k.cuda(), v.cuda(), None if mask is None else mask.cuda(), out_dtype=torch.float32).cpu()
+    assert torch.isnan(got[1]).all()
+    heads = [h for h in range(B) if h != 1]
+    got = got[heads]
+    assert not torch.isfinite(got[:, :, 1::2]).any()
+    scores = q.float() @ k.float().transpose(1, 2) / math.sqrt(D) + (0.0 if mask is None else mask.float())
+    want = torch.softmax(scores[heads], dim=-1) @ v[heads][:, :, ::2].float()
+    assert (got[:, :, ::2] - want).abs().max() <= (5e-3 if dtype == torch.float16 else 3e-2)
