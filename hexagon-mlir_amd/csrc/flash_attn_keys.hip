@@ -477,9 +477,8 @@ void flash_merge_kernel(const float* __restrict__ part, OutT* __restrict__ O, in
 template <typename T, typename OutT, int D>
 int launch_keys(const void* Q, const void* K, const void* V, const void* mask, void* O, int64_t ZH, int64_t S,
                 int64_t Skv, int head_dim, float sm_scale, bool causal, const FlashKeysPlan& plan, float* part, hipStream_t st) {
-  const int64_t blocks = (S + kRows - 1) / kRows * ZH * plan.splits, rows = ZH * S;
+  const int64_t blocks = (S + kRows - 1) / kRows * ZH * plan.splits, rows = ZH * S;     // see plan_flash_keys
   const int64_t merge_blocks = (rows + 1024 / D - 1) / (1024 / D);
-  if (blocks > 0x7fffffff || merge_blocks > 0x7fffffff) return HEXMI_ENOTSUP;
   const float unit = mask != nullptr ? kLog2e : 1.0f, scale = mask != nullptr ? sm_scale : sm_scale * kLog2e;
 #define HEXMI_KEYS(C, M, P, F)                                                                                        \
   hipLaunchKernelGGL((flash_keys_kernel<T, OutT, D, C, M, P, F>), dim3((unsigned)blocks), dim3(512), 0, st,           \
@@ -532,7 +531,7 @@ FlashKeysPlan plan_flash_keys(int64_t ZH, int64_t S, int64_t Skv, int64_t D, boo
                               bool may_split) {
   FlashKeysPlan p;
   const int64_t cus = hexmi_num_cus(), units = (S + kRows - 1) / kRows * ZH;
-  if (D % 8 != 0 || D > 128 || cus <= 0) return p;
+  if (D % 8 != 0 || D > 128 || cus <= 0 || !grid_fits(units, 512)) return p;
   if (!any_mask && (Skv <= 64 || (causal && S >= 4096))) return p;
   D = D <= 64 ? 64 : 128;                                  // narrower heads on tiles padded with zero columns
   bool take = units <= cus;

@@ -172,7 +172,7 @@ int launch_decode(const void* Q, const void* K, const void* V, const void* mask,
 // 64 5.2 / 5.6 -> 3.9 / 3.7, x 2048 29.5 / 42 -> 14.8 / 13.6; 256 x 2048 of 128 43 / 61 -> 41 / 40; 2048 x 512 of 128
 // 103 / 107 -> 81 / 78. Up to 64 keys those kernels are one block and stay.
 bool flash_decode_takes(int64_t ZH, int64_t S, int64_t Skv, int64_t D) {
-  return S == 1 && (D == 64 || D == 128) && Skv > 64 && 2 * ZH > hexmi_num_cus();
+  return S == 1 && (D == 64 || D == 128) && Skv > 64 && 2 * ZH > hexmi_num_cus() && grid_fits(ZH, kWaves * kWave);
 }
 
 int flash_decode(const void* Q, const void* K, const void* V, const void* mask, void* O, int64_t ZH, int64_t Skv,

@@ -146,6 +146,9 @@ inline hipStream_t as_stream(hexmi_stream_t s) { return reinterpret_cast<hipStre
 // the launch_status() of the next launch here.
 inline void begin_call() { (void)hipGetLastError(); }
 
+// A launch holds at most 2^32 - 1 threads per dimension.
+inline bool grid_fits(int64_t blocks, int threads) { return blocks <= 0xffffffffll / threads; }
+
 inline int launch_status() {
   return hipGetLastError() == hipSuccess ? HEXMI_OK : HEXMI_ELAUNCH;
 }

@@ -665,3 +665,23 @@ def test_attention_infinities_in_the_last_row_of_v(hexmi, case, dtype, with_mask
     scores = q.float() @ k.float().transpose(1, 2) / math.sqrt(D) + (0.0 if mask is None else mask.float())
     want = torch.softmax(scores[heads], dim=-1) @ v[heads][:, :, ::2].float()
     assert (got[:, :, ::2] - want).abs().max() <= (5e-3 if dtype == torch.float16 else 3e-2)
+
+
+@pytest.mark.parametrize("with_mask", [False, True])
+def test_attention_more_heads_than_a_grid_of_512_threads_holds(hexmi, with_mask):
+    # 2^23 workgroups of 512 threads are more than a launch takes: the persistent kernel (without a mask) and the row-wise
+    # one (with this one, rows of 65 keys) do. K is V here; four heads against the fp32 sums, bound as in the parity tests
+    B, Skv, D = (1 << 23) + 3, 65, 8
+    g = torch.Generator(device="cuda").manual_seed(77)
+    q = torch.randn(B, 1, D, generator=g, device="cuda", dtype=torch.float16)
+    k = torch.randn(B, Skv, D, generator=g, device="cuda", dtype=torch.float16)
+    mask = torch.randn(B, 1, Skv, generator=g, device="cuda", dtype=torch.float16) if with_mask else None
+    out = torch.full_like(q, float("nan"))
+    hexmi.attention(q, k, k, mask, out=out)
+    assert torch.isfinite(out).all()
+    pick = [0, 1, 1 << 22, B - 1]
+    scores = q[pick].float() @ k[pick].float().transpose(1, 2).contiguous() / math.sqrt(D)
+    if with_mask:
+        scores = scores + mask[pick].float()
+    want = torch.softmax(scores, dim=-1) @ k[pick].float()
+    assert (out[pick].float() - want).abs().max() <= 2e-2
