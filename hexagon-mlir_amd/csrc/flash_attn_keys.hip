@@ -114,19 +114,25 @@ void flash_keys_kernel(const T* __restrict__ Q, const T* __restrict__ K, const T
   const int lane = threadIdx.x % kWave, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   const int rt = wave % 2, ks = wave / 2, half = lane / 32;
 
-  // Workgroup -> (head, query block, key chunk). Workgroup ids go round robin to the 8 XCDs (one L2 each): whole heads
-  // stay on one of them. Causal: the longest query blocks of all its heads first.
+  // Workgroup -> (head, query block, key chunk). Workgroup ids go round robin to the 8 XCDs (one L2 each), and a head's
+  // workgroups share one: an XCD takes an eighth of the list of all units, head by head. (Spread
+  // over the XCDs, as head counts off the multiple of 8 were: 127 heads x 207 x 3967 of 64 76 us, 51 this way; 51 heads x
+  // 1000 of 64 causal 21.2, 17.6.) Causal: the longest query blocks of all heads first, head h on XCD h % 8;
+  // the last ZH % 8 heads wander.
   const int nqb = (S + kRows - 1) / kRows;
   int zh, qb, split;
-  {
-    const bool by_xcd = ZH % 8 == 0;
-    const int heads = by_xcd ? ZH / 8 : ZH;
-    const int u = by_xcd ? blockIdx.x / 8 : blockIdx.x;
+  const unsigned b = blockIdx.x, xcd = b % 8;
+  if (CAUSAL) {
+    const int c = b % ZH;
+    zh = c < ZH / 8 * 8 ? c / 8 * 8 + xcd : c;
+    qb = nqb - 1 - b / ZH;
+    split = 0;
+  } else {
+    const unsigned each = gridDim.x / 8, more = gridDim.x % 8;
+    const unsigned u = xcd * each + (xcd < more ? xcd : more) + b / 8, r = u / splits;
     split = u % splits;
-    const int r = u / splits;
-    const int h = CAUSAL ? r % heads : r / nqb;
-    qb = nqb - 1 - (CAUSAL ? r / heads : r % nqb);
-    zh = by_xcd ? blockIdx.x % 8 + 8 * h : h;
+    zh = r / nqb;
+    qb = nqb - 1 - r % nqb;
   }
   const int key_end = CAUSAL ? ((qb + 1) * kRows < S ? (qb + 1) * kRows : S) : Skv;
   const int unit_steps = (key_end + kStepKeys - 1) / kStepKeys;
@@ -514,12 +520,14 @@ int launch_keys(const void* Q, const void* K, const void* V, const void* mask, v
 // 64 queries. The lines are where the measured ratio to the kernels of flash_attn.hip crosses 1 (fp16, graph replay, 8 to
 // 256 heads, 64 to 8192 keys; us there -> here):
 //  - up to one workgroup per compute unit they win by 1.1 to 2.1 (one 64-key block excepted): 16 heads x 1024 queries and
-//    keys of 128 25 -> 17, with a mask 39 -> 20; 12 heads x 1000 of 64 causal 18 -> 11; 8 heads x 2048 causal 40 -> 24;
-//  - heads of 64 fit two workgroups on a compute unit: with up to 64 queries always ahead (512 heads x 1 x 2048 56 -> 51),
-//    else up to two per unit from 512 keys on (16 heads x 2048: 32 -> 28); 128 heads x 192: 8.0 -> 8.5, left where it was;
+//    keys of 128 25 -> 17, with a mask 38 -> 20; 12 heads x 1000 of 64 causal 16.5 -> 9.2; 8 heads x 2048 causal 38 -> 23;
+//  - heads of 64: with up to 64 queries ahead at any count (512 heads x 16 x 2048 46 -> 41), else up to two per compute unit
+//    from 512 keys on (84 heads x 317 x 635 14.0 -> 12.6; 128 heads x 192 x 200 would go 8.0 -> 8.5). With a mask only one
+//    fits at a time (166 registers against 112), but so it is with the other kernel's larger tiles: from 512 keys on still
+//    ahead (512 heads x 16 x 2048 69 -> 53, 226 heads x 78 x 1452 39 -> 34, 128 heads x 200 x 2000 56 -> 42);
 //  - causal units differ in length and the longest start first, which balances more than one per unit where the units are
-//    long: heads of 128 up to two from 768 keys on (16 heads x 2048: 42 -> 32; 48 heads x 512: 16 -> 17), heads of 64 up to
-//    two from 256 and four from 768 keys on (24 heads x 2048: 41 -> 27; 48 heads x 1500: 28 -> 30);
+//    long: heads of 128 up to two from 768 keys on (16 heads x 2048: 40 -> 30; 48 heads x 512 would go 15 -> 16), heads of
+//    64 up to two from 256 and four from 768 keys on (24 heads x 2048: 39 -> 26; 35 heads x 1839: 30 -> 28);
 //  - from 4096 keys on causal heads stay with those kernels, whose result for a head is the same bits however many heads
 //    run beside it (one head alone against the benchmark's 128); 8 heads x 4096 would take 51 us here against 75;
 //  - beyond, the kernels whose waves share more queries do the same work with fewer copies and steps (128 heads x 1024 of

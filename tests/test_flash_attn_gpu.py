@@ -685,3 +685,23 @@ def test_attention_more_heads_than_a_grid_of_512_threads_holds(hexmi, with_mask)
         scores = scores + mask[pick].float()
     want = torch.softmax(scores, dim=-1) @ k[pick].float()
     assert (out[pick].float() - want).abs().max() <= 2e-2
+
+
+@pytest.mark.parametrize("case", [(9, 130, 300, 64, False), (11, 3, 4000, 128, False), (63, 300, 520, 64, False), (1, 700, 700, 64, True),
+                                  (9, 260, 260, 128, True), (35, 800, 800, 64, True), (16, 200, 200, 128, True)])
+def test_attention_head_counts_off_the_multiple_of_eight(hexmi, case):
+    # units are dealt to the 8 XCDs in parts of the list of all of them (causal: the last ZH % 8 heads apart): each must be
+    # visited exactly once, so the output starts as NaN. Bound: the parity tests'
+    B, Sq, Skv, D, causal = case
+    g = _gen(79)
+    q, k, v = (torch.randn(B, n, D, generator=g).half() for n in (Sq, Skv, Skv))
+    out = torch.full((B, Sq, D), float("nan"), dtype=torch.float32, device="cuda")
+    if causal:
+        hexmi.flash_attention(q[None].cuda(), k[None].cuda(), v[None].cuda(), None, True, out=out[None])
+    else:
+        hexmi.attention(q.cuda(), k.cuda(), v.cuda(), out=out)
+    scores = q.float() @ k.float().transpose(1, 2) / math.sqrt(D)
+    if causal:
+        scores = scores.masked_fill(torch.ones(Sq, Skv).triu(1).bool(), float("-inf"))
+    want = torch.softmax(scores, dim=-1) @ v.float()
+    assert (out.cpu() - want).abs().max() <= 5e-3
