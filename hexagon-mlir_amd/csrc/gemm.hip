@@ -1581,17 +1581,14 @@ int dispatch_gemm(const void* Av, const void* Bv, void* Cv, int64_t M, int64_t N
 #undef HEXMI_GEMV
     return launch_status();
   }
-  // Up to 64 rows: the weight stream of gemm_skinny.hip where its estimate is below that of the tiles, whose time is the
-  // walk of K by N / 128 workgroups and the weights, in microseconds on cold weights (16 / 32 / 64 rows against the tiles,
-  // N = K = 4096: 8.7 / 10.3 / 14 against 24; N = 4096, K = 11008: 20 / 25 / 34 against 57; N = 11008, K = 4096:
-  // 19 / 23 / 28 against 32 to 35; N = 50264, K = 768: 17 / 22 / 33 against 26.5).
+  // Up to 64 rows: the weight stream of gemm_skinny.hip, except for 33 rows and more against very many channels, where the
+  // tiles read the rows less often (plan_gemm_skinny; on cold weights, us for 16 / 32 / 64 rows against the tiles, N = K = 4096:
+  // 9.6 / 11 / 15 against 24; N = 4096, K = 11008: 20 / 25 / 34 against 57; N = 11008, K = 4096: 19 / 24 / 29 against 36).
   if (TRANS_B && M <= 64 && N >= 64 && K % 32 == 0 && lda % 8 == 0 && ldb % 8 == 0 && aligned_to(A, 16) &&
       aligned_to(B, 16)) {
-    const double tiles_us = std::max(23.0, 4.0 + 5.2e-3 * (double)K * (double)((N + 128 * 512 - 1) / (128 * 512)) +
-                                               (double)N * (double)K / 4.5e6);
     const GemmSkinnyPlan plan = plan_gemm_skinny(M, N, K);
-    if (plan.us < 0.95 * tiles_us)
-      return launch_gemm_skinny<T, OutT>(plan.channels, A, B, C, M, N, K, lda, ldb, ldc, s, bias, resid, ldr);
+    if (plan.channels > 0)
+      return launch_gemm_skinny<T, OutT>(plan, A, B, C, M, N, K, lda, ldb, ldc, s, bias, resid, ldr);
   }
   const bool fast = K % BK == 0 && lda % 8 == 0 && ldb % 8 == 0 && ldc % 4 == 0 && N % 8 == 0 && N >= 8 &&
                     aligned_to(A, 16) && aligned_to(B, 16) && aligned_to(C, 16) && (!bias || aligned_to(bias, run)) &&

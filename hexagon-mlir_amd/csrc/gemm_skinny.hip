@@ -10,7 +10,7 @@
 // the K walk) and reads the operands from there, chunk c of row r at c ^ ((r / 2) % 8). Cold weights, us, before -> now:
 //   N = 4096, K = 4096:   16 rows 11.8 -> 8.7, 32 rows 15.2 -> 10.3, 64 rows 23 -> 14
 //   N = 4096, K = 11008:  27.7 -> 19.7, 36 -> 24.6, 57 -> 33.7        N = 768, K = 3072: 9.3 -> 4.4, 12 -> 5.6, 18 -> 8.1
-//   N = 11008, K = 4096 (on the 128 x 128 tiles before): 31.7 -> 19, 32.4 -> 22.9, 35.2 -> 28.4
+//   N = 11008, K = 4096 (on the 128 x 128 tiles before): 31.7 -> 19, 32.4 -> 24.2, 35.2 -> 29.5
 // Three and four stages, and counted waits in place of the loop's full ones, measured equal.
 #include <algorithm>
 
@@ -166,29 +166,42 @@ void gemm_nt_skinny_kernel(const T* __restrict__ A, const T* __restrict__ W, Out
 
 }  // namespace
 
-// Channels per workgroup by what the busiest CU takes in: its workgroups times (channels + rows) of K elements at about
-// 42 GB/s (fitted on 256 CUs: 39 to 60 over the shapes above), and two microseconds between workgroups that do not share
-// a CU. Up to 16 rows 16 channels are ahead (N = 11008, K = 4096: 20.5 against 24.5 us with 32) until a CU has more than
-// eight workgroups of them (N = 50264, K = 768: 21.8 against 17.4); at 32 rows N = 4096 gives 10.3 / 14.2 / 18.7 us with
-// 16 / 32 / 64 channels, N = 11008 26.9 / 27.8 / 23.9, N = 50264 35.4 / 21.9 / 26.2; at 64 rows N = 11008 37.3 / 38.4 / 28.9.
+// Channels and waves of a workgroup, or none of them (the 128 x 128 tiles). Few groups of 16 channels and a long K want many
+// waves to a group, many groups or a short K few (a wave without a round costs its LDS and its part of the sum), rows the
+// wider groups that read them less often. The lines are where both sides cross over 6 row counts x 19 N x 19 K on 256 CUs,
+// cold weights; channels x waves in us:
+//   16 rows: N = 4096: K = 256 16x8 3.3, 16x2 3.2; K = 4096 9.7, 15.0. N = 16384, K = 512: 16x8 7.5, 16x2 5.7. N = 40000,
+//     K = 1024: 16x2 18.2, 32x4 16.5. N = 28672, K = 6144: 16x2 72, 16x8 66
+//   32 rows: N = 8192: K = 512 16x2 4.6, 32x4 4.6; K = 4096 19.1, 18.5. K = 2048: N = 11008 16x2 13.5, 32x2 14.7; N = 14336
+//     17.1, 15.9. N = 14336, K = 8192: 32x2 51, 64x4 47. N = 50264, K = 2048: 32x2 53, 32x4 48
+//   64 rows: N = 4096: K = 256 16x8 4.3, 16x4 4.0; K = 4096 14.8, 16.3. N = 8192, K = 4096: 32x4 22.9, 64x4 27.5. N = 11008:
+//     K = 256 16x2 5.7, 64x4 6.6; K = 4096 64x4 29, tiles 36. N = 32768: K = 512 64x4 16.5, tiles 12.0; K = 1024 24, 20
 GemmSkinnyPlan plan_gemm_skinny(int64_t M, int64_t N, int64_t K) {
-  const int64_t cus = std::max(1, hexmi_num_cus());
-  const int mt = M <= 16 ? 1 : (M <= 32 ? 2 : 4);
-  GemmSkinnyPlan best = {0, 0.0};
-  for (int nt = 1; nt <= (mt == 1 ? 2 : 4); nt *= 2) {
-    if (mt == 1 && (nt == 2) != (N > 16 * 8 * cus)) continue;
-    const int64_t groups = ((N + 16 * nt - 1) / (16 * nt) + cus - 1) / cus;
-    const bool shares = mt == 1 || (mt == 2 && nt == 2);          // 64 KiB of LDS or less
-    const double us = 1.0 + (double)groups * ((shares ? 0.4 : 2.0) + (double)(16 * (nt + mt)) * (double)K * 2.0 / 42.0e3);
-    if (best.channels == 0 || us < best.us) best = {16 * nt, us};
+  const int64_t cus = std::max(1, hexmi_num_cus()), groups = (N + 15) / 16;
+  if (M <= 16) {
+    if (K <= 256) return {16, 2};
+    if (groups <= 2 * cus) return {16, 8};
+    if (groups > 8 * cus && K >= 768) return {32, 4};
+    return {16, groups > 4 * cus && K >= 3072 ? 8 : 2};
   }
-  return best;
+  if (M <= 32) {
+    if (groups <= 5 * cus && K <= 256) return {16, 2};
+    if (groups <= cus) return {16, 8};
+    if (groups <= 2 * cus) return K < 768 ? GemmSkinnyPlan{16, 2} : GemmSkinnyPlan{32, 4};
+    if (groups <= 4 * cus && K >= 4096) return {64, 4};
+    if (groups <= 3 * cus) return {16, 2};
+    return {32, groups > 8 * cus && K >= 768 ? 4 : 2};
+  }
+  if (groups > 5 * cus || (groups > 4 * cus && K > 512)) return {0, 0};
+  if (groups <= cus) return {16, K <= 512 ? 4 : 8};
+  if (K <= 512) return groups <= 3 * cus ? GemmSkinnyPlan{16, 2} : GemmSkinnyPlan{32, 2};
+  return {groups <= 2 * cus ? 32 : 64, 4};
 }
 
 template <typename T, typename OutT>
-int launch_gemm_skinny(int channels, const T* A, const T* B, OutT* C, int64_t M, int64_t N, int64_t K, int64_t lda,
-                       int64_t ldb, int64_t ldc, hipStream_t s, const OutT* bias, const OutT* resid, int64_t ldr) {
-  const dim3 grid((unsigned)((N + channels - 1) / channels));
+int launch_gemm_skinny(const GemmSkinnyPlan& plan, const T* A, const T* B, OutT* C, int64_t M, int64_t N, int64_t K,
+                       int64_t lda, int64_t ldb, int64_t ldc, hipStream_t s, const OutT* bias, const OutT* resid, int64_t ldr) {
+  const dim3 grid((unsigned)((N + plan.channels - 1) / plan.channels));
   // Weights beyond 64 MB are gone from the 256 MB last-level cache when a program comes back to them. Non-temporal reads of
   // them gain 1 to 1.4 us of 21 to 36 (N = 4096, K = 11008) and cost as much where the weights stay (N = 768, K = 3072: 5.6 -> 7.8).
   const bool once = N * K > (int64_t)32 << 20;
@@ -202,19 +215,30 @@ int launch_gemm_skinny(int channels, const T* A, const T* B, OutT* C, int64_t M,
                          (int)N, (int)K, lda, ldb, ldc, bias, resid, ldr);                                                    \
   } while (0)
   if (M <= 16) {
-    if (channels == 16) HEXMI_SKINNY(1, 1, 8); else HEXMI_SKINNY(1, 2, 4);
+    if (plan.channels == 32) HEXMI_SKINNY(1, 2, 4);
+    else if (plan.waves == 8) HEXMI_SKINNY(1, 1, 8);
+    else HEXMI_SKINNY(1, 1, 2);
   } else if (M <= 32) {
-    if (channels == 16) HEXMI_SKINNY(2, 1, 8); else if (channels == 32) HEXMI_SKINNY(2, 2, 4); else HEXMI_SKINNY(2, 4, 4);
+    if (plan.channels == 64) HEXMI_SKINNY(2, 4, 4);
+    else if (plan.channels == 32 && plan.waves == 4) HEXMI_SKINNY(2, 2, 4);
+    else if (plan.channels == 32) HEXMI_SKINNY(2, 2, 2);
+    else if (plan.waves == 8) HEXMI_SKINNY(2, 1, 8);
+    else HEXMI_SKINNY(2, 1, 2);
   } else {
-    if (channels == 16) HEXMI_SKINNY(4, 1, 8); else if (channels == 32) HEXMI_SKINNY(4, 2, 4); else HEXMI_SKINNY(4, 4, 4);
+    if (plan.channels == 64) HEXMI_SKINNY(4, 4, 4);
+    else if (plan.channels == 32 && plan.waves == 4) HEXMI_SKINNY(4, 2, 4);
+    else if (plan.channels == 32) HEXMI_SKINNY(4, 2, 2);
+    else if (plan.waves == 8) HEXMI_SKINNY(4, 1, 8);
+    else if (plan.waves == 4) HEXMI_SKINNY(4, 1, 4);
+    else HEXMI_SKINNY(4, 1, 2);
   }
 #undef HEXMI_SKINNY
   return launch_status();
 }
 
 #define HEXMI_INSTANCE(T, OutT)                                                                                              \
-  template int launch_gemm_skinny<T, OutT>(int, const T*, const T*, OutT*, int64_t, int64_t, int64_t, int64_t, int64_t, \
-                                           int64_t, hipStream_t, const OutT*, const OutT*, int64_t);
+  template int launch_gemm_skinny<T, OutT>(const GemmSkinnyPlan&, const T*, const T*, OutT*, int64_t, int64_t, int64_t,   \
+                                           int64_t, int64_t, int64_t, hipStream_t, const OutT*, const OutT*, int64_t);
 HEXMI_INSTANCE(f16, f16)
 HEXMI_INSTANCE(f16, float)
 HEXMI_INSTANCE(bf16, bf16)

@@ -223,13 +223,13 @@ inline bool two_pass_sum(int64_t n, int64_t block) {
 // partials == nullptr: one pass; otherwise two_pass_sum(n, block) holds and partials has room for every run.
 int block_sum_any(const void* x, void* out, int64_t n, int64_t block, int dtype, float* partials, hipStream_t s);
 
-// Up to 64 rows against [N,K] weights (gemm_skinny.hip): output channels per workgroup and the estimated time, and the
-// launch. K % 32 == 0, operand rows on 16-byte boundaries; bias and residual may be null.
-struct GemmSkinnyPlan { int channels; double us; };
+// Up to 64 rows against [N,K] weights (gemm_skinny.hip): output channels and waves of a workgroup (0: leave it to the tiles),
+// and the launch. K % 32 == 0, operand rows on 16-byte boundaries; bias and residual may be null.
+struct GemmSkinnyPlan { int channels, waves; };
 GemmSkinnyPlan plan_gemm_skinny(int64_t M, int64_t N, int64_t K);
 template <typename T, typename OutT>
-int launch_gemm_skinny(int channels, const T* A, const T* B, OutT* C, int64_t M, int64_t N, int64_t K, int64_t lda,
-                       int64_t ldb, int64_t ldc, hipStream_t s, const OutT* bias, const OutT* resid, int64_t ldr);
+int launch_gemm_skinny(const GemmSkinnyPlan& plan, const T* A, const T* B, OutT* C, int64_t M, int64_t N, int64_t K,
+                       int64_t lda, int64_t ldb, int64_t ldc, hipStream_t s, const OutT* bias, const OutT* resid, int64_t ldr);
 
 // Tiled W8A16 GEMM for many activation rows (gemm.hip): C[M,N] = (A[M,K] * W[N,K]^T) * scales[N].
 int gemm_w8a16_tiled(int64_t M, int64_t N, int64_t K, const f16* A, const int8_t* W, const f16* scales, f16* C,

@@ -110,6 +110,26 @@ def test_gemm_few_rows_wide_workgroups(hexmi, dtype, M, N, K):
     assert close16(fused, (want + bias.double() + resid.double()).to(dtype), max_ulp=1, atol=2e-5 * float(mag.max()))
 
 
+# every (channels, waves) that plan_gemm_skinny picks on 256 CUs, at widths off the workgroup's, with K of a few rounds of 64,
+# fewer rounds than waves, and the last 32 of K on its own: 16x2, 16x8, 32x4 (16 rows); 16x2, 16x8, 32x2, 32x4, 64x4 (32
+# rows); 16x4, 16x8, 16x2, 32x2, 32x4, 64x4 and the tiles (64 rows)
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("M,N,K", [(5, 401, 160), (16, 8195, 480), (16, 401, 736), (3, 33001, 800), (12, 16501, 3104),
+                                   (17, 10003, 96), (32, 8999, 992), (25, 77, 1056), (32, 14007, 544), (20, 5003, 800),
+                                   (31, 14005, 4128), (32, 33003, 800),
+                                   (33, 100, 480), (64, 333, 1056), (47, 9001, 160), (64, 17003, 224), (50, 7001, 544),
+                                   (64, 12005, 544), (64, 20500, 96)])
+def test_gemm_few_rows_every_workgroup_shape(hexmi, dtype, M, N, K):
+    a, b = _inputs(M, N, K, dtype, True, seed=M + N)
+    want, mag = a.double() @ b.double().t(), a.double().abs() @ b.double().t().abs()
+    out = torch.full((M + 1, N), float("nan"), dtype=torch.float32, device="cuda")
+    hexmi.matmul(a.cuda(), b.cuda(), out=out[:M], trans_b=True)
+    got = out.cpu()
+    # fp32 products summed in parts: K roundings of at most 2^-24 of the magnitude, far fewer in effect
+    assert ((got[:M].double() - want).abs() <= 1e-5 * mag + 1e-30).all()
+    assert torch.isnan(got[M]).all()
+
+
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("M", [1, 2, 3, 4])
 @pytest.mark.parametrize("N,K", [(64, 8), (104, 64), (4096, 2048), (1000, 2056), (256, 4096), (136, 11008)])
