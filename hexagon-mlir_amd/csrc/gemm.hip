@@ -1481,10 +1481,17 @@ int launch_f32(bool trans_b, const void* A, const void* B, void* C, int64_t M, i
 
 // 128 x 128 tiles: four LDS stages (128 KiB, one workgroup per CU) hide the copies of a tile's short slabs, two (64 KiB)
 // let two workgroups share a CU, one's first copies and last stores under the other's MFMAs and no round of its own for
-// what the first round leaves over. With a tile or less per CU four are ahead (us, four / two: 172 tiles of K = 4096
-// 37.6 / 53.4, 256 of 2048 20.3 / 26.4, 96 of 768 11.1 / 13.2), with more two (288 tiles of K = 768 with bias 19.8 / 14.7, 384
-// of 768 20.5 / 15.4, 344 of 4096 67.5 / 61.3, 480 of 3072 50.4 / 46.0, 1024 of 4096 132 / 126, 1536 of 768 65.5 / 47.7).
-inline bool two_per_cu(int64_t tiles) { return tiles > hexmi_num_cus(); }
+// what the first round leaves over. With a tile or less per CU four are ahead (16-bit operands, us, four / two: 172 tiles of
+// K = 4096 37.6 / 53.4, 256 of 2048 20.3 / 26.4, 96 of 768 11.1 / 13.2), with more two (288 tiles of K = 768 with bias
+// 19.8 / 14.7, 384 of 768 20.5 / 15.4, 344 of 4096 67.5 / 61.3, 480 of 3072 50.4 / 46.0, 1024 of 4096 132 / 126, 1536 of 768
+// 65.5 / 47.7) -- unless the rounds of two leave a tile or less per CU over and K is long: such a tile runs alone on its CU,
+// at the pace of 172 tiles above, which a round of two that came before makes good up to K of about 1536 (580 tiles: K = 1088
+// 40.8 / 35.4, 2304 57.6 / 61.8, 4352 102 / 114, 7872 177 / 212; 1140 tiles: K = 2688 121 / 109, 3840 149 / 152, 5824 233 / 254).
+// int8 weights: 300 tiles of K = 11968 202 / 181, 428 of 3840 61.6 / 56.3, 468 of 256 12.2 / 9.6.
+inline bool two_per_cu(int64_t tiles, int64_t K) {
+  const int64_t cus = hexmi_num_cus(), pairs = tiles / (2 * cus), over = tiles % (2 * cus);
+  return tiles > cus && (pairs == 0 || over == 0 || over > cus || K < 1536 * pairs);
+}
 
 // out_elems: 16-bit results leave the paired-slab kernel one element per lane (the caller has checked that this
 // kernel takes the product: K % 64 == 0, short rows, no bias or residual).
@@ -1504,7 +1511,7 @@ int launch_tiled(const T* A, const T* B, OutT* C, int64_t M, int64_t N, int64_t 
 #define HEXMI_K64_TAIL(NS, EPI) \
   do { if ((K / BK2) % NS == 0) HEXMI_K64(false, NS, EPI); else HEXMI_K64(true, NS, EPI); } while (0)
     if constexpr (WM == 2 && WN == 2) {
-      const bool two = two_per_cu((int64_t)tiles_m * tiles_n);
+      const bool two = two_per_cu((int64_t)tiles_m * tiles_n, K);
       if (bias || resid) {                          // the instantiations that carry the epilogue operands
         if (two) HEXMI_K64_TAIL(2, true); else HEXMI_K64_TAIL(4, true);
       } else {
@@ -1648,7 +1655,7 @@ int launch_w8a16(const f16* A, const int8_t* W, const f16* scales, f16* C, int64
                      static_cast<const void*>(W), C, (int)M, (int)N, (int)K, K, K, N, tiles_m, tiles_n, scales)
 #define HEXMI_K64_TAIL(NS) do { if ((K / BK2) % NS == 0) HEXMI_K64(false, NS); else HEXMI_K64(true, NS); } while (0)
     if constexpr (WM <= 2) {
-      if (two_per_cu((int64_t)tiles_m * tiles_n)) HEXMI_K64_TAIL(2); else HEXMI_K64_TAIL(4);
+      if (two_per_cu((int64_t)tiles_m * tiles_n, K)) HEXMI_K64_TAIL(2); else HEXMI_K64_TAIL(4);
     } else {
       HEXMI_K64_TAIL(2);
     }

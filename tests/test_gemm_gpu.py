@@ -171,6 +171,20 @@ def test_gemm_two_small_tiles_per_cu(hexmi, dtype, trans_b, K):
         assert close16(fused, (want + bias.double() + resid.double()).to(dtype), max_ulp=1, atol=2e-5 * mag)
 
 
+@pytest.mark.parametrize("trans_b", [False, True])
+@pytest.mark.parametrize("K", [1472, 1536, 1600])
+def test_gemm_tiles_left_over_after_a_round_of_two_per_cu(hexmi, trans_b, K):
+    # 8 x 70 tiles of 128 x 128 with epilogue operands: two stages below K = 1536, four from there on
+    M, N, dtype = 1000, 8896, torch.float16
+    a, b = _inputs(M, N, K, dtype, trans_b, seed=K)
+    bt = b.double().t() if trans_b else b.double()
+    g = _gen(K)
+    bias = torch.randn(N, generator=g).to(dtype)
+    want, mag = a.double() @ bt + bias.double(), float((a.double().abs() @ bt.abs()).max())
+    got = hexmi.matmul(a.cuda(), b.cuda(), trans_b=trans_b, bias=bias.cuda()).cpu()
+    assert close16(got, want.to(dtype), max_ulp=1, atol=2e-5 * mag)
+
+
 def test_gemm_closed_forms(hexmi):
     g = _gen(1)
     a = torch.randn(256, 128, generator=g).half()
