@@ -228,6 +228,20 @@ def test_w8a16_many_rows(hexmi, M, N, K):
     assert (got[rows].double() - want).abs().max() / math.sqrt(K) <= 2e-2
 
 
+@pytest.mark.parametrize("M,N,K", [(390, 9592, 64), (512, 8200, 128), (400, 9600, 192), (300, 12808, 448), (385, 9592, 1088)])
+def test_w8a16_two_small_tiles_per_cu(hexmi, M, N, K):
+    # more 128 x 128 tiles than CUs and too few of 256 x 256: the two-stage form, two workgroups a CU; one slab, whole and
+    # guarded last passes, ragged rows and columns. Outputs of this size need a bound in units of the accumulated magnitude
+    a, w, s = _inputs(M, N, K, seed=M + K)
+    out = torch.full((M + 1, N), float("nan"), dtype=torch.float16, device="cuda")
+    hexmi.w8a16_matmul(a.cuda(), w.cuda(), s.cuda(), out=out[:M])
+    got = out.cpu()
+    want = (a.double() @ w.double().t()) * s.double()
+    mag = float(((a.double().abs() @ w.double().abs().t()) * s.double()).max())
+    assert close16(got[:M], want.half(), max_ulp=1, atol=1e-5 * mag)
+    assert torch.isnan(got[M]).all()
+
+
 def test_w8a16_errors(hexmi):
     a = torch.zeros(2, 64, dtype=torch.float16)
     with pytest.raises(TypeError):
