@@ -1543,12 +1543,13 @@ int launch_tiled(const T* A, const T* B, OutT* C, int64_t M, int64_t N, int64_t 
 }
 
 // 256 x 256 or 128 x 128 tiles. A launch is whole rounds over the CUs and the last round may be nearly empty. With every
-// round full the large tiles run about 1.2 to 1.3 times the rate of the small ones, two of which share a CU there
-// (fp16 K = 4096: 1.34 against 1.09 PFLOP/s; three rounds at K = 1024: 1.10 against 0.94), and a round
-// that is not full runs its tiles somewhat faster: the large tiles are taken when 1.48 times the fill of their
-// rounds is at least the fill of the small tiles' rounds. (fp16, K = 4096, 256 CUs: 128 large tiles 825 TFLOP/s
-// against 1074 with small ones, 289 tiles 920 against 1019, 192 tiles 1152 against 1077, 324 tiles 1020 against 965;
-// int8 weights, N = 11008: M = 512 518 against 680, M = 768 739 against 687.)
+// round full the large tiles run about 1.2 times the rate of the small ones (two_per_cu above), and a round that is not
+// full runs its tiles somewhat faster: the large tiles are taken when 1.48 times the fill of their rounds is at least the
+// fill of the small tiles' rounds, counted one per CU. (256 CUs, K = 4096, us, large / small: fp16 128 large tiles 77 / 60, 144
+// 80 / 85, 192 85 / 93, 256 97 / 117, 289 167 / 146, 320 166 / 151, 324 167 / 160, 384 168 / 172, 512 191 / 233; K = 1024: 128
+// 26 / 20, 192 28 / 31, 289 54 / 46, 384 55 / 53, 512 65 / 70. int8 weights, N = 11008, K = 4096: M = 512 88 / 55, M = 768
+// 87 / 95, M = 1536 183 / 168, M = 2048 182 / 167. From 324 to 384 large tiles, and with int8 weights at K = 1024, the small
+// tiles are up to 17 % ahead where this line takes the large ones.)
 inline bool prefer_large_tiles(int64_t M, int64_t N) {
   const int64_t cus = hexmi_num_cus();
   if (cus <= 0) return false;
