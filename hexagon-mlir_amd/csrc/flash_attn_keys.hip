@@ -136,8 +136,7 @@ void flash_keys_kernel(const T* __restrict__ Q, const T* __restrict__ K, const T
   }
   const int key_end = CAUSAL ? ((qb + 1) * kRows < S ? (qb + 1) * kRows : S) : Skv;
   const int unit_steps = (key_end + kStepKeys - 1) / kStepKeys;
-  const int first = split * chunk;
-  if (first >= unit_steps) return;                      // a short causal unit has fewer chunks than the longest one
+  const int first = split * chunk;                      // causal units are never cut
   const int last = first + chunk < unit_steps ? first + chunk : unit_steps;
 
   const T* k_g = K + (int64_t)zh * Skv * dh;
@@ -412,7 +411,7 @@ void flash_keys_kernel(const T* __restrict__ Q, const T* __restrict__ K, const T
   }
   __syncthreads();
   const int64_t rows = (int64_t)ZH * S, row = (int64_t)zh * S + qrow;
-  const bool whole = chunk >= unit_steps;
+  const bool whole = CAUSAL || splits == 1;
   const float inv_l = 1.0f / l;
 #pragma unroll
   for (int i = 0; i < kGroups; ++i) {
@@ -444,31 +443,24 @@ void flash_keys_kernel(const T* __restrict__ Q, const T* __restrict__ K, const T
 
 // The chunks of a row added up: O = sum_s 2^(u (m_s - m)) o_s / sum_s 2^(u (m_s - m)) l_s with m the largest m_s and u the
 // log2 units of an m_s (kUnit of the kernel that wrote them). A thread
-// takes four columns; rows of units that were one chunk are already in O. Bound by reading the sums, which have just
-// been written and come from L2 / Infinity Cache.
-template <typename OutT, int D, bool CAUSAL>
+// takes four columns. Bound by reading the sums, which have just been written and come from L2 / Infinity Cache.
+template <typename OutT, int D>
 __global__ __launch_bounds__(256)
-void flash_merge_kernel(const float* __restrict__ part, OutT* __restrict__ O, int64_t rows, int S, int chunk, int splits,
-                        int head_dim, float unit) {
+void flash_merge_kernel(const float* __restrict__ part, OutT* __restrict__ O, int64_t rows, int splits, int head_dim,
+                        float unit) {
   constexpr int TPR = D / 4;                               // threads per row
   const int64_t row = (int64_t)blockIdx.x * (256 / TPR) + threadIdx.x / TPR;
   if (row >= rows) return;
-  int n = splits;
-  if constexpr (CAUSAL) {
-    const int end = ((int)(row % S) / kRows + 1) * kRows;
-    n = (((end < S ? end : S) + kStepKeys - 1) / kStepKeys + chunk - 1) / chunk;
-  }
-  if (n <= 1) return;
   const float* ml = part + (int64_t)splits * rows * D;
   float m = -INFINITY;
-  for (int s = 0; s < n; ++s) m = fmaxf(m, ml[((int64_t)s * rows + row) * 2]);
+  for (int s = 0; s < splits; ++s) m = fmaxf(m, ml[((int64_t)s * rows + row) * 2]);
   const float base = m == -INFINITY ? 0.0f : -m;           // every key of the row masked out: l stays 0, the result NaN
   const int d = threadIdx.x % TPR * 4;
   if (d >= head_dim) return;                               // padded heads
   f32x4 o = {0.0f, 0.0f, 0.0f, 0.0f};
   float l = 0.0f;
 #pragma unroll 4
-  for (int s = 0; s < n; ++s) {
+  for (int s = 0; s < splits; ++s) {
     const f32x2 v = *reinterpret_cast<const f32x2*>(ml + ((int64_t)s * rows + row) * 2);
     const f32x4 x = *reinterpret_cast<const f32x4*>(part + ((int64_t)s * rows + row) * D + d);
     const float w = __builtin_amdgcn_exp2f((v[0] + base) * unit);
@@ -503,14 +495,9 @@ int launch_keys(const void* Q, const void* K, const void* V, const void* mask, v
     else HEXMI_KEYS(false, false, false, false);
   }
 #undef HEXMI_KEYS
-  if (plan.splits > 1) {
-    if (causal)
-      hipLaunchKernelGGL((flash_merge_kernel<OutT, D, true>), dim3((unsigned)merge_blocks), dim3(256), 0, st, part,
-                         static_cast<OutT*>(O), rows, (int)S, plan.chunk, plan.splits, head_dim, unit);
-    else
-      hipLaunchKernelGGL((flash_merge_kernel<OutT, D, false>), dim3((unsigned)merge_blocks), dim3(256), 0, st, part,
-                         static_cast<OutT*>(O), rows, (int)S, plan.chunk, plan.splits, head_dim, unit);
-  }
+  if (plan.splits > 1)
+    hipLaunchKernelGGL((flash_merge_kernel<OutT, D>), dim3((unsigned)merge_blocks), dim3(256), 0, st, part,
+                       static_cast<OutT*>(O), rows, plan.splits, head_dim, unit);
   return launch_status();
 }
 
@@ -553,7 +540,7 @@ FlashKeysPlan plan_flash_keys(int64_t ZH, int64_t S, int64_t Skv, int64_t D, boo
   p.chunk = (int)steps;
   p.splits = 1;
   // self-attention without a mask is the entry point without a workspace, and gives its bits
-  may_split = may_split && (masked || S != Skv);
+  may_split = may_split && !causal && (masked || S != Skv);
   const double step_us = D == 128 ? 1.2 : 0.8, sums_us = 8.0 * (double)(ZH * S * D) / 4e6;
   double best = step_us * (double)steps;
   for (int64_t n = 2; may_split && n <= 32 && n <= steps && n * units <= cus; ++n) {
