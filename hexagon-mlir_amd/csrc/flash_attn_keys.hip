@@ -520,7 +520,7 @@ int launch_keys(const void* Q, const void* K, const void* V, const void* mask, v
 //  - beyond, the kernels whose waves share more queries do the same work with fewer copies and steps (128 heads x 1024 of
 //    128: 80 -> 113).
 // Chunks only where half the compute units would stay idle: a merge costs its launch (4 us, and 3 of the host's) and
-// the fp32 sums, a step (128 keys) about 1.2 us with heads of 128 and 0.8 with heads of 64 (8 heads x 1 x 8192: 65 us in
+// the fp32 sums (never worth it up to 768 keys), a step (128 keys) about 1.2 us with heads of 128 and 0.8 with heads of 64 (8 heads x 1 x 8192: 65 us in
 // one chunk, 15 in 16; 32 heads x 200 x 2000 of 64: 20.5 and 17.5 in two).
 FlashKeysPlan plan_flash_keys(int64_t ZH, int64_t S, int64_t Skv, int64_t D, bool causal, bool masked, bool any_mask,
                               bool may_split) {
@@ -540,7 +540,7 @@ FlashKeysPlan plan_flash_keys(int64_t ZH, int64_t S, int64_t Skv, int64_t D, boo
   p.chunk = (int)steps;
   p.splits = 1;
   // self-attention without a mask is the entry point without a workspace, and gives its bits
-  may_split = may_split && !causal && (masked || S != Skv);
+  may_split = may_split && !causal && (masked || S != Skv) && Skv > HEXMI_ATTENTION_ONE_LAUNCH_KEYS;
   const double step_us = D == 128 ? 1.2 : 0.8, sums_us = 8.0 * (double)(ZH * S * D) / 4e6;
   double best = step_us * (double)steps;
   for (int64_t n = 2; may_split && n <= 32 && n <= steps && n * units <= cus; ++n) {

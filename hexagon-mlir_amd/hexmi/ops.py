@@ -209,8 +209,9 @@ def _attention_impl(q, k, v, mask, sm_scale, out):
     Skv = k.shape[1]
     with _on(q.device):
         # few queries over many keys: the keys are cut over several workgroups when the library is handed scratch for
-        # their fp32 sums; over 768 keys and fewer a merge takes longer than it saves and the question itself costs 0.9 us
-        need = _lib.lib().hexmi_attention_workspace(B, Sq, Skv, D, 0 if mask is None else 1, _dt(q)) if Skv > 768 else 0
+        # their fp32 sums; the question costs 0.9 us and is not asked where the answer is always none
+        need = (_lib.lib().hexmi_attention_workspace(B, Sq, Skv, D, 0 if mask is None else 1, _dt(q))
+                if Skv > _lib.ATTENTION_ONE_LAUNCH_KEYS else 0)
         ws = torch.empty(need, dtype=torch.uint8, device=q.device) if need else None
         _lib.check(_lib.lib().hexmi_attention_ws(_p(q), _p(k), _p(v), _p(mask), _p(out), B, Sq, Skv, D, sm_scale,
                                                  _dt(q), _dt(out), _p(ws), need, _stream()), "hexmi_attention_ws")

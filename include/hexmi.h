@@ -356,10 +356,12 @@ int hexmi_attention(const void *Q, const void *K, const void *V,
  * test/python/triton/test_flash_attention.py:61-87).
  * hexmi_attention_workspace returns the bytes that takes for these sizes on the
  * current device, 0 when the one-launch kernels run anyway (self-attention
- * without a mask always does). workspace may be NULL (one
+ * without a mask and seq_kv up to HEXMI_ATTENTION_ONE_LAUNCH_KEYS always do,
+ * so a caller need not ask there). workspace may be NULL (one
  * launch whatever the sizes); one that is smaller than the query's answer or not
  * 16-byte aligned is HEXMI_EINVAL. It needs no initialisation and holds no state
  * between calls; two calls that overlap in time need a workspace each. */
+#define HEXMI_ATTENTION_ONE_LAUNCH_KEYS 768
 int64_t hexmi_attention_workspace(int64_t batch, int64_t seq_q, int64_t seq_kv,
                                   int64_t head_dim, int has_mask, int in_dtype);
 int hexmi_attention_ws(const void *Q, const void *K, const void *V,

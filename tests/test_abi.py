@@ -43,6 +43,12 @@ def test_loader_binds_exactly_the_header():
     assert "invalid" in _lib.strerror(_lib.EINVAL)
 
 
+def test_loader_knows_the_header_limit_of_one_launch_attention():
+    from hexmi import _lib
+    text = open(HEADER).read()
+    assert int(re.search(r"#define HEXMI_ATTENTION_ONE_LAUNCH_KEYS (\d+)", text).group(1)) == _lib.ATTENTION_ONE_LAUNCH_KEYS
+
+
 def test_argument_errors_need_no_device():
     from hexmi import _lib
     lib = _lib.lib()

@@ -564,6 +564,7 @@ def test_attention_workspace(hexmi):
     mask[2] = float("-inf")
     need = lib.hexmi_attention_workspace(B, Sq, Skv, D, 1, _lib.F16)
     assert need > 0 and lib.hexmi_attention_workspace(4096, 2048, 2048, 128, 1, _lib.F16) == 0
+    assert lib.hexmi_attention_workspace(1, 1, _lib.ATTENTION_ONE_LAUNCH_KEYS, 128, 1, _lib.F16) == 0
     assert lib.hexmi_attention_workspace(B, Sq, Skv, D, 1, _lib.F32) == 0
     ws = torch.empty(need, dtype=torch.uint8, device="cuda")
     outs = [torch.zeros(B, Sq, D, dtype=torch.float16, device="cuda") for _ in range(2)]
