@@ -58,8 +58,8 @@ def test_attention_parity_half(hexmi, oracle, case, dtype, causal):
 @pytest.mark.parametrize("case", [(1, 2, 300, 80), (2, 1, 129, 96), (1, 3, 64, 32), (1, 1, 513, 8), (2, 8, 200, 48),
                                   (1, 1, 1000, 120), (1, 2, 77, 16), (1, 1, 260, 112), (1, 16, 384, 40), (1, 1, 1, 72)])
 def test_attention_other_head_sizes(hexmi, oracle, case, dtype, causal):
-    # head sizes below 128 in multiples of 8 run the matrix-core kernel for 64 or 128 on tiles padded with zero
-    # columns; the output buffer starts as NaN and has one row more than the result, which must stay as it is
+    # head sizes below 128 in multiples of 8 run on tiles for 64 or 128 padded with zero columns (up to 64 keys the
+    # 128-query kernel, these few heads beyond that the key-group kernel; the former with more: MANY_UNIT_CASES); the output buffer starts as NaN and has one row more than the result, which must stay as it is
     Z, H, S, D = case
     q, k, v = _qkv(Z, H, S, D, dtype, seed=D + S)
     scale = 1.0 / math.sqrt(D)
@@ -98,15 +98,16 @@ def test_attention_head_sizes_up_to_256(hexmi, oracle, case, dtype, causal):
 def test_attention_padded_head_equals_the_zero_padded_problem(hexmi):
     # head size 80 on the kernel for 128 is the 128-wide problem with 48 zero columns in Q, K and V (and 1/sqrt(80)):
     # the same kernel, the same arithmetic -- bit for bit
-    Z, H, S, D = 2, 8, 700, 80
-    q, k, v = _qkv(Z, H, S, D, torch.float16, seed=31)
-    scale = 1.0 / math.sqrt(D)
-    for causal in (False, True):
-        got = hexmi.flash_attention(q.cuda(), k.cuda(), v.cuda(), scale, causal).cpu()
-        qp, kp, vp = (torch.nn.functional.pad(t, (0, 48)) for t in (q, k, v))
-        want = hexmi.flash_attention(qp.cuda(), kp.cuda(), vp.cuda(), scale, causal).cpu()
-        assert torch.equal(got, want[..., :D])
-        assert (want[..., D:] == 0).all()
+    D = 80                                               # 176 units of 64 queries: key groups; 700: the 128-query kernel
+    for Z, H, S in ((2, 8, 700), (4, 35, 260)):
+        q, k, v = _qkv(Z, H, S, D, torch.float16, seed=31)
+        scale = 1.0 / math.sqrt(D)
+        for causal in (False, True):
+            got = hexmi.flash_attention(q.cuda(), k.cuda(), v.cuda(), scale, causal).cpu()
+            qp, kp, vp = (torch.nn.functional.pad(t, (0, 48)) for t in (q, k, v))
+            want = hexmi.flash_attention(qp.cuda(), kp.cuda(), vp.cuda(), scale, causal).cpu()
+            assert torch.equal(got, want[..., :D])
+            assert (want[..., D:] == 0).all()
     # and head size 192 is the 256-wide problem with 64 zero columns (both on the two-halves form)
     q, k, v = _qkv(1, 8, 400, 192, torch.float16, seed=32)
     scale = 1.0 / math.sqrt(192)
@@ -289,12 +290,12 @@ def _mask(B, Sq, Skv, dtype, seed, drop=0.3):
 
 MASKED_CASES = [(2, 128, 128, 128), (3, 200, 72, 64), (1, 1, 64, 128), (2, 77, 516, 128), (1, 300, 4, 64),
                 (1, 130, 1024, 128), (2, 65, 66, 64), (1, 40, 100, 80),   # the last two: Skv % 4 != 0 / other D
-                # more than 128 queries and Skv % 8 == 0: mask tiles staged through LDS by 256-row workgroups
-                # (ragged last row block, ragged last key block, several row blocks, many batch entries)
+                # more than 128 queries and Skv % 8 == 0 in few units of 64 queries: the key-group kernel (the mask tiles
+                # that 256-row workgroups stage through LDS: MANY_UNIT_CASES)
                 (3, 300, 520, 128), (2, 513, 72, 64), (1, 257, 2048 + 8, 128), (40, 129, 136, 64),
-                # head sizes below 128 in multiples of 8: the 128-row kernel on tiles padded with zero columns
+                # head sizes below 128 in multiples of 8: tiles padded with zero columns
                 (2, 200, 72, 80), (1, 300, 520, 96), (3, 129, 136, 32), (1, 77, 516, 40), (2, 64, 64, 112),
-                # key counts that are not multiples of 4 (matrix-core kernel without a mask, row-wise with one)
+                # key counts that are not multiples of 4
                 (4, 1024, 77, 64), (2, 300, 1, 128), (1, 129, 515, 80)]
 
 
@@ -315,6 +316,70 @@ def test_masked_attention_parity_half(hexmi, oracle, case, dtype, with_mask):
     got32 = hexmi.attention(q.cuda(), k.cuda(), v.cuda(), None if mask is None else mask.cuda(),
                             out_dtype=torch.float32).cpu()
     assert (got32 - want).abs().max() <= (5e-3 if dtype == torch.float16 else 3e-2)
+
+
+# more units of 64 queries than the key-group kernel takes, so the 128-query kernels: masks staged through LDS (several key
+# blocks, a ragged last one, ragged rows), read in runs of four keys, no mask with an odd key count; heads of 64 and 128
+# and padded ones
+MANY_UNIT_CASES = [(100, 200, 520, 128, True), (150, 260, 712, 64, True), (100, 200, 516, 128, True), (150, 260, 524, 64, True),
+                   (100, 200, 520, 80, True), (150, 260, 516, 40, True), (100, 200, 515, 128, False), (150, 260, 77, 64, False),
+                   (100, 200, 333, 96, False), (150, 260, 515, 24, False)]
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("case", MANY_UNIT_CASES)
+def test_attention_of_many_units(hexmi, case, dtype):
+    # the bound of the parity tests (fp32 output, probabilities rounded to 16 bits)
+    B, Sq, Skv, D, with_mask = case
+    g = _gen(67)
+    q = torch.randn(B, Sq, D, generator=g).to(dtype)
+    k, v = torch.randn(B, Skv, D, generator=g).to(dtype), torch.randn(B, Skv, D, generator=g).to(dtype)
+    mask = _mask(B, Sq, Skv, dtype, 68) if with_mask else None
+    scores = q.float() @ k.float().transpose(1, 2) / math.sqrt(D)
+    if with_mask:
+        scores = scores + mask.float()
+    want = torch.softmax(scores, dim=-1) @ v.float()
+    buf = torch.full((B * Sq + 1, D), float("nan"), dtype=torch.float32, device="cuda")
+    hexmi.attention(q.cuda(), k.cuda(), v.cuda(), None if mask is None else mask.cuda(), out=buf[:B * Sq].view(B, Sq, D))
+    got = buf.cpu()
+    assert (got[:B * Sq].view(B, Sq, D) - want).abs().max() <= (5e-3 if dtype == torch.float16 else 3e-2)
+    assert torch.isnan(got[B * Sq]).all()
+
+
+def test_attention_workspace_under_capture_and_on_two_streams(hexmi):
+    # few queries over many keys: hexmi.attention hands the library scratch for the chunks' sums. Captured, the scratch is
+    # the graph's own and every replay must match the eager call; on two streams at once each call has its own
+    B, Skv, D = 4, 4096, 128
+    g = _gen(70)
+    k, v = (torch.randn(B, Skv, D, generator=g).half().cuda() for _ in range(2))
+    mask = torch.zeros(B, 2, Skv, dtype=torch.float16, device="cuda")
+    mask[:, :, :700] = float("-inf")
+    q = torch.randn(B, 2, D, generator=g).half().cuda()
+    out = torch.zeros(B, 2, D, dtype=torch.float16, device="cuda")
+    hexmi.attention(q, k, v, mask, out=out)                              # warm-up outside the capture
+    torch.cuda.synchronize()
+    stream, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    with torch.cuda.stream(stream):
+        with torch.cuda.graph(graph, stream=stream):
+            hexmi.attention(q, k, v, mask, out=out)
+    for _ in range(3):
+        q.copy_(torch.randn(B, 2, D, generator=g).half().cuda())
+        eager = hexmi.attention(q, k, v, mask)
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, eager)
+    qs = [torch.randn(B, 2, D, generator=g).half().cuda() for _ in range(2)]
+    want = [hexmi.attention(x, k, v, mask) for x in qs]
+    streams, outs = [torch.cuda.Stream(), torch.cuda.Stream()], [[], []]
+    torch.cuda.synchronize()
+    for _ in range(20):
+        for i in range(2):
+            with torch.cuda.stream(streams[i]):
+                outs[i].append(hexmi.attention(qs[i], k, v, mask))
+    torch.cuda.synchronize()
+    for i in range(2):
+        assert all(torch.equal(o, want[i]) for o in outs[i])
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
