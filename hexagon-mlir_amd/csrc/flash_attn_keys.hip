@@ -515,8 +515,8 @@ int launch_keys(const void* Q, const void* K, const void* V, const void* mask, v
 //  - causal units differ in length and the longest start first, which balances more than one per unit where the units are
 //    long: heads of 128 up to two from 768 keys on (16 heads x 2048: 40 -> 30; 48 heads x 512 would go 15 -> 16), heads of
 //    64 up to two from 256 and four from 768 keys on (24 heads x 2048: 39 -> 26; 35 heads x 1839: 30 -> 28);
-//  - from 4096 keys on causal heads stay with those kernels, whose result for a head is the same bits however many heads
-//    run beside it (one head alone against the benchmark's 128); 8 heads x 4096 would take 51 us here against 75;
+//  - causal heads of 4096 queries and more stay with those kernels whatever is faster: hexmi.h promises their callers the
+//    same bits at any number of heads, which a choice by units cannot give (8 heads x 4095: 51 us here, x 4096: 73 there);
 //  - beyond, the kernels whose waves share more queries do the same work with fewer copies and steps (128 heads x 1024 of
 //    128: 80 -> 113).
 // Chunks only where half the compute units would stay idle: a merge costs its launch (4 us, and 3 of the host's) and

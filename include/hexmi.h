@@ -315,7 +315,11 @@ int hexmi_gemm_w8a16_packed(int64_t M, int64_t N, int64_t K, const void *A,
  * multiples of 8 run them on zero-padded tiles (above 128 as two halves);
  * anything else a slow row-wise kernel (D <= 256).
  * out_dtype: in_dtype, or HEXMI_F32 with fp16 inputs (the fp16 QKV -> fp32 O
- * form of test/python/mlir/hexkl_attention/input.mlir:1-169). */
+ * form of test/python/mlir/hexkl_attention/input.mlir:1-169).
+ * The kernel is chosen by the sizes, Z * H among them: a head's result may
+ * differ in its last bits with the number of heads beside it. Causal 16-bit
+ * attention over 4096 queries and more is held to the same bits at any
+ * number of heads. */
 int hexmi_flash_attn_fwd(const void *Q, const void *K, const void *V, void *O,
                          int64_t Z, int64_t H, int64_t S, int64_t D,
                          float sm_scale, int causal, int in_dtype,

@@ -346,6 +346,22 @@ def test_attention_of_many_units(hexmi, case, dtype):
     assert torch.isnan(got[B * Sq]).all()
 
 
+@pytest.mark.parametrize("H,S,D,dtype,same_bits", [(40, 4100, 64, torch.bfloat16, True), (12, 4608, 96, torch.float16, True),
+                                                   (20, 5000, 128, torch.float16, True), (17, 2048, 128, torch.float16, False),
+                                                   (120, 300, 64, torch.float16, False)])
+def test_causal_head_beside_others(hexmi, H, S, D, dtype, same_bits):
+    # one head alone against the same head among H: the same bits from 4096 queries on; below, another kernel may run it,
+    # whose 16-bit probabilities and result round apart (fp16: a result below 4 in units of 2^-9 at most, so 2^-8)
+    q, k, v = _qkv(1, H, S, D, dtype, seed=69)
+    many = hexmi.flash_attention(q.cuda(), k.cuda(), v.cuda(), None, True).cpu()
+    for h in (0, H // 2, H - 1):
+        one = hexmi.flash_attention(*(t[:, h:h + 1].contiguous().cuda() for t in (q, k, v)), None, True).cpu()
+        if same_bits:
+            assert torch.equal(one[0, 0], many[0, h])
+        else:
+            assert (one[0, 0].float() - many[0, h].float()).abs().max() <= 2.0 ** -8
+
+
 def test_attention_workspace_under_capture_and_on_two_streams(hexmi):
     # few queries over many keys: hexmi.attention hands the library scratch for the chunks' sums. Captured, the scratch is
     # the graph's own and every replay must match the eager call; on two streams at once each call has its own
