@@ -1589,18 +1589,18 @@ int dispatch_gemm(const void* Av, const void* Bv, void* Cv, int64_t M, int64_t N
 #undef HEXMI_GEMV
     return launch_status();
   }
+  const bool fast = K % BK == 0 && lda % 8 == 0 && ldb % 8 == 0 && ldc % 4 == 0 && N % 8 == 0 && N >= 8 &&
+                    aligned_to(A, 16) && aligned_to(B, 16) && aligned_to(C, 16) && (!bias || aligned_to(bias, run)) &&
+                    (!resid || (aligned_to(resid, run) && ldr % 4 == 0));
   // Up to 64 rows: the weight stream of gemm_skinny.hip, except for 33 rows and more against very many channels, where the
   // tiles read the rows less often (plan_gemm_skinny; on cold weights, us for 16 / 32 / 64 rows against the tiles, N = K = 4096:
   // 9.6 / 11 / 15 against 24; N = 4096, K = 11008: 20 / 25 / 34 against 57; N = 11008, K = 4096: 19 / 24 / 29 against 36).
   if (TRANS_B && M <= 64 && N >= 64 && K % 32 == 0 && lda % 8 == 0 && ldb % 8 == 0 && aligned_to(A, 16) &&
       aligned_to(B, 16)) {
-    const GemmSkinnyPlan plan = plan_gemm_skinny(M, N, K);
+    const GemmSkinnyPlan plan = plan_gemm_skinny(M, N, K, fast || (!bias && !resid));
     if (plan.channels > 0)
       return launch_gemm_skinny<T, OutT>(plan, A, B, C, M, N, K, lda, ldb, ldc, s, bias, resid, ldr);
   }
-  const bool fast = K % BK == 0 && lda % 8 == 0 && ldb % 8 == 0 && ldc % 4 == 0 && N % 8 == 0 && N >= 8 &&
-                    aligned_to(A, 16) && aligned_to(B, 16) && aligned_to(C, 16) && (!bias || aligned_to(bias, run)) &&
-                    (!resid || (aligned_to(resid, run) && ldr % 4 == 0));
   if (fast) {
     const bool large = prefer_large_tiles(M, N);
     // the large-tile kernels sit at the register limit and carry no epilogue operands: a product with bias or

@@ -175,8 +175,9 @@ void gemm_nt_skinny_kernel(const T* __restrict__ A, const T* __restrict__ W, Out
 //   32 rows: N = 8192: K = 512 16x2 4.6, 32x4 4.6; K = 4096 19.1, 18.5. K = 2048: N = 11008 16x2 13.5, 32x2 14.7; N = 14336
 //     17.1, 15.9. N = 14336, K = 8192: 32x2 51, 64x4 47. N = 50264, K = 2048: 32x2 53, 32x4 48
 //   64 rows: N = 4096: K = 256 16x8 4.3, 16x4 4.0; K = 4096 14.8, 16.3. N = 8192, K = 4096: 32x4 22.9, 64x4 27.5. N = 11008:
-//     K = 256 16x2 5.7, 64x4 6.6; K = 4096 64x4 29, tiles 36. N = 32768: K = 512 64x4 16.5, tiles 12.0; K = 1024 24, 20
-GemmSkinnyPlan plan_gemm_skinny(int64_t M, int64_t N, int64_t K) {
+//     K = 256 16x2 5.7, 64x4 6.6; K = 4096 64x4 29, tiles 36. N = 32768: K = 512 64x4 16.5, tiles 12.0; K = 1024 24, 20.
+//     N = 30001 with a residual, where the tiles add it by elements: K = 256 32x2 12, tiles 22; K = 1024 64x4 23, tiles 37
+GemmSkinnyPlan plan_gemm_skinny(int64_t M, int64_t N, int64_t K, bool tiles) {
   const int64_t cus = std::max(1, hexmi_num_cus()), groups = (N + 15) / 16;
   if (M <= 16) {
     if (K <= 256) return {16, 2};
@@ -192,7 +193,10 @@ GemmSkinnyPlan plan_gemm_skinny(int64_t M, int64_t N, int64_t K) {
     if (groups <= 3 * cus) return {16, 2};
     return {32, groups > 8 * cus && K >= 768 ? 4 : 2};
   }
-  if (groups > 5 * cus || (groups > 4 * cus && K > 512)) return {0, 0};
+  if (groups > 5 * cus || (groups > 4 * cus && K > 512)) {
+    if (tiles) return {0, 0};
+    return K <= 768 ? GemmSkinnyPlan{32, 2} : GemmSkinnyPlan{64, 4};
+  }
   if (groups <= cus) return {16, K <= 512 ? 4 : 8};
   if (K <= 512) return groups <= 3 * cus ? GemmSkinnyPlan{16, 2} : GemmSkinnyPlan{32, 2};
   return {groups <= 2 * cus ? 32 : 64, 4};

@@ -224,9 +224,10 @@ inline bool two_pass_sum(int64_t n, int64_t block) {
 int block_sum_any(const void* x, void* out, int64_t n, int64_t block, int dtype, float* partials, hipStream_t s);
 
 // Up to 64 rows against [N,K] weights (gemm_skinny.hip): output channels and waves of a workgroup (0: leave it to the tiles),
-// and the launch. K % 32 == 0, operand rows on 16-byte boundaries; bias and residual may be null.
+// and the launch. K % 32 == 0, operand rows on 16-byte boundaries; bias and residual may be null. tiles: whether the tiles
+// are a choice (with bias or residual off whole runs of four columns they take twice to three times as long).
 struct GemmSkinnyPlan { int channels, waves; };
-GemmSkinnyPlan plan_gemm_skinny(int64_t M, int64_t N, int64_t K);
+GemmSkinnyPlan plan_gemm_skinny(int64_t M, int64_t N, int64_t K, bool tiles);
 template <typename T, typename OutT>
 int launch_gemm_skinny(const GemmSkinnyPlan& plan, const T* A, const T* B, OutT* C, int64_t M, int64_t N, int64_t K,
                        int64_t lda, int64_t ldb, int64_t ldc, hipStream_t s, const OutT* bias, const OutT* resid, int64_t ldr);

@@ -118,7 +118,7 @@ def test_gemm_few_rows_wide_workgroups(hexmi, dtype, M, N, K):
                                    (17, 10003, 96), (32, 8999, 992), (25, 77, 1056), (32, 14007, 544), (20, 5003, 800),
                                    (31, 14005, 4128), (32, 33003, 800),
                                    (33, 100, 480), (64, 333, 1056), (47, 9001, 160), (64, 17003, 224), (50, 7001, 544),
-                                   (64, 12005, 544), (64, 20500, 96)])
+                                   (64, 12005, 544), (64, 20500, 96), (33, 20501, 800)])
 def test_gemm_few_rows_every_workgroup_shape(hexmi, dtype, M, N, K):
     a, b = _inputs(M, N, K, dtype, True, seed=M + N)
     want, mag = a.double() @ b.double().t(), a.double().abs() @ b.double().t().abs()
@@ -128,6 +128,10 @@ def test_gemm_few_rows_every_workgroup_shape(hexmi, dtype, M, N, K):
     # fp32 products summed in parts: K roundings of at most 2^-24 of the magnitude, far fewer in effect
     assert ((got[:M].double() - want).abs() <= 1e-5 * mag + 1e-30).all()
     assert torch.isnan(got[M]).all()
+    # with a residual the widths here, off whole runs of four columns, keep the widest products from the tiles
+    resid = torch.randn(M, N, generator=_gen(K)).to(dtype)
+    fused = hexmi.matmul(a.cuda(), b.cuda(), trans_b=True, residual=resid.cuda()).cpu()
+    assert close16(fused, (want + resid.double()).to(dtype), max_ulp=1, atol=2e-5 * float(mag.max()))
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
