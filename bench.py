@@ -237,7 +237,7 @@ class GemmNT(Workload):
         self.M, self.N, self.K = M, N, K
         self.name = "gemm_f16_nt_%dx%dx%d" % (M, N, K)
         self.bound = "hbm" if M <= 64 else "mfma"
-        self.kernel = "gemv_nt_kernel" if M <= 8 else ("gemm_nt_skinny_kernel" if M <= 64 else "gemm_kernel_k64")
+        self.kernel = "gemv_nt_kernel" if M <= 2 else ("gemm_few_kernel" if M <= 64 else "gemm_kernel_k64")
         self.desc = "C = A[%d,%d] . W[%d,%d]^T fp16 U(-1,1), fp32 accumulate, fp16 out" % (M, K, N, K)
 
     def setup(self, torch, hexmi):

@@ -26,7 +26,8 @@
 // as [N,K], odd ldc, unaligned C) -> the same kernels with the tile leaving through LDS one element per lane;
 // anything else (unaligned operand rows, K % 8 != 0) -> gemm_kernel_any, which stages the slabs through registers.
 // Up to eight rows against B as [N,K] -> gemv_nt_kernel, a stream of the weights with one wave per output channel.
-// Nine to 64 rows against B as [N,K], where a fitted cost says so -> gemm_skinny.hip, a workgroup per 16 to 64 channels.
+// Up to 64 rows against B as [N,K], by measured lines -> gemm_skinny.hip, a workgroup per 16 to 64 channels. Whole chunks of K and
+// no more tiles than CUs -> gemm_few.hip, tiles of 16 x 16 to 128 x 64 that give every CU a share.
 #include <algorithm>
 #include <type_traits>
 
@@ -1571,13 +1572,17 @@ int dispatch_gemm(const void* Av, const void* Bv, void* Cv, int64_t M, int64_t N
   // chunks: K % 32 == 0, leading dimensions and N multiples of 8 elements, 16-byte aligned bases. Their epilogue
   // reads bias and residual in runs of four columns.
   const size_t run = 4 * sizeof(OutT);
-  // a few rows against [N,K] weights: the weight stream (see gemv_nt_kernel)
+  // whole 16-byte chunks on the operand side
+  const bool chunks = K % kChunk == 0 && lda % 8 == 0 && ldb % 8 == 0 && aligned_to(A, 16) && aligned_to(B, 16) &&
+                      (TRANS_B || (N % 8 == 0 && N >= 8));
+  // a row or two against [N,K] weights: the weight stream (see gemv_nt_kernel)
   // (Every workgroup stages the activation rows it multiplies, so their traffic grows with the rows while the
-  // weights' does not: up to two rows always, up to four from K = 1024, up to eight from K = 2048 on -- N = 50264,
-  // K = 768: 14.6 against 23 us on the tiles at one row, 32 against 23 at eight. Nine to sixteen rows as two passes
-  // of eight measured 21.5 against 24 us at N = K = 4096 but 48 against 26 at N = 11008: not taken.)
-  if (TRANS_B && (M <= 2 || (M <= 4 && K >= 1024) || (M <= 8 && K >= 2048)) && N >= 64 && K % kChunk == 0 &&
-      lda % 8 == 0 && ldb % 8 == 0 && aligned_to(A, 16) && aligned_to(B, 16)) {
+  // weights' does not: up to two rows always, three and four from K = 1024 on -- N = 50264, K = 768: 14.6 against 23 us on the
+  // tiles at one row, 32 against 23 at eight -- and up to eight from K = 2048 on where gemm_few.hip has no tile for them.)
+  const GemmFewTile few = chunks && M > (TRANS_B ? 2 : 0) && lda < (1 << 21) && ldb < (1 << 21) && K <= (1 << 30)
+                              ? plan_gemm_few(TRANS_B, M, N, K) : GemmFewTile{0, 0};
+  if (few.m) return launch_gemm_few<T, OutT, TRANS_B>(few, A, B, C, M, N, K, lda, ldb, ldc, s, bias, resid, ldr);
+  if (TRANS_B && (M <= 2 || (M <= 4 && K >= 1024) || (M <= 8 && K >= 2048)) && N >= 64 && chunks) {
 #define HEXMI_GEMV(MR, NW, RPW) \
   hipLaunchKernelGGL((gemv_nt_kernel<T, OutT, MR, NW, RPW>), dim3((unsigned)((N + NW * RPW - 1) / (NW * RPW))), dim3(NW * 64), 0, s, \
                      A, B, C, (int)M, (int)N, (int)K, lda, ldb, ldc, bias, resid, ldr)
@@ -1592,9 +1597,8 @@ int dispatch_gemm(const void* Av, const void* Bv, void* Cv, int64_t M, int64_t N
   const bool fast = K % BK == 0 && lda % 8 == 0 && ldb % 8 == 0 && ldc % 4 == 0 && N % 8 == 0 && N >= 8 &&
                     aligned_to(A, 16) && aligned_to(B, 16) && aligned_to(C, 16) && (!bias || aligned_to(bias, run)) &&
                     (!resid || (aligned_to(resid, run) && ldr % 4 == 0));
-  // Up to 64 rows: the weight stream of gemm_skinny.hip, except for 33 rows and more against very many channels, where the
-  // tiles read the rows less often (plan_gemm_skinny; on cold weights, us for 16 / 32 / 64 rows against the tiles, N = K = 4096:
-  // 9.6 / 11 / 15 against 24; N = 4096, K = 11008: 20 / 25 / 34 against 57; N = 11008, K = 4096: 19 / 24 / 29 against 36).
+  // Up to 64 rows that gemm_few.hip leaves: the weight stream of gemm_skinny.hip, except for 33 rows and more against very many
+  // channels, where the tiles read the rows less often (plan_gemm_skinny).
   if (TRANS_B && M <= 64 && N >= 64 && K % 32 == 0 && lda % 8 == 0 && ldb % 8 == 0 && aligned_to(A, 16) &&
       aligned_to(B, 16)) {
     const GemmSkinnyPlan plan = plan_gemm_skinny(M, N, K, fast || (!bias && !resid));
@@ -1612,8 +1616,6 @@ int dispatch_gemm(const void* Av, const void* Bv, void* Cv, int64_t M, int64_t N
   // Whole 16-byte chunks on the operand side only (K % 8 == 0; B given as [K,N] also N % 8 == 0): the 128x128 tiles
   // with a masked last slab, and an output side that may be anything ([N,K] weights with an odd N, such as a
   // vocabulary of 50257, land here: 1.0 PFLOP/s against 0.1 on the generic kernel below).
-  const bool chunks = K % kChunk == 0 && lda % 8 == 0 && ldb % 8 == 0 && aligned_to(A, 16) && aligned_to(B, 16) &&
-                      (TRANS_B || (N % 8 == 0 && N >= 8));
   // ... and with whole 64-wide slabs, a 16-bit result and no epilogue operands the paired-slab kernels take it, their
   // staged tiles leaving element by element
   if (chunks && sizeof(OutT) == 2 && K % BK2 == 0 && lda < (1 << 21) && ldb < (1 << 21) && !bias && !resid) {

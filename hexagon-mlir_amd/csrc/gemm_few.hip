@@ -1,0 +1,352 @@
+// C[M,N] = A[M,K] * op(B) where tiles of 128 x 128 would leave compute units without work (fp16 / bf16 in, fp32 sums): tiles of
+// 16 x 16 to 128 x 64 in one round, a workgroup of eight waves to a tile.
+//
+// What bounds it: a CU takes in about 90 GB/s through L2 whatever it does with it, and a tile of BM x BN asks for (BM + BN) x K
+// operands. 128 x 128 tiles run at that rate (0.31 us per 64 of K, K = 3072), so what is left is to have every CU take in a share:
+// a smaller tile reads each operand more often, but all of the chip reads. Per slab the LDS is the next limit (128 bytes a
+// clock): waves side by side read the same rows, so the shapes below give a wave 32 x 32 to 64 x 64 of the tile and let wave
+// groups take the 32-k steps of a slab in turn; their sums meet in LDS at the end, where the tile leaves in whole rows. Eight
+// waves with small accumulators beat four that own all of the tile (64 x 64, K = 3072: 11.5 against 17.5 us, a slab's reads
+// and multiplications of one wave per SIMD have nothing to run beside). Cold weights, bf16, us, before (128 x 128 tiles, for [N,K]
+// weights up to 64 rows gemm_skinny.hip) -> now:
+//   [K,N]  16 rows: 768 x 768 8.8 -> 4.3, 4096 x 4096 30 -> 18;  64 rows: 768 x 3072 20 -> 8.8, 4096 x 4096 35 -> 19
+//   [K,N]  N = 768, K = 3072: 256 rows 20.7 -> 9.3, 1000 rows 21 -> 12, 2000 rows 21.7 -> 17.4;  K = 768, 2000 rows 9.9 -> 7.8
+//   [N,K]  N = 4096, K = 4096: 64 rows 14.5 -> 12, 128 rows 37.7 -> 16, 256 rows 37 -> 20, 500 rows 37 -> 27
+#include <algorithm>
+#include <type_traits>
+
+#include "hexmi_common.h"
+
+namespace hexmi {
+namespace {
+
+__device__ __attribute__((aligned(16))) unsigned g_few_zeros[4];      // where a copy of a chunk past K points
+
+__device__ __forceinline__ f32x4 mfma16(const f16x8& b, const f16x8& a, f32x4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_f16(b, a, c, 0, 0, 0);
+}
+__device__ __forceinline__ f32x4 mfma16(const bf16x8& b, const bf16x8& a, f32x4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(b, a, c, 0, 0, 0);
+}
+template <typename T> struct Frag8;
+template <> struct Frag8<f16> { typedef f16x8 V; };
+template <> struct Frag8<bf16> { typedef bf16x8 V; };
+
+// 16 bytes a lane, global -> LDS, from an address of each lane's own; as copy_to_lds_asm (hexmi_common.h)
+__device__ __forceinline__ void copy_ptr_to_lds_asm(const char* src, char* lds) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  const uint32_t dst = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)((__attribute__((address_space(3))) void*)(lds)));
+  uint32_t saved;
+  asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %2, off\n\ts_mov_b32 m0, %0"
+               : "=&s"(saved) : "s"(dst), "v"(src) : "memory");
+#endif
+}
+
+// s_waitcnt immediate (gfx9 encoding): at most vm vector-memory operations outstanding, LDS reads returned
+constexpr int wait_imm(int vm) { return (vm & 0xF) | ((vm >> 4) << 14) | (0x7 << 4); }
+
+// TM x TN: 16 x 16 tiles of a wave; SM x SN waves side by side; KH wave groups share the 32-k steps of a slab.
+template <int TM_, int TN_, int SM_, int SN_, int KH_>
+struct Shape {
+  static constexpr int TM = TM_, TN = TN_, SM = SM_, SN = SN_, KH = KH_, kWaves = SM * SN * KH, kThreads = kWaves * kWave;
+  static constexpr int BM = SM * TM * 16, BN = SN * TN * 16, BK = KH * 32;
+  static constexpr int kStage = (BM + BN) * BK;                  // elements of a stage: rows of A, then B
+};
+
+// chunk c (16 bytes) of row r of a K-contiguous tile of BK elements a row sits at c ^ swz_row(r): sixteen rows of one chunk
+// then cover all banks
+template <int BK> __device__ __forceinline__ int swz_row(int r) { return BK == 64 ? (r >> 1) & 7 : r & 15; }
+// N-contiguous tile of BN columns a row of k: the 32 lanes of a transposing read touch k % 4, k / 8 % 2 x 32 bytes, which the
+// XOR spreads over the eight 32-byte slots of all banks
+template <int BN> __device__ __forceinline__ int swz_col(int k) {
+  return BN == 64 ? (((k >> 1) & 1) | (((k >> 3) & 1) << 1)) << 1 : ((k >> 3) & 1) << 1;
+}
+
+// NS stages of a slab of KH * 32 k: copies fill all but one while that one is read; one barrier a slab. K % 8 == 0, operand rows
+// on 16-byte boundaries ([K,N]: N % 8 == 0 too). runs: the output (and bias and residual) in runs of eight columns on
+// 16-byte boundaries; otherwise they go by elements.
+template <typename T, typename OutT, typename S, int NS, bool TRANS_B>
+__global__ __launch_bounds__(S::kThreads)
+void gemm_few_kernel(const T* __restrict__ A, const T* __restrict__ B, OutT* C, int M, int N, int K, int64_t lda, int64_t ldb,
+                     int64_t ldc, const OutT* __restrict__ bias, const OutT* resid, int64_t ldr, int tiles_m, int tiles_n,
+                     int runs) {
+  constexpr int TM = S::TM, TN = S::TN, BM = S::BM, BN = S::BN, BK = S::BK, KH = S::KH, kWaves = S::kWaves, kThreads = S::kThreads;
+  constexpr int kA = BM * BK / 512 / kWaves, kB = BN * BK / 512 / kWaves, kCopies = kA + kB;   // a wave's copies (1 KiB) of a slab
+  static_assert(kA * kWaves * 512 == BM * BK && kB * kWaves * 512 == BN * BK, "whole copies");
+  constexpr int kStageBytes = S::kStage * 2, kPitch = BN + 4;    // pitch of the sums on their way out
+  constexpr int kLds = std::max(NS * kStageBytes, KH * BM * kPitch * 4);
+  __shared__ __attribute__((aligned(16))) char lds[kLds];
+
+  const int lane = threadIdx.x % kWave, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const int r16 = lane % 16, kg = lane / 16;
+  int tm, tn;                                                    // every XCD (each its own L2) a band of tiles
+  {
+    const int total = tiles_m * tiles_n, pid = blockIdx.x;
+    const int xcd = pid % 8, per = total / 8, extra = total % 8;
+    const int logical = xcd * per + (xcd < extra ? xcd : extra) + pid / 8;
+    constexpr int kGroup = 8;
+    const int group_size = kGroup * tiles_n, group = logical / group_size, first = group * kGroup;
+    const int gm = tiles_m - first < kGroup ? tiles_m - first : kGroup;
+    tm = first + logical % group_size % gm;
+    tn = logical % group_size / gm;
+  }
+  const int m0 = tm * BM, n0 = tn * BN;
+
+  // copy i of a slab moves chunks [i * 512 + wave * 64, + 64) of the tile: A's kA, then B's kB
+  int voff[kCopies], kc[kCopies];
+#pragma unroll
+  for (int i = 0; i < kCopies; ++i) {
+    const int chunk = (i < kA ? i : i - kA) * kThreads + threadIdx.x;
+    if (i < kA || TRANS_B) {
+      const int row = chunk / (BK / 8), c = (chunk % (BK / 8)) ^ swz_row<BK>(row);
+      const int left = (i < kA ? M - m0 : N - n0) - 1;           // past the edge: the last row again, not stored
+      voff[i] = (int)((int64_t)(row < left ? row : left) * (i < kA ? lda : ldb) * 2 + c * 16);
+      kc[i] = c * 8;
+    } else {
+      const int k = chunk / (BN / 8), c = (chunk % (BN / 8)) ^ swz_col<BN>(k);
+      const int left = N - n0 - 8;
+      voff[i] = (int)((int64_t)k * ldb * 2 + (c * 8 < left ? c * 8 : left) * 2);
+      kc[i] = k;
+    }
+  }
+  const char* a_base = reinterpret_cast<const char*>(A + (int64_t)m0 * lda);
+  const char* b_base = reinterpret_cast<const char*>(TRANS_B ? B + (int64_t)n0 * ldb : B + n0);
+  const int64_t b_step = (TRANS_B ? BK : BK * ldb) * 2;
+  const int slabs = (K + BK - 1) / BK;
+  auto copy = [&](int slab, int stage, auto ragged) __attribute__((always_inline)) {
+    const char* a_from = a_base + (int64_t)slab * (BK * 2);
+    const char* b_from = b_base + slab * b_step;
+    char* to = lds + stage * kStageBytes + wave * 1024;
+#pragma unroll
+    for (int i = 0; i < kCopies; ++i) {
+      const char* from = i < kA ? a_from : b_from;
+      if constexpr (decltype(ragged)::value) {                   // the slab that reaches past K: zeros there
+        const char* src = slab * BK + kc[i] < K ? from + voff[i] : reinterpret_cast<const char*>(g_few_zeros);
+        copy_ptr_to_lds_asm(src, to + i * (kWaves * 1024));
+      } else {
+        copy_to_lds_asm(from, voff[i], to + i * (kWaves * 1024));
+      }
+    }
+  };
+  const int full = K / BK;
+  auto copy_any = [&](int slab, int stage) __attribute__((always_inline)) {
+    if (slab < full) copy(slab, stage, std::false_type{}); else copy(slab, stage, std::true_type{});
+  };
+
+  // this lane's fragments of a stage: wave group kh takes the slab's step kh (32 of K)
+  const int kh = wave / (S::SM * S::SN), wm = wave % (S::SM * S::SN) / S::SN, wn = wave % S::SN;
+    const int arow = wm * TM * 16 + r16;
+  const int a_at = (arow * BK + ((kh * 4 + kg) ^ swz_row<BK>(arow)) * 8) * 2;
+  int b_at[TN];
+#pragma unroll
+  for (int j = 0; j < TN; ++j) {
+    if (TRANS_B) {
+      const int row = (wn * TN + j) * 16 + r16;
+      b_at[j] = (BM * BK + row * BK + ((kh * 4 + kg) ^ swz_row<BK>(row)) * 8) * 2;
+    } else {                                                     // lane i of 16: row i / 4, columns 4 (i % 4) .. + 3
+      const int k = kh * 32 + kg * 8 + r16 / 4, col = (wn * TN + j) * 16 + (r16 & 3) * 4;
+      b_at[j] = (BM * BK + k * BN + ((col / 8) ^ swz_col<BN>(k)) * 8 + col % 8) * 2;
+    }
+  }
+
+  // bias and residual of this thread's runs of eight columns of the result, under the K walk
+  constexpr int kRuns = BM * BN / 8 < kThreads ? 1 : BM * BN / 8 / kThreads;
+  struct alignas(16) Run { OutT v[8]; };
+  Run add_b[kRuns], add_r[kRuns];
+  if (runs) {
+#pragma unroll
+    for (int p = 0; p < kRuns; ++p) {
+      const int idx = threadIdx.x + p * kThreads, row = idx / (BN / 8) % BM, col = idx % (BN / 8) * 8;
+      const int gm = m0 + row < M ? m0 + row : M - 1, gn = n0 + col < N ? n0 + col : N - 8;
+      if (bias) add_b[p] = *reinterpret_cast<const Run*>(bias + gn);
+      if (resid) add_r[p] = *reinterpret_cast<const Run*>(resid + (int64_t)gm * ldr + gn);
+    }
+  }
+
+  f32x4 acc[TM][TN];
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  typedef typename Frag8<T>::V Frag;
+  struct Step { Frag a[TM], b[TN]; };
+  auto read = [&](int stage, Step& f) __attribute__((always_inline)) {
+    const char* from = lds + stage * kStageBytes;
+#pragma unroll
+    for (int j = 0; j < TN; ++j) {
+      if constexpr (TRANS_B) {
+        f.b[j] = *reinterpret_cast<const Frag*>(from + b_at[j]);
+      } else {                                                   // four k on: the same place in its row
+        union { i16x4 h[2]; Frag v; } u;
+#pragma unroll
+        for (int p = 0; p < 2; ++p)
+          u.h[p] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) i16x4*)(from + b_at[j] + p * (4 * BN * 2)));
+        f.b[j] = u.v;
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < TM; ++i) f.a[i] = *reinterpret_cast<const Frag*>(from + a_at + i * (16 * BK * 2));   // the swizzle repeats
+  };
+  auto multiply = [&](const Step& f) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int j = 0; j < TN; ++j) acc[i][j] = mfma16(f.b[j], f.a[i], acc[i][j]);
+  };
+#define HEXMI_FENCE __builtin_amdgcn_sched_barrier(0)
+  // The copies are assembly: the compiler would wait for all of them before any LDS read. Here a wave waits until at most `newer`
+  // slabs of its own are in flight and its reads of the slab before have returned, then for every other wave.
+  auto landed = [&](auto newer) __attribute__((always_inline)) {
+    HEXMI_FENCE;
+    __builtin_amdgcn_s_waitcnt(wait_imm(decltype(newer)::value * kCopies));
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    HEXMI_FENCE;
+  };
+  HEXMI_FENCE;
+#pragma unroll
+  for (int j = 0; j < NS - 1; ++j)
+    if (j < slabs) copy_any(j, j);
+  int stage = 0, j = 0;
+  auto step = [&](auto newer, auto next) __attribute__((always_inline)) {   // next: the copies that follow into the free stage
+    landed(newer);
+    next();
+    HEXMI_FENCE;
+    Step f;
+    read(stage, f);
+    multiply(f);
+    stage = stage == NS - 1 ? 0 : stage + 1;
+    ++j;
+  };
+  auto free_stage = [&]() { return stage == 0 ? NS - 1 : stage - 1; };
+  constexpr std::integral_constant<int, NS - 2> kBehind{};
+  while (j + NS - 1 < full) step(kBehind, [&]() __attribute__((always_inline)) { copy(j + NS - 1, free_stage(), std::false_type{}); });
+  if (j + NS - 1 < slabs) step(kBehind, [&]() __attribute__((always_inline)) { copy(j + NS - 1, free_stage(), std::true_type{}); });
+  auto last = [&](auto left) __attribute__((always_inline)) {    // left: slabs behind this one
+    if (j + decltype(left)::value < slabs) step(left, []() __attribute__((always_inline)) {});
+  };
+  if constexpr (NS > 7) last(std::integral_constant<int, 6>{});
+  if constexpr (NS > 6) last(std::integral_constant<int, 5>{});
+  if constexpr (NS > 5) last(std::integral_constant<int, 4>{});
+  if constexpr (NS > 4) last(std::integral_constant<int, 3>{});
+  if constexpr (NS > 3) last(std::integral_constant<int, 2>{});
+  if constexpr (NS > 2) last(std::integral_constant<int, 1>{});
+  last(std::integral_constant<int, 0>{});
+  static_assert(NS >= 2 && NS <= 8, "the ladder above");
+#undef HEXMI_FENCE
+
+  // the wave groups' sums meet in LDS and leave in rows
+  __syncthreads();
+  float* red = reinterpret_cast<float*>(lds);
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int jj = 0; jj < TN; ++jj)                              // a lane: row lane % 16, columns 4 (lane / 16) .. + 3
+      *reinterpret_cast<f32x4*>(red + (kh * BM + (wm * TM + i) * 16 + r16) * kPitch + (wn * TN + jj) * 16 + kg * 4) = acc[i][jj];
+  __syncthreads();
+  if (runs) {
+#pragma unroll
+    for (int p = 0; p < kRuns; ++p) {
+      const int idx = threadIdx.x + p * kThreads, row = idx / (BN / 8), col = idx % (BN / 8) * 8;
+      if (BM * BN / 8 < kThreads && row >= BM) break;
+      f32x4 s0 = {0.f, 0.f, 0.f, 0.f}, s1 = s0;
+#pragma unroll
+      for (int h = 0; h < KH; ++h) {
+        const float* from = red + (h * BM + row) * kPitch + col;
+        s0 += *reinterpret_cast<const f32x4*>(from);
+        s1 += *reinterpret_cast<const f32x4*>(from + 4);
+      }
+      Run out;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        float v = e < 4 ? s0[e % 4] : s1[e % 4];
+        if (bias) v += to_f32<OutT>(add_b[p].v[e]);
+        if (resid) v += to_f32<OutT>(add_r[p].v[e]);
+        out.v[e] = from_f32<OutT>(v);
+      }
+      if (m0 + row < M && n0 + col < N) *reinterpret_cast<Run*>(C + (int64_t)(m0 + row) * ldc + n0 + col) = out;
+    }
+  } else {
+    // (a residual that is the output itself: an element is read and written by one thread)
+    for (int idx = threadIdx.x; idx < BM * BN; idx += kThreads) {
+      const int row = idx / BN, col = idx % BN;
+      if (m0 + row >= M || n0 + col >= N) continue;
+      float v = 0.f;
+#pragma unroll
+      for (int h = 0; h < KH; ++h) v += red[(h * BM + row) * kPitch + col];
+      if (bias) v += to_f32<OutT>(bias[n0 + col]);
+      if (resid) v += to_f32<OutT>(resid[(int64_t)(m0 + row) * ldr + n0 + col]);
+      C[(int64_t)(m0 + row) * ldc + n0 + col] = from_f32<OutT>(v);
+    }
+  }
+}
+
+template <int BM, int BN> struct FewShape;                       // waves, stages: what measured fastest of two to five forms each
+template <> struct FewShape<16, 16> { typedef Shape<1, 1, 1, 1, 8> S; static constexpr int NS = 8; };
+template <> struct FewShape<16, 32> { typedef Shape<1, 2, 1, 1, 8> S; static constexpr int NS = 6; };
+template <> struct FewShape<32, 32> { typedef Shape<2, 2, 1, 1, 8> S; static constexpr int NS = 5; };
+template <> struct FewShape<32, 64> { typedef Shape<2, 2, 1, 2, 4> S; static constexpr int NS = 6; };
+template <> struct FewShape<64, 64> { typedef Shape<2, 4, 2, 1, 4> S; static constexpr int NS = 4; };
+template <> struct FewShape<128, 64> { typedef Shape<4, 4, 2, 1, 4> S; static constexpr int NS = 3; };
+
+}  // namespace
+
+// The smallest tile of which there is at most one per CU (more tiles than CUs: a second round, at the same intake per CU as a tile of
+// twice the area; over 250 random products of up to 2000 rows no other tile was more than 6 % ahead of this choice but where K < 128),
+// none where even 128 x 64 are more. us for 128 x 64 / 64 x 64 / 32 x 64 / 32 x 32 tiles (how many), K = 3072 [K,N]: N = 768, 2000 rows
+// 17.5 (192) / 22 (384); 1000 rows 18 (96) / 12 (192) / 18 (384); 500 rows 17 / 11.6 (96) / 10 (192) / 16 (384); 256 rows 16.5 / 11.7
+// / 9.7 (96) / 9.3 (192).
+// Up to 64 rows against [N,K] weights there is the weight stream of gemm_skinny.hip, whose start and end are shorter: it stays for 33
+// rows and more up to K = 128 (50 x 176 x 32 3.3, 3.2; 38 x 320 x 64 3.1, 3.2), for 17 to 32 rows against weights of less than 2^23
+// elements (29 x 640 x 3872 5.4, 5.8; 20 x 9968 x 320 4.5, 4.6; 23 x 8728 x 896 7.5, 6.9; 32 x 4096 x 4096 11.7, 10.3) and for up to
+// 16 rows of less than 3 * 2^22 (16 x 768 x 3072 4.9, 5.1; 10 x 2800 x 3136 6.5, 7.0; 9 x 3672 x 3360 8.3, 7.8; 16 x 4096 x 4096
+// 9.9, 8.7; 13 x 7904 x 5952 19.5, 16) -- but where five to eight rows and K of 2048 and more would go by dot products, a tile is
+// always ahead (8 x 800 x 3168 8.5, 5.5; 7 x 304 x 11968 18, 11).
+GemmFewTile plan_gemm_few(bool trans_b, int64_t M, int64_t N, int64_t K) {
+  const int64_t cus = hexmi_num_cus();
+  if (trans_b && M <= 64) {
+    if (M > 32 ? K <= 128 : N * K < (int64_t)(M > 16 ? 2 : 3) << 22 && !(M >= 5 && M <= 8 && K >= 2048)) return {0, 0};
+  }
+  static constexpr GemmFewTile kTiles[] = {{16, 16}, {16, 32}, {32, 32}, {32, 64}, {64, 64}, {128, 64}};
+  for (const GemmFewTile& t : kTiles) {
+    if (t.m == 16 && (M > 64 || (t.n == 16 && !trans_b))) continue;       // sixteen columns of a row of B are a quarter of a line
+    if (((M + t.m - 1) / t.m) * ((N + t.n - 1) / t.n) <= cus) return t;
+  }
+  return {0, 0};
+}
+
+template <typename T, typename OutT, bool TRANS_B>
+int launch_gemm_few(const GemmFewTile& tile, const T* A, const T* B, OutT* C, int64_t M, int64_t N, int64_t K, int64_t lda,
+                    int64_t ldb, int64_t ldc, hipStream_t s, const OutT* bias, const OutT* resid, int64_t ldr) {
+  const int tiles_m = (int)((M + tile.m - 1) / tile.m), tiles_n = (int)((N + tile.n - 1) / tile.n);
+  const int runs = N % 8 == 0 && ldc % 8 == 0 && aligned_to(C, 16) && aligned_to(bias, 16) && aligned_to(resid, 16) &&
+                   (!resid || ldr % 8 == 0);
+#define HEXMI_FEW(BM, BN)                                                                                                    \
+  hipLaunchKernelGGL((gemm_few_kernel<T, OutT, FewShape<BM, BN>::S, FewShape<BM, BN>::NS, TRANS_B>),                         \
+                     dim3((unsigned)(tiles_m * tiles_n)), dim3(FewShape<BM, BN>::S::kThreads), 0, s, A, B, C, (int)M, (int)N, \
+                     (int)K, lda, ldb, ldc, bias, resid, ldr, tiles_m, tiles_n, runs)
+  if (tile.m == 128) HEXMI_FEW(128, 64);
+  else if (tile.m == 64) HEXMI_FEW(64, 64);
+  else if (tile.n == 64) HEXMI_FEW(32, 64);
+  else if (tile.m == 32) HEXMI_FEW(32, 32);
+  else if (tile.n == 32) HEXMI_FEW(16, 32);
+  else if constexpr (TRANS_B) HEXMI_FEW(16, 16);
+  else return HEXMI_ENOTSUP;                                     // (the plan gives [K,N] none)
+#undef HEXMI_FEW
+  return launch_status();
+}
+
+#define HEXMI_INSTANCE(T, OutT, TB)                                                                                          \
+  template int launch_gemm_few<T, OutT, TB>(const GemmFewTile&, const T*, const T*, OutT*, int64_t, int64_t, int64_t, int64_t, \
+                                            int64_t, int64_t, hipStream_t, const OutT*, const OutT*, int64_t);
+HEXMI_INSTANCE(f16, f16, false)
+HEXMI_INSTANCE(f16, f16, true)
+HEXMI_INSTANCE(f16, float, false)
+HEXMI_INSTANCE(f16, float, true)
+HEXMI_INSTANCE(bf16, bf16, false)
+HEXMI_INSTANCE(bf16, bf16, true)
+HEXMI_INSTANCE(bf16, float, false)
+HEXMI_INSTANCE(bf16, float, true)
+#undef HEXMI_INSTANCE
+
+}  // namespace hexmi

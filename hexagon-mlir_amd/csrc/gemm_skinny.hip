@@ -8,9 +8,10 @@
 // own: a CU took in 29 GB/s that way whatever was in flight (4 to 16 waves, 2 to 8 steps: 36 to 38 us). Here a
 // wave copies its rounds into LDS eight lanes to a 128-byte line (each wave its own two stages: no barrier in
 // the K walk) and reads the operands from there, chunk c of row r at c ^ ((r / 2) % 8). Cold weights, us, before -> now:
-//   N = 4096, K = 4096:   16 rows 11.8 -> 8.7, 32 rows 15.2 -> 10.3, 64 rows 23 -> 14
-//   N = 4096, K = 11008:  27.7 -> 19.7, 36 -> 24.6, 57 -> 33.7        N = 768, K = 3072: 9.3 -> 4.4, 12 -> 5.6, 18 -> 8.1
-//   N = 11008, K = 4096 (on the 128 x 128 tiles before): 31.7 -> 19, 32.4 -> 24.2, 35.2 -> 29.5
+//   N = 4096, K = 4096:   16 rows 11.8 -> 8.7, 32 rows 15.2 -> 10.3
+//   N = 4096, K = 11008:  27.7 -> 19.7, 36 -> 24.6        N = 768, K = 3072: 9.3 -> 4.4, 12 -> 5.6
+//   N = 11008, K = 4096 (on the 128 x 128 tiles before): 31.7 -> 19, 32.4 -> 24.2
+// (Larger weights, and 33 rows and more, go to gemm_few.hip wherever one round of its tiles covers them.)
 // Three and four stages, and counted waits in place of the loop's full ones, measured equal.
 #include <algorithm>
 
@@ -207,11 +208,11 @@ void gemm_nt_skinny_kernel(const T* __restrict__ A, const T* __restrict__ W, Out
 // cold weights; channels x waves in us:
 //   16 rows: N = 4096: K = 256 16x8 3.3, 16x2 3.2; K = 4096 9.7, 15.0. N = 16384, K = 512: 16x8 7.5, 16x2 5.7. N = 40000,
 //     K = 1024: 16x2 18.2, 32x4 16.5. N = 28672, K = 6144: 16x2 72, 16x8 66
-//   32 rows: N = 8192: K = 512 16x2 4.6, 32x4 4.6; K = 4096 19.1, 18.5. K = 2048: N = 11008 16x2 13.5, 32x2 14.7; N = 14336
-//     17.1, 15.9. N = 14336, K = 8192: 32x2 51, 64x4 47. N = 50264, K = 2048: 32x2 53, 32x4 48
-//   64 rows: N = 4096: K = 256 16x8 4.3, 16x4 4.0; K = 4096 14.8, 16.3. N = 8192, K = 4096: 32x4 22.9, 64x4 27.5. N = 11008:
-//     K = 256 16x2 5.7, 64x4 6.6; K = 4096 64x4 29, tiles 36. N = 32768: K = 512 64x4 16.5, tiles 12.0; K = 1024 24, 20.
-//     N = 30001 with a residual, where the tiles add it by elements: K = 256 32x2 12, tiles 22; K = 1024 64x4 23, tiles 37
+//   32 rows: N = 8192: K = 512 16x2 4.6, 32x4 4.6. K = 2048: N = 11008 16x2 13.5, 32x2 14.7; N = 14336 17.1, 15.9. N = 50264,
+//     K = 2048: 32x2 53, 32x4 48
+//   64 rows (up to N = 16384 only where K is 128 or less, or rows of 2^21 elements and more): N = 32768: K = 512 64x4 16.5, tiles
+//     12.0; K = 1024 24, 20. N = 30001 with a residual, where the tiles add it by elements: K = 256 32x2 12, tiles 22;
+//     K = 1024 64x4 23, tiles 37
 GemmSkinnyPlan plan_gemm_skinny(int64_t M, int64_t N, int64_t K, bool tiles) {
   const int64_t cus = std::max(1, hexmi_num_cus()), groups = (N + 15) / 16;
   if (M <= 16) {
@@ -224,7 +225,6 @@ GemmSkinnyPlan plan_gemm_skinny(int64_t M, int64_t N, int64_t K, bool tiles) {
     if (groups <= 5 * cus && K <= 256) return {16, 2};
     if (groups <= cus) return {16, 8};
     if (groups <= 2 * cus) return K < 768 ? GemmSkinnyPlan{16, 2} : GemmSkinnyPlan{32, 4};
-    if (groups <= 4 * cus && K >= 4096) return {64, 4};
     if (groups <= 3 * cus) return {16, 2};
     return {32, groups > 8 * cus && K >= 768 ? 4 : 2};
   }
@@ -232,9 +232,9 @@ GemmSkinnyPlan plan_gemm_skinny(int64_t M, int64_t N, int64_t K, bool tiles) {
     if (tiles) return {0, 0};
     return K <= 768 ? GemmSkinnyPlan{32, 2} : GemmSkinnyPlan{64, 4};
   }
-  if (groups <= cus) return {16, K <= 512 ? 4 : 8};
+  if (groups <= cus) return {16, 4};
   if (K <= 512) return groups <= 3 * cus ? GemmSkinnyPlan{16, 2} : GemmSkinnyPlan{32, 2};
-  return {groups <= 2 * cus ? 32 : 64, 4};
+  return {64, 4};
 }
 
 template <typename T, typename OutT>
@@ -258,16 +258,13 @@ int launch_gemm_skinny(const GemmSkinnyPlan& plan, const T* A, const T* B, OutT*
     else if (plan.waves == 8) HEXMI_SKINNY(1, 1, 8);
     else HEXMI_SKINNY(1, 1, 2);
   } else if (M <= 32) {
-    if (plan.channels == 64) HEXMI_SKINNY(2, 4, 4);
-    else if (plan.channels == 32 && plan.waves == 4) HEXMI_SKINNY(2, 2, 4);
+    if (plan.channels == 32 && plan.waves == 4) HEXMI_SKINNY(2, 2, 4);
     else if (plan.channels == 32) HEXMI_SKINNY(2, 2, 2);
     else if (plan.waves == 8) HEXMI_SKINNY(2, 1, 8);
     else HEXMI_SKINNY(2, 1, 2);
   } else {
     if (plan.channels == 64) HEXMI_SKINNY(4, 4, 4);
-    else if (plan.channels == 32 && plan.waves == 4) HEXMI_SKINNY(4, 2, 4);
     else if (plan.channels == 32) HEXMI_SKINNY(4, 2, 2);
-    else if (plan.waves == 8) HEXMI_SKINNY(4, 1, 8);
     else if (plan.waves == 4) HEXMI_SKINNY(4, 1, 4);
     else HEXMI_SKINNY(4, 1, 2);
   }

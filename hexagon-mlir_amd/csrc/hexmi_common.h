@@ -232,6 +232,14 @@ template <typename T, typename OutT>
 int launch_gemm_skinny(const GemmSkinnyPlan& plan, const T* A, const T* B, OutT* C, int64_t M, int64_t N, int64_t K,
                        int64_t lda, int64_t ldb, int64_t ldc, hipStream_t s, const OutT* bias, const OutT* resid, int64_t ldr);
 
+// Products of few 128 x 128 tiles (gemm_few.hip): the tile, m == 0 for none, and the launch. K % 8 == 0, operand rows on 16-byte
+// boundaries, leading dimensions below 2^21 (per-lane copy offsets), B as [K,N]: N % 8 == 0; any output side.
+struct GemmFewTile { int m, n; };
+GemmFewTile plan_gemm_few(bool trans_b, int64_t M, int64_t N, int64_t K);
+template <typename T, typename OutT, bool TRANS_B>
+int launch_gemm_few(const GemmFewTile& tile, const T* A, const T* B, OutT* C, int64_t M, int64_t N, int64_t K, int64_t lda,
+                    int64_t ldb, int64_t ldc, hipStream_t s, const OutT* bias, const OutT* resid, int64_t ldr);
+
 // Tiled W8A16 GEMM for many activation rows (gemm.hip): C[M,N] = (A[M,K] * W[N,K]^T) * scales[N].
 int gemm_w8a16_tiled(int64_t M, int64_t N, int64_t K, const f16* A, const int8_t* W, const f16* scales, f16* C,
                      hipStream_t stream);

@@ -111,8 +111,8 @@ def test_gemm_few_rows_wide_workgroups(hexmi, dtype, M, N, K):
 
 
 # every (channels, waves) that plan_gemm_skinny picks on 256 CUs, at widths off the workgroup's, with K of a few rounds of 64,
-# fewer rounds than waves, and the last 32 of K on its own: 16x2, 16x8, 32x4 (16 rows); 16x2, 16x8, 32x2, 32x4, 64x4 (32
-# rows); 16x4, 16x8, 16x2, 32x2, 32x4, 64x4 and the tiles (64 rows)
+# fewer rounds than waves, and the last 32 of K on its own: 16x2, 16x8, 32x4 (16 rows); 16x2, 16x8, 32x2, 32x4 (32
+# rows); 16x4, 16x2, 32x2, 64x4 and the tiles (64 rows) -- where plan_gemm_few leaves the product to it
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("M,N,K", [(5, 401, 160), (16, 8195, 480), (16, 401, 736), (3, 33001, 800), (12, 16501, 3104),
                                    (17, 10003, 96), (32, 8999, 992), (25, 77, 1056), (32, 14007, 544), (20, 5003, 800),
@@ -187,6 +187,70 @@ def test_gemm_tiles_left_over_after_a_round_of_two_per_cu(hexmi, trans_b, K):
     want, mag = a.double() @ bt + bias.double(), float((a.double().abs() @ bt.abs()).max())
     got = hexmi.matmul(a.cuda(), b.cuda(), trans_b=trans_b, bias=bias.cuda()).cpu()
     assert close16(got, want.to(dtype), max_ulp=1, atol=2e-5 * mag)
+
+
+def _against_double(hexmi, dtype, out_dtype, trans_b, M, N, K, bias, residual, seed, out=None):
+    g = _gen(seed)
+    a, b = _inputs(M, N, K, dtype, trans_b, seed=seed)
+    bi = torch.randn(N, generator=g).to(out_dtype) if bias else None
+    r = torch.randn(M, N, generator=g).to(out_dtype) if residual else None
+    ref = a.cuda().double() @ (b.cuda().double().t() if trans_b else b.cuda().double())
+    mag = a.cuda().double().abs() @ (b.cuda().double().abs().t() if trans_b else b.cuda().double().abs())
+    for t in (bi, r):
+        if t is not None:
+            ref, mag = ref + t.cuda().double(), mag + t.cuda().double().abs()
+    got = hexmi.matmul(a.cuda(), b.cuda(), trans_b=trans_b, bias=None if bi is None else bi.cuda(),
+                       residual=None if r is None else r.cuda(), out_dtype=out_dtype, out=out)
+    # sums in fp32 in another order: 1e-5 of the summed magnitudes; one rounding to the output type: half an ulp
+    eps = {torch.float16: 2.0 ** -11, torch.bfloat16: 2.0 ** -8, torch.float32: 2.0 ** -24}[out_dtype]
+    assert ((got.double() - ref).abs() <= 1e-5 * mag + eps * ref.abs() + 1e-7).all(), (M, N, K)
+
+
+# every tile of plan_gemm_few on 256 CUs: its edges (one row or column over, one short), slabs of K that are whole, short or
+# one chunk over, fewer slabs than stages and more; outputs that leave in runs of eight and that do not
+@pytest.mark.parametrize("trans_b", [False, True])
+@pytest.mark.parametrize("dtype,out_dtype", [(torch.float16, torch.float16), (torch.bfloat16, torch.float32),
+                                             (torch.bfloat16, torch.bfloat16)])
+@pytest.mark.parametrize("M,N,K", [
+    (64, 1024, 256), (33, 40, 2056), (49, 16, 136), (64, 24, 1280),      # 16 x 16 ([N,K]), 16 x 32
+    (33, 4104, 2048), (65, 4072, 264), (500, 500 // 8 * 8, 1288),        # 16 x 32 and 32 x 32 and their edges
+    (17, 16328, 520), (129, 4096, 776), (500, 1016, 896),                # 32 x 64
+    (1000, 1024, 136), (1025, 960, 640), (257, 3264, 72),                # 64 x 64
+    (1921, 1024, 392), (2000, 768, 1032), (129, 8128, 8), (2048, 1024, 128)])    # 128 x 64; the last of a round
+def test_gemm_one_round_of_tiles(hexmi, dtype, out_dtype, trans_b, M, N, K):
+    _against_double(hexmi, dtype, out_dtype, trans_b, M, N, K, True, True, M + N + K)
+    _against_double(hexmi, dtype, out_dtype, trans_b, M, N, K, False, False, M + N + K + 1)
+    if trans_b:                                                          # rows of the output off the boundaries
+        _against_double(hexmi, dtype, out_dtype, True, M, N + 1, K, True, True, M + N + K + 2)
+    # a strided output one element off, the residual the output itself, nothing written around it
+    g = _gen(3)
+    a, b = _inputs(M, N, K, dtype, trans_b, seed=5)
+    a, b = a.cuda(), b.cuda()
+    from hexmi import _lib
+    code = {torch.float16: _lib.F16, torch.bfloat16: _lib.BF16, torch.float32: _lib.F32}
+    for ldc, off in ((N + 8, 0), (N + 3, 1)):
+        c = torch.randn(M * ldc + 16, generator=g).to(out_dtype).cuda()
+        view = c[off:off + M * ldc].view(M, ldc)
+        want = a.double() @ (b.double().t() if trans_b else b.double()) + view[:, :N].double()
+        keep = view[:, N:].clone()
+        s = torch.cuda.current_stream().cuda_stream
+        assert _lib.lib().hexmi_gemm_ex(M, N, K, a.data_ptr(), K, b.data_ptr(), b.stride(0), view.data_ptr(), ldc, None,
+                                        view.data_ptr(), ldc, code[dtype], code[out_dtype], int(trans_b), s) == _lib.OK
+        eps = torch.finfo(out_dtype).eps
+        assert ((view[:, :N].double() - want).abs() <= eps * want.abs() + 2e-5 * K).all()
+        assert torch.equal(view[:, N:], keep)
+
+
+# more tiles than one round of them: the 128 x 128 and 256 x 256 kernels and the slabs, widths and outputs each is for
+@pytest.mark.parametrize("trans_b", [False, True])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("M,N,K,bias,residual", [
+    (2049, 1096, 64, False, False), (2049, 1096, 96, False, False), (2049, 1096, 160, True, True),   # whole slabs of 64 and 32
+    (2049, 1096, 72, False, False), (2049, 1096, 1000, True, False), (2100, 1096, 448, True, True),  # chunks past K masked
+    (2049, 1033, 256, False, False), (2049, 1033, 72, False, True), (2049, 1033, 96, True, False),   # odd widths
+    (2049, 1096, 77, False, False), (2049, 1033, 333, True, True)])                                  # unaligned rows
+def test_gemm_more_than_a_round_of_tiles(hexmi, dtype, trans_b, M, N, K, bias, residual):
+    _against_double(hexmi, dtype, dtype, trans_b, M, N, K, bias, residual, M + N + K)
 
 
 def test_gemm_closed_forms(hexmi):
