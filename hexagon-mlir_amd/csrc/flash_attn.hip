@@ -72,18 +72,24 @@ struct MaskTileLoader {
 // top of the block that uses them.
 // PADDED: the head is head_dim < D wide (a multiple of 8): Q, K, V and O rows are head_dim elements apart, the tiles
 // carry zero columns from head_dim to D (they add nothing to Q K^T; the output columns there are not stored).
+// PITCH: Q, K and V stand as `at` says (heads of other widths always; D columns wide: where they are not contiguous).
+// Rows of a head stay whole lines wherever they stand, so such a head is read at the same rate; what it saves is the copies, 5 us
+// and a launch each (a layer of 2 x 1000 x 768 with q, k, v as slices of one projection 117 -> 101 us). Heads that are contiguous keep
+// kernels that know it: their addresses are shifts.
 // WIDE (with PADDED, D = 128, four waves): a head of 128 < head_dim <= 256 columns as two 128-wide halves. The
 // scores are the sum over both halves' K tiles, the output two sets of accumulators, the second half's tiles padded
 // like a narrow head's; twice the LDS and about 100 registers more, so one workgroup per CU.
 template <typename T, typename OutT, int D, bool CAUSAL, bool GENERAL = false, int NW = 4, bool MASK_LDS = false,
-          bool PADDED = false, bool WIDE = false, bool MASKED = false>
+          bool PADDED = false, bool WIDE = false, bool MASKED = false, bool PITCH = PADDED && !GENERAL>
 __global__ __launch_bounds__(NW * 64, NW == 4 && !WIDE ? (D == 64 && !GENERAL ? 3 : 2) : 1)
 void flash_fwd_kernel(const T* __restrict__ Q, const T* __restrict__ K, const T* __restrict__ V,
                       OutT* __restrict__ O, int ZH, int S, float scale_log2e, const T* __restrict__ Mk = nullptr,
-                      int Skv_arg = 0, float sm_scale = 0.0f, int group_heads = 0, int head_dim = D) {
+                      int Skv_arg = 0, float sm_scale = 0.0f, int group_heads = 0, int head_dim = D, HeadRows at = {}) {
   static_assert(!(CAUSAL && GENERAL), "the causal kernel has as many keys as queries and no mask");
   static_assert(!WIDE || (PADDED && D == 128 && NW == 4 && !GENERAL), "two halves of 128 columns, four waves, no mask");
-  const int dh = PADDED ? head_dim : D;                 // elements between rows in memory
+  const int dh = PADDED ? head_dim : D;                 // columns of a head; elements between rows of O
+  const int k_row = PITCH ? (int)at.k.row : dh, v_row = PITCH ? (int)at.v.row : dh;
+  static_assert(!PITCH || !GENERAL, "strides: self-attention without a mask");
   static_assert(!MASKED || GENERAL, "masks: general kernel");
   static_assert(!MASK_LDS || (MASKED && NW == 8), "staged mask tiles: 8 waves");
   const int Skv = GENERAL ? Skv_arg : S;
@@ -163,9 +169,10 @@ void flash_fwd_kernel(const T* __restrict__ Q, const T* __restrict__ K, const T*
     }
     const int64_t base = (int64_t)zh * S * dh;
     const int64_t kv_base = (int64_t)zh * Skv * dh;
-    const T* q_g = Q + base;
-    const T* k_g = K + kv_base;
-    const T* v_g = V + kv_base;
+    const T* q_g = Q + (PITCH ? head_at(at.q, at.heads, zh) : base);
+    const T* k_g = K + (PITCH ? head_at(at.k, at.heads, zh) : kv_base);
+    const T* v_g = V + (PITCH ? head_at(at.v, at.heads, zh) : kv_base);
+    const int64_t q_row = PITCH ? at.q.row : dh;
 
     const int q0 = qb * kBlockM + wave * 32;           // first query row of this wave
     const int qrow = q0 + lane % 32;                    // the query row this lane's scores belong to
@@ -177,7 +184,7 @@ void flash_fwd_kernel(const T* __restrict__ Q, const T* __restrict__ K, const T*
       const int qr = qrow < S ? qrow : S - 1;
 #pragma unroll
       for (int ds = 0; ds < DS; ++ds) {
-        if (!PADDED || ds * 16 + half * 8 < dh) qf[ds] = *reinterpret_cast<const Frag*>(q_g + (int64_t)qr * dh + ds * 16 + half * 8);
+        if (!PADDED || ds * 16 + half * 8 < dh) qf[ds] = *reinterpret_cast<const Frag*>(q_g + qr * q_row + ds * 16 + half * 8);
         else qf[ds] = Frag{};
       }
     }
@@ -186,7 +193,7 @@ void flash_fwd_kernel(const T* __restrict__ Q, const T* __restrict__ K, const T*
       const int qr = qrow < S ? qrow : S - 1;
 #pragma unroll
       for (int ds = 0; ds < DS; ++ds) {
-        if (D + ds * 16 + half * 8 < dh) qfb[ds] = *reinterpret_cast<const Frag*>(q_g + (int64_t)qr * dh + D + ds * 16 + half * 8);
+        if (D + ds * 16 + half * 8 < dh) qfb[ds] = *reinterpret_cast<const Frag*>(q_g + qr * q_row + D + ds * 16 + half * 8);
         else qfb[ds] = Frag{};
       }
     }
@@ -206,15 +213,15 @@ void flash_fwd_kernel(const T* __restrict__ Q, const T* __restrict__ K, const T*
     const int key_end = CAUSAL ? ((qb + 1) * kBlockM < S ? (qb + 1) * kBlockM : S) : Skv;
     const int n_steps = (key_end + kBlockN - 1) / kBlockN;
 
-    KvTileLoader<T, D, false, NW, PADDED> k_loader;
-    KvTileLoader<T, D, true, NW, PADDED> v_loader;
-    k_loader.init(wave, lane, dh, dh);
-    v_loader.init(wave, lane, dh, dh);
-    KvTileLoader<T, D, false, NW, PADDED> kb_loader;   // WIDE: the second halves, from 128 columns into the rows
-    KvTileLoader<T, D, true, NW, PADDED> vb_loader;
+    KvTileLoader<T, D, false, NW, PADDED, PADDED || PITCH> k_loader;
+    KvTileLoader<T, D, true, NW, PADDED, PADDED || PITCH> v_loader;
+    k_loader.init(wave, lane, k_row, dh);
+    v_loader.init(wave, lane, v_row, dh);
+    KvTileLoader<T, D, false, NW, PADDED, PADDED || PITCH> kb_loader;   // WIDE: the second halves, from 128 columns into the rows
+    KvTileLoader<T, D, true, NW, PADDED, PADDED || PITCH> vb_loader;
     if constexpr (WIDE) {
-      kb_loader.init(wave, lane, dh, dh - D);
-      vb_loader.init(wave, lane, dh, dh - D);
+      kb_loader.init(wave, lane, k_row, dh - D);
+      vb_loader.init(wave, lane, v_row, dh - D);
     }
     MaskTileLoader<T> m_loader;
     const T* mask_wg = nullptr;
@@ -625,24 +632,27 @@ inline int plan_causal_groups(int64_t ZH, int64_t nqb, int64_t grid) {
 
 template <typename T, typename OutT, int D, bool CAUSAL, int NW>
 int launch_mfma_nw(const void* Q, const void* K, const void* V, void* O, int64_t ZH, int64_t S, float scale_log2e,
-                   hipStream_t st, int per_cu = NW == 4 ? 2 : 1) {
+                   const HeadRows& at, hipStream_t st, int per_cu = NW == 4 ? 2 : 1) {
   const int64_t nqb = (S + NW * 32 - 1) / (NW * 32);
   const int64_t units = nqb * ZH;
   if (units > 0x7fffffff) return HEXMI_ENOTSUP;
   const int64_t blocks = resident_grid(units, per_cu);
   if (blocks <= 0) return HEXMI_ELAUNCH;
   const int groups = CAUSAL ? plan_causal_groups(ZH, nqb, blocks) : 0;
-  hipLaunchKernelGGL((flash_fwd_kernel<T, OutT, D, CAUSAL, false, NW>), dim3((unsigned)blocks), dim3(NW * 64), 0, st,
-                     static_cast<const T*>(Q), static_cast<const T*>(K), static_cast<const T*>(V),
-                     static_cast<OutT*>(O), (int)ZH, (int)S, scale_log2e, static_cast<const T*>(nullptr), 0, 0.0f,
-                     groups);
+#define HEXMI_PLAIN(PITCH)                                                                                                 \
+  hipLaunchKernelGGL((flash_fwd_kernel<T, OutT, D, CAUSAL, false, NW, false, false, false, false, PITCH>),                 \
+                     dim3((unsigned)blocks), dim3(NW * 64), 0, st, static_cast<const T*>(Q), static_cast<const T*>(K),     \
+                     static_cast<const T*>(V), static_cast<OutT*>(O), (int)ZH, (int)S, scale_log2e,                        \
+                     static_cast<const T*>(nullptr), 0, 0.0f, groups, D, at)
+  if (at.contiguous) HEXMI_PLAIN(false); else HEXMI_PLAIN(true);
+#undef HEXMI_PLAIN
   return launch_status();
 }
 
 // A head of head_dim < D columns (a multiple of 8) on the kernel for D: 128-row workgroups, two per CU.
 template <typename T, typename OutT, int D, bool CAUSAL>
 int launch_mfma_padded(const void* Q, const void* K, const void* V, void* O, int64_t ZH, int64_t S, int head_dim,
-                       float scale_log2e, hipStream_t st) {
+                       float scale_log2e, const HeadRows& at, hipStream_t st) {
   const int64_t nqb = (S + 127) / 128;
   const int64_t units = nqb * ZH;
   if (units > 0x7fffffff) return HEXMI_ENOTSUP;
@@ -652,7 +662,7 @@ int launch_mfma_padded(const void* Q, const void* K, const void* V, void* O, int
   hipLaunchKernelGGL((flash_fwd_kernel<T, OutT, D, CAUSAL, false, 4, false, true>), dim3((unsigned)blocks), dim3(256), 0, st,
                      static_cast<const T*>(Q), static_cast<const T*>(K), static_cast<const T*>(V),
                      static_cast<OutT*>(O), (int)ZH, (int)S, scale_log2e, static_cast<const T*>(nullptr), 0, 0.0f,
-                     groups, head_dim);
+                     groups, head_dim, at);
   return launch_status();
 }
 
@@ -660,7 +670,7 @@ int launch_mfma_padded(const void* Q, const void* K, const void* V, void* O, int
 // workgroup per CU.
 template <typename T, typename OutT, bool CAUSAL>
 int launch_mfma_wide(const void* Q, const void* K, const void* V, void* O, int64_t ZH, int64_t S, int head_dim,
-                     float scale_log2e, hipStream_t st) {
+                     float scale_log2e, const HeadRows& at, hipStream_t st) {
   const int64_t nqb = (S + 127) / 128;
   const int64_t units = nqb * ZH;
   if (units > 0x7fffffff) return HEXMI_ENOTSUP;
@@ -670,13 +680,13 @@ int launch_mfma_wide(const void* Q, const void* K, const void* V, void* O, int64
   hipLaunchKernelGGL((flash_fwd_kernel<T, OutT, 128, CAUSAL, false, 4, false, true, true>), dim3((unsigned)blocks), dim3(256), 0,
                      st, static_cast<const T*>(Q), static_cast<const T*>(K), static_cast<const T*>(V),
                      static_cast<OutT*>(O), (int)ZH, (int)S, scale_log2e, static_cast<const T*>(nullptr), 0, 0.0f,
-                     groups, head_dim);
+                     groups, head_dim, at);
   return launch_status();
 }
 
 template <typename T, typename OutT, int D>
 int launch_mfma(const void* Q, const void* K, const void* V, void* O, int64_t ZH, int64_t S, float scale_log2e,
-                bool causal, hipStream_t st) {
+                bool causal, const HeadRows& at, hipStream_t st) {
   // 256-row workgroups halve the L2 -> LDS copy traffic (1-9 % faster from 2048 keys on), if there are enough of
   // them to fill the chip; smaller problems keep the larger number of 128-row workgroups
   const bool wide = S >= kWideMinS && ZH * ((S + 255) / 256) >= hexmi_num_cus();
@@ -684,15 +694,15 @@ int launch_mfma(const void* Q, const void* K, const void* V, void* O, int64_t ZH
   // between 2048 and 4095 keys when every workgroup still gets two units or more; fewer units balance better two per CU
   const bool three = D == 64 && S >= kWideMinS && S < 4096 && ZH * ((S + 127) / 128) >= 6 * (int64_t)hexmi_num_cus();
   if (three) {
-    if (causal) return launch_mfma_nw<T, OutT, D, true, 4>(Q, K, V, O, ZH, S, scale_log2e, st, 3);
-    return launch_mfma_nw<T, OutT, D, false, 4>(Q, K, V, O, ZH, S, scale_log2e, st, 3);
+    if (causal) return launch_mfma_nw<T, OutT, D, true, 4>(Q, K, V, O, ZH, S, scale_log2e, at, st, 3);
+    return launch_mfma_nw<T, OutT, D, false, 4>(Q, K, V, O, ZH, S, scale_log2e, at, st, 3);
   }
   if (causal) {
-    if (wide) return launch_mfma_nw<T, OutT, D, true, 8>(Q, K, V, O, ZH, S, scale_log2e, st);
-    return launch_mfma_nw<T, OutT, D, true, 4>(Q, K, V, O, ZH, S, scale_log2e, st);
+    if (wide) return launch_mfma_nw<T, OutT, D, true, 8>(Q, K, V, O, ZH, S, scale_log2e, at, st);
+    return launch_mfma_nw<T, OutT, D, true, 4>(Q, K, V, O, ZH, S, scale_log2e, at, st);
   }
-  if (wide) return launch_mfma_nw<T, OutT, D, false, 8>(Q, K, V, O, ZH, S, scale_log2e, st);
-  return launch_mfma_nw<T, OutT, D, false, 4>(Q, K, V, O, ZH, S, scale_log2e, st);
+  if (wide) return launch_mfma_nw<T, OutT, D, false, 8>(Q, K, V, O, ZH, S, scale_log2e, at, st);
+  return launch_mfma_nw<T, OutT, D, false, 4>(Q, K, V, O, ZH, S, scale_log2e, at, st);
 }
 
 // head_dim < D: the 128-row form on padded tiles (the mask comes straight from global memory)
@@ -750,32 +760,36 @@ inline bool matrix_core_operands(const void* Q, const void* K, const void* V, co
          scale_log2e > 0.0f;
 }
 
+// bytes a head's keys or values span, for those offsets
+inline int64_t head_bytes(const HeadRows& at, int64_t Skv) { return Skv * std::max(at.k.row, at.v.row) * 2; }
+
 // whether the rows of a mask are whole aligned runs of four keys
 inline bool mask_in_runs(const void* mask, int64_t Skv) { return Skv % 4 == 0 && aligned_to(mask, 8); }
 
 // mask == nullptr and Skv == S: the tuned kernels; otherwise the general ones.
 template <typename T, typename OutT>
 int dispatch_half(const void* Q, const void* K, const void* V, const void* mask, void* O, int64_t ZH, int64_t S,
-                  int64_t Skv, int64_t D, float scale_log2e, bool causal, hipStream_t st) {
-  const bool ok = matrix_core_operands(Q, K, V, O, Skv * D * (int64_t)sizeof(T), scale_log2e);
+                  int64_t Skv, int64_t D, float scale_log2e, bool causal, const HeadRows& at, hipStream_t st) {
+  const bool ok = matrix_core_operands(Q, K, V, O, head_bytes(at, Skv), scale_log2e);
   const bool plain = !mask && Skv == S;
-  if (ok && plain && D == 128) return launch_mfma<T, OutT, 128>(Q, K, V, O, ZH, S, scale_log2e, causal, st);
-  if (ok && plain && D == 64) return launch_mfma<T, OutT, 64>(Q, K, V, O, ZH, S, scale_log2e, causal, st);
+  if (ok && plain && D == 128) return launch_mfma<T, OutT, 128>(Q, K, V, O, ZH, S, scale_log2e, causal, at, st);
+  if (ok && plain && D == 64) return launch_mfma<T, OutT, 64>(Q, K, V, O, ZH, S, scale_log2e, causal, at, st);
   // other head sizes up to 128 in multiples of 8 (rows on 16-byte boundaries): the same kernels on tiles padded with
   // zero columns to 64 or 128 ([2,16,2048,80] causal: 9.9 ms on the row-wise kernel)
   if (ok && plain && D % 8 == 0 && D < 128) {
     if (D < 64) {
-      if (causal) return launch_mfma_padded<T, OutT, 64, true>(Q, K, V, O, ZH, S, (int)D, scale_log2e, st);
-      return launch_mfma_padded<T, OutT, 64, false>(Q, K, V, O, ZH, S, (int)D, scale_log2e, st);
+      if (causal) return launch_mfma_padded<T, OutT, 64, true>(Q, K, V, O, ZH, S, (int)D, scale_log2e, at, st);
+      return launch_mfma_padded<T, OutT, 64, false>(Q, K, V, O, ZH, S, (int)D, scale_log2e, at, st);
     }
-    if (causal) return launch_mfma_padded<T, OutT, 128, true>(Q, K, V, O, ZH, S, (int)D, scale_log2e, st);
-    return launch_mfma_padded<T, OutT, 128, false>(Q, K, V, O, ZH, S, (int)D, scale_log2e, st);
+    if (causal) return launch_mfma_padded<T, OutT, 128, true>(Q, K, V, O, ZH, S, (int)D, scale_log2e, at, st);
+    return launch_mfma_padded<T, OutT, 128, false>(Q, K, V, O, ZH, S, (int)D, scale_log2e, at, st);
   }
   // ... and up to 256 as two halves of 128
   if (ok && plain && D % 8 == 0 && D > 128 && D <= 256) {
-    if (causal) return launch_mfma_wide<T, OutT, true>(Q, K, V, O, ZH, S, (int)D, scale_log2e, st);
-    return launch_mfma_wide<T, OutT, false>(Q, K, V, O, ZH, S, (int)D, scale_log2e, st);
+    if (causal) return launch_mfma_wide<T, OutT, true>(Q, K, V, O, ZH, S, (int)D, scale_log2e, at, st);
+    return launch_mfma_wide<T, OutT, false>(Q, K, V, O, ZH, S, (int)D, scale_log2e, at, st);
   }
+  if (!at.contiguous) return HEXMI_ENOTSUP;
   // (a mask is read in runs of four keys; without one any key count goes: cross-attention over 77 keys, say)
   const bool general_ok = ok && !causal && (!mask || mask_in_runs(mask, Skv));
   if (general_ok && D == 128) return launch_mfma_general<T, OutT, 128>(Q, K, V, mask, O, ZH, S, Skv, scale_log2e, st);
@@ -787,27 +801,29 @@ int dispatch_half(const void* Q, const void* K, const void* V, const void* mask,
 
 int attention_any(const void* Q, const void* K, const void* V, const void* mask, void* O, int64_t ZH, int64_t S,
                   int64_t Skv, int64_t D, float sm_scale, bool cz, int in_dtype, int out_dtype, void* workspace,
-                  int64_t workspace_bytes, hipStream_t st) {
+                  int64_t workspace_bytes, const HeadRows& at, hipStream_t st) {
   const float c = sm_scale * kLog2e;
   const bool half = (in_dtype == HEXMI_F16 || in_dtype == HEXMI_BF16) && (out_dtype == in_dtype || out_dtype == HEXMI_F32);
-  if (half && flash_decode_takes(ZH, S, Skv, D) && matrix_core_operands(Q, K, V, O, Skv * D * 2, c))
-    return flash_decode(Q, K, V, mask, O, ZH, Skv, D, sm_scale, in_dtype, out_dtype, st);
+  if (half && flash_decode_takes(ZH, S, Skv, D) && matrix_core_operands(Q, K, V, O, head_bytes(at, Skv), c))
+    return !at.contiguous ? HEXMI_ENOTSUP : flash_decode(Q, K, V, mask, O, ZH, Skv, D, sm_scale, in_dtype, out_dtype, st);
   // Masks that are not whole runs of four keys: flash_keys at any size, with the probabilities in full precision (the
   // row-wise kernel, the only other one that reads such a mask, holds them in fp32: 32 heads x 509 queries x 2555 keys
   // of 128 take it 11.4 ms). It reads masks in pieces of eight.
   const bool any_mask = mask != nullptr && !mask_in_runs(mask, Skv);
-  if (half && (!any_mask || ZH * S * Skv >= 8) && matrix_core_operands(Q, K, V, O, Skv * D * 2, c)) {
+  if (half && (!any_mask || ZH * S * Skv >= 8) && matrix_core_operands(Q, K, V, O, head_bytes(at, Skv), c)) {
     const FlashKeysPlan plan = plan_flash_keys(ZH, S, Skv, D, cz, mask != nullptr, any_mask, workspace != nullptr);
     if (plan.splits > 0) {
       if (plan.splits > 1 && (workspace_bytes < flash_keys_workspace(plan, ZH, S, D) || !aligned_to(workspace, 16)))
         return HEXMI_EINVAL;
-      return flash_keys(Q, K, V, mask, O, ZH, S, Skv, D, sm_scale, cz, in_dtype, out_dtype, plan, static_cast<float*>(workspace), st);
+      return flash_keys(Q, K, V, mask, O, ZH, S, Skv, D, sm_scale, cz, in_dtype, out_dtype, plan, static_cast<float*>(workspace),
+                        at, st);
     }
   }
-  if (in_dtype == HEXMI_F16 && out_dtype == HEXMI_F16) return dispatch_half<f16, f16>(Q, K, V, mask, O, ZH, S, Skv, D, c, cz, st);
-  if (in_dtype == HEXMI_F16 && out_dtype == HEXMI_F32) return dispatch_half<f16, float>(Q, K, V, mask, O, ZH, S, Skv, D, c, cz, st);
-  if (in_dtype == HEXMI_BF16 && out_dtype == HEXMI_BF16) return dispatch_half<bf16, bf16>(Q, K, V, mask, O, ZH, S, Skv, D, c, cz, st);
-  if (in_dtype == HEXMI_BF16 && out_dtype == HEXMI_F32) return dispatch_half<bf16, float>(Q, K, V, mask, O, ZH, S, Skv, D, c, cz, st);
+  if (in_dtype == HEXMI_F16 && out_dtype == HEXMI_F16) return dispatch_half<f16, f16>(Q, K, V, mask, O, ZH, S, Skv, D, c, cz, at, st);
+  if (in_dtype == HEXMI_F16 && out_dtype == HEXMI_F32) return dispatch_half<f16, float>(Q, K, V, mask, O, ZH, S, Skv, D, c, cz, at, st);
+  if (in_dtype == HEXMI_BF16 && out_dtype == HEXMI_BF16) return dispatch_half<bf16, bf16>(Q, K, V, mask, O, ZH, S, Skv, D, c, cz, at, st);
+  if (in_dtype == HEXMI_BF16 && out_dtype == HEXMI_F32) return dispatch_half<bf16, float>(Q, K, V, mask, O, ZH, S, Skv, D, c, cz, at, st);
+  if (!at.contiguous) return HEXMI_ENOTSUP;
   if (in_dtype == HEXMI_F32 && out_dtype == HEXMI_F32) {
     int status = HEXMI_OK;
     if (flash_attn_f32_mfma(static_cast<const float*>(Q), static_cast<const float*>(K), static_cast<const float*>(V),
@@ -832,7 +848,27 @@ extern "C" int hexmi_flash_attn_fwd(const void* Q, const void* K, const void* V,
   if (S > 0x7fffffff / 2 || Z * H > 0x7fffffff) return HEXMI_ENOTSUP;
   begin_call();
   return attention_any(Q, K, V, nullptr, O, Z * H, S, S, D, sm_scale, causal != 0, in_dtype, out_dtype, nullptr, 0,
-                       as_stream(stream));
+                       contiguous_heads(S, S, D), as_stream(stream));
+}
+
+extern "C" int hexmi_flash_attn_fwd_strided(const void* Q, const void* K, const void* V, void* O, int64_t Z, int64_t H,
+                                            int64_t S, int64_t D, const int64_t* strides, float sm_scale, int causal,
+                                            int in_dtype, int out_dtype, hexmi_stream_t stream) {
+  if (Z < 0 || H < 0 || S < 0 || D < 0) return HEXMI_EINVAL;
+  if (Z == 0 || H == 0 || S == 0 || D == 0) return HEXMI_OK;
+  if (!Q || !K || !V || !O || !strides) return HEXMI_EINVAL;
+  if (S > 0x7fffffff / 2 || Z * H > 0x7fffffff) return HEXMI_ENOTSUP;
+  // rows on 16-byte boundaries, offsets of rows within a head in 32 bits; the stride of a dimension of one means nothing
+  RowStrides r[3];
+  for (int i = 0; i < 3; ++i) {
+    r[i] = {Z > 1 ? strides[3 * i] : 0, H > 1 ? strides[3 * i + 1] : 0, S > 1 ? strides[3 * i + 2] : D};
+    if (r[i].batch % 8 != 0 || r[i].head % 8 != 0 || r[i].row % 8 != 0) return HEXMI_ENOTSUP;
+    if (r[i].batch < 0 || r[i].head < 0 || r[i].row < 0 || r[i].row > 0x7fffffff / 2 / S) return HEXMI_ENOTSUP;
+  }
+  if (in_dtype != HEXMI_F16 && in_dtype != HEXMI_BF16) return HEXMI_ENOTSUP;
+  begin_call();
+  return attention_any(Q, K, V, nullptr, O, Z * H, S, S, D, sm_scale, causal != 0, in_dtype, out_dtype, nullptr, 0,
+                       HeadRows{r[0], r[1], r[2], (int)H, false}, as_stream(stream));
 }
 
 extern "C" int hexmi_attention(const void* Q, const void* K, const void* V, const void* mask, void* O, int64_t batch,
@@ -862,5 +898,5 @@ extern "C" int hexmi_attention_ws(const void* Q, const void* K, const void* V, c
   if (seq_q > 0x7fffffff / 2 || seq_kv > 0x7fffffff / 2 || batch > 0x7fffffff) return HEXMI_ENOTSUP;
   begin_call();
   return attention_any(Q, K, V, mask, O, batch, seq_q, seq_kv, head_dim, sm_scale, false, in_dtype, out_dtype, workspace,
-                       workspace_bytes, as_stream(stream));
+                       workspace_bytes, contiguous_heads(seq_q, seq_kv, head_dim), as_stream(stream));
 }

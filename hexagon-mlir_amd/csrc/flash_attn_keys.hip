@@ -27,16 +27,17 @@ constexpr int kRows = 64;                        // queries of a workgroup: two 
 // global -> LDS copy of one [32 keys][D] tile by the two waves of a group, in the swizzled layout of the 64-key tiles.
 // PADDED: the head is d < D columns wide (a multiple of 8); a lane whose chunk lies past them copies nothing, and its LDS
 // positions, which no other lane writes, are zeroed once.
-template <typename T, int D, bool IS_V, bool PADDED>
+template <typename T, int D, bool IS_V, bool PADDED, bool PITCH>
 struct GroupTileLoader {
   static constexpr int CPR = D / 8;                        // 16-byte chunks per row
   static constexpr int NI = kTileKeys * CPR / 128;         // instructions per wave
   static constexpr int kRowStep = 128 / CPR;               // rows between a wave's instructions
   int row0, col[NI], lds0;                                 // this lane's row of instruction 0, its columns, the wave's part
-  int d;                                                   // elements between rows in memory
-  __device__ __forceinline__ void init(int rt, int lane, int head_dim) {
+  int d, row_step;                                         // columns of the head; elements between rows in memory (PITCH)
+  __device__ __forceinline__ void init(int rt, int lane, int head_dim, int pitch) {
     const int lin = rt * 64 + lane;
     d = PADDED ? head_dim : D;
+    row_step = PITCH ? pitch : D;
     row0 = lin / CPR;
     lds0 = rt * 64 * 8;
 #pragma unroll
@@ -50,7 +51,7 @@ struct GroupTileLoader {
     int key = key0 + row0 + j * kRowStep;
     key = key < Skv ? key : Skv - 1;
     if (!PADDED || col[j] < d)
-      copy_to_lds(reinterpret_cast<const char*>(g), (key * d + col[j]) * (int)sizeof(T), lds + lds0 + j * (128 * 8));
+      copy_to_lds(reinterpret_cast<const char*>(g), (key * row_step + col[j]) * (int)sizeof(T), lds + lds0 + j * (128 * 8));
   }
   __device__ __forceinline__ void zero_padding(T* lds, int lane) const {
 #pragma unroll
@@ -83,11 +84,12 @@ __device__ __forceinline__ void take_part(const bf16x8& part, float* p) {
 // small probability stays above 2^-24) or 16 (bf16, whose result is rounded to 8), three 24 (bf16 with an fp32 result). For
 // an fp32 result the parts of a tile meet in registers of their own, so that the running sum is rounded once a tile.
 // A part costs its share of MFMAs: 32 heads x 509 queries x 2555 keys of 128 with a mask 40 us in one part, 46 in two.
-template <typename T, typename OutT, int D, bool CAUSAL, bool MASKED, bool PADDED, bool FULL>
+// PITCH: Q, K and V stand as `at` says (narrower heads always; D columns wide: where they are not contiguous).
+template <typename T, typename OutT, int D, bool CAUSAL, bool MASKED, bool PADDED, bool FULL, bool PITCH>
 __global__ __launch_bounds__(512, D == 64 && !MASKED ? 4 : 2)
 void flash_keys_kernel(const T* __restrict__ Q, const T* __restrict__ K, const T* __restrict__ V, OutT* __restrict__ O,
                        int ZH, int S, int Skv, float scale, const T* __restrict__ Mk, float* __restrict__ part,
-                       int chunk, int splits, int head_dim) {
+                       int chunk, int splits, int head_dim, HeadRows at) {
   const int dh = PADDED ? head_dim : D;                 // elements between rows in memory
   static_assert(!(CAUSAL && MASKED), "the causal kernel has no mask");
   static_assert(!FULL || MASKED, "full probabilities: masked kernel");
@@ -139,16 +141,17 @@ void flash_keys_kernel(const T* __restrict__ Q, const T* __restrict__ K, const T
   const int first = split * chunk;                      // causal units are never cut
   const int last = first + chunk < unit_steps ? first + chunk : unit_steps;
 
-  const T* k_g = K + (int64_t)zh * Skv * dh;
-  const T* v_g = V + (int64_t)zh * Skv * dh;
+  const T* q_g = Q + (PITCH ? head_at(at.q, at.heads, zh) : (int64_t)zh * S * D);
+  const T* k_g = K + (PITCH ? head_at(at.k, at.heads, zh) : (int64_t)zh * Skv * D);
+  const T* v_g = V + (PITCH ? head_at(at.v, at.heads, zh) : (int64_t)zh * Skv * D);
   const int q0 = qb * kRows + rt * 32;
   const int qrow = q0 + lane % 32;
   const int qr = qrow < S ? qrow : S - 1;
 
-  GroupTileLoader<T, D, false, PADDED> k_loader;
-  GroupTileLoader<T, D, true, PADDED> v_loader;
-  k_loader.init(rt, lane, dh);
-  v_loader.init(rt, lane, dh);
+  GroupTileLoader<T, D, false, PADDED, PITCH> k_loader;
+  GroupTileLoader<T, D, true, PADDED, PITCH> v_loader;
+  k_loader.init(rt, lane, dh, (int)at.k.row);
+  v_loader.init(rt, lane, dh, (int)at.v.row);
   const int lds_g = ks * kTile;
   if constexpr (PADDED) {                               // ahead of the first barrier of the key loop
     k_loader.zero_padding(k_lds0 + lds_g, lane);
@@ -156,7 +159,7 @@ void flash_keys_kernel(const T* __restrict__ Q, const T* __restrict__ K, const T
     v_loader.zero_padding(v_lds0 + lds_g, lane);
     v_loader.zero_padding(v_lds1 + lds_g, lane);
   }
-  constexpr int kCopies = 2 * GroupTileLoader<T, D, false, PADDED>::NI;
+  constexpr int kCopies = 2 * GroupTileLoader<T, D, false, PADDED, PITCH>::NI;
   auto load_one = [&](int c, int n0, T* k_dst, T* v_dst) __attribute__((always_inline)) {
     if (c < kCopies / 2) k_loader.issue_one(c, k_g, n0, Skv, k_dst + lds_g);
     else v_loader.issue_one(c - kCopies / 2, v_g, n0, Skv, v_dst + lds_g);
@@ -203,7 +206,7 @@ void flash_keys_kernel(const T* __restrict__ Q, const T* __restrict__ K, const T
 #pragma unroll
   for (int ds = 0; ds < DS; ++ds) {
     if (!PADDED || ds * 16 + half * 8 < dh)
-      qf[ds] = *reinterpret_cast<const Frag*>(Q + ((int64_t)zh * S + qr) * dh + ds * 16 + half * 8);
+      qf[ds] = *reinterpret_cast<const Frag*>(q_g + (PITCH ? qr * at.q.row : (int64_t)qr * D) + ds * 16 + half * 8);
     else
       qf[ds] = Frag{};
   }
@@ -474,25 +477,29 @@ void flash_merge_kernel(const float* __restrict__ part, OutT* __restrict__ O, in
 
 template <typename T, typename OutT, int D>
 int launch_keys(const void* Q, const void* K, const void* V, const void* mask, void* O, int64_t ZH, int64_t S,
-                int64_t Skv, int head_dim, float sm_scale, bool causal, const FlashKeysPlan& plan, float* part, hipStream_t st) {
+                int64_t Skv, int head_dim, float sm_scale, bool causal, const FlashKeysPlan& plan, float* part, const HeadRows& at,
+                hipStream_t st) {
   const int64_t blocks = (S + kRows - 1) / kRows * ZH * plan.splits, rows = ZH * S;     // see plan_flash_keys
   const int64_t merge_blocks = (rows + 1024 / D - 1) / (1024 / D);
   const float unit = mask != nullptr ? kLog2e : 1.0f, scale = mask != nullptr ? sm_scale : sm_scale * kLog2e;
-#define HEXMI_KEYS(C, M, P, F)                                                                                        \
-  hipLaunchKernelGGL((flash_keys_kernel<T, OutT, D, C, M, P, F>), dim3((unsigned)blocks), dim3(512), 0, st,           \
+#define HEXMI_KEYS(C, M, P, F, X)                                                                                     \
+  hipLaunchKernelGGL((flash_keys_kernel<T, OutT, D, C, M, P, F, X>), dim3((unsigned)blocks), dim3(512), 0, st,           \
                      static_cast<const T*>(Q), static_cast<const T*>(K), static_cast<const T*>(V),                    \
                      static_cast<OutT*>(O), (int)ZH, (int)S, (int)Skv, scale, static_cast<const T*>(mask), part,      \
-                     plan.chunk, plan.splits, head_dim)
+                     plan.chunk, plan.splits, head_dim, at)
   if (head_dim < D) {
-    if (causal) HEXMI_KEYS(true, false, true, false);
-    else if (plan.full) HEXMI_KEYS(false, true, true, true);
-    else if (mask != nullptr) HEXMI_KEYS(false, true, true, false);
-    else HEXMI_KEYS(false, false, true, false);
+    if (causal) HEXMI_KEYS(true, false, true, false, true);
+    else if (plan.full) HEXMI_KEYS(false, true, true, true, true);
+    else if (mask != nullptr) HEXMI_KEYS(false, true, true, false, true);
+    else HEXMI_KEYS(false, false, true, false, true);
+  } else if (!at.contiguous) {                             // self-attention only: no mask
+    if (causal) HEXMI_KEYS(true, false, false, false, true);
+    else HEXMI_KEYS(false, false, false, false, true);
   } else {
-    if (causal) HEXMI_KEYS(true, false, false, false);
-    else if (plan.full) HEXMI_KEYS(false, true, false, true);
-    else if (mask != nullptr) HEXMI_KEYS(false, true, false, false);
-    else HEXMI_KEYS(false, false, false, false);
+    if (causal) HEXMI_KEYS(true, false, false, false, false);
+    else if (plan.full) HEXMI_KEYS(false, true, false, true, false);
+    else if (mask != nullptr) HEXMI_KEYS(false, true, false, false, false);
+    else HEXMI_KEYS(false, false, false, false, false);
   }
 #undef HEXMI_KEYS
   if (plan.splits > 1)
@@ -561,10 +568,11 @@ int64_t flash_keys_workspace(const FlashKeysPlan& p, int64_t ZH, int64_t S, int6
 
 int flash_keys(const void* Q, const void* K, const void* V, const void* mask, void* O, int64_t ZH, int64_t S,
                int64_t Skv, int64_t D, float sm_scale, bool causal, int in_dtype, int out_dtype,
-               const FlashKeysPlan& plan, float* part, hipStream_t st) {
+               const FlashKeysPlan& plan, float* part, const HeadRows& at,
+                hipStream_t st) {
 #define HEXMI_KEYS_D(T, OutT)                                                                                          \
-  return D > 64 ? launch_keys<T, OutT, 128>(Q, K, V, mask, O, ZH, S, Skv, (int)D, sm_scale, causal, plan, part, st) \
-                : launch_keys<T, OutT, 64>(Q, K, V, mask, O, ZH, S, Skv, (int)D, sm_scale, causal, plan, part, st)
+  return D > 64 ? launch_keys<T, OutT, 128>(Q, K, V, mask, O, ZH, S, Skv, (int)D, sm_scale, causal, plan, part, at, st) \
+                : launch_keys<T, OutT, 64>(Q, K, V, mask, O, ZH, S, Skv, (int)D, sm_scale, causal, plan, part, at, st)
   if (in_dtype == HEXMI_F16 && out_dtype == HEXMI_F16) HEXMI_KEYS_D(f16, f16);
   if (in_dtype == HEXMI_F16 && out_dtype == HEXMI_F32) HEXMI_KEYS_D(f16, float);
   if (in_dtype == HEXMI_BF16 && out_dtype == HEXMI_BF16) HEXMI_KEYS_D(bf16, bf16);

@@ -61,7 +61,8 @@ template <int D> __device__ __forceinline__ int swz_vtile(int row) {
 // PADDED: the head is narrower than the tile (d % 8 == 0, d < D): rows are d elements apart in memory, and a lane
 // whose chunk lies past column d copies nothing -- its LDS positions, which no other lane ever writes, are zeroed
 // once by the kernel (zero_padding), so the tile reads as the head padded with zero columns.
-template <typename T, int D, bool IS_V, int NW = 4, bool PADDED = false>
+// PITCH: rows stand head_dim elements apart, whatever the head is wide.
+template <typename T, int D, bool IS_V, int NW = 4, bool PADDED = false, bool PITCH = PADDED>
 struct KvTileLoader {
   static constexpr int CPR = D / 8;                       // chunks per row
   static constexpr int NI = kBlockN * CPR / 64 / NW;      // instructions per wave
@@ -73,7 +74,7 @@ struct KvTileLoader {
   int off0;                                               // element offset of this lane's chunk inside a tile, j = 0
   int row0, col0;
   int lds_off0;
-  int d;                                                  // elements between rows in memory (D unless PADDED)
+  int d;                                                  // elements between rows in memory (D unless PITCH)
   bool live;                                              // this lane's chunk is inside the head
   // live_cols: columns of the tile that exist in memory (the head itself, or what is left of it for a tile that
   // starts at a column offset: the caller then passes the offset pointer)
@@ -81,7 +82,7 @@ struct KvTileLoader {
     const int lin = wave * 64 + lane;
     row0 = lin / CPR;
     col0 = ((lin % CPR) ^ (IS_V ? swz_vtile<D>(row0) : swz_ktile<D>(row0))) * 8;
-    d = PADDED ? head_dim : D;
+    d = PITCH ? head_dim : D;
     live = !PADDED || col0 < live_cols;
     off0 = row0 * d + col0;
     lds_off0 = wave * 64 * 8;

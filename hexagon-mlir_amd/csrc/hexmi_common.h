@@ -267,6 +267,24 @@ bool flash_attn_f32_mfma(const float* Q, const float* K, const float* V, const f
                          int64_t S, int64_t Skv, int64_t D, float scale_log2e, bool causal, hipStream_t stream,
                          int* status);
 
+// Where the rows of Q, K and V stand, in elements: head h of batch z starts at z * batch + h * head, its rows row apart. Contiguous
+// [Z,H,S,D] is what the attention kernels are compiled for; other strides (the slices of one projection) they take as arguments.
+struct RowStrides { int64_t batch, head, row; };
+struct HeadRows {
+  RowStrides q, k, v;
+  int heads;
+  bool contiguous;
+};
+inline HeadRows contiguous_heads(int64_t S, int64_t Skv, int64_t D) {
+  return {{S * D, S * D, D}, {Skv * D, Skv * D, D}, {Skv * D, Skv * D, D}, 1, true};
+}
+#if defined(__HIPCC__)
+__device__ __forceinline__ int64_t head_at(const RowStrides& r, int heads, int zh) {
+  const int z = zh / heads;
+  return z * r.batch + (zh - z * heads) * r.head;
+}
+#endif
+
 // 16-bit flash attention of few (head, query block) units, the keys of a unit divided inside and over workgroups
 // (flash_attn_keys.hip). plan: splits == 0, leave it to the other kernels; > 1, the fp32 sums of that many chunks of
 // the key range go through a workspace; full, the probabilities keep fp32 precision into the second product. any_mask: a
@@ -280,7 +298,7 @@ FlashKeysPlan plan_flash_keys(int64_t ZH, int64_t S, int64_t Skv, int64_t D, boo
 int64_t flash_keys_workspace(const FlashKeysPlan& plan, int64_t ZH, int64_t S, int64_t D);
 int flash_keys(const void* Q, const void* K, const void* V, const void* mask, void* O, int64_t ZH, int64_t S,
                int64_t Skv, int64_t D, float sm_scale, bool causal, int in_dtype, int out_dtype,
-               const FlashKeysPlan& plan, float* part, hipStream_t st);
+               const FlashKeysPlan& plan, float* part, const HeadRows& at, hipStream_t st);
 
 // 16-bit attention of one query per head over many heads (flash_decode.hip): whether it takes a problem, and the launch.
 bool flash_decode_takes(int64_t ZH, int64_t S, int64_t Skv, int64_t D);

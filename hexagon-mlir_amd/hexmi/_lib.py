@@ -53,6 +53,8 @@ SIGNATURES = {
     "hexmi_dequant_w8_ex": (_int, [_i64, _i64, _ptr, _ptr, _ptr, _int, _ptr, _ptr]),
     "hexmi_gemm_w8a16_ex": (_int, [_i64, _i64, _i64, _ptr, _ptr, _ptr, _ptr, _int, _ptr, _ptr]),
     "hexmi_flash_attn_fwd": (_int, [_ptr, _ptr, _ptr, _ptr, _i64, _i64, _i64, _i64, _f32, _int, _int, _int, _ptr]),
+    "hexmi_flash_attn_fwd_strided": (_int, [_ptr, _ptr, _ptr, _ptr, _i64, _i64, _i64, _i64, _ptr, _f32, _int, _int, _int,
+                                            _ptr]),
     "hexmi_attention_workspace": (_i64, [_i64, _i64, _i64, _i64, _int, _int]),
     "hexmi_attention_ws": (_int, [_ptr, _ptr, _ptr, _ptr, _ptr, _i64, _i64, _i64, _i64, _f32, _int, _int, _ptr, _i64,
                                   _ptr]),

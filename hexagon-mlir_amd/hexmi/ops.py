@@ -11,6 +11,7 @@ device results back into the tensors the user passed).
 There is no CPU implementation: without a GPU or without libhexmi.so these
 functions raise.
 """
+import ctypes
 import math
 
 import torch
@@ -204,6 +205,22 @@ def _flash_impl(q, k, v, sm_scale, causal, out):
                    "hexmi_flash_attn_fwd")
 
 
+_Strides9 = ctypes.c_int64 * 9
+
+
+def _flash_strided(q, k, v, sm_scale, causal, out):
+    """Attention over device tensors read where they stand: True if the library takes their strides."""
+    Z, H, S, D = q.shape
+    strides = _Strides9(*q.stride()[:3], *k.stride()[:3], *v.stride()[:3])
+    with _on(q.device):
+        status = _lib.lib().hexmi_flash_attn_fwd_strided(_p(q), _p(k), _p(v), _p(out), Z, H, S, D, strides, sm_scale,
+                                                         1 if causal else 0, _dt(q), _dt(out), _stream())
+    if status == _lib.ENOTSUP:
+        return False
+    _lib.check(status, "hexmi_flash_attn_fwd_strided")
+    return True
+
+
 def _attention_impl(q, k, v, mask, sm_scale, out):
     B, Sq, D = q.shape
     Skv = k.shape[1]
@@ -271,6 +288,10 @@ def _stage(t, dev):
     if t.device.type != "cuda":
         t = t.to(dev, non_blocking=False)
     return t if t.is_contiguous() else t.contiguous()
+
+
+def _shares_storage(t, *others):
+    return any(t.untyped_storage().data_ptr() == o.untyped_storage().data_ptr() for o in others)
 
 
 def _finish(result, out):
@@ -544,8 +565,14 @@ def flash_attention(q, k, v, sm_scale=None, causal=False, out=None, out_dtype=No
     if out_dtype is None:
         out_dtype = out.dtype if out is not None else q.dtype
     dev = _device() if q.device.type != "cuda" else q.device
-    qd, kd, vd = _stage(q, dev), _stage(k, dev), _stage(v, dev)
     od = _out_like(out, q.shape, out_dtype, dev)
+    # slices of one projection and transposed heads are read where they stand (three copies, 5 us each for 2 x 12 x 1000 x 64)
+    if (not _THROUGH_DISPATCHER and (out is None or not _shares_storage(od, q, k, v)) and not (q.is_contiguous() and k.is_contiguous() and v.is_contiguous())
+            and q.device == k.device == v.device == od.device
+            and q.stride(3) == k.stride(3) == v.stride(3) == 1
+            and _flash_strided(q, k, v, float(sm_scale), causal, od)):
+        return _finish(od, out)
+    qd, kd, vd = _stage(q, dev), _stage(k, dev), _stage(v, dev)
     _run("flash_attention", _flash_impl, (qd, kd, vd, float(sm_scale), bool(causal), od), qd, kd, vd, float(sm_scale), bool(causal), od)
     return _finish(od, out)
 

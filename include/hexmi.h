@@ -325,6 +325,20 @@ int hexmi_flash_attn_fwd(const void *Q, const void *K, const void *V, void *O,
                          float sm_scale, int causal, int in_dtype,
                          int out_dtype, hexmi_stream_t stream);
 
+/* hexmi_flash_attn_fwd of Q, K and V that are not contiguous (slices of one
+ * projection, transposed or expanded heads): strides holds nine element
+ * strides, batch, head and row of Q, of K and of V; the D columns of a row are
+ * adjacent. O is contiguous [Z, H, S, D]. The same kernels, and bits, as of
+ * contiguous operands. 16-bit operands on 16-byte boundaries, strides in
+ * multiples of 8 (a dimension of one has none), D % 8 == 0, D <= 256,
+ * sm_scale > 0, S * row stride below 2^30; HEXMI_ENOTSUP for anything else, and for a
+ * single query (S == 1) of very many heads: copy the operands then. */
+int hexmi_flash_attn_fwd_strided(const void *Q, const void *K, const void *V,
+                                 void *O, int64_t Z, int64_t H, int64_t S,
+                                 int64_t D, const int64_t *strides,
+                                 float sm_scale, int causal, int in_dtype,
+                                 int out_dtype, hexmi_stream_t stream);
+
 /* tm_tensor.attention: O = softmax(sm_scale * Q K^T + mask) V per batch entry,
  * "Equivalent to : softmax(QK^T / sqrt(d_k) + mask) * V"
  * (include/hexagon/Dialect/TmTensor/IR/TmTensorOps.td:28-56; lowering

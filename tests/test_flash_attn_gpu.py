@@ -787,3 +787,82 @@ def test_attention_head_counts_off_the_multiple_of_eight(hexmi, case):
         scores = scores.masked_fill(torch.ones(Sq, Skv).triu(1).bool(), float("-inf"))
     want = torch.softmax(scores, dim=-1) @ v.float()
     assert (out.cpu() - want).abs().max() <= 5e-3
+
+
+def _standing(form, Z, H, S, D, dtype, g):
+    """q, k, v of one shape that are not contiguous, as programs have them."""
+    def r(*shape):
+        return torch.randn(*shape, generator=g).to(dtype).cuda()
+    if form == "slices":                                     # one projection [Z, S, 3 H D]
+        return tuple(t.view(Z, S, H, D).transpose(1, 2) for t in r(Z, S, 3 * H * D).split(H * D, dim=-1))
+    if form == "rows first":                                 # q [Z, S, H, D], k [S, Z, H, D], v contiguous
+        return r(Z, S, H, D).transpose(1, 2), r(S, Z, H, D).permute(1, 2, 0, 3), r(Z, H, S, D)
+    if form == "expanded":                                   # one key and value head for all, batches apart
+        return r(H, Z, S, D).transpose(0, 1), r(Z, 1, S, D).expand(Z, H, S, D), r(Z, S, 1, D).transpose(1, 2).expand(Z, H, S, D)
+    if form == "padded rows":
+        return tuple(r(Z, H, S, D + 8)[..., :D] for _ in range(3))
+    if form == "odd rows":                                   # rows off the 16-byte boundaries
+        return tuple(r(Z, H, S, D + 3)[..., :D] for _ in range(3))
+    if form == "off base":
+        return tuple(r(Z, H, S, D + 8)[..., 1:D + 1] for _ in range(3))
+    return tuple(r(Z, H, D, S).transpose(2, 3) for _ in range(3))        # "columns apart"
+
+
+# the key-group and the persistent kernels (128 and 256 queries a workgroup), padded and two-half heads, one query; the last
+# three forms, one query of many heads, a zero scale and fp32 are copied first
+@pytest.mark.parametrize("form", ["slices", "rows first", "expanded", "padded rows", "odd rows", "off base", "columns apart"])
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("case", [(2, 3, 200, 64, torch.bfloat16), (2, 4, 129, 128, torch.float16), (3, 40, 300, 64, torch.float16),
+                                  (2, 70, 130, 128, torch.bfloat16), (1, 64, 2100, 64, torch.float16), (2, 32, 1100, 128, torch.float16),
+                                  (2, 16, 2049, 128, torch.bfloat16), (2, 5, 100, 80, torch.float16), (2, 24, 515, 40, torch.bfloat16),
+                                  (1, 3, 70, 256, torch.float16), (2, 3, 1, 64, torch.float16), (2, 300, 1, 128, torch.float16),
+                                  (1, 2, 65, 64, torch.float32)])
+def test_attention_of_heads_where_they_stand(hexmi, form, causal, case):
+    Z, H, S, D, dtype = case
+    q, k, v = _standing(form, Z, H, S, D, dtype, _gen(S + D + H))
+    want = hexmi.flash_attention(q.contiguous(), k.contiguous(), v.contiguous(), 0.11, causal)
+    got = hexmi.flash_attention(q, k, v, 0.11, causal)
+    assert got.is_contiguous() and torch.equal(got, want)
+    out = torch.full_like(want, float("nan"))
+    assert hexmi.flash_attention(q, k, v, 0.11, causal, out=out) is out and torch.equal(out, want)
+    if S == 200:
+        zero = hexmi.flash_attention(q, k, v, 0.0, causal)
+        assert torch.equal(zero, hexmi.flash_attention(q.contiguous(), k.contiguous(), v.contiguous(), 0.0, causal))
+
+
+def test_attention_of_heads_where_they_stand_into_their_own_memory(hexmi):
+    # out lies in the storage of the operands: they are copied before anything is written
+    g = _gen(5)
+    Z, H, S, D = 1, 4, 300, 64
+    buf = torch.randn(4, Z * H * S * D, generator=g).half().cuda()
+    q, k, v = (buf[i].view(Z, S, H, D).transpose(1, 2) for i in range(3))
+    want = hexmi.flash_attention(q.contiguous(), k.contiguous(), v.contiguous(), 0.125, True)
+    got = hexmi.flash_attention(q, k, v, 0.125, True, out=buf[0].view(Z, H, S, D))
+    assert torch.equal(got, want)
+
+
+def test_strided_entry_refuses_what_it_cannot_read(hexmi):
+    import ctypes
+    from hexmi import _lib
+    lib = _lib.lib()
+    x = torch.zeros(1, 2, 64, 64, dtype=torch.float16, device="cuda")
+    out = torch.full_like(x, 7.0)
+    s = torch.cuda.current_stream().cuda_stream
+
+    def call(strides, dtype=_lib.F16, scale=0.1, S=64):
+        a = (ctypes.c_int64 * 9)(*strides)
+        p = x.data_ptr()
+        return lib.hexmi_flash_attn_fwd_strided(p, p, p, out.data_ptr(), 1, 2, S, 64, a, scale, 0, dtype, dtype, s)
+    good = [8192, 4096, 64] * 3
+    assert call([8192, 4096, 60] + good[3:]) == _lib.ENOTSUP
+    assert call(good[:3] + [8192, 4092, 64] + good[6:]) == _lib.ENOTSUP
+    assert call(good[:6] + [8192, 4096, -64]) == _lib.ENOTSUP
+    assert call(good[:3] + [8192, 4096, 1 << 28] + good[6:]) == _lib.ENOTSUP
+    assert call(good, _lib.F32) == _lib.ENOTSUP
+    assert call(good, scale=0.0) == _lib.ENOTSUP
+    p = x.data_ptr()
+    assert lib.hexmi_flash_attn_fwd_strided(p, p, p, p, 1, 2, 64, 64, None, 0.1, 0, _lib.F16, _lib.F16, s) == _lib.EINVAL
+    assert lib.hexmi_flash_attn_fwd_strided(None, None, None, None, 1, 0, 64, 64, None, 0.1, 0, _lib.F16, _lib.F16, s) == _lib.OK
+    torch.cuda.synchronize()
+    assert (out == 7.0).all()
+    assert call([3, 4096, 64] * 3) == _lib.OK                # a single batch has no stride
