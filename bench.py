@@ -108,6 +108,8 @@ class Softmax(Workload):
         # few long rows: every row is cut into column blocks, two launches (statistics, then the normalising sweep)
         if rows < 128 and cols >= 16384:
             self.kernel = "part_stats_kernel + part_apply_kernel"
+        elif cols * (4 if dtype == "f32" else 2) > 64 << 10:
+            self.kernel = "softmax_long_kernel"
 
     def setup(self, torch, hexmi):
         from hexmi.workloads import softmax_inputs, softmax_bytes

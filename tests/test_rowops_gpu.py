@@ -395,3 +395,68 @@ def test_rows_that_are_not_whole_chunks(hexmi, oracle, dtype, cols):
     assert torch.allclose(mean.cpu(), torch.from_numpy(want_mean), rtol=1e-5, atol=1e-6)
     assert torch.allclose(rstd.cpu(), torch.from_numpy(want_rstd), rtol=1e-5)
 
+
+
+# rows off the 16-byte boundaries of 3 MiB and more in all (norms over aligned spans): every tile, rows that are no whole
+# number of workgroups, a chunk of a row before its own line, and views whose rows lie apart
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("kind", ["rms", "layer"])
+@pytest.mark.parametrize("rows,cols,ld", [(13001, 131, 131), (6003, 1001, 1001), (1709, 2001, 2005), (411, 4099, 4099), (203, 8191, 8199),
+                                          (131, 12287, 12289), (77, 30001, 30001), (61, 32763, 32763), (41, 50257, 50264)])
+def test_norms_over_spans_of_aligned_chunks(hexmi, dtype, kind, rows, cols, ld):
+    if cols * torch.empty(0, dtype=dtype).element_size() > 128 << 10:
+        pytest.skip("rows of more than 128 KiB go another way")
+    from hexmi import _lib
+    g = _gen(cols)
+    x = torch.randn(rows, ld, generator=g).to(dtype).cuda()[:, :cols]
+    y = torch.full((rows, ld), 7.0, dtype=dtype, device="cuda")
+    w, b = (torch.randn(cols, generator=g).to(dtype).cuda() for _ in range(2))
+    mean, rstd = (torch.full((rows,), float("nan"), device="cuda") for _ in range(2))
+    code = {torch.float16: _lib.F16, torch.bfloat16: _lib.BF16, torch.float32: _lib.F32}[dtype]
+    s = torch.cuda.current_stream().cuda_stream
+    lib, xd = _lib.lib(), x.double()
+    if kind == "rms":
+        assert lib.hexmi_rms_norm_ws(x.data_ptr(), w.data_ptr(), y.data_ptr(), rows, cols, ld, ld, 1e-5, 0, code, None, 0, s) == _lib.OK
+        want = xd * torch.rsqrt(xd.pow(2).mean(1, keepdim=True) + 1e-5) * w.double()
+    else:
+        assert lib.hexmi_layer_norm_ws(x.data_ptr(), w.data_ptr(), b.data_ptr(), y.data_ptr(), mean.data_ptr(), rstd.data_ptr(), rows,
+                                       cols, ld, ld, 1e-5, 0, code, None, 0, s) == _lib.OK
+        mu, var = xd.mean(1, keepdim=True), xd.var(1, unbiased=False, keepdim=True)
+        want = (xd - mu) * torch.rsqrt(var + 1e-5) * w.double() + b.double()
+        assert (mean.double() - mu[:, 0]).abs().max() <= 1e-5 and (rstd.double() * torch.sqrt(var[:, 0] + 1e-5) - 1).abs().max() <= 1e-5
+    # half an ulp of the output type, and the fp32 statistics and products (a few 2^-24 of the operands)
+    eps = torch.finfo(dtype).eps
+    assert ((y[:, :cols].double() - want).abs() <= 0.5 * eps * want.abs() + 4e-6 * (1 + want.abs()) + 1e-8).all()
+    assert (y[:, cols:] == 7.0).all()
+
+
+# rows of 64 to 128 KiB: on lines and off them, the largest tile and one over the smaller, a row per CU and less or more, views that
+# start anywhere in a line, what max / sub / exp / sum / div gives for rows with infinities and NaN
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("rows", [3, 300])
+@pytest.mark.parametrize("kib,extra,off", [(64, 1, 0), (66, 0, 0), (90, 3, 0), (96, -7, 5), (96, 9, 16), (100, 8, 0), (128, -63, 9), (128, 0, 0),
+                                           (128, -1, 0)])
+def test_softmax_long_rows(hexmi, dtype, rows, kib, extra, off):
+    es = torch.empty(0, dtype=dtype).element_size()
+    cols = (kib << 10) // es + extra
+    g = torch.Generator(device="cuda").manual_seed(kib + extra)
+    buf = torch.randn(rows * cols + off, generator=g, device="cuda").mul_(3).to(dtype)
+    x = buf[off:].view(rows, cols)
+    out = torch.full((rows * cols + off + 8,), 7.0, dtype=dtype, device="cuda")
+    x[0, -1] = 30.0                                       # the last element matters
+    x[1, 0] = 30.0                                        # and the first
+    x[2, 5:] = float("-inf")
+    y = out[off:off + rows * cols].view(rows, cols)
+    hexmi.softmax(x, out=y)
+    want = torch.softmax(x.double(), dim=1)
+    # e^(x - m) within 2^-22 relative for |x - m| <= 40 (one product and one exponential in fp32), the sum and its reciprocal 2^-22, one rounding
+    eps = torch.finfo(dtype).eps
+    assert ((y.double() - want).abs() <= (0.5 * eps + 8e-6) * want + (6e-8 if dtype == torch.float16 else 1e-30)).all()
+    assert (out[:off] == 7.0).all() and (out[off + rows * cols:] == 7.0).all()
+    x[0, 7] = float("nan")
+    x[1] = float("-inf")
+    x[2, 3] = float("inf")
+    hexmi.softmax(x, out=y)
+    assert torch.isnan(y[0]).any() and torch.isnan(y[1]).all() and torch.isnan(y[2, 3])
+    if rows > 3:
+        assert ((y[3:].double() - want[3:]).abs() <= (0.5 * eps + 8e-6) * want[3:] + (6e-8 if dtype == torch.float16 else 1e-30)).all()
