@@ -1,4 +1,4 @@
-"""Build libhexmi.so (HIP kernels + C ABI) for gfx950, in-tree.
+"""Build libhexmi.so (HIP kernels + C ABI) for gfx950 and _front.so (its Python extension over torch), in-tree.
 
     python hexagon-mlir_amd/build.py            # incremental
     python hexagon-mlir_amd/build.py --force    # recompile everything
@@ -15,6 +15,8 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 INCLUDE = os.path.join(os.path.dirname(HERE), "include")
 OUT_LIB = os.path.join(HERE, "hexmi", "libhexmi.so")
+FRONT_SRC = os.path.join(CSRC, "torch_front.cpp")
+OUT_FRONT = os.path.join(HERE, "hexmi", "_front.so")
 OBJ_DIR = os.path.join(CSRC, "build")
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
@@ -72,6 +74,25 @@ def _compile(src, force, hdr_mtime):
     return obj, True
 
 
+def build_front(force=False):
+    """hexmi/_front.so: the operators' usual calls as a Python extension over torch's C++ headers and libhexmi.so (host code only)."""
+    import sysconfig
+    import torch
+    if (not force and os.path.exists(OUT_FRONT)
+            and os.path.getmtime(OUT_FRONT) > max(os.path.getmtime(FRONT_SRC), os.path.getmtime(os.path.join(INCLUDE, "hexmi.h")))):
+        return
+    root = os.path.dirname(torch.__file__)
+    rocm = os.path.dirname(os.path.dirname(HIPCC))
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+           "-D_GLIBCXX_USE_CXX11_ABI=%d" % torch._C._GLIBCXX_USE_CXX11_ABI, "-I", INCLUDE, "-I", os.path.join(root, "include"),
+           "-I", os.path.join(root, "include", "torch", "csrc", "api", "include"), "-I", os.path.join(rocm, "include"),
+           "-I", sysconfig.get_paths()["include"], FRONT_SRC, "-o", OUT_FRONT, "-L", os.path.join(root, "lib"), "-ltorch_python", "-ltorch",
+           "-ltorch_cpu", "-ltorch_hip", "-lc10", "-lc10_hip", "-L", os.path.dirname(OUT_LIB), "-l:libhexmi.so", "-Wl,-rpath,$ORIGIN"]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError("g++ failed for torch_front.cpp:\n%s\n%s" % (r.stdout, r.stderr))
+
+
 def build(force=False, verbose=True):
     os.makedirs(OBJ_DIR, exist_ok=True)
     hdr = _headers_mtime()
@@ -85,6 +106,7 @@ def build(force=False, verbose=True):
         r = subprocess.run(cmd, capture_output=True, text=True)
         if r.returncode != 0:
             raise RuntimeError("link failed:\n%s\n%s" % (r.stdout, r.stderr))
+    build_front(force)
     if verbose:
         print("libhexmi.so: %d sources, %s" % (len(srcs), "rebuilt" if rebuilt else "up to date"))
     return OUT_LIB
