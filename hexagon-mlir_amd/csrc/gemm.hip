@@ -23,7 +23,7 @@
 // Which kernel takes a product (dispatch_gemm): operand rows on 16-byte boundaries and whole 64-wide (gemm_kernel_k64)
 // or 32-wide (gemm_kernel) slabs of K -> the tiled kernels as described; K a multiple of 8 only -> gemm_kernel with
 // the last slab's chunks past K fetched from a zero chunk; an output side without runs of four columns (odd N with B
-// as [N,K], odd ldc, unaligned C) -> the same kernels with the tile leaving through LDS one element per lane;
+// as [N,K], odd ldc, unaligned C) -> the same kernels with the tile leaving through LDS in the pieces of 16 bytes that each row holds;
 // anything else (unaligned operand rows, K % 8 != 0) -> gemm_kernel_any, which stages the slabs through registers.
 // Up to eight rows against B as [N,K] -> gemv_nt_kernel, a stream of the weights with one wave per output channel.
 // Up to 64 rows against B as [N,K], by measured lines -> gemm_skinny.hip, a workgroup per 16 to 64 channels. Whole chunks of K and
@@ -740,6 +740,27 @@ template <> struct Mfma16<bf16> {
   }
 };
 
+// sixteen 16-bit columns in two chunks, from column `by` (0 .. 7) on: eight of them
+__device__ __forceinline__ u32x4 shift_columns(const u32x4& lo, const u32x4& hi, int by) {
+  auto pick = [](bool second, uint32_t v0, uint32_t v1) { return second ? v1 : v0; };    // (values, not places: no scratch)
+  const bool by4 = by & 4, by2 = by & 2;
+  const uint32_t x0 = pick(by4, lo[0], lo[2]), x1 = pick(by4, lo[1], lo[3]), x2 = pick(by4, lo[2], hi[0]),
+                 x3 = pick(by4, lo[3], hi[1]), x4 = pick(by4, hi[0], hi[2]), x5 = pick(by4, hi[1], hi[3]);
+  const uint32_t y0 = pick(by2, x0, x1), y1 = pick(by2, x1, x2), y2 = pick(by2, x2, x3), y3 = pick(by2, x3, x4),
+                 y4 = pick(by2, x4, x5);
+  const int bits = (by & 1) * 16;
+  const u32x4 o = {__builtin_amdgcn_alignbit(y1, y0, bits), __builtin_amdgcn_alignbit(y2, y1, bits),
+                   __builtin_amdgcn_alignbit(y3, y2, bits), __builtin_amdgcn_alignbit(y4, y3, bits)};
+  return o;
+}
+// the first NC columns of a piece, at an address that is a multiple of NC columns
+template <int NC, typename OutT>
+__device__ __forceinline__ void store_cols(OutT* p, const u32x4& v) {
+  if constexpr (NC == 4) *reinterpret_cast<u32x2*>(p) = u32x2{v[0], v[1]};
+  else if constexpr (NC == 2) *reinterpret_cast<uint32_t*>(p) = v[0];
+  else *reinterpret_cast<uint16_t*>(p) = (uint16_t)v[0];
+}
+
 // Two stages of [tile x 64], MFMA 16x16x32 (on random data the chip runs at its power limit, and this shape
 // sustains about 12 % more than 32x32x16 there: it updates a quarter of the accumulators per instruction for half
 // the products). A wave owns TM x TN tiles of 16x16 and runs, per paired slab j, two steps of 32 elements of K;
@@ -1029,7 +1050,7 @@ void gemm_kernel_k64(const T* __restrict__ A, const void* __restrict__ Bv, typen
   }
   if constexpr (sizeof(OutT) == 2) {
     // (the 256x256 tiles with a guarded last pass sit at the register limit: with this form they would spill)
-    const bool by_elements = (WM <= 2 || !TAIL) && out_elems;
+    const bool by_elements = !B_I8 && !EPI && (WM <= 2 || !TAIL) && out_elems;
     if (ldc % 8 == 0 || by_elements) {
       // 16-bit results go through LDS so that a store instruction writes whole rows of the wave's tile (TN*32
       // contiguous bytes per row) instead of 8-byte pieces of 16 rows. Each wave stages its tile in one of the four
@@ -1055,32 +1076,36 @@ void gemm_kernel_k64(const T* __restrict__ A, const void* __restrict__ Bv, typen
         }
       }
       if (by_elements) {
-        // A row of C starts anywhere, but most of it is whole 16-byte pieces: a lane gathers the eight elements of
-        // one aligned piece from the staged tile (they straddle two of its chunks) and stores them at once, 64 / CP
-        // rows per instruction; what a row has before its first boundary and after its last whole piece (up to
-        // seven elements each) goes element by element, a lane per row.
+        // A row of C starts anywhere: `lead` columns, then whole 16-byte pieces, then up to seven columns. A piece straddles two
+        // staged chunks; a lane takes both and shifts (staged in 16-bit reads this took eight per piece). The two waves side by
+        // side cover the tile's row as one: the left wave has the head and the piece on the seam, the right wave the tail, so
+        // a row of 256 columns has two ragged ends, each in up to three stores of four, two and one columns with a lane per
+        // row. (By elements, both waves with ends of their own, the ends were 28 stores of 64 lines each and wave, seven times
+        // the lines of the pieces: bf16 1021 x 50257 x 768 122 -> 106 us; its aligned neighbour N = 50264 takes 100.)
+        __syncthreads();                              // the left wave reads its neighbour's first chunks
         constexpr int W = TN * 16;                    // columns of the wave's tile
         const int gbase = n0 + wn * W;
-        const int ncols = N - gbase < W ? (int)(N - gbase) : W;
+        const int ncols = N - gbase < W + (wn ? 0 : kChunk) ? (int)(N - gbase) : W + (wn ? 0 : kChunk);   // it may reach into
+        const OutT* right = wave == 0 ? reinterpret_cast<OutT*>(a_p1) : reinterpret_cast<OutT*>(b_p1);    // the neighbour's
         const int64_t c_elem = (int64_t)(reinterpret_cast<uintptr_t>(C) / sizeof(OutT));
-        auto staged = [&](int row, int col) {
-          return cs[row * PITCH + (((col / kChunk) ^ swz(row)) * kChunk) + col % kChunk];
-        };
-        // columns up to the row's first 16-byte boundary
+        // columns up to the row's first 16-byte boundary (the same for both waves: W is whole pieces)
         auto lead_of = [&](int64_t e0) { return (int)((kChunk - ((c_elem + e0) & (kChunk - 1))) & (kChunk - 1)); };
+        // the eight columns of a row from lead + 8 q on (q < CP; past the right wave's last chunk: anything)
+        auto piece = [&](int row, int q, int lead) __attribute__((always_inline)) {
+          const OutT* next = q + 1 < CP ? cs + row * PITCH + (((q + 1) ^ swz(row)) * kChunk) : right + row * PITCH + (swz(row) * kChunk);
+          return shift_columns(*reinterpret_cast<const u32x4*>(cs + row * PITCH + ((q ^ swz(row)) * kChunk)),
+                               *reinterpret_cast<const u32x4*>(next), lead);
+        };
         constexpr int RPS = 64 / CP;
 #pragma unroll 2
         for (int r0 = 0; r0 < TM * 16; r0 += RPS) {
           const int row = r0 + lane / CP, q = lane % CP;
           const int grow = m0 + wm * TM * 16 + row;
           const int64_t e0 = (int64_t)grow * ldc + gbase;
-          const int c0 = lead_of(e0) + kChunk * q;
-          if (grow < M && c0 + kChunk <= ncols) {
-            __attribute__((aligned(16))) OutT o[kChunk];
-#pragma unroll
-            for (int i = 0; i < kChunk; ++i) o[i] = staged(row, c0 + i);
-            __builtin_nontemporal_store(*reinterpret_cast<const u32x4*>(o), reinterpret_cast<u32x4*>(C + e0 + c0));
-          }
+          const int lead = lead_of(e0);
+          const u32x4 v = piece(row, q, lead);
+          if (grow < M && lead + kChunk * (q + 1) <= ncols)
+            __builtin_nontemporal_store(v, reinterpret_cast<u32x4*>(C + e0 + lead + kChunk * q));
         }
 #pragma unroll 1
         for (int r0 = 0; r0 < TM * 16; r0 += 64) {
@@ -1089,20 +1114,27 @@ void gemm_kernel_k64(const T* __restrict__ A, const void* __restrict__ Bv, typen
           if (row < TM * 16 && grow < M && ncols > 0) {
             const int64_t e0 = (int64_t)grow * ldc + gbase;
             const int lead = lead_of(e0);
-            const int head = lead < ncols ? lead : ncols;
-            const int tail = ncols > lead ? lead + ((ncols - lead) & ~(kChunk - 1)) : ncols;
-            // every read ahead of the first store, the stores under masks (one read and one store per turn of a loop
-            // would put their latencies end to end)
-            OutT hv[kChunk - 1], tv[kChunk - 1];
+            // each end in descending powers of two away from its 16-byte boundary, which keeps every store aligned
+            if (wn == 0 && lead) {
+              const u32x4 v = *reinterpret_cast<const u32x4*>(cs + row * PITCH + (swz(row) * kChunk));
+              if (ncols < lead) {                     // the whole row ends before its first boundary
 #pragma unroll
-            for (int k = 0; k < kChunk - 1; ++k) {
-              hv[k] = staged(row, k);
-              tv[k] = staged(row, tail + k < W ? tail + k : W - 1);
+                for (int k = 0; k < kChunk - 1; ++k)
+                  if (k < ncols) store_cols<1>(C + e0 + k, shift_columns(v, v, k));
+              } else {
+                if (lead & 1) store_cols<1>(C + e0, v);
+                if (lead & 2) store_cols<2>(C + e0 + (lead & 1), shift_columns(v, v, lead & 1));
+                if (lead & 4) store_cols<4>(C + e0 + (lead & 3), shift_columns(v, v, lead & 3));
+              }
             }
-#pragma unroll
-            for (int k = 0; k < kChunk - 1; ++k) {
-              if (k < head) C[e0 + k] = hv[k];
-              if (tail + k < ncols) C[e0 + tail + k] = tv[k];
+            // behind the last whole piece; the left wave has such an end only where the matrix ends
+            const int pieces = ncols > lead ? (ncols - lead) / kChunk : 0, left = ncols > lead ? (ncols - lead) % kChunk : 0;
+            if (left && pieces < CP) {
+              const u32x4 v = piece(row, pieces, lead);
+              OutT* at = C + e0 + lead + kChunk * pieces;
+              if (left & 4) store_cols<4>(at, v);
+              if (left & 2) store_cols<2>(at + (left & 4), shift_columns(v, v, left & 4));
+              if (left & 1) store_cols<1>(at + (left & 6), shift_columns(v, v, left & 6));
             }
           }
         }
@@ -1494,7 +1526,7 @@ inline bool two_per_cu(int64_t tiles, int64_t K) {
   return tiles > cus && (pairs == 0 || over == 0 || over > cus || K < 1536 * pairs);
 }
 
-// out_elems: 16-bit results leave the paired-slab kernel one element per lane (the caller has checked that this
+// out_elems: 16-bit results leave the paired-slab kernel for rows off the 16-byte boundaries (the caller has checked that this
 // kernel takes the product: K % 64 == 0, short rows, no bias or residual).
 template <typename T, typename OutT, int WM, int WN, bool TRANS_B, int NWN = 2>
 int launch_tiled(const T* A, const T* B, OutT* C, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb,
@@ -1617,7 +1649,7 @@ int dispatch_gemm(const void* Av, const void* Bv, void* Cv, int64_t M, int64_t N
   // with a masked last slab, and an output side that may be anything ([N,K] weights with an odd N, such as a
   // vocabulary of 50257, land here: 1.0 PFLOP/s against 0.1 on the generic kernel below).
   // ... and with whole 64-wide slabs, a 16-bit result and no epilogue operands the paired-slab kernels take it, their
-  // staged tiles leaving element by element
+  // staged tiles leaving in the aligned pieces of each row
   if (chunks && sizeof(OutT) == 2 && K % BK2 == 0 && lda < (1 << 21) && ldb < (1 << 21) && !bias && !resid) {
     if (prefer_large_tiles(M, N) && (K / BK2) % 2 == 0)      // the 256x256 form without a guarded last pass only
       return launch_tiled<T, OutT, 4, 4, TRANS_B>(A, B, C, M, N, K, lda, ldb, ldc, s, nullptr, nullptr, 0, 1);

@@ -328,6 +328,27 @@ def test_gemm_output_rows_off_the_boundaries(hexmi, dtype):
         assert (c_buf[:lead] == 7.0).all() and (c[:, N:] == 7.0).all() and (c_buf[lead + M * ldc:] == 7.0).all()
 
 
+# The ends of a ragged row: the last tile holds 1 to 8 columns, ends just before, on and behind the seam between two waves' halves
+# (128 columns on 256 x 256 tiles, 64 on 128 x 128), with rows starting at every offset from a 16-byte boundary.
+@pytest.mark.parametrize("M,N", [(4096, 2049), (4096, 2054), (4096, 2175), (4096, 2177), (4096, 2183), (4096, 2303),
+                                 (300, 1025), (300, 1087), (300, 1089), (300, 1095)])
+@pytest.mark.parametrize("pad,lead", [(0, 0), (1, 5)])
+def test_gemm_ragged_row_ends(hexmi, M, N, pad, lead):
+    from hexmi import _lib
+    K, ldc = 128, N + pad
+    a, b = _inputs(M, N, K, torch.bfloat16, True, seed=N)
+    ad, bd = a.cuda(), b.cuda()
+    c_buf = torch.full((M * ldc + lead + 9,), 7.0, dtype=torch.bfloat16, device="cuda")
+    rc = _lib.lib().hexmi_gemm(M, N, K, ad.data_ptr(), K, bd.data_ptr(), K, c_buf.data_ptr() + 2 * lead, ldc, _lib.BF16, _lib.BF16,
+                               1, torch.cuda.current_stream().cuda_stream)
+    assert rc == 0
+    # the dense call of the padded weight leaves in whole pieces; the sums are the same, bit for bit
+    want = hexmi.matmul(ad, torch.cat([b, torch.zeros((-N) % 8, K, dtype=b.dtype)]).cuda(), trans_b=True)[:, :N]
+    c = c_buf[lead:lead + M * ldc].view(M, ldc)
+    assert torch.equal(c[:, :N], want)
+    assert (c_buf[:lead] == 7.0).all() and (c[:, N:] == 7.0).all() and (c_buf[lead + M * ldc:] == 7.0).all()
+
+
 def test_gemm_unaligned_views(hexmi):
     # operands and result that start 2 bytes into their buffers, odd leading dimensions (C ABI only): the any-shape
     # kernel; nothing outside the result's window is written
