@@ -161,7 +161,7 @@ def scan_scratch(asm_path):
 
 
 SOURCES = ("gemm.hip", "calibrate.hip")      # the files with MFMAs written as inline assembly
-CVT_SOURCES = ("gemm.hip", "calibrate.hip", "w8a16.hip", "w8a16_split.hip")   # asm conversions or asm MFMAs
+CVT_SOURCES = ("gemm.hip", "calibrate.hip", "w8a16.hip", "w8a16_few.hip", "w8a16_split.hip")   # asm conversions or asm MFMAs
 
 
 def _assembly(name, tmp):

@@ -217,7 +217,7 @@ PyObject* w8a16_matmul(PyObject*, PyObject* const* v, Py_ssize_t n) {
     const int64_t M = a->size(0), K = a->size(1), N = w->size(0);
     const at::Tensor *s, *z;
     if (v[2] == Py_None || !optional(v[2], s, {N}, at::kHalf, *a) || !optional(v[3], z, {N}, at::kChar, *a)) HEXMI_NOT_PLAIN;
-    if (!z && hexmi_gemm_w8a16_workspace(M, N, K) != 0) HEXMI_NOT_PLAIN;      // ops.py keeps that scratch
+    if (!z && hexmi_gemm_w8a16_workspace_helps(M, N, K)) HEXMI_NOT_PLAIN;      // ops.py keeps that scratch
     const Launch at(*a);
     if (!at.ok) HEXMI_NOT_PLAIN;
     at::Tensor out = fresh({M, N}, at::kHalf, *a);

@@ -879,8 +879,8 @@ using namespace hexmi;
 
 namespace {
 // hexmi_gemm_w8a16 (zp == nullptr, pt == 0) and hexmi_gemm_w8a16_ex: one choice of kernels for both. The decode
-// kernels and the chunked kernel have a zero-point instantiation; the 128 x 128 tile kernel does not, so more than
-// 128 rows with a zero point or a per-tensor scale run the chunked kernel in passes of 128 rows.
+// kernels, the chunked kernel and the tiles of w8a16_few.hip have a zero-point instantiation; the 128 x 128 tile kernel does not, so
+// more than 128 rows with a zero point or a per-tensor scale run on w8a16_few.hip at any size.
 int gemm_w8a16_any(int64_t M, int64_t N, int64_t K, const void* A, const int8_t* W, const void* scales,
                    const int8_t* zp, int pt, void* C, hexmi_stream_t stream) {
   if (M < 0 || N < 0 || K < 0) return HEXMI_EINVAL;
@@ -916,7 +916,7 @@ int gemm_w8a16_any(int64_t M, int64_t N, int64_t K, const void* A, const int8_t*
     return launch_status();
   }
   // the fast kernels copy 16 bytes of a weight row per lane: K % 16 == 0 and aligned bases; other shapes take the
-  // generic one. (K % 64 != 0 runs the chunked kernel, in passes of 128 rows where the tile kernel does not apply.)
+  // generic one. (K % 64 != 0 runs the chunked kernel or the tiles of w8a16_few.hip.)
   const bool tile_kernel = !zp && !pt && M > 64 && K % 64 == 0 && N % 8 == 0 && aligned_to(C, 16) && aligned_to(scales, 8);
   if (K % 16 != 0 || !aligned_to(A, 16) || !aligned_to(W, 16) || (K % 64 != 0 && K > (1 << 29))) {
     // Enough output for it: 128x128 tiles on the matrix cores, the slabs staged through registers at any alignment
@@ -945,8 +945,11 @@ int gemm_w8a16_any(int64_t M, int64_t N, int64_t K, const void* A, const int8_t*
 #undef HEXMI_GEMV
     return launch_status();
   }
-  // more than 128 rows with a zero point or a per-tensor scale: the chunked kernel in passes of 128 rows (the tile
-  // kernel has no such form; M = 256, N = 11008, K = 4096: 2 x 28 us against four passes of 20 through w8a16_kernel)
+  // 33 rows and more where the tiles of w8a16_few.hip give every CU a share
+  const GemmFewTile few = plan_w8a16_few(M, N, K, tile_kernel);
+  if (few.m) return launch_w8a16_few(few, M, N, K, a, W, s, zp, pt, c, st);
+  // what is left of more than 128 rows with a zero point or a per-tensor scale, or off whole slabs (rows too long for those tiles'
+  // offsets): the chunked kernel in passes of 128 rows
   if (((zp || pt) || (K % 64 != 0 && !tile_kernel)) && M > kMidMaxM && K <= (1 << 29)) {
     int rc = HEXMI_OK;
     for (int64_t m = 0; m < M && rc == HEXMI_OK; m += kMidMaxM) {
@@ -1041,7 +1044,13 @@ bool prefer_split(int64_t M, int64_t N, int64_t K, int cus) {
   const int64_t tiles = ((M + 127) / 128) * ((N + 127) / 128);
   return tiles * 3 <= cus || (tiles * 2 <= cus && K >= 8192);
 }
+// the tiles of w8a16_few.hip, ahead of it wherever they take a call
+bool prefer_few(int64_t M, int64_t N, int64_t K) { return K % 16 == 0 && plan_w8a16_few(M, N, K, K % 64 == 0 && N % 8 == 0).m; }
 }  // namespace
+
+extern "C" int hexmi_gemm_w8a16_workspace_helps(int64_t M, int64_t N, int64_t K) {
+  return hexmi_gemm_w8a16_workspace(M, N, K) > 0 && !prefer_few(M, N, K) ? 1 : 0;
+}
 
 extern "C" int64_t hexmi_gemm_w8a16_workspace(int64_t M, int64_t N, int64_t K) {
   if (M <= 0 || N <= 0 || K <= 0) return 0;
@@ -1067,8 +1076,9 @@ extern "C" int hexmi_gemm_w8a16_ws(int64_t M, int64_t N, int64_t K, const void* 
       rc = w8a16_split_clear(workspace, w8a16_split_header(M, N, K, cus), st);
       if (rc != HEXMI_OK) return rc;
     }
-    if (w8a16_split(M, N, K, static_cast<const f16*>(A), W, static_cast<const f16*>(scales), static_cast<f16*>(C),
-                    workspace, workspace_bytes, cus, st, &rc))
+    const bool few = prefer_few(M, N, K) && aligned_to(A, 16) && aligned_to(W, 16);
+    if (!few && w8a16_split(M, N, K, static_cast<const f16*>(A), W, static_cast<const f16*>(scales), static_cast<f16*>(C),
+                            workspace, workspace_bytes, cus, st, &rc))
       return rc;
   }
   return hexmi_gemm_w8a16(M, N, K, A, W, scales, C, stream);

@@ -1,0 +1,319 @@
+// C[M,N] = (A[M,K] * (W[N,K] - zero)^T) * scales for some ten to some hundred rows against int8 weights: tiles of one round over the
+// CUs, a workgroup of eight waves to a tile.
+//
+// What bounds it: a slab of a tile is read from LDS once per wave side by side, copied into LDS, widened and multiplied, and at one
+// workgroup per CU none of the four hides behind another entirely: 256 x 11008 x 4096 on 64 x 192 tiles takes 34 us, 27 without
+// the copies, 26 without the matrix instructions, 29 without the widening and 29 without the reads. So: eight waves; the weights
+// stay int8 in LDS and a wave widens its own channels only, waves standing side by side along the channels (64 rows to a tile) so
+// that each weight is widened once; a slab multiplies from registers while the next is read; the wave groups that take the 64-k parts of
+// a slab add up in LDS at the end; scales are fetched under the K walk (at the end, by the threads that store, they cost 1 to 3 us
+// of a call). A tile of every CU's own, down to 32 x 64, is what most shapes gain by: 128 x 128 tiles left two thirds and more of the CUs
+// idle (256 x 4096 x 4096: 64 tiles), the chunked kernel of w8a16.hip pulls all rows into every CU.
+#include <algorithm>
+#include <type_traits>
+
+#include "hexmi_common.h"
+
+namespace hexmi {
+namespace {
+
+__device__ __attribute__((aligned(16))) unsigned g_w8_zeros[4];       // where a copy of a chunk past K points
+
+// 16 bytes a lane, global -> LDS, from an address of each lane's own; as copy_to_lds_asm (hexmi_common.h)
+__device__ __forceinline__ void copy_ptr_to_lds_asm(const char* src, char* lds) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  const uint32_t dst = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)((__attribute__((address_space(3))) void*)(lds)));
+  uint32_t saved;
+  asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %2, off\n\ts_mov_b32 m0, %0"
+               : "=&s"(saved) : "s"(dst), "v"(src) : "memory");
+#endif
+}
+
+// s_waitcnt immediate (gfx9 encoding): at most vm vector-memory operations outstanding, LDS reads returned
+constexpr int wait_imm(int vm) { return (vm & 0xF) | ((vm >> 4) << 14) | (0x7 << 4); }
+
+// TM x TN: 16 x 16 tiles of a wave; SM x SN waves side by side; KH wave groups take the 64-k parts of a slab; NS stages.
+template <int TM_, int TN_, int SM_, int SN_, int KH_, int NS_>
+struct Shape {
+  static constexpr int TM = TM_, TN = TN_, SM = SM_, SN = SN_, KH = KH_, NS = NS_;
+  static constexpr int kWaves = SM * SN * KH, kThreads = kWaves * kWave;
+  static constexpr int BM = SM * TM * 16, BN = SN * TN * 16, BK = KH * 64;
+  static constexpr int kStage = BM * BK * 2 + BN * BK;           // bytes of a stage: rows of A, then rows of W
+};
+
+// 16-byte chunk c of a row sits at c ^ swz(row): sixteen rows of one chunk then cover all banks
+template <int PITCH> __device__ __forceinline__ int swz_row(int r) { return PITCH == 64 ? (r >> 1) & 3 : PITCH == 128 ? (r >> 1) & 7 : r & 15; }
+
+// K % 16 == 0, operands on 16-byte boundaries. runs: the output in runs of eight columns on 16-byte boundaries. ZP: zero points.
+// pt: one scale (and zero point) for all channels.
+template <typename S, bool ZP>
+__global__ __launch_bounds__(S::kThreads)
+void w8a16_few_kernel(const f16* __restrict__ A, const int8_t* __restrict__ W, const f16* __restrict__ scales,
+                      const int8_t* __restrict__ zp, f16* __restrict__ C, int M, int N, int K, int tiles_m, int tiles_n, int pt,
+                      int runs) {
+  constexpr int TM = S::TM, TN = S::TN, BM = S::BM, BN = S::BN, BK = S::BK, KH = S::KH, NS = S::NS, kThreads = S::kThreads;
+  constexpr int kA = BM * BK * 2 / 16 / kThreads, kB = BN * BK / 16 / kThreads, kCopies = kA + kB;   // a wave's copies of a slab
+  static_assert(kA * kThreads * 16 == BM * BK * 2 && kB * kThreads * 16 == BN * BK, "whole copies");
+  constexpr int kPitch = BN + 4;                                 // pitch of the sums on their way out
+  __shared__ __attribute__((aligned(16))) char lds[std::max(NS * S::kStage, KH * BM * kPitch * 4)];
+  __shared__ __attribute__((aligned(16))) float lds_scale[BN];
+
+  const int lane = threadIdx.x % kWave, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const int r16 = lane % 16, kg = lane / 16;
+  int tm, tn;                                                    // every XCD (each its own L2) a band of tiles
+  {
+    const int total = tiles_m * tiles_n, pid = blockIdx.x;
+    const int xcd = pid % 8, per = total / 8, extra = total % 8;
+    const int logical = xcd * per + (xcd < extra ? xcd : extra) + pid / 8;
+    constexpr int kGroup = 8;
+    const int group_size = kGroup * tiles_n, group = logical / group_size, first = group * kGroup;
+    const int gm = tiles_m - first < kGroup ? tiles_m - first : kGroup;
+    tm = first + logical % group_size % gm;
+    tn = logical % group_size / gm;
+  }
+  const int m0 = tm * BM, n0 = tn * BN;
+
+  // copy i of a slab moves chunks [i * kThreads + wave * 64, + 64) of the stage: A's kA, then W's kB
+  int voff[kCopies], kc[kCopies];
+#pragma unroll
+  for (int i = 0; i < kCopies; ++i) {
+    const bool a = i < kA;
+    const int chunk = (a ? i : i - kA) * kThreads + threadIdx.x, per_row = a ? BK / 8 : BK / 16;
+    const int row = chunk / per_row, c = (chunk % per_row) ^ (a ? swz_row<BK * 2>(row) : swz_row<BK>(row));
+    const int left = (a ? M - m0 : N - n0) - 1;                  // past the edge: the last row again, not stored
+    voff[i] = (row < left ? row : left) * (a ? 2 * K : K) + c * 16;
+    kc[i] = c * (a ? 8 : 16);
+  }
+  const char* a_base = reinterpret_cast<const char*>(A + (int64_t)m0 * K);
+  const char* w_base = reinterpret_cast<const char*>(W + (int64_t)n0 * K);
+  const int slabs = (K + BK - 1) / BK, full = K / BK;
+  auto copy = [&](int slab, int stage, auto ragged) __attribute__((always_inline)) {
+    const char* a_from = a_base + (int64_t)slab * (BK * 2);
+    const char* w_from = w_base + (int64_t)slab * BK;
+    char* to = lds + stage * S::kStage + wave * 1024;
+#pragma unroll
+    for (int i = 0; i < kCopies; ++i) {
+      const char* from = i < kA ? a_from : w_from;
+      if constexpr (decltype(ragged)::value) {                   // the slab that reaches past K: zeros there
+        const char* src = slab * BK + kc[i] < K ? from + voff[i] : reinterpret_cast<const char*>(g_w8_zeros);
+        copy_ptr_to_lds_asm(src, to + i * (kThreads * 16));
+      } else {
+        copy_to_lds_asm(from, voff[i], to + i * (kThreads * 16));
+      }
+    }
+  };
+
+  // this lane's fragments of a stage: wave group kh takes 64 k, a lane of K group kg the sixteen at kh * 64 + kg * 16 (one
+  // read of W, two of A), eight per matrix instruction
+  const int kh = wave / (S::SM * S::SN), wm = wave % (S::SM * S::SN) / S::SN, wn = wave % S::SN;
+  const int arow = wm * TM * 16 + r16, brow = wn * TN * 16 + r16;       // the swizzles repeat every sixteen rows
+  int a_at[2];
+#pragma unroll
+  for (int p = 0; p < 2; ++p) a_at[p] = arow * (BK * 2) + ((kh * 8 + kg * 2 + p) ^ swz_row<BK * 2>(arow)) * 16;
+  const int b_at = BM * BK * 2 + brow * BK + ((kh * 4 + kg) ^ swz_row<BK>(brow)) * 16;
+
+  // zero points of this lane's channels
+  f16 zero[ZP ? TN : 1];
+  if constexpr (ZP) {
+#pragma unroll
+    for (int j = 0; j < TN; ++j) {
+      const int ch = n0 + brow + j * 16;
+      zero[j] = (f16)(float)zp[pt ? 0 : ch < N ? ch : N - 1];
+    }
+  }
+
+  // the scale of channel n0 + this thread, under the K walk (loads at the end would be a latency of their own)
+  static_assert(BN <= kThreads, "a channel a thread");
+  const int scale_at = n0 + (int)threadIdx.x < N ? n0 + (int)threadIdx.x : N - 1;
+  const f16 scale = scales[pt ? 0 : scale_at];
+
+  // four partial sums of an element over K, of a wave group each or two: one chain of K / 32 additions would round more than the
+  // chunked kernel's four do
+  constexpr int kParts = KH >= 4 ? 1 : 2;
+  f32x4 acc[kParts][TM][TN];
+#pragma unroll
+  for (int p = 0; p < kParts; ++p)
+#pragma unroll
+    for (int m = 0; m < TM; ++m)
+#pragma unroll
+      for (int n = 0; n < TN; ++n) acc[p][m][n] = f32x4{0.f, 0.f, 0.f, 0.f};
+#define HEXMI_FENCE __builtin_amdgcn_sched_barrier(0)
+  struct Slab { u32x4 w[TN]; f16x8 a[2][TM]; };
+  auto read = [&](int stage, Slab& f) __attribute__((always_inline)) {
+    const char* from = lds + stage * S::kStage;
+#pragma unroll
+    for (int n = 0; n < TN; ++n) f.w[n] = *reinterpret_cast<const u32x4*>(from + b_at + n * (16 * BK));
+#pragma unroll
+    for (int p = 0; p < 2; ++p)
+#pragma unroll
+      for (int m = 0; m < TM; ++m) f.a[p][m] = *reinterpret_cast<const f16x8*>(from + a_at[p] + m * (16 * BK * 2));
+  };
+  auto multiply = [&](const Slab& f) __attribute__((always_inline)) {
+#pragma unroll
+    for (int n = 0; n < TN; ++n) {
+      f16x8 b0, b1;
+      cvt16(f.w[n], b0, b1);
+      if constexpr (ZP) {                                        // whole numbers of up to 255: exact
+        b0 -= zero[n];
+        b1 -= zero[n];
+      }
+#pragma unroll
+      for (int m = 0; m < TM; ++m) acc[0][m][n] = __builtin_amdgcn_mfma_f32_16x16x32_f16(b0, f.a[0][m], acc[0][m][n], 0, 0, 0);
+#pragma unroll
+      for (int m = 0; m < TM; ++m) {
+        f32x4& c = acc[kParts - 1][m][n];
+        c = __builtin_amdgcn_mfma_f32_16x16x32_f16(b1, f.a[1][m], c, 0, 0, 0);
+      }
+    }
+  };
+  // The copies are assembly: the compiler would wait for all of them before any LDS read. Here a wave waits until at most `newer`
+  // slabs of its own are in flight and its reads of the slab before have returned, then for every other wave.
+  auto landed = [&](int newer) __attribute__((always_inline)) {
+    HEXMI_FENCE;
+    switch (newer) {
+      case 0: __builtin_amdgcn_s_waitcnt(wait_imm(0)); break;
+      case 1: __builtin_amdgcn_s_waitcnt(wait_imm(kCopies)); break;
+      case 2: __builtin_amdgcn_s_waitcnt(wait_imm(2 * kCopies)); break;
+      default: __builtin_amdgcn_s_waitcnt(wait_imm(3 * kCopies)); break;
+    }
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    HEXMI_FENCE;
+  };
+  static_assert(NS >= 2 && NS <= 4 && 3 * kCopies < 64, "the waits above");
+  // Slab j multiplies from registers while slab j + 1 is read and slabs up to j + NS are copied: its own stage is free once every
+  // wave has read it. steady: slab j + NS is a whole one.
+  int stage = 0, j = 0;
+  auto step = [&](const Slab& now, Slab& next, auto steady) __attribute__((always_inline)) {
+    constexpr bool kSteady = decltype(steady)::value;
+    const int after = stage == NS - 1 ? 0 : stage + 1;
+    if (kSteady || j + 1 < slabs) {
+      landed(kSteady ? NS - 2 : std::min(NS - 2, slabs - 2 - j));
+      if (kSteady || j + NS < full) copy(j + NS, stage, std::false_type{});
+      else if (j + NS < slabs) copy(j + NS, stage, std::true_type{});
+      HEXMI_FENCE;
+      read(after, next);
+      HEXMI_FENCE;
+    }
+    multiply(now);
+    stage = after;
+    ++j;
+  };
+  HEXMI_FENCE;
+  auto copy_any = [&](int slab) __attribute__((always_inline)) {
+    if (slab < full) copy(slab, slab, std::false_type{});
+    else if (slab < slabs) copy(slab, slab, std::true_type{});
+  };
+#pragma unroll
+  for (int s = 0; s < NS - 1; ++s) copy_any(s);
+  landed(std::min(NS - 1, slabs) - 1);
+  copy_any(NS - 1);                                              // (behind the first slab: it would hold that up)
+  HEXMI_FENCE;
+  Slab even, odd;
+  read(0, even);
+  while (j + NS + 1 < full) {
+    step(even, odd, std::true_type{});
+    step(odd, even, std::true_type{});
+  }
+  while (j < slabs) {
+    step(even, odd, std::false_type{});
+    if (j < slabs) step(odd, even, std::false_type{});
+  }
+#undef HEXMI_FENCE
+
+  // the wave groups' sums meet in LDS and leave in rows, scaled, rounded once
+  __syncthreads();
+  float* red = reinterpret_cast<float*>(lds);
+#pragma unroll
+  for (int m = 0; m < TM; ++m)
+#pragma unroll
+    for (int n = 0; n < TN; ++n) {                               // a lane: row lane % 16, columns 4 (lane / 16) .. + 3
+      f32x4 sum = acc[0][m][n];
+      if constexpr (kParts == 2) sum += acc[1][m][n];
+      *reinterpret_cast<f32x4*>(red + (kh * BM + (wm * TM + m) * 16 + r16) * kPitch + (wn * TN + n) * 16 + kg * 4) = sum;
+    }
+  if (threadIdx.x < BN) lds_scale[threadIdx.x] = (float)scale;
+  __syncthreads();
+  if (runs) {
+    for (int idx = threadIdx.x; idx < BM * BN / 8; idx += kThreads) {
+      const int row = idx / (BN / 8), col = idx % (BN / 8) * 8;
+      if (m0 + row >= M || n0 + col >= N) continue;
+      f32x4 s[2] = {};
+#pragma unroll
+      for (int h = 0; h < KH; ++h)
+#pragma unroll
+        for (int p = 0; p < 2; ++p) s[p] += *reinterpret_cast<const f32x4*>(red + (h * BM + row) * kPitch + col + 4 * p);
+      f16x8 out;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) out[e] = (f16)(s[e / 4][e % 4] * lds_scale[col + e]);
+      *reinterpret_cast<f16x8*>(C + (int64_t)(m0 + row) * N + n0 + col) = out;
+    }
+  } else {
+    for (int idx = threadIdx.x; idx < BM * BN; idx += kThreads) {
+      const int row = idx / BN, col = idx % BN;
+      if (m0 + row >= M || n0 + col >= N) continue;
+      float v = 0.f;
+#pragma unroll
+      for (int h = 0; h < KH; ++h) v += red[(h * BM + row) * kPitch + col];
+      C[(int64_t)(m0 + row) * N + n0 + col] = (f16)(v * lds_scale[col]);
+    }
+  }
+}
+
+template <int BM, int BN> struct FewShape;                       // waves, stages
+template <> struct FewShape<32, 64> { typedef Shape<2, 2, 1, 2, 4, 4> S; };
+template <> struct FewShape<64, 64> { typedef Shape<4, 2, 1, 2, 4, 3> S; };
+template <> struct FewShape<64, 128> { typedef Shape<4, 2, 1, 4, 2, 4> S; };
+template <> struct FewShape<64, 192> { typedef Shape<4, 3, 1, 4, 2, 3> S; };
+
+}  // namespace
+
+// The smallest tile of which there is at most one per CU. us for 32 x 64 / 64 x 64 / 64 x 128 / 64 x 192 tiles (how many; cold weights)
+// and what took these calls before: 128 x 4096 x 4096 10.8 (256) / 13.3 (128) / 20 (64) / 25, 22.4; 256 x 4096 x 4096 19.8 (512) /
+// 14.6 (256) / 21.5 / 25.7, 27.3; 512 x 4096 x 4096 - / 26.7 (512) / 22.2 (256) / 26.6, 31.4; 256 x 11008 x 4096 - / 44 (688) / 44
+// (344) / 30.8 (232), 36.3; 512 x 1024 x 1024 5.5 (256) / 6.6 / 8.3 / 9.8, 11.1. Over 200 random products each of 33 to 140 and of 129
+// to 1024 rows 1.23 and 2.7 times the rate before. (128 x 128 tiles, 1000 x 4096 x 4096: 35.1, gemm.hip's 34.5.)
+// The chunked kernel of w8a16.hip, a workgroup per CU with all rows and up to 48 channels, stays ahead where rows are few: up to 48
+// (48 x 9570 x 3664 14.1 against 16.5), up to 64 rows of more than a round of 32 x 64 (64 x 8608 x 10528 38.5, 48), up to 112 of
+// more than a round of 64 x 64 (80 x 11168 x 10160 55, 58) and of few tiles over a long K (64 x 1536 x 10880 20.9, 22) -- unless it
+// has more channels than that (40 x 14336 x 992 10.8, 6.9).
+// Calls that the tiles of gemm.hip do not take (zero points, K off whole slabs of 64) would go in passes of 128 rows: they come
+// here at any size, with the tile whose rounds cost least (weights: us per 3000 of K measured above; 511 x 10907 x 13056 1238 ->
+// 180, 1000 x 14336 x 992 139 -> 53, 304 x 11008 x 4368 73 -> 60).
+GemmFewTile plan_w8a16_few(int64_t M, int64_t N, int64_t K, bool tiles) {
+  const int64_t cus = hexmi_num_cus();
+  if (cus <= 0 || M <= 32 || K > (1 << 22) || M > (1 << 30) || N > (1 << 30)) return {0, 0};
+  const bool chunked = N <= 48 * cus;
+  if (M <= 48 && chunked) return {0, 0};
+  static constexpr struct { GemmFewTile tile; int weight; } kTiles[] = {{{32, 64}, 20}, {{64, 64}, 30}, {{64, 128}, 50}, {{64, 192}, 65}};
+  GemmFewTile best = {0, 0};
+  int64_t least = 0;
+  for (const auto& t : kTiles) {
+    const int64_t count = ((M + t.tile.m - 1) / t.tile.m) * ((N + t.tile.n - 1) / t.tile.n), rounds = (count + cus - 1) / cus;
+    if (rounds == 1) {
+      const int64_t rows = t.tile.n > 64 || (K > 10240 && count * 4 < cus) ? 112 : t.tile.m == 64 ? 64 : 0;
+      return chunked && M <= rows ? GemmFewTile{0, 0} : t.tile;
+    }
+    if (tiles || M <= 128 || count > 0x7fffffff) continue;
+    if (!best.m || rounds * t.weight < least) best = t.tile, least = rounds * t.weight;
+  }
+  return best;
+}
+
+int launch_w8a16_few(const GemmFewTile& tile, int64_t M, int64_t N, int64_t K, const f16* A, const int8_t* W, const f16* scales,
+                     const int8_t* zero_points, int per_tensor, f16* C, hipStream_t s) {
+  const int tiles_m = (int)((M + tile.m - 1) / tile.m), tiles_n = (int)((N + tile.n - 1) / tile.n);
+  const int runs = N % 8 == 0 && aligned_to(C, 16);
+#define HEXMI_FEW_Z(BM, BN, ZP)                                                                                               \
+  hipLaunchKernelGGL((w8a16_few_kernel<FewShape<BM, BN>::S, ZP>), dim3((unsigned)(tiles_m * tiles_n)),                        \
+                     dim3(FewShape<BM, BN>::S::kThreads), 0, s, A, W, scales, zero_points, C, (int)M, (int)N, (int)K, tiles_m, \
+                     tiles_n, per_tensor, runs)
+#define HEXMI_FEW(BM, BN) \
+  if (tile.m == BM && tile.n == BN) { if (zero_points) HEXMI_FEW_Z(BM, BN, true); else HEXMI_FEW_Z(BM, BN, false); return launch_status(); }
+  HEXMI_FEW(32, 64) HEXMI_FEW(64, 64) HEXMI_FEW(64, 128) HEXMI_FEW(64, 192)
+#undef HEXMI_FEW
+#undef HEXMI_FEW_Z
+  return HEXMI_ENOTSUP;
+}
+
+}  // namespace hexmi

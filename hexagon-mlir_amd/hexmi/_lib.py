@@ -46,6 +46,7 @@ SIGNATURES = {
     "hexmi_transpose16": (_int, [_i64, _i64, _ptr, _i64, _ptr, _i64, _ptr]),
     "hexmi_gemm_w8a16": (_int, [_i64, _i64, _i64, _ptr, _ptr, _ptr, _ptr, _ptr]),
     "hexmi_gemm_w8a16_workspace": (_i64, [_i64, _i64, _i64]),
+    "hexmi_gemm_w8a16_workspace_helps": (_int, [_i64, _i64, _i64]),
     "hexmi_gemm_w8a16_ws": (_int, [_i64, _i64, _i64, _ptr, _ptr, _ptr, _ptr, _ptr, _i64, _ptr]),
     "hexmi_pack_w8": (_int, [_i64, _i64, _ptr, _ptr, _ptr]),
     "hexmi_gemm_w8a16_packed": (_int, [_i64, _i64, _i64, _ptr, _ptr, _ptr, _ptr, _ptr]),

@@ -164,7 +164,8 @@ def _w8a16_impl(a, w, scales, out):
     with _on(a.device):
         # shapes the library sums over several K parts need fp32 scratch for the partial tiles; one buffer per device
         # and stream is kept and reused (calls on one stream are ordered, so they may share it)
-        need = _lib.lib().hexmi_gemm_w8a16_workspace(M, N, K)
+        need = (_lib.lib().hexmi_gemm_w8a16_workspace(M, N, K) if _lib.lib().hexmi_gemm_w8a16_workspace_helps(M, N, K)
+                else 0)
         ws = None
         if need:
             key = (a.device.index, _stream())

@@ -312,6 +312,54 @@ def test_packed_weights_through_a_tensor_file(hexmi, tmp_path):
     assert torch.equal(got, hexmi.w8a16_matmul_packed(a.cuda(), wp, s.cuda()).cpu())
 
 
+# ---- tiles of one round over the CUs (w8a16_few.hip) ----------------------------------------------------------
+
+# every tile on 256 CUs and its edges: one row or channel over, one short; K below one slab, whole slabs, short last slabs, fewer
+# slabs than stages and more, odd and even counts; widths that leave in runs of eight and by elements
+@pytest.mark.parametrize("mode", ["plain", "zero points", "per tensor"])
+@pytest.mark.parametrize("M,N,K", [
+    (49, 64, 256), (65, 100, 16), (97, 513, 1040), (96, 1999, 2320), (128, 4096, 768),    # 32 x 64
+    (65, 8136, 272), (129, 3264, 1280), (256, 4093, 800), (512, 1025, 2064),              # 64 x 64
+    (129, 8192, 48), (193, 7000, 656), (512, 4090, 384), (40, 16400, 144),                # 64 x 128, 64 x 64
+    (256, 11008, 400), (449, 6144, 128), (321, 9601, 912),                                # 64 x 192
+    (1000, 4096, 8192), (385, 8192, 80), (1024, 4096, 96), (300, 12000, 144)])            # 128 x 128; rounds of more than one
+def test_w8a16_one_round_of_tiles(hexmi, mode, M, N, K):
+    a, w, s = (t.cuda() for t in _inputs(M, N, K, seed=M + N + K))
+    zp = None if mode == "plain" else torch.randint(-20, 20, (N,), generator=_gen(K), dtype=torch.int8).cuda()
+    if mode == "per tensor":
+        s, zp = s[:1].contiguous(), zp[:1].contiguous()
+    wide = w.double() if zp is None else w.double() - zp.double()[:, None]
+    sums, mag = a.double() @ wide.t(), a.double().abs() @ wide.abs().t()
+    got = hexmi.w8a16_matmul(a, w, s, zero_points=zp)
+    # fp32 sums in another order: 1e-5 of the summed magnitudes; one rounding to fp16: half an ulp
+    want, slack = sums * s.double(), 1e-5 * mag * s.double().abs()
+    assert ((got.double() - want).abs() <= slack + 2.0 ** -11 * want.abs() + 1e-7).all()
+
+
+def test_w8a16_tiles_ignore_what_lies_behind_the_operands(hexmi):
+    # a short last slab, ragged rows and channels: the operands end where their buffers go on with values that would show, and
+    # nothing outside the result is written (an output two bytes off its boundary leaves by elements)
+    M, N, K = 97, 515, 1040
+    a, w, s = _inputs(M, N, K, seed=5)
+    a_buf, w_buf = torch.full((M * K + 4096,), 6e4).half().cuda(), torch.full((N * K + 4096,), 127, dtype=torch.int8).cuda()
+    a_buf[:M * K], w_buf[:N * K] = a.reshape(-1).cuda(), w.reshape(-1).cuda()
+    want = hexmi.w8a16_matmul(a.cuda(), w.cuda(), s.cuda())
+    sd, lib = s.cuda(), hexmi.lib()
+    for off in (0, 1):
+        c = torch.full((M * N + 64,), 7.0, dtype=torch.float16, device="cuda")
+        assert lib.hexmi_gemm_w8a16(M, N, K, a_buf.data_ptr(), w_buf.data_ptr(), sd.data_ptr(), c.data_ptr() + 2 * off, None) == 0
+        torch.cuda.synchronize()
+        assert torch.equal(c[off:off + M * N].view(M, N), want)
+        assert (c[:off] == 7.0).all() and (c[off + M * N:] == 7.0).all()
+
+
+def test_w8a16_workspace_query_agrees_with_the_tiles(hexmi):
+    lib = hexmi.lib()
+    assert lib.hexmi_gemm_w8a16_workspace(128, 4096, 11008) > 0 and not lib.hexmi_gemm_w8a16_workspace_helps(128, 4096, 11008)
+    # 100 rows of more channels than 64 x 64 tiles go round, a long K: the kernel with K parts stays
+    assert lib.hexmi_gemm_w8a16_workspace_helps(100, 9000, 8192) and not lib.hexmi_gemm_w8a16_workspace_helps(16, 4096, 4096)
+
+
 # ---- the (channel range x K part) kernel behind hexmi_gemm_w8a16_ws -------------------------------------------
 
 def _ws_call(hexmi, a, w, s, ws, ws_bytes=None):
