@@ -1592,6 +1592,19 @@ inline bool prefer_large_tiles(int64_t M, int64_t N) {
   return 148 * big * rounds_small >= 100 * small * rounds_big;
 }
 
+// Columns that whole rounds of 256 x 256 tiles over the CUs take, where the tiles past them would leave more than half of a round empty; N
+// where they would not. Those columns then go as a product of their own, on the tiles that give every CU a share. us, one launch / two
+// (tiles over, of 256): K = 768: 1021 x 50257 109 / 98 (20), 2000 x 17408 68 / 59 (32), 8192 x 6271 109 / 96 (32), 8192 x 10632 149 / 144
+// (64), 2000 x 27640 101 / 99 (96); K = 2048: 2000 x 16856 139 / 115 (16), 1021 x 21248 94 / 80 (76), 2000 x 11224 95 / 88 (96);
+// 4096 x 8440 x 1536 112 / 94 (16); K = 256: 4096 x 20736 76 / 73 (16), 2000 x 44032 80 / 77 (96). With half a round and more left
+// over one launch is ahead: 4096 x 6104 x 256 31 / 33 (128), 2000 x 20696 x 1536 117 / 122 (136), 700 x 33663 x 768 54 / 58 (140).
+inline int64_t whole_rounds(int64_t M, int64_t N) {
+  const int64_t cus = hexmi_num_cus(), tiles_m = (M + 255) / 256, tiles_n = (N + 255) / 256;
+  if (cus <= 0 || tiles_m > cus) return N;
+  const int64_t cols = tiles_m * tiles_n / cus * cus / tiles_m, over = (tiles_n - cols) * tiles_m;
+  return cols > 0 && over > 0 && 20 * over <= 9 * cus ? cols * 256 : N;
+}
+
 template <typename T, typename OutT, bool TRANS_B>
 int dispatch_gemm(const void* Av, const void* Bv, void* Cv, int64_t M, int64_t N, int64_t K, int64_t lda,
                   int64_t ldb, int64_t ldc, hipStream_t s, const void* bias_v, const void* resid_v, int64_t ldr) {
@@ -1626,6 +1639,13 @@ int dispatch_gemm(const void* Av, const void* Bv, void* Cv, int64_t M, int64_t N
 #undef HEXMI_GEMV
     return launch_status();
   }
+  // 256 x 256 tiles, the columns past whole rounds of them as a product of their own
+  auto launch_rounds = [&](int out_elems) {
+    const int64_t cut = whole_rounds(M, N);
+    const int rc = launch_tiled<T, OutT, 4, 4, TRANS_B>(A, B, C, M, cut, K, lda, ldb, ldc, s, nullptr, nullptr, 0, out_elems);
+    if (rc != HEXMI_OK || cut == N) return rc;
+    return dispatch_gemm<T, OutT, TRANS_B>(A, B + (TRANS_B ? cut * ldb : cut), C + cut, M, N - cut, K, lda, ldb, ldc, s, nullptr, nullptr, 0);
+  };
   const bool fast = K % BK == 0 && lda % 8 == 0 && ldb % 8 == 0 && ldc % 4 == 0 && N % 8 == 0 && N >= 8 &&
                     aligned_to(A, 16) && aligned_to(B, 16) && aligned_to(C, 16) && (!bias || aligned_to(bias, run)) &&
                     (!resid || (aligned_to(resid, run) && ldr % 4 == 0));
@@ -1641,8 +1661,7 @@ int dispatch_gemm(const void* Av, const void* Bv, void* Cv, int64_t M, int64_t N
     const bool large = prefer_large_tiles(M, N);
     // the large-tile kernels sit at the register limit and carry no epilogue operands: a product with bias or
     // residual runs on the 128x128 tiles at any size
-    if (large && !bias && !resid)
-      return launch_tiled<T, OutT, 4, 4, TRANS_B>(A, B, C, M, N, K, lda, ldb, ldc, s, nullptr, nullptr, 0);
+    if (large && !bias && !resid) return launch_rounds(0);
     return launch_tiled<T, OutT, 2, 2, TRANS_B>(A, B, C, M, N, K, lda, ldb, ldc, s, bias, resid, ldr);
   }
   // Whole 16-byte chunks on the operand side only (K % 8 == 0; B given as [K,N] also N % 8 == 0): the 128x128 tiles
@@ -1651,8 +1670,7 @@ int dispatch_gemm(const void* Av, const void* Bv, void* Cv, int64_t M, int64_t N
   // ... and with whole 64-wide slabs, a 16-bit result and no epilogue operands the paired-slab kernels take it, their
   // staged tiles leaving in the aligned pieces of each row
   if (chunks && sizeof(OutT) == 2 && K % BK2 == 0 && lda < (1 << 21) && ldb < (1 << 21) && !bias && !resid) {
-    if (prefer_large_tiles(M, N) && (K / BK2) % 2 == 0)      // the 256x256 form without a guarded last pass only
-      return launch_tiled<T, OutT, 4, 4, TRANS_B>(A, B, C, M, N, K, lda, ldb, ldc, s, nullptr, nullptr, 0, 1);
+    if (prefer_large_tiles(M, N) && (K / BK2) % 2 == 0) return launch_rounds(1);   // the 256x256 form without a guarded last pass only
     return launch_tiled<T, OutT, 2, 2, TRANS_B>(A, B, C, M, N, K, lda, ldb, ldc, s, nullptr, nullptr, 0, 1);
   }
   if (chunks) {

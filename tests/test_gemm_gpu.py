@@ -328,6 +328,16 @@ def test_gemm_output_rows_off_the_boundaries(hexmi, dtype):
         assert (c_buf[:lead] == 7.0).all() and (c[:, N:] == 7.0).all() and (c_buf[lead + M * ldc:] == 7.0).all()
 
 
+# A few 256 x 256 tiles more than whole rounds over 256 CUs: the columns past the rounds go as a product of their own. One column,
+# eight, less and more than a tile's width; rows of the output on and off the boundaries; just under and over the line.
+@pytest.mark.parametrize("out_dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("trans_b,M,N,K", [
+    (True, 4096, 8193, 128), (True, 4096, 8200, 192), (False, 4096, 8200, 128), (True, 4090, 8451, 128), (False, 4090, 8704, 96),
+    (True, 1021, 33025, 128), (False, 1021, 33280, 64), (True, 4096, 9984, 64), (True, 4096, 9985, 128)])
+def test_gemm_columns_past_whole_rounds(hexmi, out_dtype, trans_b, M, N, K):
+    _against_double(hexmi, torch.bfloat16, out_dtype, trans_b, M, N, K, False, False, N)
+
+
 # The ends of a ragged row: the last tile holds 1 to 8 columns, ends just before, on and behind the seam between two waves' halves
 # (128 columns on 256 x 256 tiles, 64 on 128 x 128), with rows starting at every offset from a 16-byte boundary.
 @pytest.mark.parametrize("M,N", [(4096, 2049), (4096, 2054), (4096, 2175), (4096, 2177), (4096, 2183), (4096, 2303),
