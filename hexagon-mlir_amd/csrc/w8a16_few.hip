@@ -5,7 +5,7 @@
 // workgroup per CU none of the four hides behind another entirely: 256 x 11008 x 4096 on 64 x 192 tiles takes 34 us, 27 without
 // the copies, 26 without the matrix instructions, 29 without the widening and 29 without the reads. So: eight waves; the weights
 // stay int8 in LDS and a wave widens its own channels only, waves standing side by side along the channels (64 rows to a tile) so
-// that each weight is widened once; a slab multiplies from registers while the next is read; the wave groups that take the 64-k parts of
+// that each weight is widened once; a slab of the larger tiles multiplies from registers while the next is read; the wave groups that take the 64-k parts of
 // a slab add up in LDS at the end; scales are fetched under the K walk (at the end, by the threads that store, they cost 1 to 3 us
 // of a call). A tile of every CU's own, down to 32 x 64, is what most shapes gain by: 128 x 128 tiles left two thirds and more of the CUs
 // idle (256 x 4096 x 4096: 64 tiles), the chunked kernel of w8a16.hip pulls all rows into every CU.
@@ -37,6 +37,7 @@ template <int TM_, int TN_, int SM_, int SN_, int KH_, int NS_>
 struct Shape {
   static constexpr int TM = TM_, TN = TN_, SM = SM_, SN = SN_, KH = KH_, NS = NS_;
   static constexpr int kWaves = SM * SN * KH, kThreads = kWaves * kWave;
+  static constexpr bool kAhead = KH < 4;                         // the next slab is read while one multiplies
   static constexpr int BM = SM * TM * 16, BN = SN * TN * 16, BK = KH * 64;
   static constexpr int kStage = BM * BK * 2 + BN * BK;           // bytes of a stage: rows of A, then rows of W
 };
@@ -181,43 +182,62 @@ void w8a16_few_kernel(const f16* __restrict__ A, const int8_t* __restrict__ W, c
     HEXMI_FENCE;
   };
   static_assert(NS >= 2 && NS <= 4 && 3 * kCopies < 64, "the waits above");
-  // Slab j multiplies from registers while slab j + 1 is read and slabs up to j + NS are copied: its own stage is free once every
-  // wave has read it. steady: slab j + NS is a whole one.
   int stage = 0, j = 0;
-  auto step = [&](const Slab& now, Slab& next, auto steady) __attribute__((always_inline)) {
-    constexpr bool kSteady = decltype(steady)::value;
-    const int after = stage == NS - 1 ? 0 : stage + 1;
-    if (kSteady || j + 1 < slabs) {
-      landed(kSteady ? NS - 2 : std::min(NS - 2, slabs - 2 - j));
-      if (kSteady || j + NS < full) copy(j + NS, stage, std::false_type{});
-      else if (j + NS < slabs) copy(j + NS, stage, std::true_type{});
-      HEXMI_FENCE;
-      read(after, next);
-      HEXMI_FENCE;
-    }
-    multiply(now);
-    stage = after;
-    ++j;
+  auto copy_any = [&](int slab, int into) __attribute__((always_inline)) {
+    if (slab < full) copy(slab, into, std::false_type{});
+    else if (slab < slabs) copy(slab, into, std::true_type{});
   };
   HEXMI_FENCE;
-  auto copy_any = [&](int slab) __attribute__((always_inline)) {
-    if (slab < full) copy(slab, slab, std::false_type{});
-    else if (slab < slabs) copy(slab, slab, std::true_type{});
-  };
 #pragma unroll
-  for (int s = 0; s < NS - 1; ++s) copy_any(s);
-  landed(std::min(NS - 1, slabs) - 1);
-  copy_any(NS - 1);                                              // (behind the first slab: it would hold that up)
-  HEXMI_FENCE;
-  Slab even, odd;
-  read(0, even);
-  while (j + NS + 1 < full) {
-    step(even, odd, std::true_type{});
-    step(odd, even, std::true_type{});
-  }
-  while (j < slabs) {
-    step(even, odd, std::false_type{});
-    if (j < slabs) step(odd, even, std::false_type{});
+  for (int s = 0; s < NS - 1; ++s) copy_any(s, s);
+  if constexpr (S::kAhead) {
+    // Slab j multiplies from registers while slab j + 1 is read and slabs up to j + NS are copied: its own stage is free once every
+    // wave has read it. steady: slab j + NS is a whole one.
+    auto step = [&](const Slab& now, Slab& next, auto steady) __attribute__((always_inline)) {
+      constexpr bool kSteady = decltype(steady)::value;
+      const int after = stage == NS - 1 ? 0 : stage + 1;
+      if (kSteady || j + 1 < slabs) {
+        landed(kSteady ? NS - 2 : std::min(NS - 2, slabs - 2 - j));
+        if (kSteady) copy(j + NS, stage, std::false_type{}); else copy_any(j + NS, stage);
+        HEXMI_FENCE;
+        read(after, next);
+        HEXMI_FENCE;
+      }
+      multiply(now);
+      stage = after;
+      ++j;
+    };
+    landed(std::min(NS - 1, slabs) - 1);
+    copy_any(NS - 1, NS - 1);                                    // (behind the first slab: it would hold that up)
+    HEXMI_FENCE;
+    Slab even, odd;
+    read(0, even);
+    while (j + NS + 1 < full) {
+      step(even, odd, std::true_type{});
+      step(odd, even, std::true_type{});
+    }
+    while (j < slabs) {
+      step(even, odd, std::false_type{});
+      if (j < slabs) step(odd, even, std::false_type{});
+    }
+  } else {
+    // The short slabs of the small tiles gain nothing by that and K is mostly the stages' own: the last slabs in a row, each
+    // with its wait known (512 x 1024 x 1024 5.5 -> 5.0 us, 66 x 1696 x 816 5.1 -> 4.6; 294 x 688 x 9600 17.9 -> 18.7).
+    auto step = [&](int newer, auto next) __attribute__((always_inline)) {   // next: the copies that follow into the free stage
+      landed(newer);
+      next(stage == 0 ? NS - 1 : stage - 1);
+      HEXMI_FENCE;
+      Slab now;
+      read(stage, now);
+      multiply(now);
+      stage = stage == NS - 1 ? 0 : stage + 1;
+      ++j;
+    };
+    while (j + NS - 1 < full) step(NS - 2, [&](int into) __attribute__((always_inline)) { copy(j + NS - 1, into, std::false_type{}); });
+    if (j + NS - 1 < slabs) step(NS - 2, [&](int into) __attribute__((always_inline)) { copy(j + NS - 1, into, std::true_type{}); });
+#pragma unroll
+    for (int left = NS - 2; left >= 0; --left)                   // slabs behind this one
+      if (j + left < slabs) step(left, [](int) __attribute__((always_inline)) {});
   }
 #undef HEXMI_FENCE
 
@@ -271,7 +291,7 @@ template <> struct FewShape<64, 192> { typedef Shape<4, 3, 1, 4, 2, 3> S; };
 // The smallest tile of which there is at most one per CU. us for 32 x 64 / 64 x 64 / 64 x 128 / 64 x 192 tiles (how many; cold weights)
 // and what took these calls before: 128 x 4096 x 4096 10.8 (256) / 13.3 (128) / 20 (64) / 25, 22.4; 256 x 4096 x 4096 19.8 (512) /
 // 14.6 (256) / 21.5 / 25.7, 27.3; 512 x 4096 x 4096 - / 26.7 (512) / 22.2 (256) / 26.6, 31.4; 256 x 11008 x 4096 - / 44 (688) / 44
-// (344) / 30.8 (232), 36.3; 512 x 1024 x 1024 5.5 (256) / 6.6 / 8.3 / 9.8, 11.1. Over 200 random products each of 33 to 140 and of 129
+// (344) / 30.8 (232), 36.3; 512 x 1024 x 1024 5.0 (256) / 6.6 / 8.3 / 9.8, 11.1. Over 200 random products each of 33 to 140 and of 129
 // to 1024 rows 1.23 and 2.7 times the rate before. (128 x 128 tiles, 1000 x 4096 x 4096: 35.1, gemm.hip's 34.5.)
 // The chunked kernel of w8a16.hip, a workgroup per CU with all rows and up to 48 channels, stays ahead where rows are few: up to 48
 // (48 x 9570 x 3664 14.1 against 16.5), up to 64 rows of more than a round of 32 x 64 (64 x 8608 x 10528 38.5, 48), up to 112 of
