@@ -266,8 +266,8 @@ class W8A16(Workload):
     bound, dtype = "hbm", "f16"
     # the kernel rocprofv3 names for each measured shape (the library picks by M, N, K)
     KERNELS = {(1, 11008): "w8a16_gemv_kernel", (16, 11008): "w8a16_mid_kernel", (64, 11008): "w8a16_mid_kernel",
-               (256, 11008): "gemm_kernel_k64", (1, 4096): "w8a16_gemv_any_kernel", (16, 4096): "w8a16_mid_kernel",
-               (64, 4096): "w8a16_split_kernel", (256, 4096): "w8a16_split_kernel"}
+               (256, 11008): "w8a16_few_kernel", (1, 4096): "w8a16_gemv_any_kernel", (16, 4096): "w8a16_mid_kernel",
+               (64, 4096): "w8a16_few_kernel", (256, 4096): "w8a16_few_kernel"}
 
     def __init__(self, M, N=11008, K=4096):
         self.M, self.N, self.K = M, N, K
