@@ -411,6 +411,12 @@ def test_w8a16_split_parity(hexmi, oracle, M, N, K):
     assert rc == 0 and torch.equal(got_p.cpu(), got.cpu()[:, perm])
 
 
+# ... and the ones it keeps beside the tiles of w8a16_few.hip: up to 32 rows of very many channels, up to 112 rows over a long K
+@pytest.mark.parametrize("M,N,K", [(32, 25000, 256), (100, 9000, 8192), (112, 1200, 12288), (66, 520, 11008)])
+def test_w8a16_split_parity_beside_the_tiles(hexmi, oracle, M, N, K):
+    test_w8a16_split_parity(hexmi, oracle, M, N, K)
+
+
 @pytest.mark.parametrize("M", [64, 128, 256])
 def test_w8a16_down_projection_sizes(hexmi, oracle, M):
     # the other projection of the benchmark's model: N = 4096, K = 11008 (the oracle on every 29th channel)
