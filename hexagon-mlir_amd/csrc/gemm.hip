@@ -1646,6 +1646,12 @@ int dispatch_gemm(const void* Av, const void* Bv, void* Cv, int64_t M, int64_t N
     if (rc != HEXMI_OK || cut == N) return rc;
     return dispatch_gemm<T, OutT, TRANS_B>(A, B + (TRANS_B ? cut * ldb : cut), C + cut, M, N - cut, K, lda, ldb, ldc, s, nullptr, nullptr, 0);
   };
+  // Where such a cut is there to make, the large tiles are ahead also of small ones whose rounds fill better, from K = 640 on, unless
+  // half of their last row of tiles is padding (us, small tiles / large ones and the rest: 2731 x 6000 x 640 35 / 31, 3762 x 4720 x 768
+  // 41 / 38, 2772 x 6976 x 2048 83 / 71, 702 x 25576 x 3072 133 / 108; 5111 x 3296 x 512 27.6 / 27.5; padded 1100 x 14000 x 1024 38 / 42,
+  // 2683 x 6048 x 640 26 / 29, 809 x 16952 x 640 28.5 / 31).
+  const bool cut_pays = K % BK2 == 0 && K >= 640 && (M + 127) / 128 % 2 == 0 && whole_rounds(M, N) < N;
+  const bool large = !bias && !resid && (prefer_large_tiles(M, N) || cut_pays);
   const bool fast = K % BK == 0 && lda % 8 == 0 && ldb % 8 == 0 && ldc % 4 == 0 && N % 8 == 0 && N >= 8 &&
                     aligned_to(A, 16) && aligned_to(B, 16) && aligned_to(C, 16) && (!bias || aligned_to(bias, run)) &&
                     (!resid || (aligned_to(resid, run) && ldr % 4 == 0));
@@ -1658,10 +1664,9 @@ int dispatch_gemm(const void* Av, const void* Bv, void* Cv, int64_t M, int64_t N
       return launch_gemm_skinny<T, OutT>(plan, A, B, C, M, N, K, lda, ldb, ldc, s, bias, resid, ldr);
   }
   if (fast) {
-    const bool large = prefer_large_tiles(M, N);
     // the large-tile kernels sit at the register limit and carry no epilogue operands: a product with bias or
     // residual runs on the 128x128 tiles at any size
-    if (large && !bias && !resid) return launch_rounds(0);
+    if (large) return launch_rounds(0);
     return launch_tiled<T, OutT, 2, 2, TRANS_B>(A, B, C, M, N, K, lda, ldb, ldc, s, bias, resid, ldr);
   }
   // Whole 16-byte chunks on the operand side only (K % 8 == 0; B given as [K,N] also N % 8 == 0): the 128x128 tiles
@@ -1670,7 +1675,7 @@ int dispatch_gemm(const void* Av, const void* Bv, void* Cv, int64_t M, int64_t N
   // ... and with whole 64-wide slabs, a 16-bit result and no epilogue operands the paired-slab kernels take it, their
   // staged tiles leaving in the aligned pieces of each row
   if (chunks && sizeof(OutT) == 2 && K % BK2 == 0 && lda < (1 << 21) && ldb < (1 << 21) && !bias && !resid) {
-    if (prefer_large_tiles(M, N) && (K / BK2) % 2 == 0) return launch_rounds(1);   // the 256x256 form without a guarded last pass only
+    if (large && (K / BK2) % 2 == 0) return launch_rounds(1);   // the 256x256 form without a guarded last pass only
     return launch_tiled<T, OutT, 2, 2, TRANS_B>(A, B, C, M, N, K, lda, ldb, ldc, s, nullptr, nullptr, 0, 1);
   }
   if (chunks) {

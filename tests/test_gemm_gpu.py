@@ -333,7 +333,8 @@ def test_gemm_output_rows_off_the_boundaries(hexmi, dtype):
 @pytest.mark.parametrize("out_dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("trans_b,M,N,K", [
     (True, 4096, 8193, 128), (True, 4096, 8200, 192), (False, 4096, 8200, 128), (True, 4090, 8451, 128), (False, 4090, 8704, 96),
-    (True, 1021, 33025, 128), (False, 1021, 33280, 64), (True, 4096, 9984, 64), (True, 4096, 9985, 128)])
+    (True, 1021, 33025, 128), (False, 1021, 33280, 64), (True, 4096, 9984, 64), (True, 4096, 9985, 128),
+    (True, 3762, 4721, 768), (False, 3762, 4720, 832), (True, 3700, 4720, 704)])      # 1.1 rounds; half a tile of padded rows
 def test_gemm_columns_past_whole_rounds(hexmi, out_dtype, trans_b, M, N, K):
     _against_double(hexmi, torch.bfloat16, out_dtype, trans_b, M, N, K, False, False, N)
 
