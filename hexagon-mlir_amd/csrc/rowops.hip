@@ -82,10 +82,6 @@ __device__ __forceinline__ float block_reduce(float v, float* red, int wave_in_r
 }
 
 constexpr int kLine = 128;                           // bytes of a cache line
-// What the chunks of a SPAN row are counted from: its line; within a wave (THREADS == 64) the 16-byte boundary, where the up to
-// seven chunks more would cost a larger tile for what little the lines gain (softmax of 50050 x 999 fp16 42.4 us from the line,
-// 37.0; 12204 x 4097, several waves a row, 37.6 and 38.2).
-constexpr int span_granule(int threads) { return threads > kWave ? kLine : 16; }
 
 enum RowOp { kSoftmax = 0, kRmsNorm = 1, kLayerNorm = 2 };
 
@@ -133,15 +129,14 @@ __device__ __forceinline__ float rsqrt_newton(float x) {
 // issue of the next ones.
 // Without PIPE a workgroup handles exactly one row group (gridDim.x == number of groups) and accesses are masked.
 // RAGGED (never with PIPE): rows at any alignment and of any length; the masks are per element.
-// SPAN (RAGGED, x and y rows equally far off a 16-byte boundary): the row is walked as the aligned 16-byte
-// chunks that cover it, counted from the 128-byte line its first element is in. Whole chunks are read and
+// SPAN (RAGGED, x and y rows equally far off a 16-byte boundary; 0: no): the row is walked as the aligned 16-byte
+// chunks that cover it, counted from the SPAN bytes its first element is in, a 128-byte line or a chunk. Whole chunks are read and
 // written aligned (the bytes of the first and last chunk outside the row are read, sit inside the same 16 aligned
 // bytes as the row's own, and are masked); only the row's two end chunks are stored element by element. Counted from the line
-// a wave's accesses are whole lines; from the 16-byte boundary each wave shared its first and last with its neighbours
-// (softmax of 994 x 50257 fp16 44.5 -> 39.1 us). An access
+// a wave's accesses are whole lines; from the chunk each wave shares its first and last with its neighbours. An access
 // at the alignment of the element type costs about 1.6 times an aligned one. Weight and bias, which stay in the caches, are
 // read at that alignment.
-template <typename T, int OP, int CHUNKS, int THREADS, int ROWS_PER_BLOCK, bool PIPE, bool RAGGED = false, bool SPAN = false>
+template <typename T, int OP, int CHUNKS, int THREADS, int ROWS_PER_BLOCK, bool PIPE, bool RAGGED = false, int SPAN = 0>
 __global__ __launch_bounds__(THREADS * ROWS_PER_BLOCK)
 void row_kernel(const T* __restrict__ x, T* __restrict__ y, const T* __restrict__ w,
                 const T* __restrict__ b, float* __restrict__ mean_out, float* __restrict__ rstd_out,
@@ -193,11 +188,11 @@ void row_kernel(const T* __restrict__ x, T* __restrict__ y, const T* __restrict_
   };
   // Chunks past the end of the row load column 0 instead (and are ignored): the loads stay free of branches,
   // which lets them be issued back to back and waited for only where their values are used.
-  // SPAN: elements between the line boundary at or below the row's first element and that element; positions
+  // SPAN: elements between that boundary at or below the row's first element and that element; positions
   // count from the boundary, the row is positions lead .. lead + cols - 1
   int lead = 0;
   if constexpr (SPAN)
-    lead = (int)(reinterpret_cast<uintptr_t>(x + row_of(blockIdx.x) * ld_x) % span_granule(THREADS) / sizeof(T));
+    lead = (int)(reinterpret_cast<uintptr_t>(x + row_of(blockIdx.x) * ld_x) % SPAN / sizeof(T));
   const int span = cols + lead, start = lead / N * N;
   int load_col[CHUNKS];
 #pragma unroll
@@ -427,7 +422,7 @@ void row_kernel(const T* __restrict__ x, T* __restrict__ y, const T* __restrict_
 // loaded, convert it anew in every pass and take the exponentials twice, so that several rows are resident per CU and one's
 // reductions pass under another's loads and stores. 1024 rows of 50257 fp16: 48 -> 40 us, 1024 of 24576 fp32 39.7 -> 36, 762 of 65536 fp16 41.5 -> 36.4.
 // (One workgroup per CU walking its rows, the next one copied into LDS meanwhile: 43.7 us; what a CU has in flight is one row.)
-// The row is walked as the aligned 16-byte chunks that cover it (as SPAN in row_kernel; lead is 0 for aligned rows).
+// The row is walked as the aligned 16-byte chunks that cover it (SPAN as in row_kernel; lead is 0 for aligned rows).
 constexpr int kLongThreads = 512;
 
 template <typename T>
@@ -445,14 +440,14 @@ __device__ __forceinline__ float chunk_max(const Vec16<T>& r) {
   }
 }
 
-template <typename T, int CHUNKS>
+template <typename T, int CHUNKS, int SPAN>
 __global__ __launch_bounds__(kLongThreads, 4)
 void softmax_long_kernel(const T* __restrict__ x, T* __restrict__ y, int64_t rows, int cols, int64_t ld_x, int64_t ld_y) {
   constexpr int N = Vec16<T>::N, WAVES = kLongThreads / kWave;
   __shared__ float red_max[WAVES], red_sum[WAVES];
   const int t = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(t / kWave);
   const int64_t row = blockIdx.x;
-  const int lead = (int)(reinterpret_cast<uintptr_t>(x + row * ld_x) % kLine / sizeof(T)), span = cols + lead;
+  const int lead = (int)(reinterpret_cast<uintptr_t>(x + row * ld_x) % SPAN / sizeof(T)), span = cols + lead;
   const char* xr = reinterpret_cast<const char*>(x + row * ld_x - lead);
   auto first = [&](int c) { return (c * kLongThreads + wave * kWave) * N; };                 // wave-uniform, as the next two
   auto some = [&](int c) { return first(c) < span; };
@@ -853,10 +848,13 @@ int dispatch_rows(const void* xv, void* yv, const void* wv, const void* bv, floa
   if constexpr (OP == kSoftmax) {
     // (a row or less per CU: sixteen waves shorten its chain. 190 rows of 65536 fp16 12.0 us on them, 13.7 here; but 248 of 50257
     // 13.7, 12.7, and 312 of 20001 fp32 15.1, 10.5: rows off the chunks always come here)
-    if (same_offset && chunks > 1024 * 4 && line_chunks <= kLongThreads * 16 && rows <= 0x7fffffff &&
-        (!vec_ok || rows > hexmi_num_cus())) {
-#define HEXMI_LONG(C) hipLaunchKernelGGL((softmax_long_kernel<T, C>), dim3((unsigned)rows), dim3(kLongThreads), 0, s, x, y, rows, (int)cols, ld_x, ld_y)
-      if (line_chunks <= kLongThreads * 12) HEXMI_LONG(12); else HEXMI_LONG(16);
+    const bool eight_waves = !vec_ok || rows > hexmi_num_cus();
+    if (same_offset && chunks > 1024 * 4 && span_chunks <= kLongThreads * 16 && rows <= 0x7fffffff && eight_waves) {
+#define HEXMI_LONG(C, SPAN) \
+  hipLaunchKernelGGL((softmax_long_kernel<T, C, SPAN>), dim3((unsigned)rows), dim3(kLongThreads), 0, s, x, y, rows, (int)cols, ld_x, ld_y)
+      if (line_chunks <= kLongThreads * 12) HEXMI_LONG(12, kLine);
+      else if (line_chunks <= kLongThreads * 16) HEXMI_LONG(16, kLine);
+      else HEXMI_LONG(16, 16);                            // up to seven chunks short of counting from the line
 #undef HEXMI_LONG
       return launch_status();
     }
@@ -888,17 +886,26 @@ int dispatch_rows(const void* xv, void* yv, const void* wv, const void* bv, floa
   {
     const bool pays = OP == kSoftmax || rows >= (((int64_t)3 << 20) / (int64_t)sizeof(T) + cols - 1) / cols;
     if (!vec_ok && same_offset && pays && rows <= 0x7fffffff && cols < 0x7ffffff0) {
-#define HEXMI_SPAN(C, TH, RPB) \
-  { hipLaunchKernelGGL((row_kernel<T, OP, C, TH, RPB, false, true, true>), dim3((unsigned)((rows + RPB - 1) / RPB)), dim3(TH * RPB), 0, \
+#define HEXMI_SPAN(C, TH, RPB, SPAN) \
+  { hipLaunchKernelGGL((row_kernel<T, OP, C, TH, RPB, false, true, SPAN>), dim3((unsigned)((rows + RPB - 1) / RPB)), dim3(TH * RPB), 0, \
                        s, x, y, w, b, mean, rstd, rows, (int)cols, ld_x, ld_y, eps); return launch_status(); }
-      if (span_chunks <= 64 * 1) HEXMI_SPAN(1, 64, 4);
-      if (span_chunks <= 64 * 2) HEXMI_SPAN(2, 64, 4);
-      if (span_chunks <= 64 * 4) HEXMI_SPAN(4, 64, 4);
-      if (line_chunks <= 256 * 2) HEXMI_SPAN(2, 256, 1);
-      if (line_chunks <= 256 * 4) HEXMI_SPAN(4, 256, 1);
-      if (line_chunks <= 512 * 4) HEXMI_SPAN(4, 512, 1);
-      if (line_chunks <= 1024 * 4) HEXMI_SPAN(4, 1024, 1);
-      if (line_chunks <= 1024 * 8) HEXMI_SPAN(8, 1024, 1);
+#define HEXMI_SPAN_WAVES(C, TH) \
+  { if (kLines && line_chunks <= TH * C) HEXMI_SPAN(C, TH, 1, kLines ? kLine : 16) \
+    if (span_chunks <= TH * C) HEXMI_SPAN(C, TH, 1, 16) }
+      // Several waves to a row: counted from the line (us, from the chunk / the line: softmax of 9996 x 3001 fp32 42.6 / 40.9, 3332 x 9001
+      // 45.6 / 44.2, RMSNorm of 500 x 12001 10.5 / 9.7) where the up to seven chunks more do not cost the next larger tile, half of it
+      // empty: chunk / line with that tile, RMSNorm of 1835 x 16343 fp16 27.1 / 39.1, LayerNorm 32.1 / 50.8, softmax of 916 x 32727
+      // 25.9 / 36.9. 16-bit softmax always from the chunk (14641 x 2049 31.1 / 32.5, 4999 x 6001 24.2 / 24.0).
+      constexpr bool kLines = !(OP == kSoftmax && sizeof(T) == 2);
+      if (span_chunks <= 64 * 1) HEXMI_SPAN(1, 64, 4, 16);
+      if (span_chunks <= 64 * 2) HEXMI_SPAN(2, 64, 4, 16);
+      if (span_chunks <= 64 * 4) HEXMI_SPAN(4, 64, 4, 16);
+      HEXMI_SPAN_WAVES(2, 256);
+      HEXMI_SPAN_WAVES(4, 256);
+      HEXMI_SPAN_WAVES(4, 512);
+      HEXMI_SPAN_WAVES(4, 1024);
+      HEXMI_SPAN_WAVES(8, 1024);
+#undef HEXMI_SPAN_WAVES
 #undef HEXMI_SPAN
     }
   }

@@ -457,6 +457,36 @@ def test_softmax_long_rows(hexmi, dtype, rows, kib, extra, off):
     x[1] = float("-inf")
     x[2, 3] = float("inf")
     hexmi.softmax(x, out=y)
-    assert torch.isnan(y[0]).any() and torch.isnan(y[1]).all() and torch.isnan(y[2, 3])
+    assert torch.isnan(y[0]).all() and torch.isnan(y[1]).all() and torch.isnan(y[2]).all()
     if rows > 3:
         assert ((y[3:].double() - want[3:]).abs() <= (0.5 * eps + 8e-6) * want[3:] + (6e-8 if dtype == torch.float16 else 1e-30)).all()
+
+
+# rows off the chunks whose span fits a tile when counted from the 16-byte boundary, with up to seven chunks more from the line also
+# or not: the last widths of each tile, a few rows and more than one per CU, buffers that start anywhere in a line
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("chunks", [512, 1024, 2048, 4096, 6144, 8192])
+@pytest.mark.parametrize("short", [0, 1, 2, 7, 8])                      # 16-byte chunks (and an element) short of the tile
+@pytest.mark.parametrize("rows,off", [(3, 0), (261, 5)])
+def test_rows_at_the_ends_of_the_tiles(hexmi, dtype, chunks, short, rows, off):
+    es = torch.empty(0, dtype=dtype).element_size()
+    per = 16 // es
+    cols = (chunks - short) * per - 1
+    g = torch.Generator(device="cuda").manual_seed(cols)
+    x = torch.randn(rows * cols + off, generator=g, device="cuda").to(dtype)[off:].view(rows, cols)
+    w, b = (torch.randn(cols, generator=g, device="cuda").to(dtype) for _ in range(2))
+    xd = x.double()
+    mu, ms, var = xd.mean(1, keepdim=True), xd.pow(2).mean(1, keepdim=True), xd.var(1, unbiased=False, keepdim=True)
+    eps = torch.finfo(dtype).eps
+    for call, want, slack in (
+            (lambda y: hexmi.softmax(x, out=y), torch.softmax(xd, 1), 8e-6),
+            (lambda y: hexmi.rms_norm(x, w, 1e-5, out=y), xd * torch.rsqrt(ms + 1e-5) * w.double(), 4e-6),
+            (lambda y: hexmi.layer_norm(x, w, b, 1e-5, out=y), (xd - mu) * torch.rsqrt(var + 1e-5) * w.double() + b.double(), 4e-6)):
+        out = torch.full((rows * cols + off + 9,), 7.0, dtype=dtype, device="cuda")
+        y = out[off:off + rows * cols].view(rows, cols)
+        call(y)
+        # half an ulp of the output type (fp16 softmax: 2^-25 below the normal numbers), and the fp32 statistics, products and
+        # exponentials: slack of the result, for the norms of one more than it
+        tol = (0.5 * eps + slack) * want.abs() + (3e-8 if slack == 8e-6 and dtype == torch.float16 else 1e-8 if slack == 8e-6 else slack)
+        assert ((y.double() - want).abs() <= tol).all()
+        assert (out[:off] == 7.0).all() and (out[off + rows * cols:] == 7.0).all()
