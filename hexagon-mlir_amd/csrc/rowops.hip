@@ -846,9 +846,17 @@ int dispatch_rows(const void* xv, void* yv, const void* wv, const void* bv, floa
   const int64_t line_chunks = (cols * (int64_t)sizeof(T) + (on_lines ? 0 : kLine - (int64_t)sizeof(T)) + 15) / 16;
   const int64_t span_chunks = (cols + 2 * N - 2) / N;        // from the 16-byte boundary
   if constexpr (OP == kSoftmax) {
-    // (a row or less per CU: sixteen waves shorten its chain. 190 rows of 65536 fp16 12.0 us on them, 13.7 here; but 248 of 50257
-    // 13.7, 12.7, and 312 of 20001 fp32 15.1, 10.5: rows off the chunks always come here)
-    const bool eight_waves = !vec_ok || rows > hexmi_num_cus();
+    // A row or less per CU: sixteen waves shorten its chain, and their loads and stores of rows off the chunks cost more (us, sixteen
+    // waves / eight: 190 rows of 65536 fp16 12.0 / 13.7; off the chunks fp16 100 of 40001 9.6 / 9.4, 100 of 50257 10.1 / 10.9, 200
+    // 12.2 / 12.1, 230 13.2 / 12.7, 230 of 65471 15.4 / 15.4; fp32 100 of 20001 7.3 / 7.1, 48 of 25001 7.3 / 7.7, 160 9.2 / 8.9).
+    // bf16, whose conversions are instructions of their own, later (240 rows of 40001 11.7 / 11.9, 300 19.3 / 16.8; 300 of 65536
+    // 21.1 / 24.4, 520 33.8 / 33.4).
+    const int64_t cus = hexmi_num_cus();
+    bool eight_waves = rows > cus;
+    if constexpr (std::is_same<T, bf16>::value)
+      eight_waves = eight_waves && (line_chunks <= kLongThreads * 12 || rows > 2 * cus);
+    else
+      eight_waves = eight_waves || (!vec_ok && (line_chunks <= kLongThreads * 10 || 8 * rows > 7 * cus));
     if (same_offset && chunks > 1024 * 4 && span_chunks <= kLongThreads * 16 && rows <= 0x7fffffff && eight_waves) {
 #define HEXMI_LONG(C, SPAN) \
   hipLaunchKernelGGL((softmax_long_kernel<T, C, SPAN>), dim3((unsigned)rows), dim3(kLongThreads), 0, s, x, y, rows, (int)cols, ld_x, ld_y)
