@@ -25,9 +25,10 @@
 // the last slab's chunks past K fetched from a zero chunk; an output side without runs of four columns (odd N with B
 // as [N,K], odd ldc, unaligned C) -> the same kernels with the tile leaving through LDS in the pieces of 16 bytes that each row holds;
 // anything else (unaligned operand rows, K % 8 != 0) -> gemm_kernel_any, which stages the slabs through registers.
-// Up to eight rows against B as [N,K] -> gemv_nt_kernel, a stream of the weights with one wave per output channel.
-// Up to 64 rows against B as [N,K], by measured lines -> gemm_skinny.hip, a workgroup per 16 to 64 channels. Whole chunks of K and
-// no more tiles than CUs -> gemm_few.hip, tiles of 16 x 16 to 128 x 64 that give every CU a share.
+// Whole chunks of K and no more tiles than CUs -> gemm_few.hip, tiles of 16 x 16 to 128 x 64 that give every CU a share, beyond the
+// lines of plan_gemm_few where B is [N,K] and rows are few. Of what it leaves: up to eight rows against B as [N,K] -> gemv_nt_kernel, a
+// stream of the weights with one wave per output channel; up to 64, by measured lines -> gemm_skinny.hip, a workgroup per 16 to
+// 64 channels.
 #include <algorithm>
 #include <type_traits>
 
@@ -1622,8 +1623,9 @@ int dispatch_gemm(const void* Av, const void* Bv, void* Cv, int64_t M, int64_t N
                       (TRANS_B || (N % 8 == 0 && N >= 8));
   // a row or two against [N,K] weights: the weight stream (see gemv_nt_kernel)
   // (Every workgroup stages the activation rows it multiplies, so their traffic grows with the rows while the
-  // weights' does not: up to two rows always, three and four from K = 1024 on -- N = 50264, K = 768: 14.6 against 23 us on the
-  // tiles at one row, 32 against 23 at eight -- and up to eight from K = 2048 on where gemm_few.hip has no tile for them.)
+  // weights' does not: up to two rows always -- N = 50264, K = 768: 14.6 against 23 us on the 128 x 128 tiles at one row, 32
+  // against 23 at eight --, three and four from K = 1024 and up to eight from K = 2048 on where plan_gemm_few has no tile for them:
+  // five to eight where there would be more tiles than CUs.)
   const GemmFewTile few = chunks && M > (TRANS_B ? 2 : 0) && lda < (1 << 21) && ldb < (1 << 21) && K <= (1 << 30)
                               ? plan_gemm_few(TRANS_B, M, N, K) : GemmFewTile{0, 0};
   if (few.m) return launch_gemm_few<T, OutT, TRANS_B>(few, A, B, C, M, N, K, lda, ldb, ldc, s, bias, resid, ldr);

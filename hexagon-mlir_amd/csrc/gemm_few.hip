@@ -301,16 +301,39 @@ template <> struct FewShape<128, 64> { typedef Shape<4, 4, 2, 1, 4> S; static co
 // elements (29 x 640 x 3872 5.4, 5.8; 20 x 9968 x 320 4.5, 4.6; 23 x 8728 x 896 7.5, 6.9; 32 x 4096 x 4096 11.7, 10.3) and for up to
 // 16 rows of less than 3 * 2^22 (16 x 768 x 3072 4.9, 5.1; 10 x 2800 x 3136 6.5, 7.0; 9 x 3672 x 3360 8.3, 7.8; 16 x 4096 x 4096
 // 9.9, 8.7; 13 x 7904 x 5952 19.5, 16) -- but where five to eight rows and K of 2048 and more would go by dot products, a tile is
-// always ahead (8 x 800 x 3168 8.5, 5.5; 7 x 304 x 11968 18, 11).
+// always ahead (8 x 800 x 3168 8.5, 5.5; 7 x 304 x 11968 18, 11). Of the tiles beyond those lines, what would take the call instead first,
+// us on weights from HBM / on weights three times which about fill the 256 MiB behind L2:
+//   three and four rows from K = 1024 on (dot products): the tiles ahead at 4 x 4096 x 4096 (9.9, 8.9 / 9.4, 7.9), 4 x 11008 x 4096
+//   (19.5, 19.7 / 19.2, 17.5), 3 x 14336 x 1024 (9.6, 8.2 / 9.2, 7.4), 4 x 4096 x 11008 (21.9, 21.2 / 21.5, 16.7); not with weights of 3 * 2^24
+//   elements and more (3 x 16384 x 4096 25.9, 29.6 / 25.7, 29.5; 4 x 14336 x 4096 24.3, 25.5 / 23.9, 26.0; 3 x 8192 x 8192 26.0, 27.1 /
+//   25.2, 26.8) nor where tiles of 32 columns and more leave three eighths of the CUs without one (3 x 4192 x 3560 9.8, 11.5;
+//   4 x 9527 x 6416 28, 33);
+//   up to sixteen rows, half of a tile of 32 x 64 (weight stream): 16 x 14336 x 4096 22.8, 25.8 / 22.4, 24.9; 10 x 8666 x 10432 41.4, 45.1 /
+//   41.6, 45.2; 13 x 11368 x 1664 11.7, 12.2 / 8.0, 8.8 (16 x 11008 x 4096 18.9, 20.7 / 19.1, 18.0); or tiles of 16 x 16 for fewer than half
+//   of the CUs: 9 x 1208 x 15232 17.9, 17.9 / 11.2, 13.8; 12 x 1422 x 9408 13.2, 13.2 / 8.5, 9.4;
+//   up to 32 rows, up to sixteen channels per CU, weights of 3 * 2^24 elements and more (weight stream): 16 x 4096 x 14336 25.3, 27.2 / 24.5,
+//   26.1; 17 x 4096 x 12288 23.2, 25.8 / 23.1, 25.8; 32 x 4096 x 12288 29.4, 31.4 / 29.3, 31.2 -- unless its rows stand a power of two
+//   apart (16 x 4096 x 16384 33.5, 28.2 / 33.5, 28.0);
+//   17 to 24 rows, two tiles of 16 x 32, weights of less than 2^25 elements (weight stream): 17 x 3072 x 5120 12.5, 13.2 / 8.0, 8.7;
+//   24 x 3072 x 2752 8.1, 9.0 / 5.8, 6.4; 17 x 2560 x 6912 14.3, 15.0 / 8.6, 9.8 (32 rows 16.7, 16.4 / 11.2, 10.4).
 GemmFewTile plan_gemm_few(bool trans_b, int64_t M, int64_t N, int64_t K) {
   const int64_t cus = hexmi_num_cus();
   if (trans_b && M <= 64) {
     if (M > 32 ? K <= 128 : N * K < (int64_t)(M > 16 ? 2 : 3) << 22 && !(M >= 5 && M <= 8 && K >= 2048)) return {0, 0};
   }
+  const bool dots = trans_b && N >= 64 && ((M <= 4 && K >= 1024) || (M <= 8 && K >= 2048));
+  const bool stream = trans_b && N >= 64 && !dots && K % 32 == 0;
   static constexpr GemmFewTile kTiles[] = {{16, 16}, {16, 32}, {32, 32}, {32, 64}, {64, 64}, {128, 64}};
   for (const GemmFewTile& t : kTiles) {
     if (t.m == 16 && (M > 64 || (t.n == 16 && !trans_b))) continue;       // sixteen columns of a row of B are a quarter of a line
-    if (((M + t.m - 1) / t.m) * ((N + t.n - 1) / t.n) <= cus) return t;
+    const int64_t count = ((M + t.m - 1) / t.m) * ((N + t.n - 1) / t.n);
+    if (count > cus) continue;
+    if (dots && M <= 4 && (N * K >= (int64_t)3 << 24 || (t.n > 16 && 8 * count < 5 * cus))) return {0, 0};
+    if (stream && M <= 16 && (t.n == 64 || (t.n == 16 && 2 * count < cus))) return {0, 0};
+    const bool narrow = stream && M <= 32 && t.m == 16 && N <= 16 * cus;    // a channel group of sixteen per CU at most
+    if (narrow && M > 16 && M <= 24 && t.n == 32 && N * K < (int64_t)1 << 25) return {0, 0};
+    if (narrow && N * K >= (int64_t)3 << 24 && (K & (K - 1)) != 0) return {0, 0};
+    return t;
   }
   return {0, 0};
 }

@@ -75,9 +75,8 @@ def test_gemm_parity(hexmi, oracle, shape, dtype, trans_b):
 @pytest.mark.parametrize("M", [1, 2, 3, 4, 5, 8, 9, 12, 13, 16, 17, 32, 33, 48, 64])
 @pytest.mark.parametrize("N,K", [(64, 8), (100, 64), (4096, 2048), (1000, 2056), (257, 4096), (130, 11008)])
 def test_gemm_few_rows_against_transposed_weights(hexmi, oracle, dtype, M, N, K):
-    # up to 64 rows with B as [N,K]: the weight-streaming kernels (a wave per output channel up to eight rows, a
-    # workgroup per 16 channels on the matrix cores beyond), with and without the epilogue operands, 16-bit and fp32
-    # results
+    # up to 64 rows with B as [N,K]: a wave per output channel up to four rows, a workgroup per 16 channels or the tiles of
+    # gemm_few.hip beyond, with and without the epilogue operands, 16-bit and fp32 results
     a, b = _inputs(M, N, K, dtype, True, seed=M + N)
     got32 = hexmi.matmul(a.cuda(), b.cuda(), out_dtype=torch.float32, trans_b=True).cpu()
     want32 = _oracle_mm(oracle, a, b, torch.float32, True)
@@ -132,6 +131,20 @@ def test_gemm_few_rows_every_workgroup_shape(hexmi, dtype, M, N, K):
     resid = torch.randn(M, N, generator=_gen(K)).to(dtype)
     fused = hexmi.matmul(a.cuda(), b.cuda(), trans_b=True, residual=resid.cuda()).cpu()
     assert close16(fused, (want + resid.double()).to(dtype), max_ulp=1, atol=2e-5 * float(mag.max()))
+
+
+# both sides of the lines of plan_gemm_few on 256 CUs: three and four rows on tiles and, where the weights are large or the tiles few,
+# by dot products; five to eight rows by dot products of sixteen waves where there are more tiles than CUs; half a tile of 32 x 64 and
+# two of 16 x 32 where K keeps the weight stream from the call or does not
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("M,N,K", [(3, 4094, 3080), (4, 5200, 2424), (3, 16380, 1032), (3, 4099, 3104), (4, 9001, 1408), (4, 6151, 8192),
+                                   (5, 16401, 2056), (8, 50257, 2048), (6, 17001, 2112), (7, 20011, 2048), (16, 9001, 1408), (9, 16380, 1032),
+                                   (20, 3001, 2816), (20, 3001, 2808), (25, 3001, 2816), (24, 4090, 8256),
+                                   (11, 2030, 6400), (30, 4090, 12352)])
+def test_gemm_few_rows_at_the_lines_between_kernels(hexmi, dtype, M, N, K):
+    for out_dtype in (dtype, torch.float32):
+        _against_double(hexmi, dtype, out_dtype, True, M, N, K, False, False, M + N)
+        _against_double(hexmi, dtype, out_dtype, True, M, N, K, True, True, M + K)
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
