@@ -59,7 +59,8 @@ struct Launch {
 at::Tensor fresh(at::IntArrayRef sizes, at::ScalarType type, const at::Tensor& like) {
   return at::Tensor(at::detail::empty_cuda(sizes, type, like.device(), c10::nullopt));
 }
-void* ptr(const at::Tensor* t) { return t ? t->data_ptr() : nullptr; }
+// an operand is only read: a copy-on-write one stays shared
+const void* in(const at::Tensor* t) { return t ? t->const_data_ptr() : nullptr; }
 
 // an operand that may be None: true if absent or plain, of `sizes` and `type` beside `like`
 bool optional(PyObject* o, const at::Tensor*& t, at::IntArrayRef sizes, at::ScalarType type, const at::Tensor& like) {
@@ -101,12 +102,19 @@ PyObject* guarded(F&& f) {
   END_HANDLE_TH_ERRORS
 }
 #define HEXMI_NOT_PLAIN Py_RETURN_NONE
-template <typename F>
-int without_gil(F&& f) {
+// f(a...) without the interpreter lock, which is back before anything leaves this function. The arguments, pointers of tensors that
+// other threads may hold too, are taken under the lock.
+template <typename... P, typename... A>
+int unlocked(int (*f)(P...), A... a) {
+  PyThreadState* state = PyEval_SaveThread();
   int status;
-  Py_BEGIN_ALLOW_THREADS
-  status = f();
-  Py_END_ALLOW_THREADS
+  try {
+    status = f(static_cast<P>(a)...);
+  } catch (...) {
+    PyEval_RestoreThread(state);
+    throw;
+  }
+  PyEval_RestoreThread(state);
   return status;
 }
 
@@ -139,9 +147,8 @@ PyObject* softmax(PyObject*, PyObject* const* a, Py_ssize_t n) {
     at::Tensor out = fresh(r.x->sizes(), r.x->scalar_type(), *r.x);
     int64_t bytes;
     const at::Tensor ws = r.scratch(bytes);
-    return finish(without_gil([&]() {
-      return hexmi_softmax_ws(ptr(r.x), ptr(&out), r.rows, r.cols, r.cols, r.cols, 0, r.code, bytes ? ptr(&ws) : nullptr, bytes, at.stream);
-    }), "hexmi_softmax_ws", std::move(out));
+    return finish(unlocked(hexmi_softmax_ws, in(r.x), out.mutable_data_ptr(), r.rows, r.cols, r.cols, r.cols, 0, r.code,
+                           bytes ? ws.mutable_data_ptr() : nullptr, bytes, at.stream), "hexmi_softmax_ws", std::move(out));
   });
 }
 
@@ -157,10 +164,8 @@ PyObject* rms_norm(PyObject*, PyObject* const* a, Py_ssize_t n) {
     at::Tensor out = fresh(r.x->sizes(), r.x->scalar_type(), *r.x);
     int64_t bytes;
     const at::Tensor ws = r.scratch(bytes);
-    return finish(without_gil([&]() {
-      return hexmi_rms_norm_ws(ptr(r.x), ptr(w), ptr(&out), r.rows, r.cols, r.cols, r.cols, (float)eps, 0, r.code,
-                               bytes ? ptr(&ws) : nullptr, bytes, at.stream);
-    }), "hexmi_rms_norm_ws", std::move(out));
+    return finish(unlocked(hexmi_rms_norm_ws, in(r.x), in(w), out.mutable_data_ptr(), r.rows, r.cols, r.cols, r.cols, (float)eps, 0,
+                           r.code, bytes ? ws.mutable_data_ptr() : nullptr, bytes, at.stream), "hexmi_rms_norm_ws", std::move(out));
   });
 }
 
@@ -177,10 +182,9 @@ PyObject* layer_norm(PyObject*, PyObject* const* a, Py_ssize_t n) {
     at::Tensor out = fresh(r.x->sizes(), r.x->scalar_type(), *r.x);
     int64_t bytes;
     const at::Tensor ws = r.scratch(bytes);
-    return finish(without_gil([&]() {
-      return hexmi_layer_norm_ws(ptr(r.x), ptr(w), ptr(b), ptr(&out), nullptr, nullptr, r.rows, r.cols, r.cols, r.cols, (float)eps, 0,
-                                 r.code, bytes ? ptr(&ws) : nullptr, bytes, at.stream);
-    }), "hexmi_layer_norm_ws", std::move(out));
+    return finish(unlocked(hexmi_layer_norm_ws, in(r.x), in(w), in(b), out.mutable_data_ptr(), nullptr, nullptr, r.rows, r.cols, r.cols,
+                           r.cols, (float)eps, 0, r.code, bytes ? ws.mutable_data_ptr() : nullptr, bytes, at.stream),
+                  "hexmi_layer_norm_ws", std::move(out));
   });
 }
 
@@ -200,10 +204,8 @@ PyObject* matmul(PyObject*, PyObject* const* v, Py_ssize_t n) {
     const Launch at(*a);
     if (!at.ok) HEXMI_NOT_PLAIN;
     at::Tensor out = fresh({M, N}, a->scalar_type(), *a);
-    return finish(without_gil([&]() {
-      return hexmi_gemm_ex(M, N, K, ptr(a), K, ptr(b), tb ? K : N, ptr(&out), N, ptr(bias), ptr(res), res ? N : 0, code, code,
-                           tb ? 1 : 0, at.stream);
-    }), "hexmi_gemm_ex", std::move(out));
+    return finish(unlocked(hexmi_gemm_ex, M, N, K, in(a), K, in(b), tb ? K : N, out.mutable_data_ptr(), N, in(bias), in(res), res ? N : 0,
+                           code, code, tb ? 1 : 0, at.stream), "hexmi_gemm_ex", std::move(out));
   });
 }
 
@@ -222,13 +224,10 @@ PyObject* w8a16_matmul(PyObject*, PyObject* const* v, Py_ssize_t n) {
     if (!at.ok) HEXMI_NOT_PLAIN;
     at::Tensor out = fresh({M, N}, at::kHalf, *a);
     if (z)
-      return finish(without_gil([&]() {
-        return hexmi_gemm_w8a16_ex(M, N, K, ptr(a), static_cast<const int8_t*>(ptr(w)), ptr(s), static_cast<const int8_t*>(ptr(z)), 0,
-                                   ptr(&out), at.stream);
-      }), "hexmi_gemm_w8a16_ex", std::move(out));
-    return finish(without_gil([&]() {
-      return hexmi_gemm_w8a16_ws(M, N, K, ptr(a), static_cast<const int8_t*>(ptr(w)), ptr(s), ptr(&out), nullptr, 0, at.stream);
-    }), "hexmi_gemm_w8a16_ws", std::move(out));
+      return finish(unlocked(hexmi_gemm_w8a16_ex, M, N, K, in(a), in(w), in(s), in(z), 0, out.mutable_data_ptr(), at.stream),
+                    "hexmi_gemm_w8a16_ex", std::move(out));
+    return finish(unlocked(hexmi_gemm_w8a16_ws, M, N, K, in(a), in(w), in(s), out.mutable_data_ptr(), nullptr, 0, at.stream),
+                  "hexmi_gemm_w8a16_ws", std::move(out));
   });
 }
 
@@ -250,15 +249,12 @@ PyObject* flash_attention(PyObject*, PyObject* const* v, Py_ssize_t n) {
     if (!at.ok) HEXMI_NOT_PLAIN;
     at::Tensor out = fresh(q->sizes(), q->scalar_type(), *q);
     if (whole)
-      return finish(without_gil([&]() {
-        return hexmi_flash_attn_fwd(ptr(q), ptr(k), ptr(w), ptr(&out), Z, H, S, D, (float)scale, causal ? 1 : 0, code, code, at.stream);
-      }), "hexmi_flash_attn_fwd", std::move(out));
+      return finish(unlocked(hexmi_flash_attn_fwd, in(q), in(k), in(w), out.mutable_data_ptr(), Z, H, S, D, (float)scale, causal ? 1 : 0,
+                             code, code, at.stream), "hexmi_flash_attn_fwd", std::move(out));
     const int64_t strides[9] = {q->stride(0), q->stride(1), q->stride(2), k->stride(0), k->stride(1), k->stride(2),
                                 w->stride(0), w->stride(1), w->stride(2)};
-    const int status = without_gil([&]() {
-      return hexmi_flash_attn_fwd_strided(ptr(q), ptr(k), ptr(w), ptr(&out), Z, H, S, D, strides, (float)scale, causal ? 1 : 0, code, code,
-                                          at.stream);
-    });
+    const int status = unlocked(hexmi_flash_attn_fwd_strided, in(q), in(k), in(w), out.mutable_data_ptr(), Z, H, S, D, strides,
+                                (float)scale, causal ? 1 : 0, code, code, at.stream);
     if (status == HEXMI_ENOTSUP) HEXMI_NOT_PLAIN;                            // ops.py copies the operands
     return finish(status, "hexmi_flash_attn_fwd_strided", std::move(out));
   });
@@ -281,10 +277,8 @@ PyObject* attention(PyObject*, PyObject* const* v, Py_ssize_t n) {
     at::Tensor out = fresh(q->sizes(), q->scalar_type(), *q);
     const int64_t bytes = Skv > HEXMI_ATTENTION_ONE_LAUNCH_KEYS ? hexmi_attention_workspace(B, Sq, Skv, D, mask ? 1 : 0, code) : 0;
     const at::Tensor ws = bytes ? fresh({bytes}, at::kByte, *q) : at::Tensor();
-    return finish(without_gil([&]() {
-      return hexmi_attention_ws(ptr(q), ptr(k), ptr(w), ptr(mask), ptr(&out), B, Sq, Skv, D, (float)scale, code, code,
-                                bytes ? ptr(&ws) : nullptr, bytes, at.stream);
-    }), "hexmi_attention_ws", std::move(out));
+    return finish(unlocked(hexmi_attention_ws, in(q), in(k), in(w), in(mask), out.mutable_data_ptr(), B, Sq, Skv, D, (float)scale, code,
+                           code, bytes ? ws.mutable_data_ptr() : nullptr, bytes, at.stream), "hexmi_attention_ws", std::move(out));
   });
 }
 
@@ -298,7 +292,7 @@ PyObject* unary(PyObject*, PyObject* const* v, Py_ssize_t n) {
     const Launch at(*x);
     if (!at.ok) HEXMI_NOT_PLAIN;
     at::Tensor out = fresh(x->sizes(), x->scalar_type(), *x);
-    return finish(without_gil([&]() { return hexmi_unary(op, ptr(x), ptr(&out), x->numel(), code, at.stream); }), "hexmi_unary",
+    return finish(unlocked(hexmi_unary, op, in(x), out.mutable_data_ptr(), x->numel(), code, at.stream), "hexmi_unary",
                   std::move(out));
   });
 }
@@ -313,7 +307,7 @@ PyObject* binary(PyObject*, PyObject* const* v, Py_ssize_t n) {
     const Launch at(*a);
     if (!at.ok) HEXMI_NOT_PLAIN;
     at::Tensor out = fresh(a->sizes(), a->scalar_type(), *a);
-    return finish(without_gil([&]() { return hexmi_binary(op, ptr(a), ptr(b), ptr(&out), a->numel(), code, at.stream); }), "hexmi_binary",
+    return finish(unlocked(hexmi_binary, op, in(a), in(b), out.mutable_data_ptr(), a->numel(), code, at.stream), "hexmi_binary",
                   std::move(out));
   });
 }

@@ -75,6 +75,29 @@ def test_front_on_streams_threads_and_under_capture(hexmi):
             assert torch.equal(a, b), name
 
 
+def test_front_only_reads_its_operands(hexmi):
+    # A copy-on-write operand stays shared: reading it neither copies it nor needs the memory of a copy (whose allocation may fail).
+    f = hexmi.ops._front
+    hexmi.lib()
+    g = torch.Generator().manual_seed(3)
+
+    def lazy(*shape, dtype=torch.float16):
+        base = torch.randn(*shape, generator=g).to(dtype).cuda()
+        t = torch._lazy_clone(base)
+        assert torch._C._is_cow_tensor(t)
+        return base, t
+    x, w, b, m, q, kv, ks = (lazy(*s) for s in ((5, 768), (768,), (768,), (768, 64), (2, 3, 130, 64), (4, 1000, 64), (1, 200, 2, 64)))
+    wi, s = torch.ones(64, 768, dtype=torch.int8, device="cuda"), torch.ones(64, device="cuda").half()
+    for call, operands in ((lambda x, w: f.rms_norm(x, w, 1e-5), (x, w)), (lambda x, w, b: f.layer_norm(x, w, b, 1e-5), (x, w, b)),
+                           (f.softmax, (x,)), (lambda x, m: f.matmul(x, m, False, None, None), (x, m)),
+                           (lambda x: f.w8a16_matmul(x, wi, s, None), (x,)), (lambda q: f.flash_attention(q, q, q, None, True), (q,)),
+                           (lambda k: f.flash_attention(k.transpose(1, 2), k.transpose(1, 2), k.transpose(1, 2), None, True), (ks,)),
+                           (lambda k: f.attention(k, k, k, None, None), (kv,)), (lambda x: f.unary(0, x), (x,)),
+                           (lambda x: f.binary(0, x, x), (x,))):
+        want, got = call(*(t[0] for t in operands)), call(*(t[1] for t in operands))
+        assert want is not None and torch.equal(got, want) and all(torch._C._is_cow_tensor(t[1]) for t in operands)
+
+
 class _Sub(torch.Tensor):
     pass
 
