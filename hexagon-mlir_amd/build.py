@@ -84,6 +84,7 @@ def build_front(force=False):
     root = os.path.dirname(torch.__file__)
     rocm = os.path.dirname(os.path.dirname(HIPCC))
     cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+           '-DHEXMI_TORCH_VERSION="%s"' % torch.__version__,
            "-D_GLIBCXX_USE_CXX11_ABI=%d" % torch._C._GLIBCXX_USE_CXX11_ABI, "-I", INCLUDE, "-I", os.path.join(root, "include"),
            "-I", os.path.join(root, "include", "torch", "csrc", "api", "include"), "-I", os.path.join(rocm, "include"),
            "-I", sysconfig.get_paths()["include"], FRONT_SRC, "-o", OUT_FRONT, "-L", os.path.join(root, "lib"), "-ltorch_python", "-ltorch",

@@ -327,4 +327,9 @@ PyModuleDef g_module = {PyModuleDef_HEAD_INIT, "_front", "The operators' usual c
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit__front() { return PyModule_Create(&g_module); }
+// torch_version: what it was built for (HEXMI_TORCH_VERSION, from the build)
+PyMODINIT_FUNC PyInit__front() {
+  PyObject* m = PyModule_Create(&g_module);
+  if (m && PyModule_AddStringConstant(m, "torch_version", HEXMI_TORCH_VERSION) != 0) Py_CLEAR(m);
+  return m;
+}

@@ -13,6 +13,7 @@ functions raise.
 """
 import ctypes
 import math
+import warnings
 
 import torch
 
@@ -337,18 +338,31 @@ def through_dispatcher(enable=True):
 
 class _Front:
     """hexmi._front (csrc/torch_front.cpp), imported at the first call: a function of it takes a call of the plain form (dense
-    device tensors, nothing optional but operands) and returns its result, or None for any other call."""
+    device tensors, nothing optional but operands) and returns its result, or None for any other call. Where it is not built or
+    was built for another torch or Python, a warning, and every call goes through ctypes."""
 
     def __getattr__(self, name):
         _lib.lib()
+        names = ("softmax", "rms_norm", "layer_norm", "matmul", "w8a16_matmul", "flash_attention", "attention", "unary", "binary")
+        if name not in names:
+            raise AttributeError(name)
         try:
             from . import _front as native
+            if native.torch_version != torch.__version__:
+                raise ImportError("built for torch %s, not %s" % (native.torch_version, torch.__version__))
         except ImportError as e:
-            raise RuntimeError("hexmi/_front.so is missing or does not load: build it with `python hexagon-mlir_amd/build.py`") from e
-        native.set_check(_lib.check)
-        for f in ("softmax", "rms_norm", "layer_norm", "matmul", "w8a16_matmul", "flash_attention", "attention", "unary", "binary"):
-            setattr(self, f, getattr(native, f))
-        return getattr(native, name)
+            warnings.warn("hexmi/_front.so is missing or does not load (%s): every call takes the slower route through ctypes; "
+                          "build it with `python hexagon-mlir_amd/build.py`" % e, RuntimeWarning, stacklevel=3)
+            native = None
+        else:
+            native.set_check(_lib.check)
+        for f in names:
+            setattr(self, f, getattr(native, f) if native else _not_plain)
+        return getattr(self, name)
+
+
+def _not_plain(*args):
+    return None
 
 
 _front = _Front()
