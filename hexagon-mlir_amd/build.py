@@ -8,8 +8,10 @@ hexagon-mlir_amd/hexmi/libhexmi.so (next to the Python loader).
 """
 import concurrent.futures
 import os
+import shutil
 import subprocess
 import sys
+import sysconfig
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
@@ -18,6 +20,7 @@ OUT_LIB = os.path.join(HERE, "hexmi", "libhexmi.so")
 FRONT_SRC = os.path.join(CSRC, "torch_front.cpp")
 OUT_FRONT = os.path.join(HERE, "hexmi", "_front.so")
 OBJ_DIR = os.path.join(CSRC, "build")
+FRONT_STAMP = os.path.join(OBJ_DIR, "torch_front.cmd")
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 # -packed-fp32-ops off: hipcc must not form v_pk_*_f32 from float code.
@@ -74,24 +77,42 @@ def _compile(src, force, hdr_mtime):
     return obj, True
 
 
+def rocm_root():
+    """The ROCm tree that hipcc is from."""
+    found = shutil.which(HIPCC)
+    root = os.path.dirname(os.path.dirname(os.path.realpath(found))) if found else ""
+    return root if os.path.isdir(os.path.join(root, "include", "hip")) else os.environ.get("ROCM_PATH", "/opt/rocm")
+
+
 def build_front(force=False):
-    """hexmi/_front.so: the operators' usual calls as a Python extension over torch's C++ headers and libhexmi.so (host code only)."""
-    import sysconfig
-    import torch
-    if (not force and os.path.exists(OUT_FRONT)
-            and os.path.getmtime(OUT_FRONT) > max(os.path.getmtime(FRONT_SRC), os.path.getmtime(os.path.join(INCLUDE, "hexmi.h")))):
+    """hexmi/_front.so: the operators' usual calls as a Python extension over torch's C++ headers and libhexmi.so (host code only).
+    It is for the torch and Python it was built with; without torch there is none, and the C ABI needs none."""
+    try:
+        import torch
+    except ImportError:
+        print("hexmi/_front.so: not built, no torch")
         return
-    root = os.path.dirname(torch.__file__)
-    rocm = os.path.dirname(os.path.dirname(HIPCC))
+    root, rocm = os.path.dirname(torch.__file__), rocm_root()
     cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
            '-DHEXMI_TORCH_VERSION="%s"' % torch.__version__,
            "-D_GLIBCXX_USE_CXX11_ABI=%d" % torch._C._GLIBCXX_USE_CXX11_ABI, "-I", INCLUDE, "-I", os.path.join(root, "include"),
            "-I", os.path.join(root, "include", "torch", "csrc", "api", "include"), "-I", os.path.join(rocm, "include"),
            "-I", sysconfig.get_paths()["include"], FRONT_SRC, "-o", OUT_FRONT, "-L", os.path.join(root, "lib"), "-ltorch_python", "-ltorch",
            "-ltorch_cpu", "-ltorch_hip", "-lc10", "-lc10_hip", "-L", os.path.dirname(OUT_LIB), "-l:libhexmi.so", "-Wl,-rpath,$ORIGIN"]
+    built_as = "\n".join([sys.version] + cmd)               # torch's version and place, Python's, the ABI
+    try:
+        with open(FRONT_STAMP) as f:
+            same = f.read() == built_as
+    except OSError:
+        same = False
+    if (not force and same and os.path.exists(OUT_FRONT)
+            and os.path.getmtime(OUT_FRONT) > max(os.path.getmtime(FRONT_SRC), os.path.getmtime(os.path.join(INCLUDE, "hexmi.h")))):
+        return
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:
         raise RuntimeError("g++ failed for torch_front.cpp:\n%s\n%s" % (r.stdout, r.stderr))
+    with open(FRONT_STAMP, "w") as f:
+        f.write(built_as)
 
 
 def build(force=False, verbose=True):

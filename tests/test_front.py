@@ -1,5 +1,8 @@
 """The package where the native front (hexmi/_front.so) is absent or was built for another torch: the operators keep their route
 through ctypes. No GPU."""
+import importlib.util
+import os
+import subprocess
 import sys
 import types
 import warnings
@@ -42,3 +45,32 @@ def test_the_native_front_is_the_one_that_is_built():
     assert type(front.softmax).__name__ == "builtin_function_or_method"
     with pytest.raises(AttributeError):
         front.no_such_operator
+
+
+def test_the_front_is_built_again_for_another_torch(monkeypatch, tmp_path):
+    path = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(hexmi.__file__))), "build.py")
+    spec = importlib.util.spec_from_file_location("hexmi_build_under_test", path)
+    build = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(build)
+    ran = []
+
+    def run(cmd, **kw):
+        ran.append(cmd)
+        open(cmd[cmd.index("-o") + 1], "w").close()
+        return subprocess.CompletedProcess(cmd, 0, "", "")
+    monkeypatch.setattr(build.subprocess, "run", run)
+    monkeypatch.setattr(build, "OUT_FRONT", str(tmp_path / "_front.so"))
+    monkeypatch.setattr(build, "FRONT_STAMP", str(tmp_path / "torch_front.cmd"))
+    build.build_front()
+    build.build_front()
+    assert len(ran) == 1                                  # up to date
+    monkeypatch.setattr(torch, "__version__", "99.0")
+    build.build_front()
+    assert len(ran) == 2 and '-DHEXMI_TORCH_VERSION="99.0"' in ran[1]
+    monkeypatch.setattr(build, "HIPCC", "hipcc")          # found on PATH, or the usual place
+    build.build_front()
+    assert all(os.path.isdir(d) for c in ran for flag, d in zip(c, c[1:]) if flag == "-I")
+    before = len(ran)
+    monkeypatch.setitem(sys.modules, "torch", None)       # the C ABI's users need none
+    build.build_front(force=True)
+    assert len(ran) == before
