@@ -292,8 +292,15 @@ def _stage(t, dev):
     return t if t.is_contiguous() else t.contiguous()
 
 
-def _shares_storage(t, *others):
-    return any(t.untyped_storage().data_ptr() == o.untyped_storage().data_ptr() for o in others)
+def _span(t):
+    """The addresses from a tensor's first element to behind its last."""
+    return t.data_ptr(), t.data_ptr() + (sum((n - 1) * s for n, s in zip(t.shape, t.stride())) + 1) * t.element_size()
+
+
+def _overlaps(t, *others):
+    """Whether t may share memory with any of others, of one storage or not (an import over DLPack has a storage of its own)."""
+    lo, hi = _span(t)
+    return any(a < hi and lo < b for a, b in map(_span, others))
 
 
 def _finish(result, out):
@@ -626,7 +633,8 @@ def flash_attention(q, k, v, sm_scale=None, causal=False, out=None, out_dtype=No
     dev = _device() if q.device.type != "cuda" else q.device
     od = _out_like(out, q.shape, out_dtype, dev)
     # slices of one projection and transposed heads are read where they stand (three copies, 5 us each for 2 x 12 x 1000 x 64)
-    if (not _THROUGH_DISPATCHER and (out is None or not _shares_storage(od, q, k, v)) and not (q.is_contiguous() and k.is_contiguous() and v.is_contiguous())
+    if (not _THROUGH_DISPATCHER and (out is None or not _overlaps(od, q, k, v))
+            and not (q.is_contiguous() and k.is_contiguous() and v.is_contiguous())
             and q.device == k.device == v.device == od.device
             and q.stride(3) == k.stride(3) == v.stride(3) == 1
             and _flash_strided(q, k, v, float(sm_scale), causal, od)):

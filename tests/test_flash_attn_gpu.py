@@ -837,8 +837,14 @@ def test_attention_of_heads_where_they_stand_into_their_own_memory(hexmi):
     buf = torch.randn(4, Z * H * S * D, generator=g).half().cuda()
     q, k, v = (buf[i].view(Z, S, H, D).transpose(1, 2) for i in range(3))
     want = hexmi.flash_attention(q.contiguous(), k.contiguous(), v.contiguous(), 0.125, True)
-    got = hexmi.flash_attention(q, k, v, 0.125, True, out=buf[0].view(Z, H, S, D))
-    assert torch.equal(got, want)
+    keep = buf.clone()
+    for i in range(4):                                       # of q, k, v and of none of them
+        for alias in (buf[i], torch.from_dlpack(buf[i]), torch.from_dlpack(buf.view(-1)[i * Z * H * S * D - (i > 0) * 64:][:Z * H * S * D])):
+            got = hexmi.flash_attention(q, k, v, 0.125, True, out=alias.view(Z, H, S, D))
+            assert torch.equal(got, want) and got.data_ptr() == alias.data_ptr()
+            buf.copy_(keep)
+    assert hexmi.ops._overlaps(buf[1], k) and not hexmi.ops._overlaps(buf[3], q, k, v)
+    assert hexmi.ops._overlaps(torch.from_dlpack(buf[2])[-1:], v) and not hexmi.ops._overlaps(buf[0], k, v)
 
 
 def test_strided_entry_refuses_what_it_cannot_read(hexmi):
