@@ -864,6 +864,7 @@ extern "C" int hexmi_flash_attn_fwd_strided(const void* Q, const void* K, const 
     r[i] = {Z > 1 ? strides[3 * i] : 0, H > 1 ? strides[3 * i + 1] : 0, S > 1 ? strides[3 * i + 2] : D};
     if (r[i].batch % 8 != 0 || r[i].head % 8 != 0 || r[i].row % 8 != 0) return HEXMI_ENOTSUP;
     if (r[i].batch < 0 || r[i].head < 0 || r[i].row < 0 || r[i].row > 0x7fffffff / 2 / S) return HEXMI_ENOTSUP;
+    if (i > 0 && (S - 1) * r[i].row + D > 0x7fffffff / 2) return HEXMI_ENOTSUP;          // rows closer than D columns
   }
   if (in_dtype != HEXMI_F16 && in_dtype != HEXMI_BF16) return HEXMI_ENOTSUP;
   begin_call();

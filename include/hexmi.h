@@ -337,8 +337,9 @@ int hexmi_flash_attn_fwd(const void *Q, const void *K, const void *V, void *O,
  * adjacent. O is contiguous [Z, H, S, D]. The same kernels, and bits, as of
  * contiguous operands. 16-bit operands on 16-byte boundaries, strides in
  * multiples of 8 (a dimension of one has none), D % 8 == 0, D <= 256,
- * sm_scale > 0, S * row stride below 2^30; HEXMI_ENOTSUP for anything else, and for a
- * single query (S == 1) of very many heads: copy the operands then. */
+ * sm_scale > 0, S * row stride and the end of the last row below 2^30;
+ * HEXMI_ENOTSUP for anything else, and for a single query (S == 1) of very
+ * many heads: copy the operands then. */
 int hexmi_flash_attn_fwd_strided(const void *Q, const void *K, const void *V,
                                  void *O, int64_t Z, int64_t H, int64_t S,
                                  int64_t D, const int64_t *strides,

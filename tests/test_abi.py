@@ -123,3 +123,18 @@ def test_bench_refuses_more_than_one_gpu():
     r = subprocess.run([sys.executable, os.path.join(ROOT, "bench.py"), "--gpus", "2"], capture_output=True, text=True)
     assert r.returncode != 0
     assert "one GPU" in (r.stderr + r.stdout)
+
+
+def test_strided_attention_refuses_rows_past_its_offsets():
+    # rows that overlap: S * row stride is below 2^30, the last row's last columns are not (nothing is launched for such a call)
+    import ctypes
+    from hexmi import _lib
+    lib = _lib.lib()
+    S, D = (1 << 27) - 1, 64
+    for i in (1, 2):                                         # K and V
+        strides = [0, 0, 0] * 3
+        strides[3 * i + 2] = 8
+        assert S * 8 < 1 << 30 <= (S - 1) * 8 + D
+        rc = lib.hexmi_flash_attn_fwd_strided(4096, 4096, 4096, 4096, 1, 1, S, D, (ctypes.c_int64 * 9)(*strides), 0.1, 0, _lib.F16,
+                                              _lib.F16, None)
+        assert rc == _lib.ENOTSUP
