@@ -9,120 +9,12 @@
 // The per-channel scale multiplies the finished fp32 sum (it is constant over k), which differs from
 // "dequantise, then multiply" only by fp32 rounding; hexmi_dequant_w8 exposes the element-wise dequantisation.
 //
-// Work split: a workgroup of 4 waves owns one tile of 16 output channels; the waves split K four ways and their
-// partial tiles are summed through LDS.
+// Zero points, the asymmetric forms of quant.dcast, f = (float(q) - zero_point) * scale with per-channel or per-tensor parameters:
+// the zero point (an int8, exact in fp16, as is every difference q - zero_point) is subtracted from the widened weights.
 #include "hexmi_common.h"
 
 namespace hexmi {
 namespace {
-
-constexpr int kWaves = 4;
-constexpr int kThreads = kWaves * kWave;
-
-// One workgroup (4 waves) per tile of 16 output channels; wave w owns the K range [w*K/4, (w+1)*K/4) in steps of
-// 64 (one 16-byte weight load per lane = two MFMAs). All weight loads of a round are issued before the first
-// conversion so a wave keeps up to 8 KiB of the weight stream in flight; with every tile a separate workgroup
-// the whole grid is resident at once and nothing synchronises across tiles. Activation fragments are read
-// through L1/L2 (the activations are M*K*2 bytes, at most 128 KiB per 16 rows, shared by every workgroup).
-// MT: number of 16-row activation tiles handled per pass (rows m_base .. m_base + 16*MT).
-// ZP: the asymmetric forms of quant.dcast, f = (float(q) - zero_point) * scale with per-channel or per-tensor
-// parameters: the zero point (an int8, exact in fp16, as is every difference q - zero_point) is subtracted from the
-// widened weights; per_tensor reads scale and zero point at index 0 for every channel.
-template <int MT, bool ZP = false>
-__global__ __launch_bounds__(kThreads)
-void w8a16_kernel(const f16* __restrict__ A, const int8_t* __restrict__ W, const f16* __restrict__ scales,
-                  f16* __restrict__ C, int M, int N, int K, int m_base, const int8_t* __restrict__ zero_points = nullptr,
-                  int per_tensor = 0) {
-  __shared__ __attribute__((aligned(16))) float red[kWaves * MT * 256];
-
-  const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
-  const int r16 = lane % 16, kg = lane / 16;               // tile row / 16-byte k group of this lane
-  const int tile = blockIdx.x;
-  const int n = tile * 16 + r16;
-  const int nc = n < N ? n : N - 1;
-  const int8_t* wrow = W + (int64_t)nc * K + kg * 16;
-  f16 zp_h = (f16)0.0f;
-  if constexpr (ZP) {
-    if (zero_points) zp_h = (f16)(float)zero_points[per_tensor ? 0 : nc];
-  }
-
-  const int steps = K / 64;
-  const int per_wave = (steps + kWaves - 1) / kWaves;       // consecutive steps per wave: whole 128-byte lines
-  const int s_begin = wave * per_wave;
-  const int s_end = s_begin + per_wave < steps ? s_begin + per_wave : steps;
-
-  const f16* arow[MT];
-  bool avalid[MT];
-#pragma unroll
-  for (int t = 0; t < MT; ++t) {
-    const int gm = m_base + t * 16 + r16;
-    avalid[t] = gm < M;
-    arow[t] = A + (int64_t)(avalid[t] ? gm : 0) * K + kg * 16;
-  }
-
-  f32x4 acc[MT];
-#pragma unroll
-  for (int t = 0; t < MT; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-
-  // A round issues U weight loads and the 2*U*MT activation loads that go with them before anything is
-  // consumed, so the HBM latency of the weights and the L2 latency of the activations overlap.
-  constexpr int U = MT == 1 ? 8 : (MT == 2 ? 4 : 2);
-  for (int s0 = s_begin; s0 < s_end; s0 += U) {
-    u32x4 wv[U];
-    f16x8 av[U][MT][2];
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      wv[u] = u32x4{0u, 0u, 0u, 0u};
-      if (s0 + u < s_end) wv[u] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(wrow + (int64_t)(s0 + u) * 64));
-    }
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int k = (s0 + u) * 64;
-#pragma unroll
-      for (int t = 0; t < MT; ++t) {
-        av[u][t][0] = f16x8{0, 0, 0, 0, 0, 0, 0, 0};
-        av[u][t][1] = av[u][t][0];
-        if (avalid[t] && s0 + u < s_end) {
-          av[u][t][0] = *reinterpret_cast<const f16x8*>(arow[t] + k);
-          av[u][t][1] = *reinterpret_cast<const f16x8*>(arow[t] + k + 8);
-        }
-      }
-    }
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      f16x8 w0, w1;
-      cvt16(wv[u], w0, w1);                                 // a skipped step has zero weights and activations
-      if constexpr (ZP) {
-        w0 -= zp_h;                                         // exact: integers of magnitude <= 255
-        w1 -= zp_h;
-      }
-#pragma unroll
-      for (int t = 0; t < MT; ++t) {
-        // D[i = channel][j = activation row]: lane holds row j = lane%16, channels 4*(lane/16) + 0..3
-        acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(w0, av[u][t][0], acc[t], 0, 0, 0);
-        acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(w1, av[u][t][1], acc[t], 0, 0, 0);
-      }
-    }
-  }
-
-  // sum the K-partials of the waves
-#pragma unroll
-  for (int t = 0; t < MT; ++t) *reinterpret_cast<f32x4*>(red + ((wave * MT + t) * 64 + lane) * 4) = acc[t];
-  __syncthreads();
-  for (int idx = threadIdx.x; idx < MT * 64; idx += kThreads) {
-    const int t = idx / 64, l = idx % 64;
-    f32x4 sum = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int w = 0; w < kWaves; ++w) sum += *reinterpret_cast<const f32x4*>(red + ((w * MT + t) * 64 + l) * 4);
-    const int gm = m_base + t * 16 + l % 16;
-    const int gn = tile * 16 + (l / 16) * 4;
-    if (gm < M) {
-#pragma unroll
-      for (int e = 0; e < 4; ++e)
-        if (gn + e < N) C[(int64_t)gm * N + gn + e] = (f16)(sum[e] * (float)scales[ZP && per_tensor ? 0 : gn + e]);
-    }
-  }
-}
 
 // Up to 16 activation rows on pre-packed weights, K <= 4096 (plain weights go through the chunked kernel further
 // down, which is faster at every row count: 11.3 against 11.8-12.3 us at M = 4 and 8, N = 11008, K = 4096; 6.9
@@ -287,7 +179,7 @@ template <int CH> __device__ __forceinline__ int mid_w_pos(int c, int row) {
 // path for them costs the kernel registers it does not have.
 // KC: K per chunk. K need not be a multiple of it: copies of a last, shorter chunk are
 // clamped to the row and the 64-k units past K are multiplied as zeros.
-// ZP: a zero point is subtracted from the widened weights (exact in fp16), as in w8a16_kernel above; per_tensor
+// ZP: a zero point is subtracted from the widened weights (exact in fp16); per_tensor
 // reads scale and zero point at index 0 for every channel (with or without ZP).
 // TAIL: K % KC != 0 allowed. Without it the copies take a uniform chunk offset and the weights go unmasked, which
 // the forms with more than 32 rows, short of registers and issue slots, run 5 % faster (M = 64: 17.0 against 18.0 us).
@@ -856,22 +748,6 @@ void w8a16_generic_kernel(const f16* __restrict__ A, const int8_t* __restrict__ 
   }
 }
 
-template <int MT>
-int launch_pass(const f16* A, const int8_t* W, const f16* s, f16* C, int M, int N, int K, int m_base,
-                hipStream_t st) {
-  const int n_tiles = (N + 15) / 16;
-  hipLaunchKernelGGL((w8a16_kernel<MT>), dim3(n_tiles), dim3(kThreads), 0, st, A, W, s, C, M, N, K, m_base);
-  return launch_status();
-}
-template <int MT>
-int launch_pass_zp(const f16* A, const int8_t* W, const f16* s, f16* C, int M, int N, int K, int m_base,
-                   const int8_t* zp, int per_tensor, hipStream_t st) {
-  const int n_tiles = (N + 15) / 16;
-  hipLaunchKernelGGL((w8a16_kernel<MT, true>), dim3(n_tiles), dim3(kThreads), 0, st, A, W, s, C, M, N, K, m_base, zp,
-                     per_tensor);
-  return launch_status();
-}
-
 }  // namespace
 }  // namespace hexmi
 
@@ -916,9 +792,9 @@ int gemm_w8a16_any(int64_t M, int64_t N, int64_t K, const void* A, const int8_t*
     return launch_status();
   }
   // the fast kernels copy 16 bytes of a weight row per lane: K % 16 == 0 and aligned bases; other shapes take the
-  // generic one. (K % 64 != 0 runs the chunked kernel or the tiles of w8a16_few.hip.)
+  // generic one, as do rows past the offsets of the others. (K % 64 != 0 runs the chunked kernel or the tiles of w8a16_few.hip.)
   const bool tile_kernel = !zp && !pt && M > 64 && K % 64 == 0 && N % 8 == 0 && aligned_to(C, 16) && aligned_to(scales, 8);
-  if (K % 16 != 0 || !aligned_to(A, 16) || !aligned_to(W, 16) || (K % 64 != 0 && K > (1 << 29))) {
+  if (K % 16 != 0 || !aligned_to(A, 16) || !aligned_to(W, 16) || (!tile_kernel && K > (1 << 29))) {
     // Enough output for it: 128x128 tiles on the matrix cores, the slabs staged through registers at any alignment
     // (N = 11008, K = 4040: M = 64 1.43 -> 0.14 ms, M = 1024 22.5 -> 0.23 ms). With few tiles that kernel waits out a
     // memory latency per slab (about 110 us at K = 4040 whatever the rows), and the kernel below, a wave per channel
@@ -948,9 +824,9 @@ int gemm_w8a16_any(int64_t M, int64_t N, int64_t K, const void* A, const int8_t*
   // 33 rows and more where the tiles of w8a16_few.hip give every CU a share
   const GemmFewTile few = plan_w8a16_few(M, N, K, tile_kernel);
   if (few.m) return launch_w8a16_few(few, M, N, K, a, W, s, zp, pt, c, st);
-  // what is left of more than 128 rows with a zero point or a per-tensor scale, or off whole slabs (rows too long for those tiles'
-  // offsets): the chunked kernel in passes of 128 rows
-  if (((zp || pt) || (K % 64 != 0 && !tile_kernel)) && M > kMidMaxM && K <= (1 << 29)) {
+  // what is left of more than 128 rows that the 128 x 128 tiles do not take (rows too long for those tiles' offsets): the chunked
+  // kernel in passes of 128 rows (130 x 1001 x 4194368 22.5 ms; a workgroup per 16 channels in passes of 64 rows took 34.0)
+  if (!tile_kernel && M > kMidMaxM) {
     int rc = HEXMI_OK;
     for (int64_t m = 0; m < M && rc == HEXMI_OK; m += kMidMaxM) {
       const int64_t rows = M - m < kMidMaxM ? M - m : kMidMaxM;
@@ -1003,19 +879,7 @@ int gemm_w8a16_any(int64_t M, int64_t N, int64_t K, const void* A, const int8_t*
 #undef HEXMI_MID_T
     return launch_status();
   }
-  if (tile_kernel) return gemm_w8a16_tiled(M, N, K, a, W, s, c, st);
-  int rc = HEXMI_OK;
-  for (int64_t m = 0; m < M && rc == HEXMI_OK; m += 64) {
-    const int64_t left = M - m;
-    if (zp || pt) {
-      if (left > 32) rc = launch_pass_zp<4>(a, W, s, c, (int)M, (int)N, (int)K, (int)m, zp, pt, st);
-      else if (left > 16) rc = launch_pass_zp<2>(a, W, s, c, (int)M, (int)N, (int)K, (int)m, zp, pt, st);
-      else rc = launch_pass_zp<1>(a, W, s, c, (int)M, (int)N, (int)K, (int)m, zp, pt, st);
-    } else if (left > 32) rc = launch_pass<4>(a, W, s, c, (int)M, (int)N, (int)K, (int)m, st);
-    else if (left > 16) rc = launch_pass<2>(a, W, s, c, (int)M, (int)N, (int)K, (int)m, st);
-    else rc = launch_pass<1>(a, W, s, c, (int)M, (int)N, (int)K, (int)m, st);
-  }
-  return rc;
+  return gemm_w8a16_tiled(M, N, K, a, W, s, c, st);
 }
 }  // namespace
 

@@ -353,6 +353,23 @@ def test_w8a16_tiles_ignore_what_lies_behind_the_operands(hexmi):
         assert (c[:off] == 7.0).all() and (c[off + M * N:] == 7.0).all()
 
 
+# rows past the tiles' offsets (K > 2^22): the chunked kernel in passes of 128 rows, symmetric and with zero points
+@pytest.mark.parametrize("zero_points", [False, True])
+def test_w8a16_rows_past_the_offsets_of_the_tiles(hexmi, zero_points):
+    M, N, K = 130, 17, (1 << 22) + 64
+    g = torch.Generator(device="cuda").manual_seed(7)
+    a = torch.randn(M, K, generator=g, device="cuda").half()
+    w = torch.randint(-127, 128, (N, K), generator=g, device="cuda", dtype=torch.int8)
+    s = torch.rand(N, generator=g, device="cuda").mul_(0.001).half()
+    zp = torch.randint(-20, 20, (N,), generator=g, device="cuda", dtype=torch.int8) if zero_points else None
+    wide = w.double() if zp is None else w.double() - zp.double()[:, None]
+    want = (a.double() @ wide.t()) * s.double()
+    mag = (a.double().abs() @ wide.abs().t()) * s.double()
+    got = hexmi.w8a16_matmul(a, w, s, zero_points=zp)
+    # four chains of K / 128 additions an element: far fewer than their 2^15 roundings of 2^-24 in effect; one rounding to fp16
+    assert ((got.double() - want).abs() <= 1e-5 * mag + 2.0 ** -11 * want.abs() + 1e-7).all()
+
+
 def test_w8a16_workspace_query_agrees_with_the_tiles(hexmi):
     lib = hexmi.lib()
     assert lib.hexmi_gemm_w8a16_workspace(128, 4096, 11008) > 0 and not lib.hexmi_gemm_w8a16_workspace_helps(128, 4096, 11008)
