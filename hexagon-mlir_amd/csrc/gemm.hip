@@ -63,9 +63,6 @@ __device__ __attribute__((aligned(16))) unsigned g_zero_chunk[4];
 __device__ __forceinline__ int swz_k(int row) { return (row >> 2) & 3; }      // K-contiguous tiles
 __device__ __forceinline__ int swz_n(int k) { return (k & 3) << 2; }          // N-contiguous tiles
 
-// s_waitcnt immediate (gfx9 encoding): at most `vm` vector-memory operations outstanding, all LDS reads returned.
-constexpr int waitcnt_imm(int vm) { return (vm & 0xF) | ((vm >> 4) << 14) | (7 << 4) | (0 << 8); }
-
 // global -> LDS copy of a [ROWS x 32] K-contiguous slab: ROWS/64 wave-wide instructions per wave, 16 rows each.
 // Rows past row_max are clamped (their products are never stored).
 template <typename T, int ROWS, int NW = 4>
@@ -202,24 +199,6 @@ __device__ __forceinline__ typename Mfma<T>::Frag read_nmajor(const T* lds, int 
     u.h[p] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) i16x4*)(addr));
   }
   return u.f;
-}
-
-// Map the linear workgroup id to a C tile: consecutive ids go to different XCDs (each with its own L2), so
-// first give every XCD a contiguous run of logical ids, then walk tiles in bands of GROUP_M tile-rows so the
-// tiles resident on one XCD share A and B panels.
-__device__ __forceinline__ void tile_of_block(int pid, int tiles_m, int tiles_n, int& tm, int& tn) {
-  const int total = tiles_m * tiles_n;
-  // XCD x runs ids x, x + 8, ...: total/8 of them, one more on the first total%8 XCDs
-  const int xcd = pid % 8, per = total / 8, extra = total % 8;
-  const int logical = xcd * per + (xcd < extra ? xcd : extra) + pid / 8;
-  constexpr int GROUP_M = 4;
-  const int group_size = GROUP_M * tiles_n;
-  const int group = logical / group_size;
-  const int first_m = group * GROUP_M;
-  const int gm = (tiles_m - first_m) < GROUP_M ? (tiles_m - first_m) : GROUP_M;
-  const int in_group = logical % group_size;
-  tm = first_m + in_group % gm;
-  tn = in_group / gm;
 }
 
 // Epilogue operands of hexmi_gemm_ex: C = A B + bias[column] + residual[row, column], both of the output type, added
@@ -379,7 +358,7 @@ void gemm_kernel(const T* __restrict__ A, const void* __restrict__ Bv, typename 
   const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
   const int wm = wave / NWN, wn = wave % NWN;
   int tm, tn;
-  tile_of_block(blockIdx.x, tiles_m, tiles_n, tm, tn);
+  tile_of_block<4>(blockIdx.x, tiles_m, tiles_n, tm, tn);
   const int m0 = tm * BM, n0 = tn * BN;
 
   f32x16 acc[WM][WN];
@@ -802,7 +781,7 @@ void gemm_kernel_k64(const T* __restrict__ A, const void* __restrict__ Bv, typen
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);   // scalar: LDS destinations stay scalar
   const int wm = wave / 2, wn = wave % 2;
   int tm, tn;
-  tile_of_block(blockIdx.x, tiles_m, tiles_n, tm, tn);
+  tile_of_block<4>(blockIdx.x, tiles_m, tiles_n, tm, tn);
   const int m0 = tm * BM, n0 = tn * BN;
 
   f32x4 acc[TM][TN];
@@ -1226,7 +1205,7 @@ void gemm_kernel_any(const T* __restrict__ A, const void* __restrict__ Bv, OutT*
   const int tid = threadIdx.x, lane = tid % kWave, wave = tid / kWave;
   const int wm = wave / 2, wn = wave % 2;
   int tm, tn;
-  tile_of_block(blockIdx.x, tiles_m, tiles_n, tm, tn);
+  tile_of_block<4>(blockIdx.x, tiles_m, tiles_n, tm, tn);
   const int m0 = tm * BM, n0 = tn * BN;
 
   f32x16 acc[WM][WN];

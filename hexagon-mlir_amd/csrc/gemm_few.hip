@@ -32,19 +32,6 @@ template <typename T> struct Frag8;
 template <> struct Frag8<f16> { typedef f16x8 V; };
 template <> struct Frag8<bf16> { typedef bf16x8 V; };
 
-// 16 bytes a lane, global -> LDS, from an address of each lane's own; as copy_to_lds_asm (hexmi_common.h)
-__device__ __forceinline__ void copy_ptr_to_lds_asm(const char* src, char* lds) {
-#if defined(__HIP_DEVICE_COMPILE__)
-  const uint32_t dst = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)((__attribute__((address_space(3))) void*)(lds)));
-  uint32_t saved;
-  asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %2, off\n\ts_mov_b32 m0, %0"
-               : "=&s"(saved) : "s"(dst), "v"(src) : "memory");
-#endif
-}
-
-// s_waitcnt immediate (gfx9 encoding): at most vm vector-memory operations outstanding, LDS reads returned
-constexpr int wait_imm(int vm) { return (vm & 0xF) | ((vm >> 4) << 14) | (0x7 << 4); }
-
 // TM x TN: 16 x 16 tiles of a wave; SM x SN waves side by side; KH wave groups share the 32-k steps of a slab.
 template <int TM_, int TN_, int SM_, int SN_, int KH_>
 struct Shape {
@@ -79,17 +66,8 @@ void gemm_few_kernel(const T* __restrict__ A, const T* __restrict__ B, OutT* C, 
 
   const int lane = threadIdx.x % kWave, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   const int r16 = lane % 16, kg = lane / 16;
-  int tm, tn;                                                    // every XCD (each its own L2) a band of tiles
-  {
-    const int total = tiles_m * tiles_n, pid = blockIdx.x;
-    const int xcd = pid % 8, per = total / 8, extra = total % 8;
-    const int logical = xcd * per + (xcd < extra ? xcd : extra) + pid / 8;
-    constexpr int kGroup = 8;
-    const int group_size = kGroup * tiles_n, group = logical / group_size, first = group * kGroup;
-    const int gm = tiles_m - first < kGroup ? tiles_m - first : kGroup;
-    tm = first + logical % group_size % gm;
-    tn = logical % group_size / gm;
-  }
+  int tm, tn;
+  tile_of_block<8>(blockIdx.x, tiles_m, tiles_n, tm, tn);
   const int m0 = tm * BM, n0 = tn * BN;
 
   // copy i of a slab moves chunks [i * 512 + wave * 64, + 64) of the tile: A's kA, then B's kB
@@ -135,7 +113,7 @@ void gemm_few_kernel(const T* __restrict__ A, const T* __restrict__ B, OutT* C, 
 
   // this lane's fragments of a stage: wave group kh takes the slab's step kh (32 of K)
   const int kh = wave / (S::SM * S::SN), wm = wave % (S::SM * S::SN) / S::SN, wn = wave % S::SN;
-    const int arow = wm * TM * 16 + r16;
+  const int arow = wm * TM * 16 + r16;
   const int a_at = (arow * BK + ((kh * 4 + kg) ^ swz_row<BK>(arow)) * 8) * 2;
   int b_at[TN];
 #pragma unroll
@@ -198,7 +176,7 @@ void gemm_few_kernel(const T* __restrict__ A, const T* __restrict__ B, OutT* C, 
   // slabs of its own are in flight and its reads of the slab before have returned, then for every other wave.
   auto landed = [&](auto newer) __attribute__((always_inline)) {
     HEXMI_FENCE;
-    __builtin_amdgcn_s_waitcnt(wait_imm(decltype(newer)::value * kCopies));
+    __builtin_amdgcn_s_waitcnt(waitcnt_imm(decltype(newer)::value * kCopies));
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
     HEXMI_FENCE;

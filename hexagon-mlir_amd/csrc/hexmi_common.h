@@ -200,6 +200,37 @@ __device__ __forceinline__ void copy_to_lds_asm(const char* base, int voff, T* l
 #endif
 }
 
+// The same from an address of each lane's own.
+__device__ __forceinline__ void copy_ptr_to_lds_asm(const char* src, char* lds) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  const uint32_t dst = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)((__attribute__((address_space(3))) void*)(lds)));
+  uint32_t saved;
+  asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %2, off\n\ts_mov_b32 m0, %0"
+               : "=&s"(saved) : "s"(dst), "v"(src) : "memory");
+#endif
+}
+
+// s_waitcnt immediate (gfx9 encoding): at most `vm` vector-memory operations outstanding, all LDS reads returned.
+constexpr int waitcnt_imm(int vm) { return (vm & 0xF) | ((vm >> 4) << 14) | (7 << 4) | (0 << 8); }
+
+// Map the linear workgroup id to a C tile: consecutive ids go to different XCDs (each with its own L2), so
+// first give every XCD a contiguous run of logical ids, then walk tiles in bands of GROUP_M tile-rows so the
+// tiles resident on one XCD share A and B panels.
+template <int GROUP_M>
+__device__ __forceinline__ void tile_of_block(int pid, int tiles_m, int tiles_n, int& tm, int& tn) {
+  const int total = tiles_m * tiles_n;
+  // XCD x runs ids x, x + 8, ...: total/8 of them, one more on the first total%8 XCDs
+  const int xcd = pid % 8, per = total / 8, extra = total % 8;
+  const int logical = xcd * per + (xcd < extra ? xcd : extra) + pid / 8;
+  const int group_size = GROUP_M * tiles_n;
+  const int group = logical / group_size;
+  const int first_m = group * GROUP_M;
+  const int gm = (tiles_m - first_m) < GROUP_M ? (tiles_m - first_m) : GROUP_M;
+  const int in_group = logical % group_size;
+  tm = first_m + in_group % gm;
+  tn = in_group / gm;
+}
+
 inline bool aligned_to(const void* p, size_t a) { return (reinterpret_cast<uintptr_t>(p) % a) == 0; }
 
 inline int dtype_size(int dtype) {

@@ -19,19 +19,6 @@ namespace {
 
 __device__ __attribute__((aligned(16))) unsigned g_w8_zeros[4];       // where a copy of a chunk past K points
 
-// 16 bytes a lane, global -> LDS, from an address of each lane's own; as copy_to_lds_asm (hexmi_common.h)
-__device__ __forceinline__ void copy_ptr_to_lds_asm(const char* src, char* lds) {
-#if defined(__HIP_DEVICE_COMPILE__)
-  const uint32_t dst = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)((__attribute__((address_space(3))) void*)(lds)));
-  uint32_t saved;
-  asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %2, off\n\ts_mov_b32 m0, %0"
-               : "=&s"(saved) : "s"(dst), "v"(src) : "memory");
-#endif
-}
-
-// s_waitcnt immediate (gfx9 encoding): at most vm vector-memory operations outstanding, LDS reads returned
-constexpr int wait_imm(int vm) { return (vm & 0xF) | ((vm >> 4) << 14) | (0x7 << 4); }
-
 // TM x TN: 16 x 16 tiles of a wave; SM x SN waves side by side; KH wave groups take the 64-k parts of a slab; NS stages.
 template <int TM_, int TN_, int SM_, int SN_, int KH_, int NS_>
 struct Shape {
@@ -61,17 +48,8 @@ void w8a16_few_kernel(const f16* __restrict__ A, const int8_t* __restrict__ W, c
 
   const int lane = threadIdx.x % kWave, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   const int r16 = lane % 16, kg = lane / 16;
-  int tm, tn;                                                    // every XCD (each its own L2) a band of tiles
-  {
-    const int total = tiles_m * tiles_n, pid = blockIdx.x;
-    const int xcd = pid % 8, per = total / 8, extra = total % 8;
-    const int logical = xcd * per + (xcd < extra ? xcd : extra) + pid / 8;
-    constexpr int kGroup = 8;
-    const int group_size = kGroup * tiles_n, group = logical / group_size, first = group * kGroup;
-    const int gm = tiles_m - first < kGroup ? tiles_m - first : kGroup;
-    tm = first + logical % group_size % gm;
-    tn = logical % group_size / gm;
-  }
+  int tm, tn;
+  tile_of_block<8>(blockIdx.x, tiles_m, tiles_n, tm, tn);
   const int m0 = tm * BM, n0 = tn * BN;
 
   // copy i of a slab moves chunks [i * kThreads + wave * 64, + 64) of the stage: A's kA, then W's kB
@@ -172,10 +150,10 @@ void w8a16_few_kernel(const f16* __restrict__ A, const int8_t* __restrict__ W, c
   auto landed = [&](int newer) __attribute__((always_inline)) {
     HEXMI_FENCE;
     switch (newer) {
-      case 0: __builtin_amdgcn_s_waitcnt(wait_imm(0)); break;
-      case 1: __builtin_amdgcn_s_waitcnt(wait_imm(kCopies)); break;
-      case 2: __builtin_amdgcn_s_waitcnt(wait_imm(2 * kCopies)); break;
-      default: __builtin_amdgcn_s_waitcnt(wait_imm(3 * kCopies)); break;
+      case 0: __builtin_amdgcn_s_waitcnt(waitcnt_imm(0)); break;
+      case 1: __builtin_amdgcn_s_waitcnt(waitcnt_imm(kCopies)); break;
+      case 2: __builtin_amdgcn_s_waitcnt(waitcnt_imm(2 * kCopies)); break;
+      default: __builtin_amdgcn_s_waitcnt(waitcnt_imm(3 * kCopies)); break;
     }
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
