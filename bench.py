@@ -201,14 +201,14 @@ class Gemm(Workload):
         self.name = "gemm_%s_%d%s" % (dtype_name, size, "_packed_weight" if packed else "")
         self.desc = "C=A.B %s [%d,%d]x[%d,%d] U(-1,1), fp32 accumulate, %s out" % (dtype_name, size, size, size, size,
                                                                                    dtype_name)
+        if dtype_name == "f32":
+            self.kernel, self.peak = "gemm_f32_mfma_kernel", MFMA_F32_PEAK_TFLOPS
         if packed:
             self.desc += "; B re-laid-out once to [N,K] (hexmi_transpose16, outside the timed region) and multiplied as B^T"
 
     def setup(self, torch, hexmi):
         from hexmi.workloads import gemm_inputs, gemm_flops
         dt = {"f16": torch.float16, "bf16": torch.bfloat16, "f32": torch.float32}[self.dtype]
-        if self.dtype == "f32":
-            self.kernel, self.peak = "gemm_f32_mfma_kernel", MFMA_F32_PEAK_TFLOPS
         self.hexmi, self.host = hexmi, gemm_inputs(self.size, self.size, self.size, dt)
         self.work = gemm_flops(self.size, self.size, self.size)
         self.sets = _sets(torch, self.host, 0, rotate=False)
@@ -515,9 +515,12 @@ class AddMatmulSoftmax(Workload):
     """softmax((x + y) z) in one launch against add -> GEMM -> softmax (three launches)."""
     bound, kernel = "mfma", "add_matmul_softmax_kernel"
     launches_separate = 3
+    ONE_LAUNCH_MACS = 1 << 20       # beyond, the operator runs the three kernels
 
     def __init__(self, M, N, K, dtype_name):
         self.M, self.N, self.K, self.dtype = M, N, K, dtype_name
+        if M * N * K > self.ONE_LAUNCH_MACS:
+            self.kernel = "binary_kernel + gemm_few_kernel + row_kernel"
         self.name = "add_matmul_softmax_%s_%dx%dx%d" % (dtype_name, M, N, K)
         self.desc = "softmax((x + y)[%d,%d] . z[%d,%d]) over rows, %s, N(0,1) inputs" % (M, K, K, N, dtype_name)
 
@@ -527,8 +530,7 @@ class AddMatmulSoftmax(Workload):
             self.peak = MFMA_F32_PEAK_TFLOPS
         g = torch.Generator().manual_seed(9)
         self.hexmi = hexmi
-        if self.M * self.N * self.K > hexmi.ops._FUSED_MAX_MACS:       # the operator then runs the three kernels
-            self.kernel = "binary_kernel + gemm_kernel_k64 + row_kernel"
+        assert hexmi.ops._FUSED_MAX_MACS == self.ONE_LAUNCH_MACS
         self.host = {"x": torch.randn(self.M, self.K, generator=g).to(dt), "y": torch.randn(self.M, self.K, generator=g).to(dt),
                      "z": torch.randn(self.K, self.N, generator=g).mul_(self.K ** -0.5).to(dt)}
         self.work = 2.0 * self.M * self.N * self.K
@@ -688,12 +690,14 @@ def measure_hot(torch, wl, steps, warmup, use_graph):
 
 
 def measured_traffic(wl):
-    """HBM bytes per step from the committed rocprofv3 counter runs (profiles/traffic.json), or None."""
+    """HBM bytes per step from the committed rocprofv3 counter runs (profiles/traffic.json), or None: no run, or a run in which
+    another kernel took the workload."""
     try:
         with open(os.path.join(ROOT, "profiles", "traffic.json")) as f:
             table = json.load(f)["traffic"]
         per_kernel = table[wl.name]
-        return sum(per_kernel.values())
+        measured = {name.split("<")[0] for name in per_kernel}
+        return sum(per_kernel.values()) if measured.issuperset(wl.kernel.split(" + ")) else None
     except (OSError, KeyError, ValueError):
         return None
 
