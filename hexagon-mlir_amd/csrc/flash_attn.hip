@@ -72,23 +72,25 @@ struct MaskTileLoader {
 // top of the block that uses them.
 // PADDED: the head is head_dim < D wide (a multiple of 8): Q, K, V and O rows are head_dim elements apart, the tiles
 // carry zero columns from head_dim to D (they add nothing to Q K^T; the output columns there are not stored).
-// PITCH: Q, K and V stand as `at` says (heads of other widths always; D columns wide: where they are not contiguous).
+// PITCH: Q, K and V stand as `at` says (where they are not contiguous).
 // Rows of a head stay whole lines wherever they stand, so such a head is read at the same rate; what it saves is the copies, 5 us
 // and a launch each (a layer of 2 x 1000 x 768 with q, k, v as slices of one projection 117 -> 101 us). Heads that are contiguous keep
-// kernels that know it: their addresses are shifts.
+// kernels that know it: their addresses are shifts or one product (padded heads through `at` lost 0.3 us of a small call and 2 to 3 % of a
+// large one: 5 x 16 x 320 x 40 8.9 -> 9.6, 1 x 12 x 2816 x 80 causal 52.7 -> 54.4).
 // WIDE (with PADDED, D = 128, four waves): a head of 128 < head_dim <= 256 columns as two 128-wide halves. The
 // scores are the sum over both halves' K tiles, the output two sets of accumulators, the second half's tiles padded
 // like a narrow head's; twice the LDS and about 100 registers more, so one workgroup per CU.
 template <typename T, typename OutT, int D, bool CAUSAL, bool GENERAL = false, int NW = 4, bool MASK_LDS = false,
-          bool PADDED = false, bool WIDE = false, bool MASKED = false, bool PITCH = PADDED && !GENERAL>
+          bool PADDED = false, bool WIDE = false, bool MASKED = false, bool PITCH = false>
 __global__ __launch_bounds__(NW * 64, NW == 4 && !WIDE ? (D == 64 && !GENERAL ? 3 : 2) : 1)
 void flash_fwd_kernel(const T* __restrict__ Q, const T* __restrict__ K, const T* __restrict__ V,
                       OutT* __restrict__ O, int ZH, int S, float scale_log2e, const T* __restrict__ Mk = nullptr,
-                      int Skv_arg = 0, float sm_scale = 0.0f, int group_heads = 0, int head_dim = D, HeadRows at = {}) {
+                      int Skv_arg = 0, float sm_scale = 0.0f, int group_heads = 0, int head_dim = D, RowsArg<PITCH> at = {}) {
   static_assert(!(CAUSAL && GENERAL), "the causal kernel has as many keys as queries and no mask");
   static_assert(!WIDE || (PADDED && D == 128 && NW == 4 && !GENERAL), "two halves of 128 columns, four waves, no mask");
   const int dh = PADDED ? head_dim : D;                 // columns of a head; elements between rows of O
-  const int k_row = PITCH ? (int)at.k.row : dh, v_row = PITCH ? (int)at.v.row : dh;
+  int k_row = dh, v_row = dh;                           // elements between rows of K and of V
+  if constexpr (PITCH) k_row = (int)at.k.row, v_row = (int)at.v.row;
   static_assert(!PITCH || !GENERAL, "strides: self-attention without a mask");
   static_assert(!MASKED || GENERAL, "masks: general kernel");
   static_assert(!MASK_LDS || (MASKED && NW == 8), "staged mask tiles: 8 waves");
@@ -169,10 +171,14 @@ void flash_fwd_kernel(const T* __restrict__ Q, const T* __restrict__ K, const T*
     }
     const int64_t base = (int64_t)zh * S * dh;
     const int64_t kv_base = (int64_t)zh * Skv * dh;
-    const T* q_g = Q + (PITCH ? head_at(at.q, at.heads, zh) : base);
-    const T* k_g = K + (PITCH ? head_at(at.k, at.heads, zh) : kv_base);
-    const T* v_g = V + (PITCH ? head_at(at.v, at.heads, zh) : kv_base);
-    const int64_t q_row = PITCH ? at.q.row : dh;
+    const T *q_g = Q + base, *k_g = K + kv_base, *v_g = V + kv_base;
+    int64_t q_row = dh;
+    if constexpr (PITCH) {
+      q_g = Q + head_at(at.q, at.heads, zh);
+      k_g = K + head_at(at.k, at.heads, zh);
+      v_g = V + head_at(at.v, at.heads, zh);
+      q_row = at.q.row;
+    }
 
     const int q0 = qb * kBlockM + wave * 32;           // first query row of this wave
     const int qrow = q0 + lane % 32;                    // the query row this lane's scores belong to
@@ -643,7 +649,7 @@ int launch_mfma_nw(const void* Q, const void* K, const void* V, void* O, int64_t
   hipLaunchKernelGGL((flash_fwd_kernel<T, OutT, D, CAUSAL, false, NW, false, false, false, false, PITCH>),                 \
                      dim3((unsigned)blocks), dim3(NW * 64), 0, st, static_cast<const T*>(Q), static_cast<const T*>(K),     \
                      static_cast<const T*>(V), static_cast<OutT*>(O), (int)ZH, (int)S, scale_log2e,                        \
-                     static_cast<const T*>(nullptr), 0, 0.0f, groups, D, at)
+                     static_cast<const T*>(nullptr), 0, 0.0f, groups, D, rows_arg<PITCH>(at))
   if (at.contiguous) HEXMI_PLAIN(false); else HEXMI_PLAIN(true);
 #undef HEXMI_PLAIN
   return launch_status();
@@ -659,10 +665,13 @@ int launch_mfma_padded(const void* Q, const void* K, const void* V, void* O, int
   const int64_t blocks = resident_grid(units, 2);
   if (blocks <= 0) return HEXMI_ELAUNCH;
   const int groups = CAUSAL ? plan_causal_groups(ZH, nqb, blocks) : 0;
-  hipLaunchKernelGGL((flash_fwd_kernel<T, OutT, D, CAUSAL, false, 4, false, true>), dim3((unsigned)blocks), dim3(256), 0, st,
-                     static_cast<const T*>(Q), static_cast<const T*>(K), static_cast<const T*>(V),
-                     static_cast<OutT*>(O), (int)ZH, (int)S, scale_log2e, static_cast<const T*>(nullptr), 0, 0.0f,
-                     groups, head_dim, at);
+#define HEXMI_PADDED(PITCH)                                                                                               \
+  hipLaunchKernelGGL((flash_fwd_kernel<T, OutT, D, CAUSAL, false, 4, false, true, false, false, PITCH>), dim3((unsigned)blocks), \
+                     dim3(256), 0, st, static_cast<const T*>(Q), static_cast<const T*>(K), static_cast<const T*>(V),       \
+                     static_cast<OutT*>(O), (int)ZH, (int)S, scale_log2e, static_cast<const T*>(nullptr), 0, 0.0f,         \
+                     groups, head_dim, rows_arg<PITCH>(at))
+  if (at.contiguous) HEXMI_PADDED(false); else HEXMI_PADDED(true);
+#undef HEXMI_PADDED
   return launch_status();
 }
 
@@ -677,10 +686,13 @@ int launch_mfma_wide(const void* Q, const void* K, const void* V, void* O, int64
   const int64_t blocks = resident_grid(units, 1);
   if (blocks <= 0) return HEXMI_ELAUNCH;
   const int groups = CAUSAL ? plan_causal_groups(ZH, nqb, blocks) : 0;
-  hipLaunchKernelGGL((flash_fwd_kernel<T, OutT, 128, CAUSAL, false, 4, false, true, true>), dim3((unsigned)blocks), dim3(256), 0,
-                     st, static_cast<const T*>(Q), static_cast<const T*>(K), static_cast<const T*>(V),
-                     static_cast<OutT*>(O), (int)ZH, (int)S, scale_log2e, static_cast<const T*>(nullptr), 0, 0.0f,
-                     groups, head_dim, at);
+#define HEXMI_WIDE(PITCH)                                                                                                 \
+  hipLaunchKernelGGL((flash_fwd_kernel<T, OutT, 128, CAUSAL, false, 4, false, true, true, false, PITCH>), dim3((unsigned)blocks), \
+                     dim3(256), 0, st, static_cast<const T*>(Q), static_cast<const T*>(K), static_cast<const T*>(V),       \
+                     static_cast<OutT*>(O), (int)ZH, (int)S, scale_log2e, static_cast<const T*>(nullptr), 0, 0.0f,         \
+                     groups, head_dim, rows_arg<PITCH>(at))
+  if (at.contiguous) HEXMI_WIDE(false); else HEXMI_WIDE(true);
+#undef HEXMI_WIDE
   return launch_status();
 }
 

@@ -33,11 +33,11 @@ struct GroupTileLoader {
   static constexpr int NI = kTileKeys * CPR / 128;         // instructions per wave
   static constexpr int kRowStep = 128 / CPR;               // rows between a wave's instructions
   int row0, col[NI], lds0;                                 // this lane's row of instruction 0, its columns, the wave's part
-  int d, row_step;                                         // columns of the head; elements between rows in memory (PITCH)
+  int d, row_step;                                         // columns of the head; elements between rows in memory
   __device__ __forceinline__ void init(int rt, int lane, int head_dim, int pitch) {
     const int lin = rt * 64 + lane;
     d = PADDED ? head_dim : D;
-    row_step = PITCH ? pitch : D;
+    row_step = PITCH ? pitch : d;
     row0 = lin / CPR;
     lds0 = rt * 64 * 8;
 #pragma unroll
@@ -84,12 +84,12 @@ __device__ __forceinline__ void take_part(const bf16x8& part, float* p) {
 // small probability stays above 2^-24) or 16 (bf16, whose result is rounded to 8), three 24 (bf16 with an fp32 result). For
 // an fp32 result the parts of a tile meet in registers of their own, so that the running sum is rounded once a tile.
 // A part costs its share of MFMAs: 32 heads x 509 queries x 2555 keys of 128 with a mask 40 us in one part, 46 in two.
-// PITCH: Q, K and V stand as `at` says (narrower heads always; D columns wide: where they are not contiguous).
+// PITCH: Q, K and V stand as `at` says (where they are not contiguous).
 template <typename T, typename OutT, int D, bool CAUSAL, bool MASKED, bool PADDED, bool FULL, bool PITCH>
 __global__ __launch_bounds__(512, D == 64 && !MASKED ? 4 : 2)
 void flash_keys_kernel(const T* __restrict__ Q, const T* __restrict__ K, const T* __restrict__ V, OutT* __restrict__ O,
                        int ZH, int S, int Skv, float scale, const T* __restrict__ Mk, float* __restrict__ part,
-                       int chunk, int splits, int head_dim, HeadRows at) {
+                       int chunk, int splits, int head_dim, RowsArg<PITCH> at) {
   const int dh = PADDED ? head_dim : D;                 // elements between rows in memory
   static_assert(!(CAUSAL && MASKED), "the causal kernel has no mask");
   static_assert(!FULL || MASKED, "full probabilities: masked kernel");
@@ -141,17 +141,24 @@ void flash_keys_kernel(const T* __restrict__ Q, const T* __restrict__ K, const T
   const int first = split * chunk;                      // causal units are never cut
   const int last = first + chunk < unit_steps ? first + chunk : unit_steps;
 
-  const T* q_g = Q + (PITCH ? head_at(at.q, at.heads, zh) : (int64_t)zh * S * D);
-  const T* k_g = K + (PITCH ? head_at(at.k, at.heads, zh) : (int64_t)zh * Skv * D);
-  const T* v_g = V + (PITCH ? head_at(at.v, at.heads, zh) : (int64_t)zh * Skv * D);
+  const T *q_g = Q + (int64_t)zh * S * dh, *k_g = K + (int64_t)zh * Skv * dh, *v_g = V + (int64_t)zh * Skv * dh;
+  int64_t q_row = dh;
+  int k_row = dh, v_row = dh;
+  if constexpr (PITCH) {
+    q_g = Q + head_at(at.q, at.heads, zh);
+    k_g = K + head_at(at.k, at.heads, zh);
+    v_g = V + head_at(at.v, at.heads, zh);
+    q_row = at.q.row;
+    k_row = (int)at.k.row, v_row = (int)at.v.row;
+  }
   const int q0 = qb * kRows + rt * 32;
   const int qrow = q0 + lane % 32;
   const int qr = qrow < S ? qrow : S - 1;
 
   GroupTileLoader<T, D, false, PADDED, PITCH> k_loader;
   GroupTileLoader<T, D, true, PADDED, PITCH> v_loader;
-  k_loader.init(rt, lane, dh, (int)at.k.row);
-  v_loader.init(rt, lane, dh, (int)at.v.row);
+  k_loader.init(rt, lane, dh, k_row);
+  v_loader.init(rt, lane, dh, v_row);
   const int lds_g = ks * kTile;
   if constexpr (PADDED) {                               // ahead of the first barrier of the key loop
     k_loader.zero_padding(k_lds0 + lds_g, lane);
@@ -206,7 +213,7 @@ void flash_keys_kernel(const T* __restrict__ Q, const T* __restrict__ K, const T
 #pragma unroll
   for (int ds = 0; ds < DS; ++ds) {
     if (!PADDED || ds * 16 + half * 8 < dh)
-      qf[ds] = *reinterpret_cast<const Frag*>(q_g + (PITCH ? qr * at.q.row : (int64_t)qr * D) + ds * 16 + half * 8);
+      qf[ds] = *reinterpret_cast<const Frag*>(q_g + qr * q_row + ds * 16 + half * 8);
     else
       qf[ds] = Frag{};
   }
@@ -486,15 +493,16 @@ int launch_keys(const void* Q, const void* K, const void* V, const void* mask, v
   hipLaunchKernelGGL((flash_keys_kernel<T, OutT, D, C, M, P, F, X>), dim3((unsigned)blocks), dim3(512), 0, st,           \
                      static_cast<const T*>(Q), static_cast<const T*>(K), static_cast<const T*>(V),                    \
                      static_cast<OutT*>(O), (int)ZH, (int)S, (int)Skv, scale, static_cast<const T*>(mask), part,      \
-                     plan.chunk, plan.splits, head_dim, at)
-  if (head_dim < D) {
-    if (causal) HEXMI_KEYS(true, false, true, false, true);
-    else if (plan.full) HEXMI_KEYS(false, true, true, true, true);
-    else if (mask != nullptr) HEXMI_KEYS(false, true, true, false, true);
-    else HEXMI_KEYS(false, false, true, false, true);
-  } else if (!at.contiguous) {                             // self-attention only: no mask
-    if (causal) HEXMI_KEYS(true, false, false, false, true);
-    else HEXMI_KEYS(false, false, false, false, true);
+                     plan.chunk, plan.splits, head_dim, rows_arg<X>(at))
+  const bool narrow = head_dim < D;
+  if (!at.contiguous) {                                    // self-attention only: no mask
+    if (narrow) { if (causal) HEXMI_KEYS(true, false, true, false, true); else HEXMI_KEYS(false, false, true, false, true); }
+    else { if (causal) HEXMI_KEYS(true, false, false, false, true); else HEXMI_KEYS(false, false, false, false, true); }
+  } else if (narrow) {
+    if (causal) HEXMI_KEYS(true, false, true, false, false);
+    else if (plan.full) HEXMI_KEYS(false, true, true, true, false);
+    else if (mask != nullptr) HEXMI_KEYS(false, true, true, false, false);
+    else HEXMI_KEYS(false, false, true, false, false);
   } else {
     if (causal) HEXMI_KEYS(true, false, false, false, false);
     else if (plan.full) HEXMI_KEYS(false, true, false, true, false);

@@ -1,5 +1,6 @@
 // Shared device/host helpers for the hexmi kernels (gfx950 only).
 #pragma once
+#include <type_traits>
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 #include "hexmi.h"
@@ -319,6 +320,12 @@ inline HeadRows contiguous_heads(int64_t S, int64_t Skv, int64_t D) {
 __device__ __forceinline__ int64_t head_at(const RowStrides& r, int heads, int zh) {
   const int z = zh / heads;
   return z * r.batch + (zh - z * heads) * r.head;
+}
+// the kernel argument: heads that are contiguous need none
+struct NoRows {};
+template <bool PITCH> using RowsArg = std::conditional_t<PITCH, HeadRows, NoRows>;
+template <bool PITCH> inline RowsArg<PITCH> rows_arg(const HeadRows& at) {
+  if constexpr (PITCH) return at; else return {};
 }
 #endif
 
