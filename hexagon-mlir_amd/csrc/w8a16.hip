@@ -908,8 +908,15 @@ bool prefer_split(int64_t M, int64_t N, int64_t K, int cus) {
   const int64_t tiles = ((M + 127) / 128) * ((N + 127) / 128);
   return tiles * 3 <= cus || (tiles * 2 <= cus && K >= 8192);
 }
-// the tiles of w8a16_few.hip, ahead of it wherever they take a call
-bool prefer_few(int64_t M, int64_t N, int64_t K) { return K % 16 == 0 && plan_w8a16_few(M, N, K, K % 64 == 0 && N % 8 == 0).m; }
+// The tiles of w8a16_few.hip, ahead of it wherever they take a call, but where a quarter of the CUs or fewer would have one over a long K
+// (us, K parts / tiles, on weights from HBM and on weights in the cache behind L2: 64 x 2048 x 14336 23.6 / 32.2 and 23.2 / 26.6, 128 x 512 x
+// 14336 24.4 / 29.4 and 24.4 / 26.6, 192 x 512 x 14336 25.7 / 30.2 and 24.8 / 26.5; 128 x 1024 x 11392 23.4 / 26.8 and 24.2 / 22.6; half of the
+// CUs 128 x 2048 x 14336 30.2 / 32.5 and 29.0 / 26.8).
+bool prefer_few(int64_t M, int64_t N, int64_t K) {
+  if (K % 16 != 0) return false;
+  const GemmFewTile t = plan_w8a16_few(M, N, K, K % 64 == 0 && N % 8 == 0);
+  return t.m && !(K > 12288 && 4 * ((M + t.m - 1) / t.m) * ((N + t.n - 1) / t.n) <= hexmi_num_cus());
+}
 }  // namespace
 
 extern "C" int hexmi_gemm_w8a16_workspace_helps(int64_t M, int64_t N, int64_t K) {

@@ -247,7 +247,7 @@ int hexmi_gemm_w8a16(int64_t M, int64_t N, int64_t K, const void *A,
  * The reference's counterpart is the scratch its matmul runtime routine sets up
  * per call (bin/runtime/src/HexKLAPI.cpp:15-68: VTCM for tiles and the
  * accumulator read-back).
- * From 49 rows on most of these shapes have since got tiles of their own that
+ * From 49 rows on most of these shapes have got tiles of their own that
  * need no workspace and are ahead of that kernel (N = 4096, K = 11008, M = 128:
  * 26 us against 38): hexmi_gemm_w8a16_workspace_helps answers 0 there, and
  * the calls with and without a workspace run the same kernel (with one, its

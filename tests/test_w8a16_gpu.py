@@ -375,6 +375,8 @@ def test_w8a16_workspace_query_agrees_with_the_tiles(hexmi):
     assert lib.hexmi_gemm_w8a16_workspace(128, 4096, 11008) > 0 and not lib.hexmi_gemm_w8a16_workspace_helps(128, 4096, 11008)
     # 100 rows of more channels than 64 x 64 tiles go round, a long K: the kernel with K parts stays
     assert lib.hexmi_gemm_w8a16_workspace_helps(100, 9000, 8192) and not lib.hexmi_gemm_w8a16_workspace_helps(16, 4096, 4096)
+    assert lib.hexmi_gemm_w8a16_workspace_helps(128, 1000, 13312) and not lib.hexmi_gemm_w8a16_workspace_helps(128, 1088, 13312)
+    assert not lib.hexmi_gemm_w8a16_workspace_helps(128, 1000, 12288)
 
 
 # ---- the (channel range x K part) kernel behind hexmi_gemm_w8a16_ws -------------------------------------------
@@ -428,8 +430,10 @@ def test_w8a16_split_parity(hexmi, oracle, M, N, K):
     assert rc == 0 and torch.equal(got_p.cpu(), got.cpu()[:, perm])
 
 
-# ... and the ones it keeps beside the tiles of w8a16_few.hip: up to 32 rows of very many channels, up to 112 rows over a long K
-@pytest.mark.parametrize("M,N,K", [(32, 25000, 256), (100, 9000, 8192), (112, 1200, 12288), (66, 520, 11008)])
+# ... and the ones it keeps beside the tiles of w8a16_few.hip: up to 32 rows of very many channels, up to 112 rows over a long K, few
+# tiles over a long K
+@pytest.mark.parametrize("M,N,K", [(32, 25000, 256), (100, 9000, 8192), (112, 1200, 12288), (66, 520, 11008), (64, 2048, 12352),
+                                   (128, 1000, 13312), (250, 512, 12544)])
 def test_w8a16_split_parity_beside_the_tiles(hexmi, oracle, M, N, K):
     test_w8a16_split_parity(hexmi, oracle, M, N, K)
 
