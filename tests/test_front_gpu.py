@@ -157,3 +157,16 @@ def test_front_errors_are_those_of_ops(hexmi):
         hexmi.matmul(q[0], q[0])
     with pytest.raises(TypeError):
         hexmi.softmax(q.double())
+
+
+def test_front_is_left_out_while_dynamo_traces(hexmi):
+    import warnings
+    x, w = torch.randn(8, 64, device="cuda"), torch.ones(64, device="cuda")
+    for f in (lambda t: hexmi.softmax(t * 2) + 1, lambda t: hexmi.layer_norm(t, w, w, 1e-5) * 2, lambda t: hexmi.gelu(t + 1),
+              lambda t: hexmi.binary("add", t, t) * 2, lambda t: hexmi.matmul(t + 1, t, trans_b=True)):
+        want = f(x)
+        torch._dynamo.reset()
+        with warnings.catch_warnings(record=True) as seen:
+            warnings.simplefilter("always")
+            assert torch.equal(torch.compile(f, backend="eager")(x), want)
+        assert not [s for s in seen if "_front" in str(s.message) or "C/C++" in str(s.message)]
