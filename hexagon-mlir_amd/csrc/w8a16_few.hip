@@ -2,8 +2,8 @@
 // CUs, a workgroup of eight waves to a tile.
 //
 // What bounds it: a slab of a tile is read from LDS once per wave side by side, copied into LDS, widened and multiplied, and at one
-// workgroup per CU none of the four hides behind another entirely: 256 x 11008 x 4096 on 64 x 192 tiles takes 34 us, 27 without
-// the copies, 26 without the matrix instructions, 29 without the widening and 29 without the reads. So: eight waves; the weights
+// workgroup per CU none of the four hides behind another entirely: an earlier form of 64 x 192 tiles took 34 us for 256 x 11008 x 4096
+// on cold weights, 27 without the copies, 26 without the matrix instructions, 29 without the widening and 29 without the reads (this one 31). So: eight waves; the weights
 // stay int8 in LDS and a wave widens its own channels only, waves standing side by side along the channels (64 rows to a tile) so
 // that each weight is widened once; a slab of the larger tiles multiplies from registers while the next is read; the wave groups that take the 64-k parts of
 // a slab add up in LDS at the end; scales are fetched under the K walk (at the end, by the threads that store, they cost 1 to 3 us
@@ -269,7 +269,7 @@ template <> struct FewShape<64, 192> { typedef Shape<4, 3, 1, 4, 2, 3> S; };
 // The smallest tile of which there is at most one per CU. us for 32 x 64 / 64 x 64 / 64 x 128 / 64 x 192 tiles (how many; cold weights)
 // and what took these calls before: 128 x 4096 x 4096 10.8 (256) / 13.3 (128) / 20 (64) / 25, 22.4; 256 x 4096 x 4096 19.8 (512) /
 // 14.6 (256) / 21.5 / 25.7, 27.3; 512 x 4096 x 4096 - / 26.7 (512) / 22.2 (256) / 26.6, 31.4; 256 x 11008 x 4096 - / 44 (688) / 44
-// (344) / 30.8 (232), 36.3; 512 x 1024 x 1024 5.0 (256) / 6.6 / 8.3 / 9.8, 11.1. Over 200 random products each of 33 to 140 and of 129
+// (344) / 31 (232), 36.3; 512 x 1024 x 1024 5.0 (256) / 6.6 / 8.3 / 9.8, 11.1. Over 200 random products each of 33 to 140 and of 129
 // to 1024 rows 1.23 and 2.7 times the rate before. (128 x 128 tiles, 1000 x 4096 x 4096: 35.1, gemm.hip's 34.5.)
 // The chunked kernel of w8a16.hip, a workgroup per CU with all rows and up to 48 channels, stays ahead where rows are few: up to 48
 // (48 x 9570 x 3664 14.1 against 16.5), up to 64 rows of more than a round of 32 x 64 (64 x 8608 x 10528 38.5, 48), up to 112 of
