@@ -890,9 +890,11 @@ int dispatch_rows(const void* xv, void* yv, const void* wv, const void* bv, floa
   // x and y rows equally far off a 16-byte boundary (contiguous tensors with an odd number of columns, equal column slices of
   // aligned ones): aligned chunks over the span that covers the row. The norms from 3 MiB on, where that is 1.05 to 1.7 times as fast
   // (fp16, us: 4999 x 10001 RMSNorm 74.7 -> 44.9, LayerNorm 87.0 -> 55.8; 3000 x 777 fp32 8.0 -> 7.0); fewer rows wait for a row's
-  // two ends, which go by elements with weight and bias (1573 x 463 3.9 -> 4.3, 15 x 705 3.9 -> 4.6)
+  // two ends, which go by elements with weight and bias (1573 x 463 3.9 -> 4.3, 15 x 705 3.9 -> 4.6), unless sixteen waves share them (in
+  // accesses at the element's alignment / on spans: LayerNorm of 9 x 10246 fp32 6.3 / 5.0, 40 x 12001 7.5 / 6.7, 9 x 20001 fp16 10.5 / 7.5)
   {
-    const bool pays = OP == kSoftmax || rows >= (((int64_t)3 << 20) / (int64_t)sizeof(T) + cols - 1) / cols;
+    const bool pays = OP == kSoftmax || rows >= (((int64_t)3 << 20) / (int64_t)sizeof(T) + cols - 1) / cols ||
+                      span_chunks > 512 * 4;
     if (!vec_ok && same_offset && pays && rows <= 0x7fffffff && cols < 0x7ffffff0) {
 #define HEXMI_SPAN(C, TH, RPB, SPAN) \
   { hipLaunchKernelGGL((row_kernel<T, OP, C, TH, RPB, false, true, SPAN>), dim3((unsigned)((rows + RPB - 1) / RPB)), dim3(TH * RPB), 0, \
