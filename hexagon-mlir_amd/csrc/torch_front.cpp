@@ -15,6 +15,7 @@
 #include <torch/csrc/autograd/python_variable.h>
 
 #include <cmath>
+#include <cstddef>
 
 #include "hexmi.h"
 
@@ -319,17 +320,52 @@ PyObject* set_check(PyObject*, PyObject* f) {
   Py_RETURN_NONE;
 }
 
-#define HEXMI_FAST(f) {#f, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(f)), METH_FASTCALL, nullptr}
-PyMethodDef g_methods[] = {HEXMI_FAST(softmax), HEXMI_FAST(rms_norm), HEXMI_FAST(layer_norm), HEXMI_FAST(matmul),
-                           HEXMI_FAST(w8a16_matmul), HEXMI_FAST(flash_attention), HEXMI_FAST(attention), HEXMI_FAST(unary),
-                           HEXMI_FAST(binary), {"set_check", set_check, METH_O, nullptr}, {nullptr, nullptr, 0, nullptr}};
+// A function above as an object of a type of its own: dynamo breaks its graph at such a call without a word, at a built-in function's
+// with a warning. Called as fast.
+typedef PyObject* (*Function)(PyObject*, PyObject* const*, Py_ssize_t);
+struct Operator {
+  PyObject_HEAD
+  vectorcallfunc call;
+  Function f;
+};
+PyObject* call_operator(PyObject* self, PyObject* const* args, size_t n, PyObject* names) {
+  if (names && PyTuple_GET_SIZE(names) != 0) {
+    PyErr_SetString(PyExc_TypeError, "positional arguments only");
+    return nullptr;
+  }
+  return reinterpret_cast<Operator*>(self)->f(nullptr, args, PyVectorcall_NARGS(n));
+}
+PyTypeObject g_operator_type = {PyVarObject_HEAD_INIT(nullptr, 0)};
+bool add_operator(PyObject* m, const char* name, Function f) {
+  Operator* o = PyObject_New(Operator, &g_operator_type);
+  if (!o) return false;
+  o->call = call_operator;
+  o->f = f;
+  if (PyModule_AddObject(m, name, reinterpret_cast<PyObject*>(o)) == 0) return true;
+  Py_DECREF(o);
+  return false;
+}
+
+PyMethodDef g_methods[] = {{"set_check", set_check, METH_O, nullptr}, {nullptr, nullptr, 0, nullptr}};
 PyModuleDef g_module = {PyModuleDef_HEAD_INIT, "_front", "The operators' usual calls, natively.", -1, g_methods};
 
 }  // namespace
 
 // torch_version: what it was built for (HEXMI_TORCH_VERSION, from the build)
 PyMODINIT_FUNC PyInit__front() {
+  g_operator_type.tp_name = "hexmi._front.Operator";
+  g_operator_type.tp_basicsize = sizeof(Operator);
+  g_operator_type.tp_flags = Py_TPFLAGS_DEFAULT | Py_TPFLAGS_HAVE_VECTORCALL;
+  g_operator_type.tp_vectorcall_offset = offsetof(Operator, call);
+  g_operator_type.tp_call = PyVectorcall_Call;
+  if (PyType_Ready(&g_operator_type) != 0) return nullptr;
   PyObject* m = PyModule_Create(&g_module);
-  if (m && PyModule_AddStringConstant(m, "torch_version", HEXMI_TORCH_VERSION) != 0) Py_CLEAR(m);
+  if (!m) return nullptr;
+#define HEXMI_OPERATOR(f) add_operator(m, #f, f)
+  if (!(HEXMI_OPERATOR(softmax) && HEXMI_OPERATOR(rms_norm) && HEXMI_OPERATOR(layer_norm) && HEXMI_OPERATOR(matmul) &&
+        HEXMI_OPERATOR(w8a16_matmul) && HEXMI_OPERATOR(flash_attention) && HEXMI_OPERATOR(attention) && HEXMI_OPERATOR(unary) &&
+        HEXMI_OPERATOR(binary) && PyModule_AddStringConstant(m, "torch_version", HEXMI_TORCH_VERSION) == 0))
+    Py_CLEAR(m);
+#undef HEXMI_OPERATOR
   return m;
 }

@@ -373,7 +373,6 @@ def _not_plain(*args):
 
 
 _front = _Front()
-_compiling = torch.compiler.is_dynamo_compiling      # torch.compile breaks its graph at either route; at the native one it warns
 
 
 def _run(name, impl, simple, *args):
@@ -410,7 +409,7 @@ def softmax(x, out=None, dim=-1, block_cols=0):
     """Softmax over the last dimension (`F.softmax(x, dim=1)` of
     test/python/triton/test_softmax.py:93 for 2-D input). block_cols > 0: the two-phase (online) form of
     test/python/triton/test_online_softmax.py:31-81 over column blocks of that size."""
-    if out is None and dim == -1 and not block_cols and not _THROUGH_DISPATCHER and not _compiling():
+    if out is None and dim == -1 and not block_cols and not _THROUGH_DISPATCHER:
         y = _front.softmax(x)
         if y is not None:
             return y
@@ -426,7 +425,7 @@ def softmax(x, out=None, dim=-1, block_cols=0):
 
 def rms_norm(x, weight=None, eps=1e-5, out=None, block_cols=0):
     """`F.rms_norm(x, (C,), weight, eps)` (test/python/triton/test_rms_norm.py:85-87)."""
-    if out is None and not block_cols and not _THROUGH_DISPATCHER and not _compiling():
+    if out is None and not block_cols and not _THROUGH_DISPATCHER:
         y = _front.rms_norm(x, weight, eps)
         if y is not None:
             return y
@@ -444,7 +443,7 @@ def rms_norm(x, weight=None, eps=1e-5, out=None, block_cols=0):
 def layer_norm(x, weight=None, bias=None, eps=1e-5, out=None, mean=None, rstd=None, block_cols=0):
     """`F.layer_norm(x, (C,), weight, bias, eps)` (test/python/triton/test_layer_norm.py:111-113);
     `mean` / `rstd` (fp32, one per row) are filled when given, as the reference kernel does."""
-    if out is None and mean is None and rstd is None and not block_cols and not _THROUGH_DISPATCHER and not _compiling():
+    if out is None and mean is None and rstd is None and not block_cols and not _THROUGH_DISPATCHER:
         y = _front.layer_norm(x, weight, bias, eps)
         if y is not None:
             return y
@@ -475,7 +474,7 @@ def matmul(a, b, out=None, out_dtype=None, trans_b=False, bias=None, residual=No
     reference's fusion pass pulls the consumers of a matmul into its loop nest
     (qcom_hexagon_backend/lib/Conversion/LinalgToLLVM/LinalgToLLVMPass.cpp:280-283): C = A @ B + bias + residual
     with one rounding and no extra launch."""
-    if out is None and out_dtype is None and not _THROUGH_DISPATCHER and not _compiling():
+    if out is None and out_dtype is None and not _THROUGH_DISPATCHER:
         y = _front.matmul(a, b, trans_b, bias, residual)
         if y is not None:
             return y
@@ -540,7 +539,7 @@ def _quant_params(name, w_int8, scales, zero_points):
 def w8a16_matmul(a, w_int8, scales, out=None, zero_points=None):
     """C[m,n] = sum_k A[m,k] * ((W[n,k] - zero_points[n]) * scales[n]); A fp16 [M,K], W int8 [N,K], scales fp16 [N]
     (or [1]: one scale and zero point for the tensor), zero_points int8 or None (symmetric)."""
-    if out is None and not _THROUGH_DISPATCHER and not _compiling():
+    if out is None and not _THROUGH_DISPATCHER:
         y = _front.w8a16_matmul(a, w_int8, scales, zero_points)
         if y is not None:
             return y
@@ -619,7 +618,7 @@ def dequant_w8(w_int8, scales, out=None, zero_points=None):
 def flash_attention(q, k, v, sm_scale=None, causal=False, out=None, out_dtype=None):
     """softmax(sm_scale * Q K^T [+causal]) V for [Z,H,S,D] tensors
     (`F.scaled_dot_product_attention(q, k, v, scale=...)`, test/python/triton/test_flash_attention.py:212)."""
-    if out is None and out_dtype is None and not _THROUGH_DISPATCHER and not _compiling():
+    if out is None and out_dtype is None and not _THROUGH_DISPATCHER:
         y = _front.flash_attention(q, k, v, sm_scale, causal)
         if y is not None:
             return y
@@ -649,7 +648,7 @@ def attention(q, k, v, mask=None, sm_scale=None, out=None, out_dtype=None):
     """tm_tensor.attention: softmax(Q K^T / sqrt(d) + mask) V for q [B,Sq,D], k / v [B,Skv,D] and an additive
     mask [B,Sq,Skv] (or None) (include/hexagon/Dialect/TmTensor/IR/TmTensorOps.td:28-56,
     lib/Transforms/LowerTmTensor.cpp:70-235); `F.scaled_dot_product_attention(q, k, v, attn_mask=mask)`."""
-    if out is None and out_dtype is None and not _compiling():
+    if out is None and out_dtype is None:
         y = _front.attention(q, k, v, mask, sm_scale)
         if y is not None:
             return y
@@ -681,7 +680,7 @@ def unary(op, x, out=None):
     "rsqrt": test_rsqrt.py:20-24, "sin" / "cos": test_math_ops.py:25-38, "exp")."""
     if op not in UNARY_OPS:
         raise ValueError("hexmi.unary: unknown op %r" % (op,))
-    if out is None and not _compiling():
+    if out is None:
         y = _front.unary(UNARY_OPS[op], x)
         if y is not None:
             return y
@@ -707,7 +706,7 @@ def binary(op, a, b, out=None):
     test_vec_div_2d.py:21-55)."""
     if op not in BINARY_OPS:
         raise ValueError("hexmi.binary: unknown op %r" % (op,))
-    if out is None and not _compiling():
+    if out is None:
         y = _front.binary(BINARY_OPS[op], a, b)
         if y is not None:
             return y

@@ -42,9 +42,11 @@ def test_the_native_front_is_the_one_that_is_built():
     with warnings.catch_warnings():
         warnings.simplefilter("error")
         assert front.softmax(torch.zeros(4, 8)) is None   # a host tensor is not of the plain form
-    assert type(front.softmax).__name__ == "builtin_function_or_method"
+    assert type(front.softmax).__name__ == "Operator"
     with pytest.raises(AttributeError):
         front.no_such_operator
+    with pytest.raises(TypeError):
+        front.softmax(x=torch.zeros(4, 8))
 
 
 def test_the_front_is_built_again_for_another_torch(monkeypatch, tmp_path):

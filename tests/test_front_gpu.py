@@ -159,7 +159,7 @@ def test_front_errors_are_those_of_ops(hexmi):
         hexmi.softmax(q.double())
 
 
-def test_front_is_left_out_while_dynamo_traces(hexmi):
+def test_dynamo_breaks_its_graph_at_the_front_without_a_warning(hexmi):
     import warnings
     x, w = torch.randn(8, 64, device="cuda"), torch.ones(64, device="cuda")
     for f in (lambda t: hexmi.softmax(t * 2) + 1, lambda t: hexmi.layer_norm(t, w, w, 1e-5) * 2, lambda t: hexmi.gelu(t + 1),
