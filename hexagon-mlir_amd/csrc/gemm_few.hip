@@ -294,13 +294,16 @@ template <> struct FewShape<128, 64> { typedef Shape<4, 4, 2, 1, 4> S; static co
 //   apart (16 x 4096 x 16384 33.5, 28.2 / 33.5, 28.0);
 //   17 to 24 rows, two tiles of 16 x 32, weights of less than 2^25 elements (weight stream): 17 x 3072 x 5120 12.5, 13.2 / 8.0, 8.7;
 //   24 x 3072 x 2752 8.1, 9.0 / 5.8, 6.4; 17 x 2560 x 6912 14.3, 15.0 / 8.6, 9.8 (32 rows 16.7, 16.4 / 11.2, 10.4).
+// The weight stream takes whole 32s of K and 64 channels and more; what neither it nor the dot products take has its tile at any size of the
+// weights (on the 128 x 128 tiles, us, before / now: 16 x 272 x 4264 40 / 6.8, 30 x 3000 x 2504 24.6 / 6.4, 16 x 11008 x 1000 15.8 / 7.8,
+// 12 x 4096 x 776 12.6 / 4.5, 50 x 3000 x 104 4.9 / 3.5).
 GemmFewTile plan_gemm_few(bool trans_b, int64_t M, int64_t N, int64_t K) {
   const int64_t cus = hexmi_num_cus();
-  if (trans_b && M <= 64) {
-    if (M > 32 ? K <= 128 : N * K < (int64_t)(M > 16 ? 2 : 3) << 22 && !(M >= 5 && M <= 8 && K >= 2048)) return {0, 0};
-  }
   const bool dots = trans_b && N >= 64 && ((M <= 4 && K >= 1024) || (M <= 8 && K >= 2048));
   const bool stream = trans_b && N >= 64 && !dots && K % 32 == 0;
+  if ((dots || stream) && M <= 64) {
+    if (M > 32 ? K <= 128 : N * K < (int64_t)(M > 16 ? 2 : 3) << 22 && !(M >= 5 && M <= 8 && K >= 2048)) return {0, 0};
+  }
   static constexpr GemmFewTile kTiles[] = {{16, 16}, {16, 32}, {32, 32}, {32, 64}, {64, 64}, {128, 64}};
   for (const GemmFewTile& t : kTiles) {
     if (t.m == 16 && (M > 64 || (t.n == 16 && !trans_b))) continue;       // sixteen columns of a row of B are a quarter of a line

@@ -254,6 +254,16 @@ def test_gemm_one_round_of_tiles(hexmi, dtype, out_dtype, trans_b, M, N, K):
         assert torch.equal(view[:, N:], keep)
 
 
+# up to 64 rows against [N,K] weights that the weight stream does not take: K off whole 32s, fewer than 64 channels
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("M,N,K", [(3, 64, 8), (8, 700, 1000), (9, 65, 40), (16, 272, 4264), (17, 257, 1128), (32, 384, 856), (33, 2000, 72),
+                                   (64, 513, 2056), (3, 63, 1056), (40, 50, 2048), (64, 1, 256), (16, 4097, 776)])
+def test_gemm_few_rows_the_weight_stream_leaves(hexmi, dtype, M, N, K):
+    for out_dtype in (dtype, torch.float32):
+        _against_double(hexmi, dtype, out_dtype, True, M, N, K, False, False, M + N)
+        _against_double(hexmi, dtype, out_dtype, True, M, N, K, True, True, M + K)
+
+
 # more tiles than one round of them: the 128 x 128 and 256 x 256 kernels and the slabs, widths and outputs each is for
 @pytest.mark.parametrize("trans_b", [False, True])
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
