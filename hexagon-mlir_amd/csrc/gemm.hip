@@ -24,7 +24,7 @@
 // or 32-wide (gemm_kernel) slabs of K -> the tiled kernels as described; K a multiple of 8 only -> gemm_kernel with
 // the last slab's chunks past K fetched from a zero chunk; an output side without runs of four columns (odd N with B
 // as [N,K], odd ldc, unaligned C) -> the same kernels with the tile leaving through LDS in the pieces of 16 bytes that each row holds;
-// anything else (unaligned operand rows, K % 8 != 0) -> gemm_kernel_any, which stages the slabs through registers.
+// anything else (unaligned operand rows, K % 8 != 0) -> the tiles of gemm_few.hip with slabs that come through registers.
 // Whole chunks of K and no more tiles than CUs -> gemm_few.hip, tiles of 16 x 16 to 128 x 64 that give every CU a share, beyond the
 // lines of plan_gemm_few where B is [N,K] and rows are few. Of what it leaves: up to eight rows against B as [N,K] -> gemv_nt_kernel, a
 // stream of the weights with one wave per output channel; up to 64, by measured lines -> gemm_skinny.hip, a workgroup per 16 to
@@ -720,19 +720,6 @@ template <> struct Mfma16<bf16> {
   }
 };
 
-// sixteen 16-bit columns in two chunks, from column `by` (0 .. 7) on: eight of them
-__device__ __forceinline__ u32x4 shift_columns(const u32x4& lo, const u32x4& hi, int by) {
-  auto pick = [](bool second, uint32_t v0, uint32_t v1) { return second ? v1 : v0; };    // (values, not places: no scratch)
-  const bool by4 = by & 4, by2 = by & 2;
-  const uint32_t x0 = pick(by4, lo[0], lo[2]), x1 = pick(by4, lo[1], lo[3]), x2 = pick(by4, lo[2], hi[0]),
-                 x3 = pick(by4, lo[3], hi[1]), x4 = pick(by4, hi[0], hi[2]), x5 = pick(by4, hi[1], hi[3]);
-  const uint32_t y0 = pick(by2, x0, x1), y1 = pick(by2, x1, x2), y2 = pick(by2, x2, x3), y3 = pick(by2, x3, x4),
-                 y4 = pick(by2, x4, x5);
-  const int bits = (by & 1) * 16;
-  const u32x4 o = {__builtin_amdgcn_alignbit(y1, y0, bits), __builtin_amdgcn_alignbit(y2, y1, bits),
-                   __builtin_amdgcn_alignbit(y3, y2, bits), __builtin_amdgcn_alignbit(y4, y3, bits)};
-  return o;
-}
 // the first NC columns of a piece, at an address that is a multiple of NC columns
 template <int NC, typename OutT>
 __device__ __forceinline__ void store_cols(OutT* p, const u32x4& v) {
@@ -1146,15 +1133,12 @@ void gemm_kernel_k64(const T* __restrict__ A, const void* __restrict__ Bv, typen
   }
 }
 
-// Any shape, any alignment: what the kernels above do not take -- operand rows that do not start on 16-byte
-// boundaries (an odd leading dimension, a base that is a view into a larger tensor), K not a multiple of 8, B given as
-// [K,N] with a ragged N. 128x128 tiles, four waves of 2x2 MFMA tiles, the LDS layouts and fragment reads of
-// gemm_kernel; but the slabs come through registers: 16-byte global loads at whatever alignment the rows have (the
+// int8 weights of any shape, any alignment (K off whole 16s, odd bases). 128x128 tiles, four waves of 2x2 MFMA tiles, the LDS layouts and
+// fragment reads of gemm_kernel; but the slabs come through registers: 16-byte global loads at whatever alignment the rows have (the
 // hardware takes them at 2-byte alignment; the global -> LDS copy path is kept for aligned chunks), issued for slab
 // kt + 1 before slab kt is multiplied and written to the other LDS stage after it, one barrier per slab. A chunk that
-// reaches past K (or, B as [K,N], past N) is put together from guarded element loads with zeros behind the edge; rows
-// past M (and past N, B as [N,K]) are clamped, their products never stored. The result leaves in rows through LDS
-// (store_tile_by_rows). About 0.5 PFLOP/s where the one-MFMA-per-barrier kernel this replaces ran 0.07.
+// reaches past K is put together from guarded element loads with zeros behind the edge; rows past M and N are clamped, their
+// products never stored. The result leaves in rows through LDS (store_tile_by_rows).
 template <typename T>
 __device__ __forceinline__ u32x4 load_chunk_any(const T* p, int valid) {
   u32x4 v;
@@ -1185,23 +1169,18 @@ __device__ __forceinline__ u32x4 load_chunk_i8(const int8_t* p, int valid, int z
   return u.v;
 }
 
-// B_I8: B is int8 [N,K] (needs TRANS_B, fp16 A and C): (W - zero_point) is formed in fp16 on the way into LDS and the
-// finished sums are multiplied by scales[column] (one scale and zero point for the tensor with per_tensor).
-template <typename T, typename OutT, bool TRANS_B, bool B_I8 = false>
+// (W - zero_point) is formed in fp16 on the way into LDS and the finished sums are multiplied by scales[column] (one scale and zero
+// point for the tensor with per_tensor).
 __global__ __launch_bounds__(256)
-void gemm_kernel_any(const T* __restrict__ A, const void* __restrict__ Bv, OutT* C, int M, int N, int K, int64_t lda,
-                     int64_t ldb, int64_t ldc, int tiles_m, int tiles_n, const OutT* __restrict__ bias = nullptr,
-                     const OutT* resid = nullptr, int64_t ldr = 0, const f16* __restrict__ scales = nullptr,
-                     const int8_t* __restrict__ zero_points = nullptr, int per_tensor = 0) {
-  static_assert(sizeof(T) == 2, "16-bit operands");
-  static_assert(!B_I8 || (TRANS_B && std::is_same<T, f16>::value), "int8 B is [N,K] and multiplies fp16 A");
-  const T* B = static_cast<const T*>(Bv);
-  const int8_t* B8 = static_cast<const int8_t*>(Bv);
-  typedef typename Mfma<T>::Frag Frag;
+void gemm_kernel_any_i8(const f16* __restrict__ A, const int8_t* __restrict__ B, f16* __restrict__ C, int M, int N, int K, int tiles_m,
+                        int tiles_n, const f16* __restrict__ scales, const int8_t* __restrict__ zero_points, int per_tensor) {
+  typedef f16 T;
+  typedef Mfma<T>::Frag Frag;
+  const int64_t lda = K, ldb = K;
   constexpr int WM = 2, WN = 2, NW = 4, BM = 128, BN = 128;
   __shared__ __attribute__((aligned(16))) T a_s[2][BM * BK];
   __shared__ __attribute__((aligned(16))) T b_s[2][BN * BK];
-  __shared__ __attribute__((aligned(16))) OutT c_s[RaggedStage<OutT>::kRows * RaggedStage<OutT>::pitch(BN)];
+  __shared__ __attribute__((aligned(16))) f16 c_s[RaggedStage<f16>::kRows * RaggedStage<f16>::pitch(BN)];
   const int tid = threadIdx.x, lane = tid % kWave, wave = tid / kWave;
   const int wm = wave / 2, wn = wave % 2;
   int tm, tn;
@@ -1216,66 +1195,36 @@ void gemm_kernel_any(const T* __restrict__ A, const void* __restrict__ Bv, OutT*
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
 
-  // Two chunks of each operand per thread and slab. K-contiguous tile: chunk e -> row e / 4, source chunk e % 4.
-  // [K,N] tile: chunk e -> slab row e / 16, source chunk e % 16. LDS positions as in KMajorLoader / NMajorLoader.
+  // Two chunks of each operand per thread and slab: chunk e -> row e / 4, source chunk e % 4. LDS positions as in KMajorLoader.
   const T* a_ptr[2];
-  const T* b_ptr[2];
-  const int8_t* b8_ptr[2];
-  int a_k[2], b_k[2], a_pos[2], b_pos[2], b_valid_n[2], b_zero[2];
+  const int8_t* b_ptr[2];
+  int a_k[2], a_pos[2], b_zero[2];
 #pragma unroll
   for (int j = 0; j < 2; ++j) {
-    const int e = j * 256 + tid;
-    {
-      const int row = e / 4, c = e % 4;
-      int grow = m0 + row;
-      grow = grow < M - 1 ? grow : M - 1;
-      a_ptr[j] = A + (int64_t)grow * lda + c * kChunk;
-      a_k[j] = c * kChunk;
-      a_pos[j] = row * BK + ((c ^ swz_k(row)) * kChunk);
-    }
-    if constexpr (TRANS_B) {
-      const int row = e / 4, c = e % 4;
-      int grow = n0 + row;
-      grow = grow < N - 1 ? grow : N - 1;
-      if constexpr (B_I8) b8_ptr[j] = B8 + (int64_t)grow * ldb + c * kChunk;
-      else b_ptr[j] = B + (int64_t)grow * ldb + c * kChunk;
-      b_k[j] = c * kChunk;
-      b_pos[j] = row * BK + ((c ^ swz_k(row)) * kChunk);
-      b_valid_n[j] = kChunk;
-      b_zero[j] = B_I8 && zero_points ? (int)zero_points[per_tensor ? 0 : grow] : 0;
-    } else {
-      constexpr int CPR = BN / kChunk;
-      const int k = e / CPR, c = e % CPR;
-      const int gcol = n0 + c * kChunk;
-      b_valid_n[j] = gcol >= N ? 0 : (N - gcol < kChunk ? N - gcol : kChunk);   // columns of this chunk inside the matrix
-      b_ptr[j] = B + (int64_t)k * ldb + (gcol < N ? gcol : 0);
-      b_k[j] = k;
-      b_pos[j] = (k * CPR + (c ^ swz_n(k))) * kChunk;
-    }
+    const int e = j * 256 + tid, row = e / 4, c = e % 4;
+    const int am = m0 + row < M - 1 ? m0 + row : M - 1, bn = n0 + row < N - 1 ? n0 + row : N - 1;
+    a_ptr[j] = A + (int64_t)am * lda + c * kChunk;
+    b_ptr[j] = B + (int64_t)bn * ldb + c * kChunk;
+    a_k[j] = c * kChunk;
+    a_pos[j] = row * BK + ((c ^ swz_k(row)) * kChunk);
+    b_zero[j] = zero_points ? (int)zero_points[per_tensor ? 0 : bn] : 0;
   }
   u32x4 ra[2], rb[2];
   auto fetch = [&](int kt) {
     const int k0 = kt * BK;
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
-      const int left = K - (k0 + a_k[j]);                    // elements of this chunk before the end of K
-      ra[j] = load_chunk_any<T>(a_ptr[j] + k0, left < 0 ? 0 : left);
-      if constexpr (B_I8) {
-        const int leftb = K - (k0 + b_k[j]);
-        rb[j] = load_chunk_i8(b8_ptr[j] + k0, leftb < 0 ? 0 : leftb, b_zero[j]);
-      } else if constexpr (TRANS_B) {
-        const int leftb = K - (k0 + b_k[j]);
-        rb[j] = load_chunk_any<T>(b_ptr[j] + k0, leftb < 0 ? 0 : leftb);
-      } else {
-        rb[j] = load_chunk_any<T>(b_ptr[j] + (int64_t)k0 * ldb, k0 + b_k[j] < K ? b_valid_n[j] : 0);
-      }
+      int left = K - (k0 + a_k[j]);                          // elements of this chunk before the end of K
+      left = left < 0 ? 0 : left;
+      ra[j] = load_chunk_any<T>(a_ptr[j] + k0, left);
+      rb[j] = load_chunk_i8(b_ptr[j] + k0, left, b_zero[j]);
     }
   };
   auto stash = [&](int stage) {
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
       *reinterpret_cast<u32x4*>(&a_s[stage][a_pos[j]]) = ra[j];
-      *reinterpret_cast<u32x4*>(&b_s[stage][b_pos[j]]) = rb[j];
+      *reinterpret_cast<u32x4*>(&b_s[stage][a_pos[j]]) = rb[j];
     }
   };
   const int KT = (K + BK - 1) / BK;
@@ -1291,10 +1240,7 @@ void gemm_kernel_any(const T* __restrict__ A, const void* __restrict__ Bv, OutT*
 #pragma unroll
       for (int i = 0; i < WM; ++i) af[i] = read_kmajor<T>(a_s[stage], (wm * WM + i) * 32 + lane % 32, ks * 2 + lane / 32);
 #pragma unroll
-      for (int j = 0; j < WN; ++j) {
-        if constexpr (TRANS_B) bf[j] = read_kmajor<T>(b_s[stage], (wn * WN + j) * 32 + lane % 32, ks * 2 + lane / 32);
-        else bf[j] = read_nmajor<T, BN>(b_s[stage], (wn * WN + j) * 32, ks, lane);
-      }
+      for (int j = 0; j < WN; ++j) bf[j] = read_kmajor<T>(b_s[stage], (wn * WN + j) * 32 + lane % 32, ks * 2 + lane / 32);
 #pragma unroll
       for (int i = 0; i < WM; ++i)
 #pragma unroll
@@ -1303,8 +1249,8 @@ void gemm_kernel_any(const T* __restrict__ A, const void* __restrict__ Bv, OutT*
     if (kt + 1 < KT) stash(stage ^ 1);
     __syncthreads();
   }
-  store_tile_by_rows<OutT, WM, WN, NW, BM, BN>(acc, c_s, C, ldc, bias, resid, ldr, M, N, m0, n0, wm, wn, wave, lane,
-                                               B_I8 ? scales : nullptr, per_tensor);
+  store_tile_by_rows<f16, WM, WN, NW, BM, BN>(acc, c_s, C, N, nullptr, nullptr, 0, M, N, m0, n0, wm, wn, wave, lane, scales,
+                                              per_tensor);
 }
 
 // Up to eight activation rows against weights given as [N,K] (x @ W^T, a decode step): the product is a stream of
@@ -1652,7 +1598,7 @@ int dispatch_gemm(const void* Av, const void* Bv, void* Cv, int64_t M, int64_t N
   }
   // Whole 16-byte chunks on the operand side only (K % 8 == 0; B given as [K,N] also N % 8 == 0): the 128x128 tiles
   // with a masked last slab, and an output side that may be anything ([N,K] weights with an odd N, such as a
-  // vocabulary of 50257, land here: 1.0 PFLOP/s against 0.1 on the generic kernel below).
+  // vocabulary of 50257, land here: 1.0 PFLOP/s against 0.3 through registers).
   // ... and with whole 64-wide slabs, a 16-bit result and no epilogue operands the paired-slab kernels take it, their
   // staged tiles leaving in the aligned pieces of each row
   if (chunks && sizeof(OutT) == 2 && K % BK2 == 0 && lda < (1 << 21) && ldb < (1 << 21) && !bias && !resid) {
@@ -1669,11 +1615,7 @@ int dispatch_gemm(const void* Av, const void* Bv, void* Cv, int64_t M, int64_t N
                        bias, resid, ldr, runs ? 1 : 0);
     return launch_status();
   }
-  const int64_t tiles_m = (M + 127) / 128, tiles_n = (N + 127) / 128;
-  if (tiles_m * tiles_n > 0x7fffffff || K > 0x7fffffff - 64) return HEXMI_ENOTSUP;
-  hipLaunchKernelGGL((gemm_kernel_any<T, OutT, TRANS_B>), dim3((unsigned)(tiles_m * tiles_n)), dim3(256), 0, s, A, B, C,
-                     (int)M, (int)N, (int)K, lda, ldb, ldc, (int)tiles_m, (int)tiles_n, bias, resid, ldr);
-  return launch_status();
+  return launch_gemm_any<T, OutT, TRANS_B>(A, B, C, M, N, K, lda, ldb, ldc, s, bias, resid, ldr);
 }
 
 template <typename T, typename OutT>
@@ -1735,9 +1677,8 @@ int gemm_w8a16_any_shape(int64_t M, int64_t N, int64_t K, const f16* A, const in
                          const int8_t* zero_points, int per_tensor, f16* C, hipStream_t stream) {
   const int64_t tiles_m = (M + 127) / 128, tiles_n = (N + 127) / 128;
   if (tiles_m * tiles_n > 0x7fffffff || K > 0x7fffffff - 64) return HEXMI_ENOTSUP;
-  hipLaunchKernelGGL((gemm_kernel_any<f16, f16, true, true>), dim3((unsigned)(tiles_m * tiles_n)), dim3(256), 0, stream, A,
-                     static_cast<const void*>(W), C, (int)M, (int)N, (int)K, K, K, N, (int)tiles_m, (int)tiles_n, nullptr,
-                     nullptr, 0, scales, zero_points, per_tensor);
+  hipLaunchKernelGGL(gemm_kernel_any_i8, dim3((unsigned)(tiles_m * tiles_n)), dim3(256), 0, stream, A, W, C, (int)M, (int)N, (int)K,
+                     (int)tiles_m, (int)tiles_n, scales, zero_points, per_tensor);
   return launch_status();
 }
 

@@ -32,11 +32,11 @@ template <typename T> struct Frag8;
 template <> struct Frag8<f16> { typedef f16x8 V; };
 template <> struct Frag8<bf16> { typedef bf16x8 V; };
 
-// TM x TN: 16 x 16 tiles of a wave; SM x SN waves side by side; KH wave groups share the 32-k steps of a slab.
-template <int TM_, int TN_, int SM_, int SN_, int KH_>
+// TM x TN: 16 x 16 tiles of a wave; SM x SN waves side by side; KH wave groups share the 32-k steps of a slab, STEPS (one or two) each.
+template <int TM_, int TN_, int SM_, int SN_, int KH_, int STEPS_ = 1>
 struct Shape {
-  static constexpr int TM = TM_, TN = TN_, SM = SM_, SN = SN_, KH = KH_, kWaves = SM * SN * KH, kThreads = kWaves * kWave;
-  static constexpr int BM = SM * TM * 16, BN = SN * TN * 16, BK = KH * 32;
+  static constexpr int TM = TM_, TN = TN_, SM = SM_, SN = SN_, KH = KH_, STEPS = STEPS_, kWaves = SM * SN * KH, kThreads = kWaves * kWave;
+  static constexpr int BM = SM * TM * 16, BN = SN * TN * 16, BK = KH * STEPS * 32;
   static constexpr int kStage = (BM + BN) * BK;                  // elements of a stage: rows of A, then B
 };
 
@@ -46,22 +46,35 @@ template <int BK> __device__ __forceinline__ int swz_row(int r) { return BK == 6
 // N-contiguous tile of BN columns a row of k: the 32 lanes of a transposing read touch k % 4, k / 8 % 2 x 32 bytes, which the
 // XOR spreads over the eight 32-byte slots of all banks
 template <int BN> __device__ __forceinline__ int swz_col(int k) {
+  if (BN == 128) return ((k & 3) | (((k >> 3) & 1) << 2)) << 1;
   return BN == 64 ? (((k >> 1) & 1) | (((k >> 3) & 1) << 1)) << 1 : ((k >> 3) & 1) << 1;
 }
 
 // NS stages of a slab of KH * 32 k: copies fill all but one while that one is read; one barrier a slab. K % 8 == 0, operand rows
 // on 16-byte boundaries ([K,N]: N % 8 == 0 too). runs: the output (and bias and residual) in runs of eight columns on
 // 16-byte boundaries; otherwise they go by elements.
-template <typename T, typename OutT, typename S, int NS, bool TRANS_B>
-__global__ __launch_bounds__(S::kThreads)
+// ANY: operand rows at any alignment, any K and N ([K,N] weights with an odd N, views). A copy into LDS needs its 16 bytes on a
+// boundary, a load into registers does not: two slabs are on their way in registers while a third is multiplied from one of two
+// stages. Bound by the latency of a slab's loads as the copies are, so no load waits for a choice: a chunk that reaches past the end of K or
+// of a [K,N] row is read as the last eight elements before it and shifted into place, with zeros behind K, on its way into LDS, in
+// the last slab and the last column of tiles only. Tiles of 128 x 128 have one slab on its way, so that two fit a CU. (128 x 128 tiles that
+// put such chunks together from elements under a branch of every load had their four chunks of a slab one latency after the other, 2 us
+// for 32 of K. [K,N], us, there / here: 128 x 7219 x 6656 299 / 49, 640 x 7031 x 3584 322 / 105, 16 x 4097 x 4096 120 / 19, 50 x 1001 x 768
+// 48 / 6.8, 4000 x 4001 x 2048 160 / 110, 1021 x 50257 x 768 174 / 157; aligned neighbours with copies into LDS take 43, 61, 18, 5, 48 and
+// 102. What alignment itself costs is a tenth to a fifth: rows on the boundaries / off them, [N,K] 128 x 7224 x 6651 37 / 43,
+// [K,N] 44 / 47, 1021 x 50264 x 763 138 / 145. Two slabs on their way
+// in 128 x 128 tiles leave one to a CU: 1021 x 50257 x 768 211, 640 x 7031 x 3584 140.)
+template <typename T, typename OutT, typename S, int NS, bool TRANS_B, bool ANY>
+__global__ __launch_bounds__(S::kThreads, S::STEPS == 2 ? 4 : 2)
 void gemm_few_kernel(const T* __restrict__ A, const T* __restrict__ B, OutT* C, int M, int N, int K, int64_t lda, int64_t ldb,
                      int64_t ldc, const OutT* __restrict__ bias, const OutT* resid, int64_t ldr, int tiles_m, int tiles_n,
                      int runs) {
   constexpr int TM = S::TM, TN = S::TN, BM = S::BM, BN = S::BN, BK = S::BK, KH = S::KH, kWaves = S::kWaves, kThreads = S::kThreads;
   constexpr int kA = BM * BK / 512 / kWaves, kB = BN * BK / 512 / kWaves, kCopies = kA + kB;   // a wave's copies (1 KiB) of a slab
+  static_assert(ANY || S::STEPS == 1, "a slab is one step of a wave");
   static_assert(kA * kWaves * 512 == BM * BK && kB * kWaves * 512 == BN * BK, "whole copies");
   constexpr int kStageBytes = S::kStage * 2, kPitch = BN + 4;    // pitch of the sums on their way out
-  constexpr int kLds = std::max(NS * kStageBytes, KH * BM * kPitch * 4);
+  constexpr int kLds = std::max((ANY ? 2 : NS) * kStageBytes, KH * BM * kPitch * 4);
   __shared__ __attribute__((aligned(16))) char lds[kLds];
 
   const int lane = threadIdx.x % kWave, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
@@ -72,8 +85,29 @@ void gemm_few_kernel(const T* __restrict__ A, const T* __restrict__ B, OutT* C, 
 
   // copy i of a slab moves chunks [i * 512 + wave * 64, + 64) of the tile: A's kA, then B's kB
   int voff[kCopies], kc[kCopies];
+  const T* ptr[ANY ? kCopies : 1];
+  int by[ANY ? kCopies : 1];                                     // ANY, [K,N]: columns the chunk was moved back to end at N
+  if constexpr (ANY) {
 #pragma unroll
-  for (int i = 0; i < kCopies; ++i) {
+    for (int i = 0; i < kCopies; ++i) {
+      const int chunk = (i < kA ? i : i - kA) * kThreads + threadIdx.x;
+      if (i < kA || TRANS_B) {
+        const int row = chunk / (BK / 8), c = (chunk % (BK / 8)) ^ swz_row<BK>(row);
+        const int left = (i < kA ? M - m0 : N - n0) - 1;
+        ptr[i] = (i < kA ? A + (int64_t)m0 * lda : B + (int64_t)n0 * ldb) + (int64_t)(row < left ? row : left) * (i < kA ? lda : ldb) + c * 8;
+        kc[i] = c * 8;
+        by[i] = 0;
+      } else {
+        const int k = chunk / (BN / 8), c = (chunk % (BN / 8)) ^ swz_col<BN>(k);
+        const int col = n0 + c * 8, at = col + 8 <= N ? col : N - 8;
+        ptr[i] = B + (int64_t)k * ldb + at;
+        kc[i] = k;
+        by[i] = (col - at) & 7;                                  // (chunks wholly past N: anything, those columns are not stored)
+      }
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < (ANY ? 0 : kCopies); ++i) {
     const int chunk = (i < kA ? i : i - kA) * kThreads + threadIdx.x;
     if (i < kA || TRANS_B) {
       const int row = chunk / (BK / 8), c = (chunk % (BK / 8)) ^ swz_row<BK>(row);
@@ -130,15 +164,17 @@ void gemm_few_kernel(const T* __restrict__ A, const T* __restrict__ B, OutT* C, 
   // bias and residual of this thread's runs of eight columns of the result, under the K walk
   constexpr int kRuns = BM * BN / 8 < kThreads ? 1 : BM * BN / 8 / kThreads;
   struct alignas(16) Run { OutT v[8]; };
+  constexpr bool kEarly = kRuns <= 2;                            // (128 x 128: no registers for them)
   Run add_b[kRuns], add_r[kRuns];
-  if (runs) {
+  auto ask = [&](int p) __attribute__((always_inline)) {
+    const int idx = threadIdx.x + p * kThreads, row = idx / (BN / 8) % BM, col = idx % (BN / 8) * 8;
+    const int gm = m0 + row < M ? m0 + row : M - 1, gn = n0 + col < N ? n0 + col : N - 8;
+    if (bias) add_b[p] = *reinterpret_cast<const Run*>(bias + gn);
+    if (resid) add_r[p] = *reinterpret_cast<const Run*>(resid + (int64_t)gm * ldr + gn);
+  };
+  if (kEarly && runs) {
 #pragma unroll
-    for (int p = 0; p < kRuns; ++p) {
-      const int idx = threadIdx.x + p * kThreads, row = idx / (BN / 8) % BM, col = idx % (BN / 8) * 8;
-      const int gm = m0 + row < M ? m0 + row : M - 1, gn = n0 + col < N ? n0 + col : N - 8;
-      if (bias) add_b[p] = *reinterpret_cast<const Run*>(bias + gn);
-      if (resid) add_r[p] = *reinterpret_cast<const Run*>(resid + (int64_t)gm * ldr + gn);
-    }
+    for (int p = 0; p < kRuns; ++p) ask(p);
   }
 
   f32x4 acc[TM][TN];
@@ -148,22 +184,23 @@ void gemm_few_kernel(const T* __restrict__ A, const T* __restrict__ B, OutT* C, 
     for (int j = 0; j < TN; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
   typedef typename Frag8<T>::V Frag;
   struct Step { Frag a[TM], b[TN]; };
-  auto read = [&](int stage, Step& f) __attribute__((always_inline)) {
+  auto read = [&](int stage, int st, Step& f) __attribute__((always_inline)) {   // st: step of the wave, KH * 32 of K apart
     const char* from = lds + stage * kStageBytes;
+    const int far = st * (KH * 64), far_b = TRANS_B ? 0 : st * (KH * 32 * BN * 2);
 #pragma unroll
     for (int j = 0; j < TN; ++j) {
       if constexpr (TRANS_B) {
-        f.b[j] = *reinterpret_cast<const Frag*>(from + b_at[j]);
+        f.b[j] = *reinterpret_cast<const Frag*>(from + (b_at[j] ^ far));
       } else {                                                   // four k on: the same place in its row
         union { i16x4 h[2]; Frag v; } u;
 #pragma unroll
         for (int p = 0; p < 2; ++p)
-          u.h[p] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) i16x4*)(from + b_at[j] + p * (4 * BN * 2)));
+          u.h[p] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) i16x4*)(from + b_at[j] + far_b + p * (4 * BN * 2)));
         f.b[j] = u.v;
       }
     }
 #pragma unroll
-    for (int i = 0; i < TM; ++i) f.a[i] = *reinterpret_cast<const Frag*>(from + a_at + i * (16 * BK * 2));   // the swizzle repeats
+    for (int i = 0; i < TM; ++i) f.a[i] = *reinterpret_cast<const Frag*>(from + (a_at ^ far) + i * (16 * BK * 2));   // the swizzle repeats
   };
   auto multiply = [&](const Step& f) __attribute__((always_inline)) {
 #pragma unroll
@@ -181,36 +218,137 @@ void gemm_few_kernel(const T* __restrict__ A, const T* __restrict__ B, OutT* C, 
     asm volatile("" ::: "memory");
     HEXMI_FENCE;
   };
-  HEXMI_FENCE;
+  if constexpr (ANY) {
+    constexpr int kSets = S::STEPS == 2 ? 1 : 2;                 // slabs on their way
+    u32x4 set[kSets][kCopies];
+    // PLAIN: every chunk lies inside its row and K. The other form takes any slab, one past the last too (zeros).
+    auto fetch = [&](int slab, u32x4 (&to)[kCopies], auto plain) __attribute__((always_inline)) {
 #pragma unroll
-  for (int j = 0; j < NS - 1; ++j)
-    if (j < slabs) copy_any(j, j);
-  int stage = 0, j = 0;
-  auto step = [&](auto newer, auto next) __attribute__((always_inline)) {   // next: the copies that follow into the free stage
-    landed(newer);
-    next();
+      for (int i = 0; i < kCopies; ++i) {
+        if constexpr (decltype(plain)::value) {
+          __builtin_memcpy(&to[i], ptr[i] + (i < kA || TRANS_B ? (int64_t)slab * BK : (int64_t)slab * BK * ldb), 16);
+        } else {
+          const int k = slab * BK + kc[i];
+          if (i < kA || TRANS_B) __builtin_memcpy(&to[i], ptr[i] + (slab * BK + (k < K - 8 ? 0 : K - 8 - k)), 16);
+          else __builtin_memcpy(&to[i], ptr[i] + (int64_t)((k < K - 1 ? k : K - 1) - kc[i]) * ldb, 16);
+        }
+      }
+    };
+    auto put = [&](const u32x4 (&from)[kCopies], int slab, int stage, auto plain) __attribute__((always_inline)) {
+      char* to = lds + stage * kStageBytes + threadIdx.x * 16;
+#pragma unroll
+      for (int i = 0; i < kCopies; ++i) {
+        u32x4 v = from[i];
+        if constexpr (!decltype(plain)::value) {
+          const int left = K - slab * BK - kc[i];                // elements or rows before the end of K
+          const u32x4 zero = {0u, 0u, 0u, 0u};
+          v = shift_columns(v, zero, i < kA || TRANS_B ? (left < 8 ? 8 - left : 0) & 7 : by[i]);
+          v = left > 0 ? v : zero;
+        }
+        *reinterpret_cast<u32x4*>(to + (i < kA ? i * kThreads * 16 : BM * BK * 2 + (i - kA) * kThreads * 16)) = v;
+      }
+    };
+    auto meet = [&]() __attribute__((always_inline)) {           // every wave's writes and reads of LDS are done; loads stay in flight
+      HEXMI_FENCE;
+      __builtin_amdgcn_s_waitcnt(waitcnt_imm(63));
+      __builtin_amdgcn_s_barrier();
+      asm volatile("" ::: "memory");
+      HEXMI_FENCE;
+    };
+    if (K < 8 || (!TRANS_B && N < 8)) {                          // less than a chunk: by elements
+#pragma unroll 1
+      for (int slab = 0; slab < slabs; ++slab) {
+        __syncthreads();
+#pragma unroll 1
+        for (int e = threadIdx.x; e < (BM + BN) * BK; e += kThreads) {
+          const bool a = e < BM * BK;
+          const int q = a ? e : e - BM * BK;
+          unsigned short v = 0;
+          if (a || TRANS_B) {
+            const int row = q / BK, k = slab * BK + ((q % BK / 8) ^ swz_row<BK>(row)) * 8 + q % 8;
+            const T* base = a ? A + (int64_t)m0 * lda : B + (int64_t)n0 * ldb;
+            if (k < K && row < (a ? M - m0 : N - n0)) v = reinterpret_cast<const unsigned short*>(base)[row * (a ? lda : ldb) + k];
+          } else {
+            const int row = q / BN, col = n0 + ((q % BN / 8) ^ swz_col<BN>(row)) * 8 + q % 8;
+            if (slab * BK + row < K && col < N) v = reinterpret_cast<const unsigned short*>(B)[(int64_t)(slab * BK + row) * ldb + col];
+          }
+          reinterpret_cast<unsigned short*>(lds)[e] = v;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int st = 0; st < S::STEPS; ++st) {
+          Step f;
+          read(0, st, f);
+          multiply(f);
+        }
+      }
+    } else {
+      constexpr std::true_type kPlain{};
+      constexpr std::false_type kAny{};
+      // slab j from its stage; slab j + 1 from its set into the other stage, which slab j - 1 has left; the next slab into that set
+      auto turn = [&](int j, int stage, u32x4 (&next)[kCopies], auto plain) __attribute__((always_inline)) {
+        meet();
+#pragma unroll
+        for (int st = 0; st < S::STEPS; ++st) {
+          Step f;
+          read(stage, st, f);
+          if (st == 0) {
+            put(next, j + 1, stage ^ 1, plain);
+            fetch(j + 1 + kSets, next, plain);
+            HEXMI_FENCE;
+          }
+          multiply(f);
+        }
+      };
+      fetch(0, set[0], kAny);
+      if constexpr (kSets > 1) fetch(1, set[1], kAny);
+      put(set[0], 0, 0, kAny);
+      fetch(kSets, set[0], kAny);
+      int j = 0;
+      if (TRANS_B || n0 + BN <= N) {
+        const int whole = K / BK;
+        for (; j + 2 + kSets < whole; j += 2) {
+          turn(j, 0, set[kSets - 1], kPlain);
+          turn(j + 1, 1, set[0], kPlain);
+        }
+      }
+      for (; j < slabs; j += 2) {                                // (one slab of zeros where their number is odd)
+        turn(j, 0, set[kSets - 1], kAny);
+        turn(j + 1, 1, set[0], kAny);
+      }
+    }
+  } else {
     HEXMI_FENCE;
-    Step f;
-    read(stage, f);
-    multiply(f);
-    stage = stage == NS - 1 ? 0 : stage + 1;
-    ++j;
-  };
-  auto free_stage = [&]() { return stage == 0 ? NS - 1 : stage - 1; };
-  constexpr std::integral_constant<int, NS - 2> kBehind{};
-  while (j + NS - 1 < full) step(kBehind, [&]() __attribute__((always_inline)) { copy(j + NS - 1, free_stage(), std::false_type{}); });
-  if (j + NS - 1 < slabs) step(kBehind, [&]() __attribute__((always_inline)) { copy(j + NS - 1, free_stage(), std::true_type{}); });
-  auto last = [&](auto left) __attribute__((always_inline)) {    // left: slabs behind this one
-    if (j + decltype(left)::value < slabs) step(left, []() __attribute__((always_inline)) {});
-  };
-  if constexpr (NS > 7) last(std::integral_constant<int, 6>{});
-  if constexpr (NS > 6) last(std::integral_constant<int, 5>{});
-  if constexpr (NS > 5) last(std::integral_constant<int, 4>{});
-  if constexpr (NS > 4) last(std::integral_constant<int, 3>{});
-  if constexpr (NS > 3) last(std::integral_constant<int, 2>{});
-  if constexpr (NS > 2) last(std::integral_constant<int, 1>{});
-  last(std::integral_constant<int, 0>{});
-  static_assert(NS >= 2 && NS <= 8, "the ladder above");
+#pragma unroll
+    for (int j = 0; j < NS - 1; ++j)
+      if (j < slabs) copy_any(j, j);
+    int stage = 0, j = 0;
+    auto step = [&](auto newer, auto next) __attribute__((always_inline)) {   // next: the copies that follow into the free stage
+      landed(newer);
+      next();
+      HEXMI_FENCE;
+      Step f;
+      read(stage, 0, f);
+      multiply(f);
+      stage = stage == NS - 1 ? 0 : stage + 1;
+      ++j;
+    };
+    auto free_stage = [&]() { return stage == 0 ? NS - 1 : stage - 1; };
+    constexpr std::integral_constant<int, NS - 2> kBehind{};
+    while (j + NS - 1 < full) step(kBehind, [&]() __attribute__((always_inline)) { copy(j + NS - 1, free_stage(), std::false_type{}); });
+    if (j + NS - 1 < slabs) step(kBehind, [&]() __attribute__((always_inline)) { copy(j + NS - 1, free_stage(), std::true_type{}); });
+    auto last = [&](auto left) __attribute__((always_inline)) {    // left: slabs behind this one
+      if (j + decltype(left)::value < slabs) step(left, []() __attribute__((always_inline)) {});
+    };
+    if constexpr (NS > 7) last(std::integral_constant<int, 6>{});
+    if constexpr (NS > 6) last(std::integral_constant<int, 5>{});
+    if constexpr (NS > 5) last(std::integral_constant<int, 4>{});
+    if constexpr (NS > 4) last(std::integral_constant<int, 3>{});
+    if constexpr (NS > 3) last(std::integral_constant<int, 2>{});
+    if constexpr (NS > 2) last(std::integral_constant<int, 1>{});
+    last(std::integral_constant<int, 0>{});
+    static_assert(NS >= 2 && NS <= 8, "the ladder above");
+  }
 #undef HEXMI_FENCE
 
   // the wave groups' sums meet in LDS and leave in rows
@@ -227,6 +365,7 @@ void gemm_few_kernel(const T* __restrict__ A, const T* __restrict__ B, OutT* C, 
     for (int p = 0; p < kRuns; ++p) {
       const int idx = threadIdx.x + p * kThreads, row = idx / (BN / 8), col = idx % (BN / 8) * 8;
       if (BM * BN / 8 < kThreads && row >= BM) break;
+      if (!kEarly) ask(p);
       f32x4 s0 = {0.f, 0.f, 0.f, 0.f}, s1 = s0;
 #pragma unroll
       for (int h = 0; h < KH; ++h) {
@@ -266,6 +405,7 @@ template <> struct FewShape<32, 32> { typedef Shape<2, 2, 1, 1, 8> S; static con
 template <> struct FewShape<32, 64> { typedef Shape<2, 2, 1, 2, 4> S; static constexpr int NS = 6; };
 template <> struct FewShape<64, 64> { typedef Shape<2, 4, 2, 1, 4> S; static constexpr int NS = 4; };
 template <> struct FewShape<128, 64> { typedef Shape<4, 4, 2, 1, 4> S; static constexpr int NS = 3; };
+template <> struct FewShape<128, 128> { typedef Shape<4, 2, 2, 4, 1, 2> S; static constexpr int NS = 2; };   // (ANY only)
 
 }  // namespace
 
@@ -319,6 +459,36 @@ GemmFewTile plan_gemm_few(bool trans_b, int64_t M, int64_t N, int64_t K) {
   return {0, 0};
 }
 
+// The tile of a product on operand rows at any alignment: the smallest of which there is at most one per CU, 128 x 128 beyond.
+static GemmFewTile plan_gemm_any(int64_t M, int64_t N) {
+  static constexpr GemmFewTile kTiles[] = {{16, 32}, {32, 32}, {32, 64}, {64, 64}, {128, 64}};
+  for (const GemmFewTile& t : kTiles)
+    if ((t.m > 16 || M <= 64) && ((M + t.m - 1) / t.m) * ((N + t.n - 1) / t.n) <= hexmi_num_cus()) return t;
+  return {128, 128};
+}
+
+template <typename T, typename OutT, bool TRANS_B>
+int launch_gemm_any(const T* A, const T* B, OutT* C, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, int64_t ldc, hipStream_t s,
+                    const OutT* bias, const OutT* resid, int64_t ldr) {
+  const GemmFewTile tile = plan_gemm_any(M, N);
+  const int64_t tiles_m = (M + tile.m - 1) / tile.m, tiles_n = (N + tile.n - 1) / tile.n;
+  if (!grid_fits(tiles_m * tiles_n, 512) || tiles_m * tiles_n > 0x7fffffff || K > 0x7fffffff - 256) return HEXMI_ENOTSUP;
+  const int runs = N % 8 == 0 && ldc % 8 == 0 && aligned_to(C, 16) && aligned_to(bias, 16) && aligned_to(resid, 16) &&
+                   (!resid || ldr % 8 == 0);
+#define HEXMI_ANY(BM, BN)                                                                                                     \
+  hipLaunchKernelGGL((gemm_few_kernel<T, OutT, FewShape<BM, BN>::S, 2, TRANS_B, true>), dim3((unsigned)(tiles_m * tiles_n)),   \
+                     dim3(FewShape<BM, BN>::S::kThreads), 0, s, A, B, C, (int)M, (int)N, (int)K, lda, ldb, ldc, bias, resid, ldr, \
+                     (int)tiles_m, (int)tiles_n, runs)
+  if (tile.n == 128) HEXMI_ANY(128, 128);
+  else if (tile.m == 128) HEXMI_ANY(128, 64);
+  else if (tile.m == 64) HEXMI_ANY(64, 64);
+  else if (tile.n == 64) HEXMI_ANY(32, 64);
+  else if (tile.m == 32) HEXMI_ANY(32, 32);
+  else HEXMI_ANY(16, 32);
+#undef HEXMI_ANY
+  return launch_status();
+}
+
 template <typename T, typename OutT, bool TRANS_B>
 int launch_gemm_few(const GemmFewTile& tile, const T* A, const T* B, OutT* C, int64_t M, int64_t N, int64_t K, int64_t lda,
                     int64_t ldb, int64_t ldc, hipStream_t s, const OutT* bias, const OutT* resid, int64_t ldr) {
@@ -326,7 +496,7 @@ int launch_gemm_few(const GemmFewTile& tile, const T* A, const T* B, OutT* C, in
   const int runs = N % 8 == 0 && ldc % 8 == 0 && aligned_to(C, 16) && aligned_to(bias, 16) && aligned_to(resid, 16) &&
                    (!resid || ldr % 8 == 0);
 #define HEXMI_FEW(BM, BN)                                                                                                    \
-  hipLaunchKernelGGL((gemm_few_kernel<T, OutT, FewShape<BM, BN>::S, FewShape<BM, BN>::NS, TRANS_B>),                         \
+  hipLaunchKernelGGL((gemm_few_kernel<T, OutT, FewShape<BM, BN>::S, FewShape<BM, BN>::NS, TRANS_B, false>),                         \
                      dim3((unsigned)(tiles_m * tiles_n)), dim3(FewShape<BM, BN>::S::kThreads), 0, s, A, B, C, (int)M, (int)N, \
                      (int)K, lda, ldb, ldc, bias, resid, ldr, tiles_m, tiles_n, runs)
   if (tile.m == 128) HEXMI_FEW(128, 64);
@@ -342,7 +512,9 @@ int launch_gemm_few(const GemmFewTile& tile, const T* A, const T* B, OutT* C, in
 
 #define HEXMI_INSTANCE(T, OutT, TB)                                                                                          \
   template int launch_gemm_few<T, OutT, TB>(const GemmFewTile&, const T*, const T*, OutT*, int64_t, int64_t, int64_t, int64_t, \
-                                            int64_t, int64_t, hipStream_t, const OutT*, const OutT*, int64_t);
+                                            int64_t, int64_t, hipStream_t, const OutT*, const OutT*, int64_t);                 \
+  template int launch_gemm_any<T, OutT, TB>(const T*, const T*, OutT*, int64_t, int64_t, int64_t, int64_t, int64_t, int64_t,   \
+                                            hipStream_t, const OutT*, const OutT*, int64_t);
 HEXMI_INSTANCE(f16, f16, false)
 HEXMI_INSTANCE(f16, f16, true)
 HEXMI_INSTANCE(f16, float, false)

@@ -211,6 +211,19 @@ __device__ __forceinline__ void copy_ptr_to_lds_asm(const char* src, char* lds) 
 #endif
 }
 
+// sixteen 16-bit columns in two chunks, from column `by` (0 .. 7) on: eight of them
+__device__ __forceinline__ u32x4 shift_columns(const u32x4& lo, const u32x4& hi, int by) {
+  auto pick = [](bool second, uint32_t v0, uint32_t v1) { return second ? v1 : v0; };    // (values, not places: no scratch)
+  const bool by4 = by & 4, by2 = by & 2;
+  const uint32_t x0 = pick(by4, lo[0], lo[2]), x1 = pick(by4, lo[1], lo[3]), x2 = pick(by4, lo[2], hi[0]),
+                 x3 = pick(by4, lo[3], hi[1]), x4 = pick(by4, hi[0], hi[2]), x5 = pick(by4, hi[1], hi[3]);
+  const uint32_t y0 = pick(by2, x0, x1), y1 = pick(by2, x1, x2), y2 = pick(by2, x2, x3), y3 = pick(by2, x3, x4),
+                 y4 = pick(by2, x4, x5);
+  const int bits = (by & 1) * 16;
+  const u32x4 o = {__builtin_amdgcn_alignbit(y1, y0, bits), __builtin_amdgcn_alignbit(y2, y1, bits),
+                   __builtin_amdgcn_alignbit(y3, y2, bits), __builtin_amdgcn_alignbit(y4, y3, bits)};
+  return o;
+}
 // s_waitcnt immediate (gfx9 encoding): at most `vm` vector-memory operations outstanding, all LDS reads returned.
 constexpr int waitcnt_imm(int vm) { return (vm & 0xF) | ((vm >> 4) << 14) | (7 << 4) | (0 << 8); }
 
@@ -271,6 +284,10 @@ GemmFewTile plan_gemm_few(bool trans_b, int64_t M, int64_t N, int64_t K);
 template <typename T, typename OutT, bool TRANS_B>
 int launch_gemm_few(const GemmFewTile& tile, const T* A, const T* B, OutT* C, int64_t M, int64_t N, int64_t K, int64_t lda,
                     int64_t ldb, int64_t ldc, hipStream_t s, const OutT* bias, const OutT* resid, int64_t ldr);
+// ... and products on operand rows at any alignment, any K, any strides.
+template <typename T, typename OutT, bool TRANS_B>
+int launch_gemm_any(const T* A, const T* B, OutT* C, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, int64_t ldc, hipStream_t s,
+                    const OutT* bias, const OutT* resid, int64_t ldr);
 
 // Tiled W8A16 GEMM for many activation rows (gemm.hip): C[M,N] = (A[M,K] * W[N,K]^T) * scales[N].
 int gemm_w8a16_tiled(int64_t M, int64_t N, int64_t K, const f16* A, const int8_t* W, const f16* scales, f16* C,

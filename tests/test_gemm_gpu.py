@@ -264,6 +264,38 @@ def test_gemm_few_rows_the_weight_stream_leaves(hexmi, dtype, M, N, K):
         _against_double(hexmi, dtype, out_dtype, True, M, N, K, True, True, M + K)
 
 
+# operand rows off the boundaries: every tile of plan_gemm_any on 256 CUs and its edges, K of fewer slabs than are on their way, of whole
+# slabs and one element over and short, rows of fewer columns than a chunk
+@pytest.mark.parametrize("trans_b", [False, True])
+@pytest.mark.parametrize("dtype,out_dtype", [(torch.float16, torch.float16), (torch.bfloat16, torch.float32)])
+@pytest.mark.parametrize("M,N,K", [
+    (1, 1, 1), (3, 5, 7), (5, 9, 300), (2, 7, 1000), (16, 4097, 257), (17, 33, 2049), (64, 2047, 255), (33, 1025, 1281),    # 16 x 32
+    (65, 2049, 513), (200, 501, 767), (97, 1999, 264), (500, 993, 1024),                                        # 32 x 32, 32 x 64
+    (300, 3001, 129), (1000, 1001, 1000), (1900, 1023, 333),                                                    # 64 x 64, 128 x 64
+    (2100, 2049, 63), (2049, 2050, 193), (2177, 2191, 256), (70, 33001, 65), (33025, 129, 127)])                # 128 x 128
+def test_gemm_operand_rows_off_the_boundaries(hexmi, dtype, out_dtype, trans_b, M, N, K):
+    _against_double(hexmi, dtype, out_dtype, trans_b, M, N, K, False, False, M + N + K)
+    _against_double(hexmi, dtype, out_dtype, trans_b, M, N, K, True, True, M + N + K + 1)
+    # views one and three elements into larger buffers of infinities: nothing outside the operands reaches a sum
+    from hexmi import _lib
+    code = {torch.float16: _lib.F16, torch.bfloat16: _lib.BF16, torch.float32: _lib.F32}
+    a, b = _inputs(M, N, K, dtype, trans_b, seed=7)
+    br, bc = b.shape
+    lda, ldb = K + 3, bc + 5
+    ab, bb = torch.full((M * lda + 8,), math.inf, dtype=dtype), torch.full((br * ldb + 8,), math.inf, dtype=dtype)
+    ab[1:1 + M * lda].view(M, lda)[:, :K] = a
+    bb[3:3 + br * ldb].view(br, ldb)[:, :bc] = b
+    ab, bb = ab.cuda(), bb.cuda()
+    c = torch.full((M, N), math.nan, dtype=out_dtype, device="cuda")
+    assert _lib.lib().hexmi_gemm_ex(M, N, K, ab.data_ptr() + 2, lda, bb.data_ptr() + 6, ldb, c.data_ptr(), N, None, None, 0, code[dtype],
+                                    code[out_dtype], int(trans_b), torch.cuda.current_stream().cuda_stream) == _lib.OK
+    a, b = a.cuda().double(), b.cuda().double()
+    b = b.t() if trans_b else b
+    # sums in fp32 in another order: 1e-5 of the summed magnitudes; one rounding to the output type: half an ulp
+    eps = {torch.float16: 2.0 ** -11, torch.bfloat16: 2.0 ** -8, torch.float32: 2.0 ** -24}[out_dtype]
+    assert ((c.double() - a @ b).abs() <= 1e-5 * (a.abs() @ b.abs()) + eps * (a @ b).abs() + 1e-7).all()
+
+
 # more tiles than one round of them: the 128 x 128 and 256 x 256 kernels and the slabs, widths and outputs each is for
 @pytest.mark.parametrize("trans_b", [False, True])
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
