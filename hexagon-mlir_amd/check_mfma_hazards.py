@@ -160,8 +160,8 @@ def scan_scratch(asm_path):
     return bad
 
 
-SOURCES = ("gemm.hip", "calibrate.hip")      # the files with MFMAs written as inline assembly
-CVT_SOURCES = ("gemm.hip", "calibrate.hip", "w8a16.hip", "w8a16_few.hip", "w8a16_split.hip")   # asm conversions or asm MFMAs
+SOURCES = ("gemm.hip", "gemm_mid.hip", "calibrate.hip")      # the files with MFMAs written as inline assembly
+CVT_SOURCES = ("gemm.hip", "gemm_mid.hip", "calibrate.hip", "w8a16.hip", "w8a16_few.hip", "w8a16_split.hip")   # asm conversions or asm MFMAs
 
 
 def _assembly(name, tmp):

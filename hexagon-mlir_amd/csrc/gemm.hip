@@ -25,6 +25,7 @@
 // the last slab's chunks past K fetched from a zero chunk; an output side without runs of four columns (odd N with B
 // as [N,K], odd ldc, unaligned C) -> the same kernels with the tile leaving through LDS in the pieces of 16 bytes that each row holds;
 // anything else (unaligned operand rows, K % 8 != 0) -> the tiles of gemm_few.hip with slabs that come through registers.
+// Between them, and for K off whole 64s, gemm_mid.hip where results are 16-bit in whole runs of eight columns.
 // Whole chunks of K and no more tiles than CUs -> gemm_few.hip, tiles of 16 x 16 to 128 x 64 that give every CU a share, beyond the
 // lines of plan_gemm_few where B is [N,K] and rows are few. Of what it leaves: up to eight rows against B as [N,K] -> gemv_nt_kernel, a
 // stream of the weights with one wave per output channel; up to 64, by measured lines -> gemm_skinny.hip, a workgroup per 16 to
@@ -1589,6 +1590,15 @@ int dispatch_gemm(const void* Av, const void* Bv, void* Cv, int64_t M, int64_t N
     const GemmSkinnyPlan plan = plan_gemm_skinny(M, N, K, fast || (!bias && !resid));
     if (plan.channels > 0)
       return launch_gemm_skinny<T, OutT>(plan, A, B, C, M, N, K, lda, ldb, ldc, s, bias, resid, ldr);
+  }
+  // 16-bit results in whole runs of eight columns: the tiles between 128 x 128 and 256 x 256
+  if constexpr (std::is_same<T, OutT>::value) {
+    if (chunks && N % 8 == 0 && ldc % 8 == 0 && aligned_to(C, 16) && lda < (1 << 21) && ldb < (1 << 21) && K <= (1 << 30) &&
+        (!bias || aligned_to(bias, run)) && (!resid || (aligned_to(resid, run) && ldr % 4 == 0))) {
+      const int now = K % BK2 != 0 ? 0 : large ? 256 : two_per_cu(((M + 127) / 128) * ((N + 127) / 128), K) ? 2 : 1;
+      const GemmMidTile mid = plan_gemm_mid(M, N, K, now, resid != nullptr);
+      if (mid.m) return launch_gemm_mid<T, TRANS_B>(mid, A, B, C, M, N, K, lda, ldb, ldc, s, bias, resid, ldr);
+    }
   }
   if (fast) {
     // the large-tile kernels sit at the register limit and carry no epilogue operands: a product with bias or

@@ -254,6 +254,37 @@ def test_gemm_one_round_of_tiles(hexmi, dtype, out_dtype, trans_b, M, N, K):
         assert torch.equal(view[:, N:], keep)
 
 
+# the tiles of plan_gemm_mid on 256 CUs: one row and one run of columns over and short of them, K of fewer slabs than stages, of whole slabs
+# and chunks over, slabs that the stages do not divide
+@pytest.mark.parametrize("trans_b", [False, True])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("M,N,K,bias,residual", [
+    (1025, 4096, 8, False, False), (2049, 1096, 72, False, False), (1153, 4104, 200, True, True), (2047, 4088, 120, False, True),
+    (2049, 1096, 1000, True, False),                                              # 128 x 128, two and one to a CU
+    (1345, 6216, 1608, False, True), (1291, 3096, 2552, True, False), (2177, 2056, 640, False, False),           # 192 x 128
+    (4097, 4104, 1016, False, False), (1300, 6400, 1600, True, False), (1345, 6344, 1600, True, True),           # 192 x 192
+    (700, 9000, 1000, False, True), (511, 16376, 1160, True, False),                                          # 256 x 128
+    (645, 12456, 704, True, False), (1009, 24000, 328, True, False), (3073, 3080, 128, True, False)])           # 256 x 192
+def test_gemm_tiles_between_128_and_256(hexmi, dtype, trans_b, M, N, K, bias, residual):
+    _against_double(hexmi, dtype, dtype, trans_b, M, N, K, bias, residual, M + N + K)
+    # a strided output, the residual the output itself, nothing written around it
+    from hexmi import _lib
+    a, b = _inputs(M, N, K, dtype, trans_b, seed=5)
+    a, b = a.cuda(), b.cuda()
+    view = torch.randn(M, N + 8, generator=_gen(3)).to(dtype).cuda()
+    want, mag = a.double() @ (b.double().t() if trans_b else b.double()), a.double().abs() @ (b.double().abs().t() if trans_b else b.double().abs())
+    if residual:
+        want, mag = want + view[:, :N].double(), mag + view[:, :N].double().abs()
+    keep = view[:, N:].clone()
+    code = {torch.float16: _lib.F16, torch.bfloat16: _lib.BF16}[dtype]
+    assert _lib.lib().hexmi_gemm_ex(M, N, K, a.data_ptr(), K, b.data_ptr(), b.stride(0), view.data_ptr(), N + 8, None,
+                                    view.data_ptr() if residual else None, N + 8 if residual else 0, code, code, int(trans_b),
+                                    torch.cuda.current_stream().cuda_stream) == _lib.OK
+    # fp32 sums in another order, then one rounding to the output type
+    assert ((view[:, :N].double() - want).abs() <= 1e-5 * mag + torch.finfo(dtype).eps / 2 * want.abs() + 1e-7).all()
+    assert torch.equal(view[:, N:], keep)
+
+
 # up to 64 rows against [N,K] weights that the weight stream does not take: K off whole 32s, fewer than 64 channels
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("M,N,K", [(3, 64, 8), (8, 700, 1000), (9, 65, 40), (16, 272, 4264), (17, 257, 1128), (32, 384, 856), (33, 2000, 72),
