@@ -1,5 +1,5 @@
 // C[M,N] = A[M,K] * op(B) where tiles of 128 x 128 would leave compute units without work (fp16 / bf16 in, fp32 sums): tiles of
-// 16 x 16 to 128 x 64 in one round, a workgroup of eight waves to a tile.
+// 16 x 16 to 128 x 64 and 96 x 96 in one round, a workgroup of eight waves to a tile.
 //
 // What bounds it: a CU takes in about 90 GB/s through L2 whatever it does with it, and a tile of BM x BN asks for (BM + BN) x K
 // operands. 128 x 128 tiles run at that rate (0.31 us per 64 of K, K = 3072), so what is left is to have every CU take in a share:
@@ -46,6 +46,7 @@ template <int BK> __device__ __forceinline__ int swz_row(int r) { return BK == 6
 // N-contiguous tile of BN columns a row of k: the 32 lanes of a transposing read touch k % 4, k / 8 % 2 x 32 bytes, which the
 // XOR spreads over the eight 32-byte slots of all banks
 template <int BN> __device__ __forceinline__ int swz_col(int k) {
+  if (BN == 96) return ((k >> 3) & 1) << 1;                     // (rows of three quarters of the banks: four start on different ones)
   if (BN == 128) return ((k & 3) | (((k >> 3) & 1) << 2)) << 1;
   return BN == 64 ? (((k >> 1) & 1) | (((k >> 3) & 1) << 1)) << 1 : ((k >> 3) & 1) << 1;
 }
@@ -162,9 +163,9 @@ void gemm_few_kernel(const T* __restrict__ A, const T* __restrict__ B, OutT* C, 
   }
 
   // bias and residual of this thread's runs of eight columns of the result, under the K walk
-  constexpr int kRuns = BM * BN / 8 < kThreads ? 1 : BM * BN / 8 / kThreads;
+  constexpr int kRuns = (BM * BN / 8 + kThreads - 1) / kThreads;
   struct alignas(16) Run { OutT v[8]; };
-  constexpr bool kEarly = kRuns <= 2;                            // (128 x 128: no registers for them)
+  constexpr bool kEarly = !ANY || kRuns <= 2;                    // (128 x 128, two to a CU: no registers for them)
   Run add_b[kRuns], add_r[kRuns];
   auto ask = [&](int p) __attribute__((always_inline)) {
     const int idx = threadIdx.x + p * kThreads, row = idx / (BN / 8) % BM, col = idx % (BN / 8) * 8;
@@ -364,7 +365,7 @@ void gemm_few_kernel(const T* __restrict__ A, const T* __restrict__ B, OutT* C, 
 #pragma unroll
     for (int p = 0; p < kRuns; ++p) {
       const int idx = threadIdx.x + p * kThreads, row = idx / (BN / 8), col = idx % (BN / 8) * 8;
-      if (BM * BN / 8 < kThreads && row >= BM) break;
+      if (BM * BN / 8 % kThreads && row >= BM) break;
       if (!kEarly) ask(p);
       f32x4 s0 = {0.f, 0.f, 0.f, 0.f}, s1 = s0;
 #pragma unroll
@@ -405,13 +406,18 @@ template <> struct FewShape<32, 32> { typedef Shape<2, 2, 1, 1, 8> S; static con
 template <> struct FewShape<32, 64> { typedef Shape<2, 2, 1, 2, 4> S; static constexpr int NS = 6; };
 template <> struct FewShape<64, 64> { typedef Shape<2, 4, 2, 1, 4> S; static constexpr int NS = 4; };
 template <> struct FewShape<128, 64> { typedef Shape<4, 4, 2, 1, 4> S; static constexpr int NS = 3; };
-template <> struct FewShape<128, 128> { typedef Shape<4, 2, 2, 4, 1, 2> S; static constexpr int NS = 2; };   // (ANY only)
+template <> struct FewShape<96, 96> { typedef Shape<3, 6, 2, 1, 4> S; static constexpr int NS = 3; };
+typedef Shape<4, 2, 2, 4, 1, 2> AnyShape128;                     // 128 x 128, ANY: two to a CU
 
 }  // namespace
 
+// (96 x 96 asks for what 128 x 64 does, an eighth more of C to a tile; us on 128 x 128 tiles two to a CU or one / here: 1336 x 1600 x 1600
+// 20.2 / 16.2, 330 x 5672 x 7232 72 / 56, 3209 x 592 x 9064 101 / 71, 165 x 8632 x 1984 19.7 / 15.2, 189 x 9704 x 384 10.2 / 8.1; 1.15 times
+// the rate over 56 products, two of them slower: 77 x 17216 x 3840 27.6 / 28.6, 1510 x 1512 x 6912 48 / 58. 128 x 128 on eight waves: equal
+// to gemm.hip's.)
 // The smallest tile of which there is at most one per CU (more tiles than CUs: a second round, at the same intake per CU as a tile of
 // twice the area; over 250 random products of up to 2000 rows no other tile was more than 6 % ahead of this choice but where K < 128),
-// none where even 128 x 64 are more. us for 128 x 64 / 64 x 64 / 32 x 64 / 32 x 32 tiles (how many), K = 3072 [K,N]: N = 768, 2000 rows
+// none where even 128 x 64 and 96 x 96 are more. us for 128 x 64 / 64 x 64 / 32 x 64 / 32 x 32 tiles (how many), K = 3072 [K,N]: N = 768, 2000 rows
 // 17.5 (192) / 22 (384); 1000 rows 18 (96) / 12 (192) / 18 (384); 500 rows 17 / 11.6 (96) / 10 (192) / 16 (384); 256 rows 16.5 / 11.7
 // / 9.7 (96) / 9.3 (192).
 // Up to 64 rows against [N,K] weights there is the weight stream of gemm_skinny.hip, whose start and end are shorter: it stays for 33
@@ -444,7 +450,7 @@ GemmFewTile plan_gemm_few(bool trans_b, int64_t M, int64_t N, int64_t K) {
   if ((dots || stream) && M <= 64) {
     if (M > 32 ? K <= 128 : N * K < (int64_t)(M > 16 ? 2 : 3) << 22 && !(M >= 5 && M <= 8 && K >= 2048)) return {0, 0};
   }
-  static constexpr GemmFewTile kTiles[] = {{16, 16}, {16, 32}, {32, 32}, {32, 64}, {64, 64}, {128, 64}};
+  static constexpr GemmFewTile kTiles[] = {{16, 16}, {16, 32}, {32, 32}, {32, 64}, {64, 64}, {128, 64}, {96, 96}};
   for (const GemmFewTile& t : kTiles) {
     if (t.m == 16 && (M > 64 || (t.n == 16 && !trans_b))) continue;       // sixteen columns of a row of B are a quarter of a line
     const int64_t count = ((M + t.m - 1) / t.m) * ((N + t.n - 1) / t.n);
@@ -475,16 +481,17 @@ int launch_gemm_any(const T* A, const T* B, OutT* C, int64_t M, int64_t N, int64
   if (!grid_fits(tiles_m * tiles_n, 512) || tiles_m * tiles_n > 0x7fffffff || K > 0x7fffffff - 256) return HEXMI_ENOTSUP;
   const int runs = N % 8 == 0 && ldc % 8 == 0 && aligned_to(C, 16) && aligned_to(bias, 16) && aligned_to(resid, 16) &&
                    (!resid || ldr % 8 == 0);
-#define HEXMI_ANY(BM, BN)                                                                                                     \
-  hipLaunchKernelGGL((gemm_few_kernel<T, OutT, FewShape<BM, BN>::S, 2, TRANS_B, true>), dim3((unsigned)(tiles_m * tiles_n)),   \
-                     dim3(FewShape<BM, BN>::S::kThreads), 0, s, A, B, C, (int)M, (int)N, (int)K, lda, ldb, ldc, bias, resid, ldr, \
-                     (int)tiles_m, (int)tiles_n, runs)
-  if (tile.n == 128) HEXMI_ANY(128, 128);
-  else if (tile.m == 128) HEXMI_ANY(128, 64);
-  else if (tile.m == 64) HEXMI_ANY(64, 64);
-  else if (tile.n == 64) HEXMI_ANY(32, 64);
-  else if (tile.m == 32) HEXMI_ANY(32, 32);
-  else HEXMI_ANY(16, 32);
+#define HEXMI_ANY(S_)                                                                                                         \
+  hipLaunchKernelGGL((gemm_few_kernel<T, OutT, S_, 2, TRANS_B, true>), dim3((unsigned)(tiles_m * tiles_n)), dim3(S_::kThreads), 0, s, A, B, \
+                     C, (int)M, (int)N, (int)K, lda, ldb, ldc, bias, resid, ldr, (int)tiles_m, (int)tiles_n, runs)
+  typedef FewShape<128, 64>::S Any12864; typedef FewShape<64, 64>::S Any6464; typedef FewShape<32, 64>::S Any3264;
+  typedef FewShape<32, 32>::S Any3232; typedef FewShape<16, 32>::S Any1632;
+  if (tile.n == 128) HEXMI_ANY(AnyShape128);
+  else if (tile.m == 128) HEXMI_ANY(Any12864);
+  else if (tile.m == 64) HEXMI_ANY(Any6464);
+  else if (tile.n == 64) HEXMI_ANY(Any3264);
+  else if (tile.m == 32) HEXMI_ANY(Any3232);
+  else HEXMI_ANY(Any1632);
 #undef HEXMI_ANY
   return launch_status();
 }
@@ -500,6 +507,7 @@ int launch_gemm_few(const GemmFewTile& tile, const T* A, const T* B, OutT* C, in
                      dim3((unsigned)(tiles_m * tiles_n)), dim3(FewShape<BM, BN>::S::kThreads), 0, s, A, B, C, (int)M, (int)N, \
                      (int)K, lda, ldb, ldc, bias, resid, ldr, tiles_m, tiles_n, runs)
   if (tile.m == 128) HEXMI_FEW(128, 64);
+  else if (tile.m == 96) HEXMI_FEW(96, 96);
   else if (tile.m == 64) HEXMI_FEW(64, 64);
   else if (tile.n == 64) HEXMI_FEW(32, 64);
   else if (tile.m == 32) HEXMI_FEW(32, 32);
