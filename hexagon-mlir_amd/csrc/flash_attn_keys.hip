@@ -84,8 +84,8 @@ __device__ __forceinline__ void take_part(const bf16x8& part, float* p) {
 // small probability stays above 2^-24) or 16 (bf16, whose result is rounded to 8), three 24 (bf16 with an fp32 result). For
 // an fp32 result the parts of a tile meet in registers of their own, so that the running sum is rounded once a tile.
 // A part costs its share of MFMAs: 32 heads x 509 queries x 2555 keys of 128 with a mask 40 us in one part, 46 in two.
-// PITCH: Q, K and V stand as `at` says (where they are not contiguous).
-template <typename T, typename OutT, int D, bool CAUSAL, bool MASKED, bool PADDED, bool FULL, bool PITCH>
+// PITCH: Q, K and V stand as `at` says (where they are not contiguous). COLS (with PADDED): as in flash_attn.hip.
+template <typename T, typename OutT, int D, bool CAUSAL, bool MASKED, bool PADDED, bool FULL, bool PITCH, int COLS = D>
 __global__ __launch_bounds__(512, D == 64 && !MASKED ? 4 : 2)
 void flash_keys_kernel(const T* __restrict__ Q, const T* __restrict__ K, const T* __restrict__ V, OutT* __restrict__ O,
                        int ZH, int S, int Skv, float scale, const T* __restrict__ Mk, float* __restrict__ part,
@@ -103,7 +103,7 @@ void flash_keys_kernel(const T* __restrict__ Q, const T* __restrict__ K, const T
   // of 128), and a maximum that was multiplied and rounded was off by more than an exponent holds from about -2e9 on.
   constexpr float kUnit = MASKED ? kLog2e : 1.0f, kLag = kRescaleLag / kUnit;
   typedef typename MfmaT<T>::Frag Frag;
-  constexpr int DS = D / 16, DT = D / 32, CPR = D / 8;
+  constexpr int DS = (COLS + 15) / 16, DT = (COLS + 31) / 32, CPR = D / 8;
   constexpr int kTile = kTileKeys * D;
   __shared__ __attribute__((aligned(16))) T k_lds0[kGroups * kTile];
   __shared__ __attribute__((aligned(16))) T k_lds1[kGroups * kTile];
@@ -389,7 +389,8 @@ void flash_keys_kernel(const T* __restrict__ Q, const T* __restrict__ K, const T
 
   // ---- the four groups' sums: scaled to the largest of their maxima, then group i adds up the i-th quarter of the
   // output registers (float4 units u = dt * 4 + q4). The pieces for group i go through the i-th tile array.
-  constexpr int kUnits = DT * 4 / kGroups;              // units of a group
+  constexpr int kUnits = D / 32 * 4 / kGroups;          // units of a group: of the whole tile, so that a column's sums meet in the
+                                                        // same order at any COLS
   auto ml_of = [&](int g) __attribute__((always_inline)) {
     return reinterpret_cast<f32x2*>(w_lds + (g * 2 + rt) * kWaveBytes) + lane;
   };
@@ -415,6 +416,7 @@ void flash_keys_kernel(const T* __restrict__ Q, const T* __restrict__ K, const T
 #pragma unroll
     for (int j = 0; j < kUnits; ++j) {
       const int u = i * kUnits + j;
+      if (u >= DT * 4) continue;
       dst[j * 64] = f32x4{o_acc[u / 4][u % 4 * 4 + 0] * w, o_acc[u / 4][u % 4 * 4 + 1] * w,
                           o_acc[u / 4][u % 4 * 4 + 2] * w, o_acc[u / 4][u % 4 * 4 + 3] * w};
     }
@@ -429,6 +431,7 @@ void flash_keys_kernel(const T* __restrict__ Q, const T* __restrict__ K, const T
 #pragma unroll
     for (int j = 0; j < kUnits; ++j) {
       const int u = i * kUnits + j;
+      if (u >= DT * 4) continue;
       f32x4 o;
 #pragma unroll
       for (int e = 0; e < 4; ++e) o[e] = o_acc[u / 4][u % 4 * 4 + e] * w;
@@ -489,27 +492,37 @@ int launch_keys(const void* Q, const void* K, const void* V, const void* mask, v
   const int64_t blocks = (S + kRows - 1) / kRows * ZH * plan.splits, rows = ZH * S;     // see plan_flash_keys
   const int64_t merge_blocks = (rows + 1024 / D - 1) / (1024 / D);
   const float unit = mask != nullptr ? kLog2e : 1.0f, scale = mask != nullptr ? sm_scale : sm_scale * kLog2e;
-#define HEXMI_KEYS(C, M, P, F, X)                                                                                     \
-  hipLaunchKernelGGL((flash_keys_kernel<T, OutT, D, C, M, P, F, X>), dim3((unsigned)blocks), dim3(512), 0, st,           \
+#define HEXMI_KEYS_AS(C, M, P, F, X, COLS)                                                                            \
+  hipLaunchKernelGGL((flash_keys_kernel<T, OutT, D, C, M, P, F, X, COLS>), dim3((unsigned)blocks), dim3(512), 0, st,           \
                      static_cast<const T*>(Q), static_cast<const T*>(K), static_cast<const T*>(V),                    \
                      static_cast<OutT*>(O), (int)ZH, (int)S, (int)Skv, scale, static_cast<const T*>(mask), part,      \
                      plan.chunk, plan.splits, head_dim, rows_arg<X>(at))
+#define HEXMI_KEYS(C, M, P, F, X) HEXMI_KEYS_AS(C, M, P, F, X, D)
+  // heads of up to 80 and 96 columns without a mask
+#define HEXMI_KEYS_NARROW(C, X)                                                                                       \
+  do {                                                                                                                \
+    if (D == 128 && head_dim <= 80) HEXMI_KEYS_AS(C, false, true, false, X, (D == 128 ? 80 : D));                      \
+    else if (D == 128 && head_dim <= 96) HEXMI_KEYS_AS(C, false, true, false, X, (D == 128 ? 96 : D));                 \
+    else HEXMI_KEYS(C, false, true, false, X);                                                                        \
+  } while (0)
   const bool narrow = head_dim < D;
   if (!at.contiguous) {                                    // self-attention only: no mask
-    if (narrow) { if (causal) HEXMI_KEYS(true, false, true, false, true); else HEXMI_KEYS(false, false, true, false, true); }
+    if (narrow) { if (causal) HEXMI_KEYS_NARROW(true, true); else HEXMI_KEYS_NARROW(false, true); }
     else { if (causal) HEXMI_KEYS(true, false, false, false, true); else HEXMI_KEYS(false, false, false, false, true); }
   } else if (narrow) {
-    if (causal) HEXMI_KEYS(true, false, true, false, false);
+    if (causal) HEXMI_KEYS_NARROW(true, false);
     else if (plan.full) HEXMI_KEYS(false, true, true, true, false);
     else if (mask != nullptr) HEXMI_KEYS(false, true, true, false, false);
-    else HEXMI_KEYS(false, false, true, false, false);
+    else HEXMI_KEYS_NARROW(false, false);
   } else {
     if (causal) HEXMI_KEYS(true, false, false, false, false);
     else if (plan.full) HEXMI_KEYS(false, true, false, true, false);
     else if (mask != nullptr) HEXMI_KEYS(false, true, false, false, false);
     else HEXMI_KEYS(false, false, false, false, false);
   }
+#undef HEXMI_KEYS_NARROW
 #undef HEXMI_KEYS
+#undef HEXMI_KEYS_AS
   if (plan.splits > 1)
     hipLaunchKernelGGL((flash_merge_kernel<OutT, D>), dim3((unsigned)merge_blocks), dim3(256), 0, st, part,
                        static_cast<OutT*>(O), rows, plan.splits, head_dim, unit);

@@ -95,6 +95,21 @@ def test_attention_head_sizes_up_to_256(hexmi, oracle, case, dtype, causal):
     assert (got32 - want).abs().max() <= (5e-3 if dtype == torch.float16 else 3e-2)
 
 
+# widths on both sides of 80 and 96 columns (the instances that leave the rest of 128 out), both kernels, heads where they stand
+@pytest.mark.parametrize("D", [72, 80, 88, 96, 104])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("Z,H,S", [(1, 2, 33), (2, 8, 700), (4, 35, 260)])
+def test_attention_narrow_heads_equal_the_zero_padded_problem(hexmi, D, dtype, Z, H, S):
+    q, k, v = (t.cuda() for t in _qkv(Z, H, S, D, dtype, seed=D))
+    scale = 1.0 / math.sqrt(D)
+    for causal in (False, True):
+        qp, kp, vp = (torch.nn.functional.pad(t, (0, 128 - D)) for t in (q, k, v))
+        want = hexmi.flash_attention(qp, kp, vp, scale, causal)[..., :D]
+        assert torch.equal(hexmi.flash_attention(q, k, v, scale, causal), want)
+        wide = [t.transpose(1, 2).contiguous().transpose(1, 2) for t in (q, k, v)]
+        assert torch.equal(hexmi.flash_attention(*wide, scale, causal), want)
+
+
 def test_attention_padded_head_equals_the_zero_padded_problem(hexmi):
     # head size 80 on the kernel for 128 is the 128-wide problem with 48 zero columns in Q, K and V (and 1/sqrt(80)):
     # the same kernel, the same arithmetic -- bit for bit
