@@ -1591,13 +1591,15 @@ int dispatch_gemm(const void* Av, const void* Bv, void* Cv, int64_t M, int64_t N
     if (plan.channels > 0)
       return launch_gemm_skinny<T, OutT>(plan, A, B, C, M, N, K, lda, ldb, ldc, s, bias, resid, ldr);
   }
-  // 16-bit results in whole runs of eight columns: the tiles between 128 x 128 and 256 x 256
+  // 16-bit results: the tiles between 128 x 128 and 256 x 256; of output rows off the boundaries those that the paired-slab kernels leave
   if constexpr (std::is_same<T, OutT>::value) {
-    if (chunks && N % 8 == 0 && ldc % 8 == 0 && aligned_to(C, 16) && lda < (1 << 21) && ldb < (1 << 21) && K <= (1 << 30) &&
-        (!bias || aligned_to(bias, run)) && (!resid || (aligned_to(resid, run) && ldr % 4 == 0))) {
-      const int now = K % BK2 != 0 ? 0 : large ? 256 : two_per_cu(((M + 127) / 128) * ((N + 127) / 128), K) ? 2 : 1;
+    const bool aligned = N % 8 == 0 && ldc % 8 == 0 && aligned_to(C, 16) && (!bias || aligned_to(bias, run)) &&
+                         (!resid || (aligned_to(resid, run) && ldr % 4 == 0));
+    const bool whole = K % BK2 == 0, odd = TRANS_B && !aligned && (bias || resid || !whole);
+    if (chunks && (aligned || odd) && lda < (1 << 21) && ldb < (1 << 21) && K <= (1 << 30)) {
+      const int now = odd || !whole ? 0 : large ? 256 : two_per_cu(((M + 127) / 128) * ((N + 127) / 128), K) ? 2 : 1;
       const GemmMidTile mid = plan_gemm_mid(M, N, K, now, resid != nullptr);
-      if (mid.m) return launch_gemm_mid<T, TRANS_B>(mid, A, B, C, M, N, K, lda, ldb, ldc, s, bias, resid, ldr);
+      if (mid.m) return launch_gemm_mid<T, TRANS_B>(mid, A, B, C, M, N, K, lda, ldb, ldc, s, bias, resid, ldr, odd);
     }
   }
   if (fast) {

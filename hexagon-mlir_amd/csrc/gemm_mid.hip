@@ -42,13 +42,18 @@ template <int BN> __device__ __forceinline__ int swz_col(int k) {
 
 constexpr int kPast = (int)0x80000000u;     // a copy's offset past the end of its descriptor: zeros
 
-template <typename T, int TM, int TN, int NS, bool TRANS_B, bool EPI>
+// ODD: output rows of any length at any place, with or without bias and residual: a wave's sums pass through LDS 16 rows at a time and
+// leave, and take bias and residual, by elements, 64 columns of a row to an instruction; the residual of the next rows is on its way meanwhile.
+// (us on 128 x 128 tiles of 32-k slabs, bias and residual one load after the other / here: 6177 x 869 x 1344 + residual 61 / 32, 896 x 35335 x 400 +
+// residual 190 / 88, 1021 x 50257 x 768 + bias 239 / 159, 2942 x 3571 x 3984 163 / 118, 4524 x 3741 x 384 + both 133 / 53; 1.83 times the rate over 40.)
+template <typename T, int TM, int TN, int NS, bool TRANS_B, bool EPI, bool ODD = false>
 __global__ __launch_bounds__(256)
 void gemm_mid_kernel(const T* __restrict__ A, const T* __restrict__ B, T* C, int M, int N, int K, int64_t lda, int64_t ldb, int64_t ldc,
                      int tiles_m, int tiles_n, const T* __restrict__ bias, const T* resid, int64_t ldr) {
   typedef typename Types<T>::Frag Frag;
   typedef typename Types<T>::Run Run;
   constexpr int BM = 32 * TM, BN = 32 * TN;
+  static_assert(!(EPI && ODD), "ODD takes bias and residual its own way");
   static_assert(NS >= 2 && NS <= 4 && TM % 2 == 0 && TN % 2 == 0 && TM >= 4 && TN >= 4, "shapes");
   __shared__ __attribute__((aligned(16))) T a_p0[BM * BK];
   __shared__ __attribute__((aligned(16))) T a_p1[BM * BK];
@@ -247,6 +252,43 @@ void gemm_mid_kernel(const T* __restrict__ A, const T* __restrict__ B, T* C, int
       }
   }
   __syncthreads();
+  if constexpr (ODD) {
+    constexpr int W = TN * 16, PW = W + 4, EACH = W / 4;           // columns of the wave's tile, pitch, elements a lane takes of 16 rows
+    float* st = reinterpret_cast<float*>(wave == 0 ? a_p0 : wave == 1 ? a_p1 : wave == 2 ? b_p0 : b_p1);
+    static_assert(16 * PW * 4 <= BN * BK * 2 && 16 * PW * 4 <= BM * BK * 2, "16 rows of sums fit one stage");
+    const int row0 = m0 + wm * TM * 16, col0 = n0 + wn * W;
+    T add[EACH], res[2][EACH];
+    auto ask = [&](int i, T* to) __attribute__((always_inline)) {
+#pragma unroll
+      for (int t = 0; t < EACH; ++t) {
+        const int e = lane + 64 * t, row = row0 + i * 16 + e / W, col = col0 + e % W;
+        to[t] = resid[(int64_t)(row < M ? row : M - 1) * ldr + (col < N ? col : N - 1)];
+      }
+    };
+    if (bias) {
+#pragma unroll
+      for (int t = 0; t < EACH; ++t) {
+        const int col = col0 + (lane + 64 * t) % W;
+        add[t] = bias[col < N ? col : N - 1];
+      }
+    }
+    if (resid) ask(0, res[0]);
+#pragma unroll
+    for (int i = 0; i < TM; ++i) {
+#pragma unroll
+      for (int j = 0; j < TN; ++j) *reinterpret_cast<f32x4*>(st + (lane % 16) * PW + j * 16 + 4 * (lane / 16)) = acc[i][j];
+      if (resid && i + 1 < TM) ask(i + 1, res[(i + 1) & 1]);
+#pragma unroll
+      for (int t = 0; t < EACH; ++t) {
+        const int e = lane + 64 * t, row = row0 + i * 16 + e / W, col = col0 + e % W;
+        float v = st[e / W * PW + e % W];
+        if (bias) v += to_f32<T>(add[t]);
+        if (resid) v += to_f32<T>(res[i & 1][t]);
+        if (row < M && col < N) C[(int64_t)row * ldc + col] = from_f32<T>(v);
+      }
+    }
+    return;
+  }
   T* cs = wave == 0 ? a_p0 : wave == 1 ? a_p1 : wave == 2 ? b_p0 : b_p1;
   constexpr int CP = TN * 2, PITCH = TN * 16;          // 16-byte chunks and elements of a row of the wave's tile
   static_assert(TM * 16 * PITCH <= BM * BK && TM * 16 * PITCH <= BN * BK, "a wave's tile fits one stage");
@@ -308,13 +350,19 @@ GemmMidTile plan_gemm_mid(int64_t M, int64_t N, int64_t K, int now, bool resid) 
 
 template <typename T, bool TRANS_B>
 int launch_gemm_mid(const GemmMidTile& tile, const T* A, const T* B, T* C, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb,
-                    int64_t ldc, hipStream_t s, const T* bias, const T* resid, int64_t ldr) {
+                    int64_t ldc, hipStream_t s, const T* bias, const T* resid, int64_t ldr, bool odd) {
   const int64_t tiles_m = (M + tile.m - 1) / tile.m, tiles_n = (N + tile.n - 1) / tile.n;
   if (tiles_m * tiles_n > 0x7fffffff / 256 || (resid && tile.m * tile.n > 192 * 192)) return HEXMI_ENOTSUP;
-#define HEXMI_MID_AS(TM, TN, NS, EPI)                                                                                           \
-  hipLaunchKernelGGL((gemm_mid_kernel<T, TM, TN, NS, TRANS_B, EPI>), dim3((unsigned)(tiles_m * tiles_n)), dim3(256), 0, s, A, B, C, \
+#define HEXMI_MID_AS(TM, TN, NS, EPI, ODD)                                                                                           \
+  hipLaunchKernelGGL((gemm_mid_kernel<T, TM, TN, NS, TRANS_B, EPI, ODD>), dim3((unsigned)(tiles_m * tiles_n)), dim3(256), 0, s, A, B, C, \
                      (int)M, (int)N, (int)K, lda, ldb, ldc, (int)tiles_m, (int)tiles_n, bias, resid, ldr)
-#define HEXMI_MID(TM, TN, NS) do { if (bias || resid) HEXMI_MID_AS(TM, TN, NS, true); else HEXMI_MID_AS(TM, TN, NS, false); } while (0)
+#define HEXMI_MID(TM, TN, NS)                                                                                                  \
+  do {                                                                                                                         \
+    if (TRANS_B && odd) HEXMI_MID_AS(TM, TN, NS, false, TRANS_B);                                                               \
+    else if (bias || resid) HEXMI_MID_AS(TM, TN, NS, true, false);                                                              \
+    else HEXMI_MID_AS(TM, TN, NS, false, false);                                                                                \
+  } while (0)
+  if (odd && !TRANS_B) return HEXMI_ENOTSUP;
   if (tile.m == 128 && tile.per_cu == 2) HEXMI_MID(4, 4, 2);
   else if (tile.m == 128) HEXMI_MID(4, 4, 4);
   else if (tile.m == 192 && tile.n == 128) HEXMI_MID(6, 4, 4);
@@ -328,7 +376,7 @@ int launch_gemm_mid(const GemmMidTile& tile, const T* A, const T* B, T* C, int64
 
 #define HEXMI_INSTANCE(T, TB)                                                                                                  \
   template int launch_gemm_mid<T, TB>(const GemmMidTile&, const T*, const T*, T*, int64_t, int64_t, int64_t, int64_t, int64_t, int64_t, \
-                                      hipStream_t, const T*, const T*, int64_t);
+                                      hipStream_t, const T*, const T*, int64_t, bool);
 HEXMI_INSTANCE(f16, false)
 HEXMI_INSTANCE(f16, true)
 HEXMI_INSTANCE(bf16, false)

@@ -291,13 +291,13 @@ int launch_gemm_any(const T* A, const T* B, OutT* C, int64_t M, int64_t N, int64
 
 // Tiles of 128 x 128 to 256 x 192 for products of 16-bit results (gemm_mid.hip): the tile, m == 0 for none, and the launch. K % 8 == 0,
 // operand rows on 16-byte boundaries, leading dimensions below 2^21 (per-lane copy offsets), B as [K,N]: N % 8 == 0; the output on 16-byte
-// boundaries too, in whole runs of eight columns, bias and residual on 8-byte ones. now: what takes the call otherwise, 256 x 256 tiles
+// boundaries too, in whole runs of eight columns, bias and residual on 8-byte ones, or, odd (B as [N,K]), any of them anywhere. now: what takes the call otherwise, 256 x 256 tiles
 // (256), 128 x 128 two (2) or one (1) to a CU, or nothing of that rate (0).
 struct GemmMidTile { int m, n, per_cu; };
 GemmMidTile plan_gemm_mid(int64_t M, int64_t N, int64_t K, int now, bool resid);
 template <typename T, bool TRANS_B>
 int launch_gemm_mid(const GemmMidTile& tile, const T* A, const T* B, T* C, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb,
-                    int64_t ldc, hipStream_t s, const T* bias, const T* resid, int64_t ldr);
+                    int64_t ldc, hipStream_t s, const T* bias, const T* resid, int64_t ldr, bool odd);
 
 // Tiled W8A16 GEMM for many activation rows (gemm.hip): C[M,N] = (A[M,K] * W[N,K]^T) * scales[N].
 int gemm_w8a16_tiled(int64_t M, int64_t N, int64_t K, const f16* A, const int8_t* W, const f16* scales, f16* C,

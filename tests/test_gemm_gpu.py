@@ -286,6 +286,34 @@ def test_gemm_tiles_between_128_and_256(hexmi, dtype, trans_b, M, N, K, bias, re
     assert torch.equal(view[:, N:], keep)
 
 
+# ... and output rows of any length at any place, which take bias and residual by elements
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("M,N,K,bias,residual", [
+    (1025, 4097, 8, False, False), (2049, 1097, 72, True, True), (482, 4069, 1024, True, True), (2177, 1033, 136, False, True),   # 128 x 128
+    (2049, 1095, 1000, True, False), (1345, 6215, 1608, False, True), (1300, 6401, 1600, True, False), (1300, 6401, 1600, False, True),
+    (700, 9001, 1000, False, True), (645, 12457, 704, True, False), (1009, 24001, 328, True, False)])
+def test_gemm_tiles_between_128_and_256_odd_rows(hexmi, dtype, M, N, K, bias, residual):
+    _against_double(hexmi, dtype, dtype, True, M, N, K, bias, residual, M + N + K)
+    # an output one element off in rows three longer, the residual the output itself, nothing written around it
+    from hexmi import _lib
+    a, b = _inputs(M, N, K, dtype, True, seed=5)
+    a, b = a.cuda(), b.cuda()
+    bi = torch.randn(N + 1, generator=_gen(4)).to(dtype).cuda()[1:]
+    buf = torch.randn(M * (N + 3) + 8, generator=_gen(3)).to(dtype).cuda()
+    view = buf[1:1 + M * (N + 3)].view(M, N + 3)
+    want, mag = a.double() @ b.double().t() + bi.double(), a.double().abs() @ b.double().abs().t() + bi.double().abs()
+    if residual:
+        want, mag = want + view[:, :N].double(), mag + view[:, :N].double().abs()
+    keep, ends = view[:, N:].clone(), torch.cat([buf[:1], buf[1 + M * (N + 3):]]).clone()
+    code = {torch.float16: _lib.F16, torch.bfloat16: _lib.BF16}[dtype]
+    assert _lib.lib().hexmi_gemm_ex(M, N, K, a.data_ptr(), K, b.data_ptr(), K, view.data_ptr(), N + 3, bi.data_ptr(),
+                                    view.data_ptr() if residual else None, N + 3 if residual else 0, code, code, 1,
+                                    torch.cuda.current_stream().cuda_stream) == _lib.OK
+    # fp32 sums in another order, then one rounding to the output type
+    assert ((view[:, :N].double() - want).abs() <= 1e-5 * mag + torch.finfo(dtype).eps / 2 * want.abs() + 1e-7).all()
+    assert torch.equal(view[:, N:], keep) and torch.equal(torch.cat([buf[:1], buf[1 + M * (N + 3):]]), ends)
+
+
 # up to 64 rows against [N,K] weights that the weight stream does not take: K off whole 32s, fewer than 64 channels
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("M,N,K", [(3, 64, 8), (8, 700, 1000), (9, 65, 40), (16, 272, 4264), (17, 257, 1128), (32, 384, 856), (33, 2000, 72),
