@@ -406,11 +406,18 @@ template <> struct FewShape<32, 32> { typedef Shape<2, 2, 1, 1, 8> S; static con
 template <> struct FewShape<32, 64> { typedef Shape<2, 2, 1, 2, 4> S; static constexpr int NS = 6; };
 template <> struct FewShape<64, 64> { typedef Shape<2, 4, 2, 1, 4> S; static constexpr int NS = 4; };
 template <> struct FewShape<128, 64> { typedef Shape<4, 4, 2, 1, 4> S; static constexpr int NS = 3; };
+template <> struct FewShape<48, 32> { typedef Shape<3, 2, 1, 1, 8> S; static constexpr int NS = 4; };
+template <> struct FewShape<96, 64> { typedef Shape<3, 4, 2, 1, 4> S; static constexpr int NS = 3; };
+template <> struct FewShape<64, 96> { typedef Shape<4, 3, 1, 2, 4> S; static constexpr int NS = 3; };
 template <> struct FewShape<96, 96> { typedef Shape<3, 6, 2, 1, 4> S; static constexpr int NS = 3; };
 typedef Shape<4, 2, 2, 4, 1, 2> AnyShape128;                     // 128 x 128, ANY: two to a CU
 
 }  // namespace
 
+// (64 x 96 and 96 x 64 ask for an eighth less than the tile of 128 x 64 that took their calls and leave fewer CUs idle: 2638 x 512 x 5600 40 /
+// 31, 168 x 6128 x 9520 86 / 68, 1725 x 624 x 9728 64 / 53, 583 x 2144 x 4288 24 / 20, 2751 x 488 x 5312 28.8 / 23.8, 280 x 4992 x 384 6.8 / 6.2; 1.12
+// and 1.07 times the rate over 60 and 25 products, none slower. 48 x 32 before 32 x 64: 92 x 3304 x 8832 33 / 27.6, 687 x 400 x 3680 13.2 / 11.6,
+// level or a few hundredths slower below K of about 1000. 48 x 64 with two stages of 256 of K loses 10 % to 64 x 64.)
 // (96 x 96 asks for what 128 x 64 does, an eighth more of C to a tile; us on 128 x 128 tiles two to a CU or one / here: 1336 x 1600 x 1600
 // 20.2 / 16.2, 330 x 5672 x 7232 72 / 56, 3209 x 592 x 9064 101 / 71, 165 x 8632 x 1984 19.7 / 15.2, 189 x 9704 x 384 10.2 / 8.1; 1.15 times
 // the rate over 56 products, two of them slower: 77 x 17216 x 3840 27.6 / 28.6, 1510 x 1512 x 6912 48 / 58. 128 x 128 on eight waves: equal
@@ -450,8 +457,9 @@ GemmFewTile plan_gemm_few(bool trans_b, int64_t M, int64_t N, int64_t K) {
   if ((dots || stream) && M <= 64) {
     if (M > 32 ? K <= 128 : N * K < (int64_t)(M > 16 ? 2 : 3) << 22 && !(M >= 5 && M <= 8 && K >= 2048)) return {0, 0};
   }
-  static constexpr GemmFewTile kTiles[] = {{16, 16}, {16, 32}, {32, 32}, {32, 64}, {64, 64}, {128, 64}, {96, 96}};
+  static constexpr GemmFewTile kTiles[] = {{16, 16}, {16, 32}, {32, 32}, {48, 32}, {32, 64}, {64, 64}, {64, 96}, {96, 64}, {128, 64}, {96, 96}};
   for (const GemmFewTile& t : kTiles) {
+    if (t.m == 48 && K < 1024) continue;
     if (t.m == 16 && (M > 64 || (t.n == 16 && !trans_b))) continue;       // sixteen columns of a row of B are a quarter of a line
     const int64_t count = ((M + t.m - 1) / t.m) * ((N + t.n - 1) / t.n);
     if (count > cus) continue;
@@ -507,7 +515,10 @@ int launch_gemm_few(const GemmFewTile& tile, const T* A, const T* B, OutT* C, in
                      dim3((unsigned)(tiles_m * tiles_n)), dim3(FewShape<BM, BN>::S::kThreads), 0, s, A, B, C, (int)M, (int)N, \
                      (int)K, lda, ldb, ldc, bias, resid, ldr, tiles_m, tiles_n, runs)
   if (tile.m == 128) HEXMI_FEW(128, 64);
+  else if (tile.m == 96 && tile.n == 64) HEXMI_FEW(96, 64);
   else if (tile.m == 96) HEXMI_FEW(96, 96);
+  else if (tile.m == 48) HEXMI_FEW(48, 32);
+  else if (tile.m == 64 && tile.n == 96) HEXMI_FEW(64, 96);
   else if (tile.m == 64) HEXMI_FEW(64, 64);
   else if (tile.n == 64) HEXMI_FEW(32, 64);
   else if (tile.m == 32) HEXMI_FEW(32, 32);
