@@ -821,7 +821,7 @@ int gemm_w8a16_any(int64_t M, int64_t N, int64_t K, const void* A, const int8_t*
 #undef HEXMI_GEMV
     return launch_status();
   }
-  // 33 rows and more where the tiles of w8a16_few.hip give every CU a share
+  // three rows and more where the tiles of w8a16_few.hip give every CU a share
   const GemmFewTile few = plan_w8a16_few(M, N, K, tile_kernel);
   if (few.m) return launch_w8a16_few(few, M, N, K, a, W, s, zp, pt, c, st);
   // what is left of more than 128 rows that the 128 x 128 tiles do not take (rows too long for those tiles' offsets): the chunked
@@ -908,14 +908,14 @@ bool prefer_split(int64_t M, int64_t N, int64_t K, int cus) {
   const int64_t tiles = ((M + 127) / 128) * ((N + 127) / 128);
   return tiles * 3 <= cus || (tiles * 2 <= cus && K >= 8192);
 }
-// The tiles of w8a16_few.hip, ahead of it wherever they take a call, but where a quarter of the CUs or fewer would have one over a long K
+// The tiles of w8a16_few.hip, ahead of it wherever they take a call, but where a quarter of the CUs or fewer would have one of 32 x 64 over a long K
 // (us, K parts / tiles, on weights from HBM and on weights in the cache behind L2: 64 x 2048 x 14336 23.6 / 32.2 and 23.2 / 26.6, 128 x 512 x
 // 14336 24.4 / 29.4 and 24.4 / 26.6, 192 x 512 x 14336 25.7 / 30.2 and 24.8 / 26.5; 128 x 1024 x 11392 23.4 / 26.8 and 24.2 / 22.6; half of the
 // CUs 128 x 2048 x 14336 30.2 / 32.5 and 29.0 / 26.8).
 bool prefer_few(int64_t M, int64_t N, int64_t K) {
   if (K % 16 != 0) return false;
   const GemmFewTile t = plan_w8a16_few(M, N, K, K % 64 == 0 && N % 8 == 0);
-  return t.m && !(K > 12288 && 4 * ((M + t.m - 1) / t.m) * ((N + t.n - 1) / t.n) <= hexmi_num_cus());
+  return t.m && !(K > 12288 && 4 * ((M + 31) / 32) * ((N + 63) / 64) <= hexmi_num_cus());
 }
 }  // namespace
 

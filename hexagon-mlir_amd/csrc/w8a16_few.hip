@@ -1,4 +1,4 @@
-// C[M,N] = (A[M,K] * (W[N,K] - zero)^T) * scales for some ten to some hundred rows against int8 weights: tiles of one round over the
+// C[M,N] = (A[M,K] * (W[N,K] - zero)^T) * scales for three to some hundred rows against int8 weights: tiles of one round over the
 // CUs, a workgroup of eight waves to a tile.
 //
 // What bounds it: a slab of a tile is read from LDS once per wave side by side, copied into LDS, widened and multiplied, and at one
@@ -7,7 +7,7 @@
 // stay int8 in LDS and a wave widens its own channels only, waves standing side by side along the channels (64 rows to a tile) so
 // that each weight is widened once; a slab of the larger tiles multiplies from registers while the next is read; the wave groups that take the 64-k parts of
 // a slab add up in LDS at the end; scales are fetched under the K walk (at the end, by the threads that store, they cost 1 to 3 us
-// of a call). A tile of every CU's own, down to 32 x 64, is what most shapes gain by: 128 x 128 tiles left two thirds and more of the CUs
+// of a call). A tile of every CU's own, down to 16 x 16, is what most shapes gain by: 128 x 128 tiles left two thirds and more of the CUs
 // idle (256 x 4096 x 4096: 64 tiles), the chunked kernel of w8a16.hip pulls all rows into every CU.
 #include <algorithm>
 #include <type_traits>
@@ -106,9 +106,9 @@ void w8a16_few_kernel(const f16* __restrict__ A, const int8_t* __restrict__ W, c
   const int scale_at = n0 + (int)threadIdx.x < N ? n0 + (int)threadIdx.x : N - 1;
   const f16 scale = scales[pt ? 0 : scale_at];
 
-  // four partial sums of an element over K, of a wave group each or two: one chain of K / 32 additions would round more than the
-  // chunked kernel's four do
-  constexpr int kParts = KH >= 4 ? 1 : 2;
+  // Partial sums of an element over K, one to four of a wave group each: one chain of K / 32 additions would round more than the
+  // chunked kernel's sixteen (up to 16 rows) or four to eight do.
+  constexpr int kParts = TM == 1 ? 16 / KH : KH == 4 ? 1 : 2;
   f32x4 acc[kParts][TM][TN];
 #pragma unroll
   for (int p = 0; p < kParts; ++p)
@@ -117,6 +117,8 @@ void w8a16_few_kernel(const f16* __restrict__ A, const int8_t* __restrict__ W, c
 #pragma unroll
       for (int n = 0; n < TN; ++n) acc[p][m][n] = f32x4{0.f, 0.f, 0.f, 0.f};
 #define HEXMI_FENCE __builtin_amdgcn_sched_barrier(0)
+  typedef std::integral_constant<int, 0> Part0;
+  typedef std::integral_constant<int, 1> Part1;
   struct Slab { u32x4 w[TN]; f16x8 a[2][TM]; };
   auto read = [&](int stage, Slab& f) __attribute__((always_inline)) {
     const char* from = lds + stage * S::kStage;
@@ -127,7 +129,8 @@ void w8a16_few_kernel(const f16* __restrict__ A, const int8_t* __restrict__ W, c
 #pragma unroll
       for (int m = 0; m < TM; ++m) f.a[p][m] = *reinterpret_cast<const f16x8*>(from + a_at[p] + m * (16 * BK * 2));
   };
-  auto multiply = [&](const Slab& f) __attribute__((always_inline)) {
+  auto multiply = [&](const Slab& f, auto part) __attribute__((always_inline)) {      // part: of four sums, which two take this slab
+    constexpr int kFirst = kParts == 4 ? 2 * decltype(part)::value : 0, kSecond = kParts == 1 ? 0 : kFirst + 1;
 #pragma unroll
     for (int n = 0; n < TN; ++n) {
       f16x8 b0, b1;
@@ -137,10 +140,13 @@ void w8a16_few_kernel(const f16* __restrict__ A, const int8_t* __restrict__ W, c
         b1 -= zero[n];
       }
 #pragma unroll
-      for (int m = 0; m < TM; ++m) acc[0][m][n] = __builtin_amdgcn_mfma_f32_16x16x32_f16(b0, f.a[0][m], acc[0][m][n], 0, 0, 0);
+      for (int m = 0; m < TM; ++m) {
+        f32x4& c = acc[kFirst][m][n];
+        c = __builtin_amdgcn_mfma_f32_16x16x32_f16(b0, f.a[0][m], c, 0, 0, 0);
+      }
 #pragma unroll
       for (int m = 0; m < TM; ++m) {
-        f32x4& c = acc[kParts - 1][m][n];
+        f32x4& c = acc[kSecond][m][n];
         c = __builtin_amdgcn_mfma_f32_16x16x32_f16(b1, f.a[1][m], c, 0, 0, 0);
       }
     }
@@ -181,7 +187,7 @@ void w8a16_few_kernel(const f16* __restrict__ A, const int8_t* __restrict__ W, c
         read(after, next);
         HEXMI_FENCE;
       }
-      multiply(now);
+      multiply(now, Part0{});
       stage = after;
       ++j;
     };
@@ -201,21 +207,31 @@ void w8a16_few_kernel(const f16* __restrict__ A, const int8_t* __restrict__ W, c
   } else {
     // The short slabs of the small tiles gain nothing by that and K is mostly the stages' own: the last slabs in a row, each
     // with its wait known (512 x 1024 x 1024 5.5 -> 5.0 us, 66 x 1696 x 816 5.1 -> 4.6; 294 x 688 x 9600 17.9 -> 18.7).
-    auto step = [&](int newer, auto next) __attribute__((always_inline)) {   // next: the copies that follow into the free stage
+    auto step = [&](int newer, auto part, auto next) __attribute__((always_inline)) {   // next: the copies that follow into the free stage
       landed(newer);
       next(stage == 0 ? NS - 1 : stage - 1);
       HEXMI_FENCE;
       Slab now;
       read(stage, now);
-      multiply(now);
+      multiply(now, part);
       stage = stage == NS - 1 ? 0 : stage + 1;
       ++j;
     };
-    while (j + NS - 1 < full) step(NS - 2, [&](int into) __attribute__((always_inline)) { copy(j + NS - 1, into, std::false_type{}); });
-    if (j + NS - 1 < slabs) step(NS - 2, [&](int into) __attribute__((always_inline)) { copy(j + NS - 1, into, std::true_type{}); });
+    auto whole = [&](int into) __attribute__((always_inline)) { copy(j + NS - 1, into, std::false_type{}); };
+    if constexpr (kParts == 4) {
+      while (j + NS < full) {
+        step(NS - 2, Part0{}, whole);
+        step(NS - 2, Part1{}, whole);
+      }
+    }
+    while (j + NS - 1 < full) step(NS - 2, Part0{}, whole);
+    if (j + NS - 1 < slabs) step(NS - 2, Part1{}, [&](int into) __attribute__((always_inline)) { copy(j + NS - 1, into, std::true_type{}); });
 #pragma unroll
     for (int left = NS - 2; left >= 0; --left)                   // slabs behind this one
-      if (j + left < slabs) step(left, [](int) __attribute__((always_inline)) {});
+      if (j + left < slabs) {
+        if (left & 1) step(left, Part1{}, [](int) __attribute__((always_inline)) {});
+        else step(left, Part0{}, [](int) __attribute__((always_inline)) {});
+      }
   }
 #undef HEXMI_FENCE
 
@@ -227,7 +243,8 @@ void w8a16_few_kernel(const f16* __restrict__ A, const int8_t* __restrict__ W, c
 #pragma unroll
     for (int n = 0; n < TN; ++n) {                               // a lane: row lane % 16, columns 4 (lane / 16) .. + 3
       f32x4 sum = acc[0][m][n];
-      if constexpr (kParts == 2) sum += acc[1][m][n];
+      if constexpr (kParts >= 2) sum += acc[1][m][n];
+      if constexpr (kParts == 4) sum += acc[2][m][n] + acc[3][m][n];
       *reinterpret_cast<f32x4*>(red + (kh * BM + (wm * TM + m) * 16 + r16) * kPitch + (wn * TN + n) * 16 + kg * 4) = sum;
     }
   if (threadIdx.x < BN) lds_scale[threadIdx.x] = (float)scale;
@@ -259,40 +276,63 @@ void w8a16_few_kernel(const f16* __restrict__ A, const int8_t* __restrict__ W, c
 }
 
 template <int BM, int BN> struct FewShape;                       // waves, stages
+template <> struct FewShape<16, 16> { typedef Shape<1, 1, 1, 1, 8, 4> S; };
+template <> struct FewShape<16, 32> { typedef Shape<1, 2, 1, 1, 8, 4> S; };
+template <> struct FewShape<32, 32> { typedef Shape<2, 2, 1, 1, 8, 3> S; };
+template <> struct FewShape<16, 64> { typedef Shape<1, 2, 1, 2, 4, 4> S; };
 template <> struct FewShape<32, 64> { typedef Shape<2, 2, 1, 2, 4, 4> S; };
+template <> struct FewShape<48, 64> { typedef Shape<3, 2, 1, 2, 4, 3> S; };
+template <> struct FewShape<32, 96> { typedef Shape<2, 3, 1, 2, 4, 3> S; };
 template <> struct FewShape<64, 64> { typedef Shape<4, 2, 1, 2, 4, 3> S; };
+template <> struct FewShape<64, 96> { typedef Shape<4, 3, 1, 2, 4, 2> S; };
 template <> struct FewShape<64, 128> { typedef Shape<4, 2, 1, 4, 2, 4> S; };
 template <> struct FewShape<64, 192> { typedef Shape<4, 3, 1, 4, 2, 3> S; };
 
 }  // namespace
 
 // The smallest tile of which there is at most one per CU. us for 32 x 64 / 64 x 64 / 64 x 128 / 64 x 192 tiles (how many; cold weights)
-// and what took these calls before: 128 x 4096 x 4096 10.8 (256) / 13.3 (128) / 20 (64) / 25, 22.4; 256 x 4096 x 4096 19.8 (512) /
-// 14.6 (256) / 21.5 / 25.7, 27.3; 512 x 4096 x 4096 - / 26.7 (512) / 22.2 (256) / 26.6, 31.4; 256 x 11008 x 4096 - / 44 (688) / 44
-// (344) / 31 (232), 36.3; 512 x 1024 x 1024 5.0 (256) / 6.6 / 8.3 / 9.8, 11.1. Over 200 random products each of 33 to 140 and of 129
-// to 1024 rows 1.23 and 2.7 times the rate before. (128 x 128 tiles, 1000 x 4096 x 4096: 35.1, gemm.hip's 34.5.)
-// The chunked kernel of w8a16.hip, a workgroup per CU with all rows and up to 48 channels, stays ahead where rows are few: up to 48
-// (48 x 9570 x 3664 14.1 against 16.5), up to 64 rows of more than a round of 32 x 64 (64 x 8608 x 10528 38.5, 48), up to 112 of
-// more than a round of 64 x 64 (80 x 11168 x 10160 55, 58) and of few tiles over a long K (64 x 1536 x 10880 20.9, 22) -- unless it
-// has more channels than that (40 x 14336 x 992 10.8, 6.9).
+// and what took these calls before there were any: 128 x 4096 x 4096 10.8 (256) / 13.3 (128) / 20 (64) / 25, 22.4; 256 x 4096 x 4096 19.8
+// (512) / 14.6 (256) / 21.5 / 25.7, 27.3; 512 x 4096 x 4096 - / 26.7 (512) / 22.2 (256) / 26.6, 31.4; 256 x 11008 x 4096 - / 44 (688) /
+// 44 (344) / 31 (232), 36.3. Tiles of 16 x 16 to 16 x 64 and the three between (us for these / the smallest of the four above or the
+// chunked kernel of w8a16.hip): 16 x 4096 x 4096 5.7 (16 x 16) / 7.4, 32 x 4096 x 4096 6.6 (16 x 32) / 9.6, 64 x 4096 x 11008 22.6 (32 x 32 and
+// 16 x 64) / 27.9, 95 x 912 x 3872 8.1 / 12.9, 45 x 1328 x 6464 7.0 / 15.5, 47 x 4330 x 7936 16.7 (16 x 64) / 22.7, 149 x 1504 x 8256 13.2
+// (32 x 32) / 18.2, 80 x 6272 x 10624 31.9 (48 x 64) / 38.0, 339 x 2144 x 3840 12.8 (32 x 96) / 13.9, 289 x 4223 x 3072 17.0 (64 x 96) / 23.1.
+// 16 x 64 copies fewer rows of A a CU than 32 x 32 and more of W: ahead up to K = 2048 (32 x 8192 x 2048 6.2 / 7.0, x 4096 12.3 / 12.6).
+// 64 x 96 has two stages of 56 KiB where 64 x 128 has four of 24: ahead where K is short, or not long and the weights come through L2
+// for many rows (284 x 4352 x 3968 22.6 / 26.2, 352 x 2816 x 2688 13.7 / 15.9; 600 x 1792 x 7040 35.9 / 34.0, 160 x 6992 x 3712 22.1 / 20.4).
+// (128 x 128 tiles, 1000 x 4096 x 4096: 35.1, gemm.hip's 34.5. 48 x 32, 16 x 48, 32 x 48, 48 x 96, 96 x 64 and 32 x 128 tiles: nowhere ahead of
+// both neighbours by more than 2 %.)
+// The chunked kernel, a workgroup per CU with all rows and up to 48 channels, reads each weight once: it stays ahead where the weights are
+// what counts (16 x 11008 x 4096 11.9, 12.5 on 16 x 48; 16 x 8192 x 4096 9.9, 10.6; 32 x 10064 x 3328 13.0, 13.9; 40 x 11008 x 4096 16.2, 17.1;
+// 80 x 11008 x 4096 20.6, 22.6) -- unless there are more channels than that (40 x 14336 x 992 10.8, 6.9).
 // Calls that the tiles of gemm.hip do not take (zero points, K off whole slabs of 64) would go in passes of 128 rows: they come
 // here at any size, with the tile whose rounds cost least (weights: us per 3000 of K measured above; 511 x 10907 x 13056 1238 ->
 // 180, 1000 x 14336 x 992 139 -> 53, 304 x 11008 x 4368 73 -> 60).
 GemmFewTile plan_w8a16_few(int64_t M, int64_t N, int64_t K, bool tiles) {
   const int64_t cus = hexmi_num_cus();
-  if (cus <= 0 || M <= 32 || K > (1 << 22) || M > (1 << 30) || N > (1 << 30)) return {0, 0};
-  const bool chunked = N <= 48 * cus;
-  if (M <= 48 && chunked) return {0, 0};
-  static constexpr struct { GemmFewTile tile; int weight; } kTiles[] = {{{32, 64}, 20}, {{64, 64}, 30}, {{64, 128}, 50}, {{64, 192}, 65}};
+  if (cus <= 0 || M <= 2 || K > (1 << 22) || M > (1 << 30) || N > (1 << 30)) return {0, 0};
+  const bool chunked = N <= 48 * cus, heavy = N * K >= (24 << 20);       // heavy: the stream of weights is most of the call
+  struct Tile { GemmFewTile tile; int weight; };
+  static constexpr Tile kShort[] = {{{16, 16}, 0}, {{16, 32}, 0}, {{16, 64}, 0}, {{32, 32}, 0}};
+  static constexpr Tile kLong[] = {{{16, 16}, 0}, {{16, 32}, 0}, {{32, 32}, 0}, {{16, 64}, 0}};
+  static constexpr Tile kLarge[] = {{{32, 64}, 20}, {{48, 64}, 0}, {{32, 96}, 0}, {{64, 64}, 30}, {{64, 96}, 0}, {{64, 128}, 50}, {{64, 192}, 65}};
+  auto count = [&](const GemmFewTile& t) { return ((M + t.m - 1) / t.m) * ((N + t.n - 1) / t.n); };
+  for (const Tile& t : K <= 2048 ? kShort : kLong) {
+    if (count(t.tile) > cus) continue;
+    if (chunked && heavy && (M <= 16 || (M <= 32 && t.tile.n == 64))) return {0, 0};
+    return t.tile;
+  }
   GemmFewTile best = {0, 0};
   int64_t least = 0;
-  for (const auto& t : kTiles) {
-    const int64_t count = ((M + t.tile.m - 1) / t.tile.m) * ((N + t.tile.n - 1) / t.tile.n), rounds = (count + cus - 1) / cus;
+  for (const Tile& t : kLarge) {
+    const int64_t rounds = (count(t.tile) + cus - 1) / cus;
     if (rounds == 1) {
-      const int64_t rows = t.tile.n > 64 || (K > 10240 && count * 4 < cus) ? 112 : t.tile.m == 64 ? 64 : 0;
-      return chunked && M <= rows ? GemmFewTile{0, 0} : t.tile;
+      const int area = t.tile.m * t.tile.n;
+      if (area == 64 * 96 && K > (M <= 192 ? 2048 : 4608)) continue;
+      if (chunked && ((M <= 32 && heavy) || (M <= 48 && area > 32 * 64 && K > 2048) || (M <= 112 && area >= 64 * 96 && K >= 2048))) return {0, 0};
+      return t.tile;
     }
-    if (tiles || M <= 128 || count > 0x7fffffff) continue;
+    if (!t.weight || tiles || M <= 128 || count(t.tile) > 0x7fffffff) continue;
     if (!best.m || rounds * t.weight < least) best = t.tile, least = rounds * t.weight;
   }
   return best;
@@ -308,7 +348,8 @@ int launch_w8a16_few(const GemmFewTile& tile, int64_t M, int64_t N, int64_t K, c
                      tiles_n, per_tensor, runs)
 #define HEXMI_FEW(BM, BN) \
   if (tile.m == BM && tile.n == BN) { if (zero_points) HEXMI_FEW_Z(BM, BN, true); else HEXMI_FEW_Z(BM, BN, false); return launch_status(); }
-  HEXMI_FEW(32, 64) HEXMI_FEW(64, 64) HEXMI_FEW(64, 128) HEXMI_FEW(64, 192)
+  HEXMI_FEW(16, 16) HEXMI_FEW(16, 32) HEXMI_FEW(16, 64) HEXMI_FEW(32, 32) HEXMI_FEW(32, 64) HEXMI_FEW(32, 96)
+  HEXMI_FEW(48, 64) HEXMI_FEW(64, 64) HEXMI_FEW(64, 96) HEXMI_FEW(64, 128) HEXMI_FEW(64, 192)
 #undef HEXMI_FEW
 #undef HEXMI_FEW_Z
   return HEXMI_ENOTSUP;

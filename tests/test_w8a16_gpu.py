@@ -336,6 +336,20 @@ def test_w8a16_one_round_of_tiles(hexmi, mode, M, N, K):
     assert ((got.double() - want).abs() <= slack + 2.0 ** -11 * want.abs() + 1e-7).all()
 
 
+# ... the tiles down to 16 x 16 and those between: fewer slabs than stages, odd and even counts of whole slabs, short last ones
+@pytest.mark.parametrize("mode", ["plain", "zero points", "per tensor"])
+@pytest.mark.parametrize("M,N,K", [
+    (3, 16, 64), (8, 17, 528), (16, 1000, 2048), (17, 2047, 4624), (33, 1360, 6160),      # 16 x 16
+    (16, 4097, 2064), (31, 4096, 512), (48, 2721, 3088), (113, 1024, 4112),               # 16 x 32
+    (5, 8193, 256), (16, 16384, 272), (32, 8192, 1024), (33, 5441, 1296), (80, 3264, 2048), (47, 4330, 2832),   # 16 x 64, four sums
+    (64, 4096, 2560), (95, 2720, 2064), (129, 1632, 5136),                                # 32 x 32
+    (97, 5437, 2064), (240, 3264, 96), (48, 12288, 1040), (144, 5376, 784),               # 48 x 64
+    (64, 8193, 2064), (128, 6143, 272), (256, 3072, 1296),                                # 32 x 96
+    (193, 6144, 272), (80, 11000, 1024), (257, 4889, 2576), (641, 2180, 768)])            # 64 x 96
+def test_w8a16_one_round_of_small_tiles(hexmi, mode, M, N, K):
+    test_w8a16_one_round_of_tiles(hexmi, mode, M, N, K)
+
+
 def test_w8a16_tiles_ignore_what_lies_behind_the_operands(hexmi):
     # a short last slab, ragged rows and channels: the operands end where their buffers go on with values that would show, and
     # nothing outside the result is written (an output two bytes off its boundary leaves by elements)
