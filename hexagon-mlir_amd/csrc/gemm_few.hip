@@ -69,7 +69,7 @@ template <typename T, typename OutT, typename S, int NS, bool TRANS_B, bool ANY>
 __global__ __launch_bounds__(S::kThreads, S::STEPS == 2 ? 4 : 2)
 void gemm_few_kernel(const T* __restrict__ A, const T* __restrict__ B, OutT* C, int M, int N, int K, int64_t lda, int64_t ldb,
                      int64_t ldc, const OutT* __restrict__ bias, const OutT* resid, int64_t ldr, int tiles_m, int tiles_n,
-                     int runs) {
+                     int runs, int part) {
   constexpr int TM = S::TM, TN = S::TN, BM = S::BM, BN = S::BN, BK = S::BK, KH = S::KH, kWaves = S::kWaves, kThreads = S::kThreads;
   constexpr int kA = BM * BK / 512 / kWaves, kB = BN * BK / 512 / kWaves, kCopies = kA + kB;   // a wave's copies (1 KiB) of a slab
   static_assert(ANY || S::STEPS == 1, "a slab is one step of a wave");
@@ -83,6 +83,13 @@ void gemm_few_kernel(const T* __restrict__ A, const T* __restrict__ B, OutT* C, 
   int tm, tn;
   tile_of_block<8>(blockIdx.x, tiles_m, tiles_n, tm, tn);
   const int m0 = tm * BM, n0 = tn * BN;
+  if constexpr (!ANY) {                                          // blockIdx.y: the part of K, whole slabs, whose sums go to a C of its own
+    const int k0 = blockIdx.y * part;
+    A += k0;
+    B += TRANS_B ? (int64_t)k0 : k0 * ldb;
+    C += blockIdx.y * (int64_t)M * ldc;
+    K = K - k0 < part ? K - k0 : part;
+  }
 
   // copy i of a slab moves chunks [i * 512 + wave * 64, + 64) of the tile: A's kA, then B's kB
   int voff[kCopies], kc[kCopies];
@@ -410,7 +417,31 @@ template <> struct FewShape<48, 32> { typedef Shape<3, 2, 1, 1, 8> S; static con
 template <> struct FewShape<96, 64> { typedef Shape<3, 4, 2, 1, 4> S; static constexpr int NS = 3; };
 template <> struct FewShape<64, 96> { typedef Shape<4, 3, 1, 2, 4> S; static constexpr int NS = 3; };
 template <> struct FewShape<96, 96> { typedef Shape<3, 6, 2, 1, 4> S; static constexpr int NS = 3; };
+template <> struct FewShape<16, 64> { typedef Shape<1, 4, 1, 1, 8> S; static constexpr int NS = 4; };      // parts of K only,
+template <> struct FewShape<16, 128> { typedef Shape<1, 8, 1, 1, 8> S; static constexpr int NS = 2; };     // these two
 typedef Shape<4, 2, 2, 4, 1, 2> AnyShape128;                     // 128 x 128, ANY: two to a CU
+
+// C[M,N] = the sums of the parts of K, in their order, + bias + residual: one rounding. A row of the sums is pitch floats, whole eights.
+template <typename OutT>
+__global__ __launch_bounds__(128)
+void gemm_merge_kernel(const float* __restrict__ sums, OutT* C, int M, int N, int pitch, int parts, int64_t ldc,
+                       const OutT* __restrict__ bias, const OutT* resid, int64_t ldr) {
+  const int at = blockIdx.x * 128 + threadIdx.x, per_row = pitch / 4, row = at / per_row, col = at % per_row * 4;
+  if (row >= M) return;
+  const int64_t all = (int64_t)M * pitch;
+  const float* from = sums + (int64_t)row * pitch + col;
+  f32x4 s = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 8
+  for (int p = 0; p < parts; ++p) s += *reinterpret_cast<const f32x4*>(from + p * all);
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    if (col + e >= N) break;
+    float v = s[e];
+    if (bias) v += to_f32<OutT>(bias[col + e]);
+    if (resid) v += to_f32<OutT>(resid[(int64_t)row * ldr + col + e]);
+    C[(int64_t)row * ldc + col + e] = from_f32<OutT>(v);
+  }
+}
 
 }  // namespace
 
@@ -418,8 +449,8 @@ typedef Shape<4, 2, 2, 4, 1, 2> AnyShape128;                     // 128 x 128, A
 // 9.9 / 8.3; 1.12 times the rate over 50 products of 65 to 267 rows, none slower.)
 // (64 x 96 and 96 x 64 ask for an eighth less than the tile of 128 x 64 that took their calls and leave fewer CUs idle: 2638 x 512 x 5600 40 /
 // 31, 168 x 6128 x 9520 86 / 68, 1725 x 624 x 9728 64 / 53, 583 x 2144 x 4288 24 / 20, 2751 x 488 x 5312 28.8 / 23.8, 280 x 4992 x 384 6.8 / 6.2; 1.12
-// and 1.07 times the rate over 60 and 25 products, none slower. 48 x 32 before 32 x 64: 92 x 3304 x 8832 33 / 27.6, 687 x 400 x 3680 13.2 / 11.6,
-// level or a few hundredths slower below K of about 1000. 48 x 64 with two stages of 256 of K loses 10 % to 64 x 64.)
+// and 1.07 times the rate over 60 and 25 products, none slower. 48 x 32 before 32 x 64, [N,K]: 92 x 3304 x 8832 33 / 27.6, 687 x 400 x 3680 13.2 / 11.6,
+// level or a few hundredths slower below K of about 1000 and against [K,N] weights (1149 x 320 x 2752 10.5 / 11.4). 48 x 64 with two stages of 256 of K loses 10 % to 64 x 64.)
 // (96 x 96 asks for what 128 x 64 does, an eighth more of C to a tile; us on 128 x 128 tiles two to a CU or one / here: 1336 x 1600 x 1600
 // 20.2 / 16.2, 330 x 5672 x 7232 72 / 56, 3209 x 592 x 9064 101 / 71, 165 x 8632 x 1984 19.7 / 15.2, 189 x 9704 x 384 10.2 / 8.1; 1.15 times
 // the rate over 56 products, two of them slower: 77 x 17216 x 3840 27.6 / 28.6, 1510 x 1512 x 6912 48 / 58. 128 x 128 on eight waves: equal
@@ -461,7 +492,7 @@ GemmFewTile plan_gemm_few(bool trans_b, int64_t M, int64_t N, int64_t K) {
   }
   static constexpr GemmFewTile kTiles[] = {{16, 16}, {16, 32}, {32, 32}, {48, 32}, {32, 64}, {64, 64}, {64, 96}, {96, 64}, {128, 64}, {96, 96}};
   for (const GemmFewTile& t : kTiles) {
-    if (t.m == 48 && K < 1024) continue;
+    if (t.m == 48 && (K < 1024 || !trans_b)) continue;
     if (t.n == 16 && !trans_b) continue;                         // sixteen columns of a row of B are a quarter of a line
     const int64_t count = ((M + t.m - 1) / t.m) * ((N + t.n - 1) / t.n);
     if (count > cus) continue;
@@ -493,7 +524,7 @@ int launch_gemm_any(const T* A, const T* B, OutT* C, int64_t M, int64_t N, int64
                    (!resid || ldr % 8 == 0);
 #define HEXMI_ANY(S_)                                                                                                         \
   hipLaunchKernelGGL((gemm_few_kernel<T, OutT, S_, 2, TRANS_B, true>), dim3((unsigned)(tiles_m * tiles_n)), dim3(S_::kThreads), 0, s, A, B, \
-                     C, (int)M, (int)N, (int)K, lda, ldb, ldc, bias, resid, ldr, (int)tiles_m, (int)tiles_n, runs)
+                     C, (int)M, (int)N, (int)K, lda, ldb, ldc, bias, resid, ldr, (int)tiles_m, (int)tiles_n, runs, 0)
   typedef FewShape<128, 64>::S Any12864; typedef FewShape<64, 64>::S Any6464; typedef FewShape<32, 64>::S Any3264;
   typedef FewShape<32, 32>::S Any3232; typedef FewShape<16, 32>::S Any1632;
   if (tile.n == 128) HEXMI_ANY(AnyShape128);
@@ -515,7 +546,7 @@ int launch_gemm_few(const GemmFewTile& tile, const T* A, const T* B, OutT* C, in
 #define HEXMI_FEW(BM, BN)                                                                                                    \
   hipLaunchKernelGGL((gemm_few_kernel<T, OutT, FewShape<BM, BN>::S, FewShape<BM, BN>::NS, TRANS_B, false>),                         \
                      dim3((unsigned)(tiles_m * tiles_n)), dim3(FewShape<BM, BN>::S::kThreads), 0, s, A, B, C, (int)M, (int)N, \
-                     (int)K, lda, ldb, ldc, bias, resid, ldr, tiles_m, tiles_n, runs)
+                     (int)K, lda, ldb, ldc, bias, resid, ldr, tiles_m, tiles_n, runs, (int)K)
   if (tile.m == 128) HEXMI_FEW(128, 64);
   else if (tile.m == 96 && tile.n == 64) HEXMI_FEW(96, 64);
   else if (tile.m == 96) HEXMI_FEW(96, 96);
@@ -531,11 +562,53 @@ int launch_gemm_few(const GemmFewTile& tile, const T* A, const T* B, OutT* C, in
   return launch_status();
 }
 
+// Parts of K where an output of few tiles leaves most CUs without a share of a long K: a tile of 32 rows of [K,N] weights takes them in at
+// 24 GB/s to a CU. Up to one tile to a CU, parts of 512 and more, three of them at least; the sums pass through memory and a second
+// launch, 3 us. us, the tiles above / parts ([K,N]): 1 x 1024 x 11376 37 / 12, 1 x 2560 x 4096 12.8 / 9.2, 16 x 2560 x 11376 52 / 20, 16 x 4096 x
+// 4096 19.7 / 13.2, 16 x 8192 x 11008 53 / 39, 32 x 2048 x 11008 44 / 15.6, 64 x 4096 x 4096 20.9 / 15.7, 113 x 304 x 11968 22.7 / 11.6, 256 x
+// 1024 x 11008 47 / 24, 512 x 512 x 8192 22.9 / 19.4. Below these lines the second launch costs what the parts give: 16 x 4096 x 2048 7.8 / 8.7,
+// 64 x 768 x 3072 8.3 / 8.8, 11 x 7296 x 3200 15.4 / 16.7, 58 x 1408 x 4352 10.7 / 11.7; 1.22 times the rate over 110 products of K = 3072 on.
+// Tiles of [N,K] weights come in whole lines and are ahead up to K of about 10000 (64 x 4096 x 4096 13.0 /
+// 14.1, 512 x 512 x 8192 14.4 / 18.9; 64 x 4096 x 11008 33 / 26, 256 x 1024 x 11008 26 / 21, 32 x 2048 x 11008 17.7 / 15.0).
+// Up to 16 rows of more than 1024 columns tiles of 128 columns: 16 x 2560 x 11376 23.0 on 64 columns, 20.2; 1 x 1024 x 11376 11.5, 12.6.
+GemmParts plan_gemm_parts(bool trans_b, int64_t M, int64_t N, int64_t K) {
+  const GemmFewTile t = M <= 16 ? GemmFewTile{16, N <= 1024 ? 64 : 128} : GemmFewTile{M <= 32 ? 32 : 64, 64};
+  const int64_t tiles = ((M + t.m - 1) / t.m) * ((N + t.n - 1) / t.n), parts = std::min(hexmi_num_cus() / std::max<int64_t>(tiles, 1), K / 512);
+  if (parts < 3 || (trans_b ? K < 10240 || M <= 16 : M <= 32 ? K < 3072 || K < N : K < 4608)) return {};
+  const int64_t part = ((K + parts - 1) / parts + 255) / 256 * 256;          // whole slabs of every shape
+  return {t, (int)((K + part - 1) / part), (int)part};
+}
+
+template <typename T, typename OutT, bool TRANS_B>
+int launch_gemm_parts(const GemmParts& plan, const T* A, const T* B, OutT* C, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb,
+                      int64_t ldc, hipStream_t s, const OutT* bias, const OutT* resid, int64_t ldr, float* sums) {
+  const int tiles_m = (int)((M + plan.tile.m - 1) / plan.tile.m), tiles_n = (int)((N + plan.tile.n - 1) / plan.tile.n);
+  const int64_t pitch = gemm_parts_pitch(N);
+#define HEXMI_PARTS(BM, BN)                                                                                                  \
+  hipLaunchKernelGGL((gemm_few_kernel<T, float, FewShape<BM, BN>::S, FewShape<BM, BN>::NS, TRANS_B, false>),                         \
+                     dim3((unsigned)(tiles_m * tiles_n), (unsigned)plan.parts), dim3(FewShape<BM, BN>::S::kThreads), 0, s, A, B, sums, \
+                     (int)M, (int)N, (int)K, lda, ldb, pitch, (const float*)nullptr, (const float*)nullptr, (int64_t)0, tiles_m, tiles_n, 1, \
+                     plan.part)
+  if (plan.tile.m == 16 && plan.tile.n == 64) HEXMI_PARTS(16, 64);
+  else if (plan.tile.m == 16) HEXMI_PARTS(16, 128);
+  else if (plan.tile.m == 32) HEXMI_PARTS(32, 64);
+  else if (plan.tile.m == 64) HEXMI_PARTS(64, 64);
+  else return HEXMI_ENOTSUP;
+#undef HEXMI_PARTS
+  const int rc = launch_status();
+  if (rc != HEXMI_OK) return rc;
+  hipLaunchKernelGGL((gemm_merge_kernel<OutT>), dim3((unsigned)((M * (pitch / 4) + 127) / 128)), dim3(128), 0, s, sums, C, (int)M, (int)N,
+                     (int)pitch, plan.parts, ldc, bias, resid, ldr);
+  return launch_status();
+}
+
 #define HEXMI_INSTANCE(T, OutT, TB)                                                                                          \
   template int launch_gemm_few<T, OutT, TB>(const GemmFewTile&, const T*, const T*, OutT*, int64_t, int64_t, int64_t, int64_t, \
                                             int64_t, int64_t, hipStream_t, const OutT*, const OutT*, int64_t);                 \
   template int launch_gemm_any<T, OutT, TB>(const T*, const T*, OutT*, int64_t, int64_t, int64_t, int64_t, int64_t, int64_t,   \
-                                            hipStream_t, const OutT*, const OutT*, int64_t);
+                                            hipStream_t, const OutT*, const OutT*, int64_t);                                     \
+  template int launch_gemm_parts<T, OutT, TB>(const GemmParts&, const T*, const T*, OutT*, int64_t, int64_t, int64_t, int64_t, int64_t, \
+                                              int64_t, hipStream_t, const OutT*, const OutT*, int64_t, float*);
 HEXMI_INSTANCE(f16, f16, false)
 HEXMI_INSTANCE(f16, f16, true)
 HEXMI_INSTANCE(f16, float, false)

@@ -205,8 +205,10 @@ PyObject* matmul(PyObject*, PyObject* const* v, Py_ssize_t n) {
     const Launch at(*a);
     if (!at.ok) HEXMI_NOT_PLAIN;
     at::Tensor out = fresh({M, N}, a->scalar_type(), *a);
-    return finish(unlocked(hexmi_gemm_ex, M, N, K, in(a), K, in(b), tb ? K : N, out.mutable_data_ptr(), N, in(bias), in(res), res ? N : 0,
-                           code, code, tb ? 1 : 0, at.stream), "hexmi_gemm_ex", std::move(out));
+    const int64_t bytes = K >= HEXMI_GEMM_ONE_LAUNCH_K ? hexmi_gemm_workspace(M, N, K, code, tb ? 1 : 0) : 0;
+    const at::Tensor ws = bytes ? fresh({bytes}, at::kByte, *a) : at::Tensor();
+    return finish(unlocked(hexmi_gemm_ws, M, N, K, in(a), K, in(b), tb ? K : N, out.mutable_data_ptr(), N, in(bias), in(res), res ? N : 0,
+                           code, code, tb ? 1 : 0, bytes ? ws.mutable_data_ptr() : nullptr, bytes, at.stream), "hexmi_gemm_ws", std::move(out));
   });
 }
 

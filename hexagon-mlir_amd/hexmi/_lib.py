@@ -12,6 +12,7 @@ LIB_PATH = os.path.join(_HERE, "libhexmi.so")
 
 OK, EINVAL, ENOTSUP, ELAUNCH, ETOOBIG = 0, -1, -2, -3, -4
 F16, F32, I8, BF16 = 1, 2, 4, 16       # hexmi_dtype: the reference's tensor.h ids, bf16 outside its table
+GEMM_ONE_LAUNCH_K = 2048                 # HEXMI_GEMM_ONE_LAUNCH_K: no workspace below so long a K
 ATTENTION_ONE_LAUNCH_KEYS = 768         # HEXMI_ATTENTION_ONE_LAUNCH_KEYS: no workspace up to so many keys
 
 
@@ -41,6 +42,9 @@ SIGNATURES = {
     "hexmi_gemm": (_int, [_i64, _i64, _i64, _ptr, _i64, _ptr, _i64, _ptr, _i64, _int, _int, _int, _ptr]),
     "hexmi_gemm_ex": (_int, [_i64, _i64, _i64, _ptr, _i64, _ptr, _i64, _ptr, _i64, _ptr, _ptr, _i64, _int, _int, _int,
                              _ptr]),
+    "hexmi_gemm_workspace": (_i64, [_i64, _i64, _i64, _int, _int]),
+    "hexmi_gemm_ws": (_int, [_i64, _i64, _i64, _ptr, _i64, _ptr, _i64, _ptr, _i64, _ptr, _ptr, _i64, _int, _int, _int,
+                             _ptr, _i64, _ptr]),
     "hexmi_add_matmul_softmax_max_n": (_i64, []),
     "hexmi_add_matmul_softmax": (_int, [_i64, _i64, _i64, _ptr, _i64, _ptr, _i64, _ptr, _i64, _ptr, _i64, _int, _ptr]),
     "hexmi_transpose16": (_int, [_i64, _i64, _ptr, _i64, _ptr, _i64, _ptr]),

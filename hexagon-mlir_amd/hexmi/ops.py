@@ -131,20 +131,20 @@ def _layer_norm_impl(x, weight, bias, eps, out, mean, rstd, rows=None, cols=None
 
 
 def _matmul_impl(a, b, trans_b, out):
-    M, K = a.shape
-    N = b.shape[0] if trans_b else b.shape[1]
-    with _on(a.device):
-        _lib.check(_lib.lib().hexmi_gemm(M, N, K, _p(a), a.stride(0), _p(b), b.stride(0), _p(out), out.stride(0),
-                                         _dt(a), _dt(out), 1 if trans_b else 0, _stream()), "hexmi_gemm")
+    _linear_impl(a, b, None, None, trans_b, out)
 
 
 def _linear_impl(a, b, bias, residual, trans_b, out):
     M, K = a.shape
     N = b.shape[0] if trans_b else b.shape[1]
     with _on(a.device):
-        _lib.check(_lib.lib().hexmi_gemm_ex(M, N, K, _p(a), a.stride(0), _p(b), b.stride(0), _p(out), out.stride(0),
+        # few tiles over a long K: several workgroups share a tile when the library is handed scratch for their fp32 sums
+        need = (_lib.lib().hexmi_gemm_workspace(M, N, K, _dt(a), 1 if trans_b else 0)
+                if K >= _lib.GEMM_ONE_LAUNCH_K and M * N <= 1 << 20 else 0)
+        ws = torch.empty(need, dtype=torch.uint8, device=a.device) if need else None
+        _lib.check(_lib.lib().hexmi_gemm_ws(M, N, K, _p(a), a.stride(0), _p(b), b.stride(0), _p(out), out.stride(0),
                                             _p(bias), _p(residual), residual.stride(0) if residual is not None else 0,
-                                            _dt(a), _dt(out), 1 if trans_b else 0, _stream()), "hexmi_gemm_ex")
+                                            _dt(a), _dt(out), 1 if trans_b else 0, _p(ws), need, _stream()), "hexmi_gemm_ws")
 
 
 def _add_matmul_softmax_impl(x, y, z, out):

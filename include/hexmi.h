@@ -187,6 +187,25 @@ int hexmi_gemm_ex(int64_t M, int64_t N, int64_t K, const void *A, int64_t lda,
                   int in_dtype, int out_dtype, int trans_b,
                   hexmi_stream_t stream);
 
+/* hexmi_gemm_ex with scratch: few rows or columns over a long K give few tiles,
+ * and with scratch for fp32 sums several workgroups take a tile's K in parts,
+ * summed in their order by a second launch. hexmi_gemm_workspace
+ * returns the bytes that takes for contiguous operands, 0 where the product
+ * goes as a whole (every fp32 product, an output of many tiles, and any K below
+ * HEXMI_GEMM_ONE_LAUNCH_K, so a caller need not ask there).
+ * workspace may be NULL (hexmi_gemm_ex for every shape); a workspace on no
+ * 16-byte boundary or smaller than the query's answer is HEXMI_EINVAL, one that
+ * is not needed is not touched. It carries nothing between calls; two
+ * calls that overlap in time need a workspace each. */
+#define HEXMI_GEMM_ONE_LAUNCH_K 2048
+int64_t hexmi_gemm_workspace(int64_t M, int64_t N, int64_t K, int in_dtype,
+                             int trans_b);
+int hexmi_gemm_ws(int64_t M, int64_t N, int64_t K, const void *A, int64_t lda,
+                  const void *B, int64_t ldb, void *C, int64_t ldc,
+                  const void *bias, const void *residual, int64_t ldr,
+                  int in_dtype, int out_dtype, int trans_b, void *workspace,
+                  int64_t workspace_bytes, hexmi_stream_t stream);
+
 /* out[M,N] = softmax((x[M,K] + y[M,K]) * z[K,N], over each row), one launch:
  * the fused kernel the reference compiles from
  * test/python/torch-mlir/test_add_matmul_softmax.py:19-29 (torch.add ->

@@ -258,6 +258,71 @@ def test_gemm_one_round_of_tiles(hexmi, dtype, out_dtype, trans_b, M, N, K):
         assert torch.equal(view[:, N:], keep)
 
 
+# parts of K through a workspace (plan_gemm_parts on 256 CUs): each tile, three parts and many, a short last part, K off whole slabs, a
+# column run and a row over and short of a tile; beside them shapes that go as a whole. Without a workspace every shape does.
+@pytest.mark.parametrize("dtype,out_dtype", [(torch.float16, torch.float16), (torch.bfloat16, torch.float32),
+                                             (torch.bfloat16, torch.bfloat16)])
+@pytest.mark.parametrize("M,N,K,trans_b,parts", [
+    (1, 8, 3072, False, True), (16, 1024, 4104, False, True), (3, 1000, 11376, False, True),                        # 16 x 64
+    (1, 1032, 4096, False, True), (16, 4096, 4096, False, True), (15, 8200, 9000, False, True),                     # 16 x 128
+    (17, 72, 3080, False, True), (32, 2048, 11008, False, True), (29, 2560, 5128, False, True),                     # 32 x 64
+    (33, 56, 4608, False, True), (113, 304, 11968, False, True), (513, 512, 8192, False, True),                     # 64 x 64
+    (17, 2047, 10240, True, True), (64, 4097, 11008, True, True), (255, 1030, 10248, True, True),
+    (16, 4104, 4096, False, False), (16, 11008, 11376, False, False), (64, 768, 4096, False, False), (16, 1024, 11008, True, False),
+    (64, 4096, 8192, True, False), (8, 1001, 4096, False, False)])
+def test_gemm_parts_of_a_long_k(hexmi, dtype, out_dtype, M, N, K, trans_b, parts):
+    from hexmi import _lib
+    lib, code = _lib.lib(), {torch.float16: _lib.F16, torch.bfloat16: _lib.BF16, torch.float32: _lib.F32}
+    need = lib.hexmi_gemm_workspace(M, N, K, code[dtype], int(trans_b))
+    assert (need > 0) == parts
+    a, b = _inputs(M, N, K, dtype, trans_b, seed=M + N + K)
+    a, b = a.cuda(), b.cuda()
+    bias = torch.randn(N, generator=_gen(4)).to(out_dtype).cuda()
+    # rows of the output three longer, the residual the output itself, nothing written around it; the scratch starts as garbage
+    view = torch.randn(M, N + 3, generator=_gen(3)).to(out_dtype).cuda()
+    keep, wide = view.clone(), b.double().t() if trans_b else b.double()
+    want = a.double() @ wide + bias.double() + view[:, :N].double()
+    mag = a.double().abs() @ wide.abs() + bias.double().abs() + view[:, :N].double().abs()
+    ws = torch.full((need + 64,), 0xFF, dtype=torch.uint8, device="cuda")
+    s = torch.cuda.current_stream().cuda_stream
+
+    def call(ws_ptr, ws_bytes):
+        view.copy_(keep)
+        return lib.hexmi_gemm_ws(M, N, K, a.data_ptr(), K, b.data_ptr(), b.stride(0), view.data_ptr(), N + 3, bias.data_ptr(), view.data_ptr(),
+                                 N + 3, code[dtype], code[out_dtype], int(trans_b), ws_ptr, ws_bytes, s)
+    for ptr, size in ((ws.data_ptr(), need), (None, 0)):
+        assert call(ptr, size) == _lib.OK
+        # fp32 sums in another order, then one rounding to the output type
+        assert ((view[:, :N].double() - want).abs() <= 1e-5 * mag + torch.finfo(out_dtype).eps / 2 * want.abs() + 1e-7).all()
+        assert torch.equal(view[:, N:], keep[:, N:])
+    assert (ws[need:] == 0xFF).all()
+    if parts:
+        assert call(ws.data_ptr(), need - 1) == _lib.EINVAL and call(ws.data_ptr() + 4, need) == _lib.EINVAL
+        assert torch.equal(view, keep)
+        # operand rows off the boundaries go as a whole, and the scratch is not touched
+        ab, ws[:] = torch.zeros(M * K + 8, dtype=dtype, device="cuda"), 0xFF
+        ab[1:1 + M * K] = a.reshape(-1)
+        view.copy_(keep)
+        assert lib.hexmi_gemm_ws(M, N, K, ab.data_ptr() + 2, K, b.data_ptr(), b.stride(0), view.data_ptr(), N + 3, bias.data_ptr(),
+                                 view.data_ptr(), N + 3, code[dtype], code[out_dtype], int(trans_b), ws.data_ptr(), need, s) == _lib.OK
+        assert ((view[:, :N].double() - want).abs() <= 1e-5 * mag + torch.finfo(out_dtype).eps / 2 * want.abs() + 1e-7).all()
+        assert (ws == 0xFF).all()
+    # the operator gives the same with an output of its own and with one it is handed, and under capture
+    if dtype == out_dtype:
+        y = hexmi.matmul(a, b, trans_b=trans_b, bias=bias)
+        assert torch.equal(y, hexmi.matmul(a, b, trans_b=trans_b, bias=bias, out=torch.empty_like(y)))
+        side = torch.cuda.Stream()
+        side.wait_stream(torch.cuda.current_stream())
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=side):
+            z = hexmi.matmul(a, b, trans_b=trans_b, bias=bias)
+        for _ in range(3):
+            z.fill_(7.0)
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(z, y)
+
+
 # the tiles of plan_gemm_mid on 256 CUs: one row and one run of columns over and short of them, K of fewer slabs than stages, of whole slabs
 # and chunks over, slabs that the stages do not divide
 @pytest.mark.parametrize("trans_b", [False, True])
