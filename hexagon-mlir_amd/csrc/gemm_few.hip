@@ -568,13 +568,14 @@ int launch_gemm_few(const GemmFewTile& tile, const T* A, const T* B, OutT* C, in
 // 4096 19.7 / 13.2, 16 x 8192 x 11008 53 / 39, 32 x 2048 x 11008 44 / 15.6, 64 x 4096 x 4096 20.9 / 15.7, 113 x 304 x 11968 22.7 / 11.6, 256 x
 // 1024 x 11008 47 / 24, 512 x 512 x 8192 22.9 / 19.4. Below these lines the second launch costs what the parts give: 16 x 4096 x 2048 7.8 / 8.7,
 // 64 x 768 x 3072 8.3 / 8.8, 11 x 7296 x 3200 15.4 / 16.7, 58 x 1408 x 4352 10.7 / 11.7; 1.22 times the rate over 110 products of K = 3072 on.
-// Tiles of [N,K] weights come in whole lines and are ahead up to K of about 10000 (64 x 4096 x 4096 13.0 /
-// 14.1, 512 x 512 x 8192 14.4 / 18.9; 64 x 4096 x 11008 33 / 26, 256 x 1024 x 11008 26 / 21, 32 x 2048 x 11008 17.7 / 15.0).
+// Tiles of [N,K] weights come in whole lines and are ahead or behind by a tenth at K of about 10000 (64 x 4096 x 4096 13.0 / 14.1,
+// 512 x 512 x 8192 14.4 / 18.9, 64 x 512 x 10240 10.3 / 11.9, 128 x 2048 x 10240 26 / 22; 64 x 4096 x 11008 33 / 26, 256 x 1024 x 11008 26 / 21,
+// 128 x 1024 x 12288 28.9 / 15.8, 32 x 2048 x 11008 17.7 / 15.0, 32 x 4096 x 11008 21.6 / 21.4).
 // Up to 16 rows of more than 1024 columns tiles of 128 columns: 16 x 2560 x 11376 23.0 on 64 columns, 20.2; 1 x 1024 x 11376 11.5, 12.6.
 GemmParts plan_gemm_parts(bool trans_b, int64_t M, int64_t N, int64_t K) {
   const GemmFewTile t = M <= 16 ? GemmFewTile{16, N <= 1024 ? 64 : 128} : GemmFewTile{M <= 32 ? 32 : 64, 64};
   const int64_t tiles = ((M + t.m - 1) / t.m) * ((N + t.n - 1) / t.n), parts = std::min(hexmi_num_cus() / std::max<int64_t>(tiles, 1), K / 512);
-  if (parts < 3 || (trans_b ? K < 10240 || M <= 16 : M <= 32 ? K < 3072 || K < N : K < 4608)) return {};
+  if (parts < 3 || (trans_b ? K < 11008 || M <= 16 || (M <= 32 && parts < 8) : M <= 32 ? K < 3072 || K < N : K < 4608)) return {};
   const int64_t part = ((K + parts - 1) / parts + 255) / 256 * 256;          // whole slabs of every shape
   return {t, (int)((K + part - 1) / part), (int)part};
 }

@@ -267,9 +267,9 @@ def test_gemm_one_round_of_tiles(hexmi, dtype, out_dtype, trans_b, M, N, K):
     (1, 1032, 4096, False, True), (16, 4096, 4096, False, True), (15, 8200, 9000, False, True),                     # 16 x 128
     (17, 72, 3080, False, True), (32, 2048, 11008, False, True), (29, 2560, 5128, False, True),                     # 32 x 64
     (33, 56, 4608, False, True), (113, 304, 11968, False, True), (513, 512, 8192, False, True),                     # 64 x 64
-    (17, 2047, 10240, True, True), (64, 4097, 11008, True, True), (255, 1030, 10248, True, True),
+    (17, 2047, 11008, True, True), (64, 4097, 11008, True, True), (255, 1030, 11016, True, True),
     (16, 4104, 4096, False, False), (16, 11008, 11376, False, False), (64, 768, 4096, False, False), (16, 1024, 11008, True, False),
-    (64, 4096, 8192, True, False), (8, 1001, 4096, False, False)])
+    (64, 4096, 8192, True, False), (32, 4096, 11008, True, False), (8, 1001, 4096, False, False)])
 def test_gemm_parts_of_a_long_k(hexmi, dtype, out_dtype, M, N, K, trans_b, parts):
     from hexmi import _lib
     lib, code = _lib.lib(), {torch.float16: _lib.F16, torch.bfloat16: _lib.BF16, torch.float32: _lib.F32}
