@@ -265,7 +265,7 @@ class GemmNT(Workload):
 class W8A16(Workload):
     bound, dtype = "hbm", "f16"
     # the kernel rocprofv3 names for each measured shape (the library picks by M, N, K)
-    KERNELS = {(1, 11008): "w8a16_gemv_kernel", (16, 11008): "w8a16_mid_kernel", (64, 11008): "w8a16_mid_kernel",
+    KERNELS = {(1, 11008): "w8a16_gemv_kernel", (16, 11008): "w8a16_mid_kernel", (64, 11008): "w8a16_few_kernel",
                (256, 11008): "w8a16_few_kernel", (1, 4096): "w8a16_gemv_any_kernel", (16, 4096): "w8a16_mid_kernel",
                (64, 4096): "w8a16_few_kernel", (256, 4096): "w8a16_few_kernel"}
 
@@ -470,7 +470,7 @@ class MaskedAttention(Workload):
 class LinearFused(Workload):
     """A GPT-2 style projection with bias and residual: one launch (hexmi_gemm_ex) against the same result from the
     GEMM followed by two element-wise add launches."""
-    bound, kernel, dtype = "mfma", "gemm_kernel_k64", "f16"
+    bound, kernel, dtype = "mfma", "gemm_mid_kernel", "f16"
     launches_separate = 3
 
     def __init__(self, M=8192, N=768, K=3072):

@@ -26,10 +26,10 @@
 // as [N,K], odd ldc, unaligned C) -> the same kernels with the tile leaving through LDS in the pieces of 16 bytes that each row holds;
 // anything else (unaligned operand rows, K % 8 != 0) -> the tiles of gemm_few.hip with slabs that come through registers.
 // Between them, and for K off whole 64s, gemm_mid.hip where results are 16-bit in whole runs of eight columns.
-// Whole chunks of K and no more tiles than CUs -> gemm_few.hip, tiles of 16 x 16 to 128 x 64 that give every CU a share, beyond the
+// Whole chunks of K and no more tiles than CUs -> gemm_few.hip, tiles of 16 x 16 to 128 x 64 and 96 x 96 that give every CU a share, beyond the
 // lines of plan_gemm_few where B is [N,K] and rows are few. Of what it leaves: up to eight rows against B as [N,K] -> gemv_nt_kernel, a
 // stream of the weights with one wave per output channel; up to 64, by measured lines -> gemm_skinny.hip, a workgroup per 16 to
-// 64 channels.
+// 64 channels. With scratch (hexmi_gemm_ws), few tiles over a long K -> parts of K on the tiles of gemm_few.hip.
 #include <algorithm>
 #include <type_traits>
 

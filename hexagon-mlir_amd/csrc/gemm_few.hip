@@ -1,5 +1,5 @@
 // C[M,N] = A[M,K] * op(B) where tiles of 128 x 128 would leave compute units without work (fp16 / bf16 in, fp32 sums): tiles of
-// 16 x 16 to 128 x 64 and 96 x 96 in one round, a workgroup of eight waves to a tile.
+// 16 x 16 to 128 x 64 and 96 x 96 in one round, a workgroup of eight waves to a tile; and parts of a long K (plan_gemm_parts).
 //
 // What bounds it: a CU takes in about 90 GB/s through L2 whatever it does with it, and a tile of BM x BN asks for (BM + BN) x K
 // operands. 128 x 128 tiles run at that rate (0.31 us per 64 of K, K = 3072), so what is left is to have every CU take in a share:
