@@ -1734,22 +1734,25 @@ extern "C" int hexmi_gemm_ex(int64_t M, int64_t N, int64_t K, const void* A, int
 namespace {
 template <typename T, typename OutT>
 int gemm_parts_trans(const GemmParts& plan, bool tb, const void* A, const void* B, void* C, int64_t M, int64_t N, int64_t K, int64_t lda,
-                     int64_t ldb, int64_t ldc, hipStream_t s, const void* bias, const void* resid, int64_t ldr, void* sums) {
+                     int64_t ldb, int64_t ldc, hipStream_t s, const void* bias, const void* resid, int64_t ldr, void* sums, bool any) {
   const auto go = tb ? launch_gemm_parts<T, OutT, true> : launch_gemm_parts<T, OutT, false>;
   return go(plan, static_cast<const T*>(A), static_cast<const T*>(B), static_cast<OutT*>(C), M, N, K, lda, ldb, ldc, s,
-            static_cast<const OutT*>(bias), static_cast<const OutT*>(resid), ldr, static_cast<float*>(sums));
+            static_cast<const OutT*>(bias), static_cast<const OutT*>(resid), ldr, static_cast<float*>(sums), any);
 }
-bool gemm_in_parts(int64_t M, int64_t N, int64_t K, int in_dtype, bool tb, GemmParts* plan) {
-  if ((in_dtype != HEXMI_F16 && in_dtype != HEXMI_BF16) || M <= 0 || N <= 0 || K < HEXMI_GEMM_ONE_LAUNCH_K || K % 8 != 0 || (!tb && N % 8 != 0) ||
+// any: rows of an operand stand off the 16-byte boundaries
+bool gemm_in_parts(int64_t M, int64_t N, int64_t K, int in_dtype, bool tb, bool any, GemmParts* plan) {
+  if ((in_dtype != HEXMI_F16 && in_dtype != HEXMI_BF16) || M <= 0 || N <= 0 || K < HEXMI_GEMM_ONE_LAUNCH_K || (tb && any) ||
       M > 0x7fffffff || N > 0x7fffffff || K > (1 << 21)) return false;
-  *plan = plan_gemm_parts(tb, M, N, K);
+  *plan = plan_gemm_parts(tb, M, N, K, any);
   return plan->parts > 1;
 }
+bool gemm_rows_off(int64_t N, int64_t K, bool tb) { return K % 8 != 0 || (!tb && N % 8 != 0); }
+int64_t gemm_parts_bytes(const GemmParts& plan, int64_t M, int64_t N) { return plan.parts * M * gemm_parts_pitch(N) * 4; }
 }  // namespace
 
 extern "C" int64_t hexmi_gemm_workspace(int64_t M, int64_t N, int64_t K, int in_dtype, int trans_b) {
   GemmParts plan;
-  return gemm_in_parts(M, N, K, in_dtype, trans_b != 0, &plan) ? plan.parts * M * gemm_parts_pitch(N) * 4 : 0;
+  return gemm_in_parts(M, N, K, in_dtype, trans_b != 0, gemm_rows_off(N, K, trans_b != 0), &plan) ? gemm_parts_bytes(plan, M, N) : 0;
 }
 
 extern "C" int hexmi_gemm_ws(int64_t M, int64_t N, int64_t K, const void* A, int64_t lda, const void* B, int64_t ldb, void* C,
@@ -1758,18 +1761,19 @@ extern "C" int hexmi_gemm_ws(int64_t M, int64_t N, int64_t K, const void* A, int
   const bool tb = trans_b != 0;
   GemmParts plan;
   if (workspace_bytes < 0) return HEXMI_EINVAL;
+  const bool off = gemm_rows_off(N, K, tb), any = off || lda % 8 != 0 || ldb % 8 != 0 || !aligned_to(A, 16) || !aligned_to(B, 16);
   if (workspace && A && B && C && lda >= K && ldc >= N && ldb >= (tb ? K : N) && !(residual && ldr < N) &&
-      (out_dtype == in_dtype || out_dtype == HEXMI_F32) && lda % 8 == 0 && ldb % 8 == 0 && lda < (1 << 21) && ldb < (1 << 21) &&
-      aligned_to(A, 16) && aligned_to(B, 16) && gemm_in_parts(M, N, K, in_dtype, tb, &plan)) {
-    if (workspace_bytes < plan.parts * M * gemm_parts_pitch(N) * 4 || !aligned_to(workspace, 16)) return HEXMI_EINVAL;
+      (out_dtype == in_dtype || out_dtype == HEXMI_F32) && any == off && lda < (1 << 21) && ldb < (1 << 21) &&
+      gemm_in_parts(M, N, K, in_dtype, tb, any, &plan)) {
+    if (workspace_bytes < gemm_parts_bytes(plan, M, N) || !aligned_to(workspace, 16)) return HEXMI_EINVAL;
     hipStream_t s = as_stream(stream);
     begin_call();
     if (in_dtype == HEXMI_F16) {
       const auto go = out_dtype == HEXMI_F32 ? gemm_parts_trans<f16, float> : gemm_parts_trans<f16, f16>;
-      return go(plan, tb, A, B, C, M, N, K, lda, ldb, ldc, s, bias, residual, ldr, workspace);
+      return go(plan, tb, A, B, C, M, N, K, lda, ldb, ldc, s, bias, residual, ldr, workspace, any);
     }
     const auto go = out_dtype == HEXMI_F32 ? gemm_parts_trans<bf16, float> : gemm_parts_trans<bf16, bf16>;
-    return go(plan, tb, A, B, C, M, N, K, lda, ldb, ldc, s, bias, residual, ldr, workspace);
+    return go(plan, tb, A, B, C, M, N, K, lda, ldb, ldc, s, bias, residual, ldr, workspace, any);
   }
   return hexmi_gemm_ex(M, N, K, A, lda, B, ldb, C, ldc, bias, residual, ldr, in_dtype, out_dtype, trans_b, stream);
 }

@@ -83,7 +83,7 @@ void gemm_few_kernel(const T* __restrict__ A, const T* __restrict__ B, OutT* C, 
   int tm, tn;
   tile_of_block<8>(blockIdx.x, tiles_m, tiles_n, tm, tn);
   const int m0 = tm * BM, n0 = tn * BN;
-  if constexpr (!ANY) {                                          // blockIdx.y: the part of K, whole slabs, whose sums go to a C of its own
+  {                                                              // blockIdx.y: the part of K, whole slabs, whose sums go to a C of its own
     const int k0 = blockIdx.y * part;
     A += k0;
     B += TRANS_B ? (int64_t)k0 : k0 * ldb;
@@ -524,7 +524,7 @@ int launch_gemm_any(const T* A, const T* B, OutT* C, int64_t M, int64_t N, int64
                    (!resid || ldr % 8 == 0);
 #define HEXMI_ANY(S_)                                                                                                         \
   hipLaunchKernelGGL((gemm_few_kernel<T, OutT, S_, 2, TRANS_B, true>), dim3((unsigned)(tiles_m * tiles_n)), dim3(S_::kThreads), 0, s, A, B, \
-                     C, (int)M, (int)N, (int)K, lda, ldb, ldc, bias, resid, ldr, (int)tiles_m, (int)tiles_n, runs, 0)
+                     C, (int)M, (int)N, (int)K, lda, ldb, ldc, bias, resid, ldr, (int)tiles_m, (int)tiles_n, runs, (int)K)
   typedef FewShape<128, 64>::S Any12864; typedef FewShape<64, 64>::S Any6464; typedef FewShape<32, 64>::S Any3264;
   typedef FewShape<32, 32>::S Any3232; typedef FewShape<16, 32>::S Any1632;
   if (tile.n == 128) HEXMI_ANY(AnyShape128);
@@ -571,10 +571,13 @@ int launch_gemm_few(const GemmFewTile& tile, const T* A, const T* B, OutT* C, in
 // Tiles of [N,K] weights come in whole lines and are ahead or behind by a tenth at K of about 10000 (64 x 4096 x 4096 13.0 / 14.1,
 // 512 x 512 x 8192 14.4 / 18.9, 64 x 512 x 10240 10.3 / 11.9, 128 x 2048 x 10240 26 / 22; 64 x 4096 x 11008 33 / 26, 256 x 1024 x 11008 26 / 21,
 // 128 x 1024 x 12288 28.9 / 15.8, 32 x 2048 x 11008 17.7 / 15.0, 32 x 4096 x 11008 21.6 / 21.4).
+// [K,N] weights whose rows stand off the boundaries, whole / in parts: 16 x 2027 x 12144 47 / 19, 128 x 1175 x 11904 49 / 24, 3 x 485 x 8704 20.6 / 11.4, 128 x
+// 2250 x 5312 28.9 / 19.9, 15 x 1601 x 4352 13.8 / 11.8, 2 x 405 x 3136 10.9 / 11.3; 1.45 times the rate over 44 (up to 16 rows parts of 256 and
+// more: a slab through registers is a latency; with 512 and more 2 x 1497 x 4512 13.2 / 13.8, with 256 and more at 64 rows 90 x 318 x 11584 13.3 -> 15.5).
 // Up to 16 rows of more than 1024 columns tiles of 128 columns: 16 x 2560 x 11376 23.0 on 64 columns, 20.2; 1 x 1024 x 11376 11.5, 12.6.
-GemmParts plan_gemm_parts(bool trans_b, int64_t M, int64_t N, int64_t K) {
-  const GemmFewTile t = M <= 16 ? GemmFewTile{16, N <= 1024 ? 64 : 128} : GemmFewTile{M <= 32 ? 32 : 64, 64};
-  const int64_t tiles = ((M + t.m - 1) / t.m) * ((N + t.n - 1) / t.n), parts = std::min(hexmi_num_cus() / std::max<int64_t>(tiles, 1), K / 512);
+GemmParts plan_gemm_parts(bool trans_b, int64_t M, int64_t N, int64_t K, bool any) {
+  const GemmFewTile t = M <= 16 ? GemmFewTile{16, N <= 1024 || any ? 64 : 128} : GemmFewTile{M <= 32 ? 32 : 64, 64};
+  const int64_t tiles = ((M + t.m - 1) / t.m) * ((N + t.n - 1) / t.n), parts = std::min(hexmi_num_cus() / std::max<int64_t>(tiles, 1), K / (any && M <= 16 ? 256 : 512));
   if (parts < 3 || (trans_b ? K < 11008 || M <= 16 || (M <= 32 && parts < 8) : M <= 32 ? K < 3072 || K < N : K < 4608)) return {};
   const int64_t part = ((K + parts - 1) / parts + 255) / 256 * 256;          // whole slabs of every shape
   return {t, (int)((K + part - 1) / part), (int)part};
@@ -582,20 +585,27 @@ GemmParts plan_gemm_parts(bool trans_b, int64_t M, int64_t N, int64_t K) {
 
 template <typename T, typename OutT, bool TRANS_B>
 int launch_gemm_parts(const GemmParts& plan, const T* A, const T* B, OutT* C, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb,
-                      int64_t ldc, hipStream_t s, const OutT* bias, const OutT* resid, int64_t ldr, float* sums) {
+                      int64_t ldc, hipStream_t s, const OutT* bias, const OutT* resid, int64_t ldr, float* sums, bool any) {
   const int tiles_m = (int)((M + plan.tile.m - 1) / plan.tile.m), tiles_n = (int)((N + plan.tile.n - 1) / plan.tile.n);
   const int64_t pitch = gemm_parts_pitch(N);
-#define HEXMI_PARTS(BM, BN)                                                                                                  \
-  hipLaunchKernelGGL((gemm_few_kernel<T, float, FewShape<BM, BN>::S, FewShape<BM, BN>::NS, TRANS_B, false>),                         \
+#define HEXMI_PARTS_AS(BM, BN, NS, ANY)                                                                                            \
+  hipLaunchKernelGGL((gemm_few_kernel<T, float, FewShape<BM, BN>::S, NS, TRANS_B, ANY>),                                             \
                      dim3((unsigned)(tiles_m * tiles_n), (unsigned)plan.parts), dim3(FewShape<BM, BN>::S::kThreads), 0, s, A, B, sums, \
                      (int)M, (int)N, (int)K, lda, ldb, pitch, (const float*)nullptr, (const float*)nullptr, (int64_t)0, tiles_m, tiles_n, 1, \
                      plan.part)
+#define HEXMI_PARTS(BM, BN)                                                                                                  \
+  do {                                                                                                                       \
+    if (!TRANS_B && any) HEXMI_PARTS_AS(BM, BN, 2, !TRANS_B);                                                                 \
+    else HEXMI_PARTS_AS(BM, BN, (FewShape<BM, BN>::NS), false);                                                               \
+  } while (0)
+  if (any && (TRANS_B || plan.tile.n > 64)) return HEXMI_ENOTSUP;
   if (plan.tile.m == 16 && plan.tile.n == 64) HEXMI_PARTS(16, 64);
-  else if (plan.tile.m == 16) HEXMI_PARTS(16, 128);
+  else if (plan.tile.m == 16) HEXMI_PARTS_AS(16, 128, (FewShape<16, 128>::NS), false);
   else if (plan.tile.m == 32) HEXMI_PARTS(32, 64);
   else if (plan.tile.m == 64) HEXMI_PARTS(64, 64);
   else return HEXMI_ENOTSUP;
 #undef HEXMI_PARTS
+#undef HEXMI_PARTS_AS
   const int rc = launch_status();
   if (rc != HEXMI_OK) return rc;
   hipLaunchKernelGGL((gemm_merge_kernel<OutT>), dim3((unsigned)((M * (pitch / 4) + 127) / 128)), dim3(128), 0, s, sums, C, (int)M, (int)N,
@@ -609,7 +619,7 @@ int launch_gemm_parts(const GemmParts& plan, const T* A, const T* B, OutT* C, in
   template int launch_gemm_any<T, OutT, TB>(const T*, const T*, OutT*, int64_t, int64_t, int64_t, int64_t, int64_t, int64_t,   \
                                             hipStream_t, const OutT*, const OutT*, int64_t);                                     \
   template int launch_gemm_parts<T, OutT, TB>(const GemmParts&, const T*, const T*, OutT*, int64_t, int64_t, int64_t, int64_t, int64_t, \
-                                              int64_t, hipStream_t, const OutT*, const OutT*, int64_t, float*);
+                                              int64_t, hipStream_t, const OutT*, const OutT*, int64_t, float*, bool);
 HEXMI_INSTANCE(f16, f16, false)
 HEXMI_INSTANCE(f16, f16, true)
 HEXMI_INSTANCE(f16, float, false)

@@ -283,11 +283,12 @@ struct GemmFewTile { int m, n; };
 GemmFewTile plan_gemm_few(bool trans_b, int64_t M, int64_t N, int64_t K);
 // ... and in parts of K whose fp32 sums go through a caller workspace: rows of gemm_parts_pitch(N) floats, M of them for each part
 struct GemmParts { GemmFewTile tile; int parts, part; };           // parts: 0 where the product goes as a whole
-GemmParts plan_gemm_parts(bool trans_b, int64_t M, int64_t N, int64_t K);
+// any: operand rows off the boundaries, [K,N] weights
+GemmParts plan_gemm_parts(bool trans_b, int64_t M, int64_t N, int64_t K, bool any);
 inline int64_t gemm_parts_pitch(int64_t N) { return (N + 7) / 8 * 8; }
 template <typename T, typename OutT, bool TRANS_B>
 int launch_gemm_parts(const GemmParts& plan, const T* A, const T* B, OutT* C, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb,
-                      int64_t ldc, hipStream_t s, const OutT* bias, const OutT* resid, int64_t ldr, float* sums);
+                      int64_t ldc, hipStream_t s, const OutT* bias, const OutT* resid, int64_t ldr, float* sums, bool any);
 template <typename T, typename OutT, bool TRANS_B>
 int launch_gemm_few(const GemmFewTile& tile, const T* A, const T* B, OutT* C, int64_t M, int64_t N, int64_t K, int64_t lda,
                     int64_t ldb, int64_t ldc, hipStream_t s, const OutT* bias, const OutT* resid, int64_t ldr);

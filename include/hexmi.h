@@ -195,7 +195,8 @@ int hexmi_gemm_ex(int64_t M, int64_t N, int64_t K, const void *A, int64_t lda,
  * HEXMI_GEMM_ONE_LAUNCH_K, so a caller need not ask there).
  * workspace may be NULL (hexmi_gemm_ex for every shape); a workspace on no
  * 16-byte boundary or smaller than the query's answer is HEXMI_EINVAL, one that
- * is not needed is not touched. It carries nothing between calls; two
+ * is not needed is not touched (operands that stand off the 16-byte boundaries
+ * though their sizes do not put them there go as a whole). It carries nothing between calls; two
  * calls that overlap in time need a workspace each. */
 #define HEXMI_GEMM_ONE_LAUNCH_K 2048
 int64_t hexmi_gemm_workspace(int64_t M, int64_t N, int64_t K, int in_dtype,

@@ -269,7 +269,9 @@ def test_gemm_one_round_of_tiles(hexmi, dtype, out_dtype, trans_b, M, N, K):
     (33, 56, 4608, False, True), (113, 304, 11968, False, True), (513, 512, 8192, False, True),                     # 64 x 64
     (17, 2047, 11008, True, True), (64, 4097, 11008, True, True), (255, 1030, 11016, True, True),
     (16, 4104, 4096, False, False), (16, 11008, 11376, False, False), (64, 768, 4096, False, False), (16, 1024, 11008, True, False),
-    (64, 4096, 8192, True, False), (32, 4096, 11008, True, False), (8, 1001, 4096, False, False)])
+    (64, 4096, 8192, True, False), (32, 4096, 11008, True, False),
+    (8, 1001, 4096, False, True), (16, 4097, 4100, False, True), (1, 3, 3075, False, True), (31, 2049, 5001, False, True),   # rows off the
+    (128, 531, 9736, False, True), (64, 1024, 4611, False, True), (64, 2047, 11009, True, False)])                          # boundaries
 def test_gemm_parts_of_a_long_k(hexmi, dtype, out_dtype, M, N, K, trans_b, parts):
     from hexmi import _lib
     lib, code = _lib.lib(), {torch.float16: _lib.F16, torch.bfloat16: _lib.BF16, torch.float32: _lib.F32}
@@ -299,7 +301,8 @@ def test_gemm_parts_of_a_long_k(hexmi, dtype, out_dtype, M, N, K, trans_b, parts
     if parts:
         assert call(ws.data_ptr(), need - 1) == _lib.EINVAL and call(ws.data_ptr() + 4, need) == _lib.EINVAL
         assert torch.equal(view, keep)
-        # operand rows off the boundaries go as a whole, and the scratch is not touched
+    if parts and K % 8 == 0 and (trans_b or N % 8 == 0):
+        # a base off the boundaries where the sizes are not: as a whole, and the scratch is not touched
         ab, ws[:] = torch.zeros(M * K + 8, dtype=dtype, device="cuda"), 0xFF
         ab[1:1 + M * K] = a.reshape(-1)
         view.copy_(keep)
