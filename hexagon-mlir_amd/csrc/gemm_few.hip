@@ -576,9 +576,11 @@ int launch_gemm_few(const GemmFewTile& tile, const T* A, const T* B, OutT* C, in
 // more: a slab through registers is a latency; with 512 and more 2 x 1497 x 4512 13.2 / 13.8, with 256 and more at 64 rows 90 x 318 x 11584 13.3 -> 15.5).
 // Up to 16 rows of more than 1024 columns tiles of 128 columns: 16 x 2560 x 11376 23.0 on 64 columns, 20.2; 1 x 1024 x 11376 11.5, 12.6.
 GemmParts plan_gemm_parts(bool trans_b, int64_t M, int64_t N, int64_t K, bool any) {
+  if (trans_b ? K < 11008 || M <= 16 : M <= 32 ? K < 3072 || K < N : K < 4608) return {};
   const GemmFewTile t = M <= 16 ? GemmFewTile{16, N <= 1024 || any ? 64 : 128} : GemmFewTile{M <= 32 ? 32 : 64, 64};
-  const int64_t tiles = ((M + t.m - 1) / t.m) * ((N + t.n - 1) / t.n), parts = std::min(hexmi_num_cus() / std::max<int64_t>(tiles, 1), K / (any && M <= 16 ? 256 : 512));
-  if (parts < 3 || (trans_b ? K < 11008 || M <= 16 || (M <= 32 && parts < 8) : M <= 32 ? K < 3072 || K < N : K < 4608)) return {};
+  const int64_t tiles = ((M + t.m - 1) / t.m) * ((N + t.n - 1) / t.n);
+  const int64_t parts = std::min(hexmi_num_cus() / std::max<int64_t>(tiles, 1), K / (any && M <= 16 ? 256 : 512));
+  if (parts < 3 || (trans_b && M <= 32 && parts < 8)) return {};
   const int64_t part = ((K + parts - 1) / parts + 255) / 256 * 256;          // whole slabs of every shape
   return {t, (int)((K + part - 1) / part), (int)part};
 }

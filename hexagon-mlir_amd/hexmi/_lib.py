@@ -12,7 +12,7 @@ LIB_PATH = os.path.join(_HERE, "libhexmi.so")
 
 OK, EINVAL, ENOTSUP, ELAUNCH, ETOOBIG = 0, -1, -2, -3, -4
 F16, F32, I8, BF16 = 1, 2, 4, 16       # hexmi_dtype: the reference's tensor.h ids, bf16 outside its table
-GEMM_ONE_LAUNCH_K = 2048                 # HEXMI_GEMM_ONE_LAUNCH_K: no workspace below so long a K
+GEMM_ONE_LAUNCH_K = 3072                 # HEXMI_GEMM_ONE_LAUNCH_K: no workspace below so long a K
 ATTENTION_ONE_LAUNCH_KEYS = 768         # HEXMI_ATTENTION_ONE_LAUNCH_KEYS: no workspace up to so many keys
 
 

@@ -198,7 +198,7 @@ int hexmi_gemm_ex(int64_t M, int64_t N, int64_t K, const void *A, int64_t lda,
  * is not needed is not touched (operands that stand off the 16-byte boundaries
  * though their sizes do not put them there go as a whole). It carries nothing between calls; two
  * calls that overlap in time need a workspace each. */
-#define HEXMI_GEMM_ONE_LAUNCH_K 2048
+#define HEXMI_GEMM_ONE_LAUNCH_K 3072
 int64_t hexmi_gemm_workspace(int64_t M, int64_t N, int64_t K, int in_dtype,
                              int trans_b);
 int hexmi_gemm_ws(int64_t M, int64_t N, int64_t K, const void *A, int64_t lda,
