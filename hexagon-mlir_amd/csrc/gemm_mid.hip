@@ -317,7 +317,7 @@ void gemm_mid_kernel(const T* __restrict__ A, const T* __restrict__ B, T* C, int
 
 // What a launch takes, us: rounds of tiles over the CUs (two tiles to a CU where two fit), slabs of K in each. A round costs a part by its
 // length and a part by how many of its tiles there are (they share L2 and the chip's power). Fitted to 370 random products of 65 to
-// 8192 rows, K = 256 to 12288, on one box (mean error 7 to 10 %); of these tiles the one it names is 1.2 % off the best.
+// 8192 rows, K = 256 to 12288, on one card (mean error 7 to 10 %); of these tiles the one it names is 1.2 % off the best.
 struct MidCost { int m, n, per_cu; double start, slab, slab_full, tile, tile_full, resid; };
 static double mid_time(const MidCost& c, int64_t M, int64_t N, int64_t K, bool resid) {
   const int64_t tiles = ((M + c.m - 1) / c.m) * ((N + c.n - 1) / c.n), slots = std::max(1, hexmi_num_cus()) * c.per_cu;

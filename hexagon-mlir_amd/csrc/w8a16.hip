@@ -17,8 +17,8 @@ namespace hexmi {
 namespace {
 
 // Up to 16 activation rows on pre-packed weights, K <= 4096 (plain weights go through the chunked kernel further
-// down, which is faster at every row count: 11.3 against 11.8-12.3 us at M = 4 and 8, N = 11008, K = 4096; 6.9
-// against 8.6 at N = K = 4096): persistent workgroups of 16 waves, one per compute unit. The per-CU rate
+// down or the tiles of w8a16_few.hip, which are faster at every row count: 11.3 against 11.8-12.3 us at M = 4 and 8, N = 11008, K = 4096;
+// 5.7 against 8.6 at N = K = 4096): persistent workgroups of 16 waves, one per compute unit. The per-CU rate
 // of the weight reads is what bounds this shape, so the output channels are dealt in equal
 // contiguous ranges over exactly as many workgroups as there are CUs (N = 11008 on 256 CUs: 43 channels each,
 // walked as tiles of 16, 16 and 11 channels; the lanes of a short tile re-read its last row and drop the result).
