@@ -51,6 +51,13 @@ template <int BN> __device__ __forceinline__ int swz_col(int k) {
   return BN == 64 ? (((k >> 1) & 1) | (((k >> 3) & 1) << 1)) << 1 : ((k >> 3) & 1) << 1;
 }
 
+// Elements of K from a slab on, zero and less for slabs past the last one. The difference fits where slab * BK passes 2^31: near the
+// longest K a slab past the last one wrapped round and was read from 2^31 elements before its row.
+__host__ __device__ constexpr int rest_of(int K, int slab, int BK) { return (int)((unsigned)K - (unsigned)slab * (unsigned)BK); }
+constexpr int kAnyMaxK = 0x7fffffff - 64;                        // the longest K of launch_gemm_any
+static_assert(rest_of(kAnyMaxK, kAnyMaxK / 256, 256) == kAnyMaxK % 256 && rest_of(kAnyMaxK, kAnyMaxK / 256 + 4, 256) < 0 &&
+              rest_of(kAnyMaxK, kAnyMaxK / 64 + 4, 64) < 0 && rest_of(kAnyMaxK, 0, 256) == kAnyMaxK, "slabs past the last one are past K");
+
 // NS stages of a slab of KH * 32 k: copies fill all but one while that one is read; one barrier a slab. K % 8 == 0, operand rows
 // on 16-byte boundaries ([K,N]: N % 8 == 0 too). runs: the output (and bias and residual) in runs of eight columns on
 // 16-byte boundaries; otherwise they go by elements.
@@ -132,7 +139,7 @@ void gemm_few_kernel(const T* __restrict__ A, const T* __restrict__ B, OutT* C, 
   const char* a_base = reinterpret_cast<const char*>(A + (int64_t)m0 * lda);
   const char* b_base = reinterpret_cast<const char*>(TRANS_B ? B + (int64_t)n0 * ldb : B + n0);
   const int64_t b_step = (TRANS_B ? BK : BK * ldb) * 2;
-  const int slabs = (K + BK - 1) / BK;
+  const int slabs = (int)(((unsigned)K + BK - 1) / BK);
   auto copy = [&](int slab, int stage, auto ragged) __attribute__((always_inline)) {
     const char* a_from = a_base + (int64_t)slab * (BK * 2);
     const char* b_from = b_base + slab * b_step;
@@ -236,9 +243,10 @@ void gemm_few_kernel(const T* __restrict__ A, const T* __restrict__ B, OutT* C, 
         if constexpr (decltype(plain)::value) {
           __builtin_memcpy(&to[i], ptr[i] + (i < kA || TRANS_B ? (int64_t)slab * BK : (int64_t)slab * BK * ldb), 16);
         } else {
-          const int k = slab * BK + kc[i];
-          if (i < kA || TRANS_B) __builtin_memcpy(&to[i], ptr[i] + (slab * BK + (k < K - 8 ? 0 : K - 8 - k)), 16);
-          else __builtin_memcpy(&to[i], ptr[i] + (int64_t)((k < K - 1 ? k : K - 1) - kc[i]) * ldb, 16);
+          const int left = rest_of(K, slab, BK) - kc[i];         // elements or rows before the end of K; from the slab's start on where
+                                                                 // eight (one) are left, and before the end of K otherwise
+          if (i < kA || TRANS_B) __builtin_memcpy(&to[i], ptr[i] + (left > 8 ? (int64_t)slab * BK : K - 8 - kc[i]), 16);
+          else __builtin_memcpy(&to[i], ptr[i] + (left > 1 ? (int64_t)slab * BK : K - 1 - kc[i]) * ldb, 16);
         }
       }
     };
@@ -248,7 +256,7 @@ void gemm_few_kernel(const T* __restrict__ A, const T* __restrict__ B, OutT* C, 
       for (int i = 0; i < kCopies; ++i) {
         u32x4 v = from[i];
         if constexpr (!decltype(plain)::value) {
-          const int left = K - slab * BK - kc[i];                // elements or rows before the end of K
+          const int left = rest_of(K, slab, BK) - kc[i];
           const u32x4 zero = {0u, 0u, 0u, 0u};
           v = shift_columns(v, zero, i < kA || TRANS_B ? (left < 8 ? 8 - left : 0) & 7 : by[i]);
           v = left > 0 ? v : zero;
@@ -273,12 +281,12 @@ void gemm_few_kernel(const T* __restrict__ A, const T* __restrict__ B, OutT* C, 
           const int q = a ? e : e - BM * BK;
           unsigned short v = 0;
           if (a || TRANS_B) {
-            const int row = q / BK, k = slab * BK + ((q % BK / 8) ^ swz_row<BK>(row)) * 8 + q % 8;
-            const T* base = a ? A + (int64_t)m0 * lda : B + (int64_t)n0 * ldb;
-            if (k < K && row < (a ? M - m0 : N - n0)) v = reinterpret_cast<const unsigned short*>(base)[row * (a ? lda : ldb) + k];
+            const int row = q / BK, k = ((q % BK / 8) ^ swz_row<BK>(row)) * 8 + q % 8;
+            const T* base = (a ? A + (int64_t)m0 * lda : B + (int64_t)n0 * ldb) + (int64_t)slab * BK;
+            if (k < rest_of(K, slab, BK) && row < (a ? M - m0 : N - n0)) v = reinterpret_cast<const unsigned short*>(base)[row * (a ? lda : ldb) + k];
           } else {
             const int row = q / BN, col = n0 + ((q % BN / 8) ^ swz_col<BN>(row)) * 8 + q % 8;
-            if (slab * BK + row < K && col < N) v = reinterpret_cast<const unsigned short*>(B)[(int64_t)(slab * BK + row) * ldb + col];
+            if (row < rest_of(K, slab, BK) && col < N) v = reinterpret_cast<const unsigned short*>(B)[((int64_t)slab * BK + row) * ldb + col];
           }
           reinterpret_cast<unsigned short*>(lds)[e] = v;
         }
@@ -519,7 +527,7 @@ int launch_gemm_any(const T* A, const T* B, OutT* C, int64_t M, int64_t N, int64
                     const OutT* bias, const OutT* resid, int64_t ldr) {
   const GemmFewTile tile = plan_gemm_any(M, N);
   const int64_t tiles_m = (M + tile.m - 1) / tile.m, tiles_n = (N + tile.n - 1) / tile.n;
-  if (!grid_fits(tiles_m * tiles_n, 512) || tiles_m * tiles_n > 0x7fffffff || K > 0x7fffffff - 256) return HEXMI_ENOTSUP;
+  if (!grid_fits(tiles_m * tiles_n, 512) || tiles_m * tiles_n > 0x7fffffff || K > kAnyMaxK) return HEXMI_ENOTSUP;
   const int runs = N % 8 == 0 && ldc % 8 == 0 && aligned_to(C, 16) && aligned_to(bias, 16) && aligned_to(resid, 16) &&
                    (!resid || ldr % 8 == 0);
 #define HEXMI_ANY(S_)                                                                                                         \

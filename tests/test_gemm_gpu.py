@@ -427,6 +427,16 @@ def test_gemm_operand_rows_off_the_boundaries(hexmi, dtype, out_dtype, trans_b, 
     assert ((c.double() - a @ b).abs() <= 1e-5 * (a.abs() @ b.abs()) + eps * (a @ b).abs() + 1e-7).all()
 
 
+def test_gemm_longest_inner_dimension(hexmi):
+    # one workgroup walks all of K: the slabs asked for past the last one lie past 2^31 elements
+    K = 0x7fffffff - 64
+    a, b = (torch.zeros(1, K, dtype=torch.float16, device="cuda") for _ in range(2))
+    at = torch.tensor([0, 1, K // 2, 1 << 30, K - 600, K - 257, K - 9, K - 8, K - 1], device="cuda")
+    a[0, at] = 2.0 ** torch.arange(9, device="cuda").half()
+    b[0, at] = 1.0
+    assert float(hexmi.matmul(a, b, trans_b=True)) == 511.0
+
+
 # more tiles than one round of them: the 128 x 128 and 256 x 256 kernels and the slabs, widths and outputs each is for
 @pytest.mark.parametrize("trans_b", [False, True])
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
