@@ -527,7 +527,15 @@ int launch_gemm_any(const T* A, const T* B, OutT* C, int64_t M, int64_t N, int64
                     const OutT* bias, const OutT* resid, int64_t ldr) {
   const GemmFewTile tile = plan_gemm_any(M, N);
   const int64_t tiles_m = (M + tile.m - 1) / tile.m, tiles_n = (N + tile.n - 1) / tile.n;
-  if (!grid_fits(tiles_m * tiles_n, 512) || tiles_m * tiles_n > 0x7fffffff || K > kAnyMaxK) return HEXMI_ENOTSUP;
+  if (K > kAnyMaxK) return HEXMI_ENOTSUP;
+  if (!grid_fits(tiles_m * tiles_n, 512)) {                      // more threads than a grid holds: half of the tiles, then the rest
+    const bool rows = tiles_m >= tiles_n;
+    const int64_t m = rows ? (tiles_m + 1) / 2 * tile.m : 0, n = rows ? 0 : (tiles_n + 1) / 2 * tile.n;
+    const int rc = launch_gemm_any<T, OutT, TRANS_B>(A, B, C, rows ? m : M, rows ? N : n, K, lda, ldb, ldc, s, bias, resid, ldr);
+    if (rc != HEXMI_OK) return rc;
+    return launch_gemm_any<T, OutT, TRANS_B>(A + m * lda, B + n * (TRANS_B ? ldb : 1), C + m * ldc + n, M - m, N - n, K, lda, ldb, ldc, s,
+                                             bias ? bias + n : nullptr, resid ? resid + m * ldr + n : nullptr, ldr);
+  }
   const int runs = N % 8 == 0 && ldc % 8 == 0 && aligned_to(C, 16) && aligned_to(bias, 16) && aligned_to(resid, 16) &&
                    (!resid || ldr % 8 == 0);
 #define HEXMI_ANY(S_)                                                                                                         \

@@ -342,6 +342,7 @@ GemmMidTile plan_gemm_mid(int64_t M, int64_t N, int64_t K, int now, bool resid) 
   for (const MidCost& c : kMidTiles) {
     if (now != 0 && c.m == 128) continue;                    // (gemm.hip's own are the better ones of whole slabs)
     if (resid && c.m * c.n > 192 * 192) continue;
+    if (!grid_fits(((M + c.m - 1) / c.m) * ((N + c.n - 1) / c.n), 256)) continue;
     const double t = mid_time(c, M, N, K, resid);
     if (t < least) least = t, best = &c;
   }
@@ -352,7 +353,7 @@ template <typename T, bool TRANS_B>
 int launch_gemm_mid(const GemmMidTile& tile, const T* A, const T* B, T* C, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb,
                     int64_t ldc, hipStream_t s, const T* bias, const T* resid, int64_t ldr, bool odd) {
   const int64_t tiles_m = (M + tile.m - 1) / tile.m, tiles_n = (N + tile.n - 1) / tile.n;
-  if (tiles_m * tiles_n > 0x7fffffff / 256 || (resid && tile.m * tile.n > 192 * 192)) return HEXMI_ENOTSUP;
+  if (!grid_fits(tiles_m * tiles_n, 256) || (resid && tile.m * tile.n > 192 * 192)) return HEXMI_ENOTSUP;
 #define HEXMI_MID_AS(TM, TN, NS, EPI, ODD)                                                                                           \
   hipLaunchKernelGGL((gemm_mid_kernel<T, TM, TN, NS, TRANS_B, EPI, ODD>), dim3((unsigned)(tiles_m * tiles_n)), dim3(256), 0, s, A, B, C, \
                      (int)M, (int)N, (int)K, lda, ldb, ldc, (int)tiles_m, (int)tiles_n, bias, resid, ldr)

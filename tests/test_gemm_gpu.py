@@ -437,6 +437,14 @@ def test_gemm_longest_inner_dimension(hexmi):
     assert float(hexmi.matmul(a, b, trans_b=True)) == 511.0
 
 
+# more tiles than a grid of 512 threads each holds: rows of eight on the tiles of 16-bit results, single columns through registers
+@pytest.mark.parametrize("N", [1, 8])
+def test_gemm_more_tiles_than_a_grid_holds(hexmi, N):
+    M = (0xffffffff // 512 + 1) * 128 + 3
+    a = torch.randint(-2048, 2049, (M, N), dtype=torch.float16, device="cuda", generator=torch.Generator("cuda").manual_seed(5))
+    assert torch.equal(hexmi.matmul(a, torch.eye(N, dtype=torch.float16, device="cuda")), a)
+
+
 # more tiles than one round of them: the 128 x 128 and 256 x 256 kernels and the slabs, widths and outputs each is for
 @pytest.mark.parametrize("trans_b", [False, True])
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
