@@ -65,7 +65,9 @@ static_assert(rest_of(kAnyMaxK, kAnyMaxK / 256, 256) == kAnyMaxK % 256 && rest_o
 // boundary, a load into registers does not: two slabs are on their way in registers while a third is multiplied from one of two
 // stages. Bound by the latency of a slab's loads as the copies are, so no load waits for a choice: a chunk that reaches past the end of K or
 // of a [K,N] row is read as the last eight elements before it and shifted into place, with zeros behind K, on its way into LDS, in
-// the last slab and the last column of tiles only. Tiles of 128 x 128 have one slab on its way, so that two fit a CU. (128 x 128 tiles that
+// the last slab and the last column of tiles only. Rows of fewer than eight columns are read with the end of the row before (the first of B from
+// its start); fewer than eight of K are one chunk, put together from elements. (By elements throughout, one latency after the other, 65536 x 1
+// x 4096 took 866 us, 65536 x 7 x 768 167 and 4096 x 4096 x 7 36; with 128 x 128 tiles of chunks under branches 203, 57 and 20; here 132, 29 and 13.) Tiles of 128 x 128 have one slab on its way, so that two fit a CU. (128 x 128 tiles that
 // put such chunks together from elements under a branch of every load had their four chunks of a slab one latency after the other, 2 us
 // for 32 of K. [K,N], us, there / here: 128 x 7219 x 6656 299 / 49, 640 x 7031 x 3584 322 / 105, 16 x 4097 x 4096 120 / 19, 50 x 1001 x 768
 // 48 / 6.8, 4000 x 4001 x 2048 160 / 110, 1021 x 50257 x 768 174 / 157; aligned neighbours with copies into LDS take 43, 61, 18, 5, 48 and
@@ -117,7 +119,7 @@ void gemm_few_kernel(const T* __restrict__ A, const T* __restrict__ B, OutT* C, 
         const int col = n0 + c * 8, at = col + 8 <= N ? col : N - 8;
         ptr[i] = B + (int64_t)k * ldb + at;
         kc[i] = k;
-        by[i] = (col - at) & 7;                                  // (chunks wholly past N: anything, those columns are not stored)
+        by[i] = (col - at) & 7;                                  // (columns past N: anything, they are not stored)
       }
     }
   }
@@ -237,7 +239,13 @@ void gemm_few_kernel(const T* __restrict__ A, const T* __restrict__ B, OutT* C, 
     constexpr int kSets = S::STEPS == 2 ? 1 : 2;                 // slabs on their way
     u32x4 set[kSets][kCopies];
     // PLAIN: every chunk lies inside its row and K. The other form takes any slab, one past the last too (zeros).
-    auto fetch = [&](int slab, u32x4 (&to)[kCopies], auto plain) __attribute__((always_inline)) {
+    // first: the slab at the start of B, whose first rows, where they are shorter than a chunk, are read from there on: so many elements
+    // on from where the chunk's end would be the row's
+    auto ahead_of = [&](int i) __attribute__((always_inline)) {
+      const int ahead = 8 - N - (kc[i] < 8 ? kc[i] : 8) * (ldb < 8 ? (int)ldb : 8);
+      return !TRANS_B && i >= kA && ahead > 0 ? ahead : 0;
+    };
+    auto fetch = [&](int slab, u32x4 (&to)[kCopies], auto plain, auto first) __attribute__((always_inline)) {
 #pragma unroll
       for (int i = 0; i < kCopies; ++i) {
         if constexpr (decltype(plain)::value) {
@@ -245,12 +253,13 @@ void gemm_few_kernel(const T* __restrict__ A, const T* __restrict__ B, OutT* C, 
         } else {
           const int left = rest_of(K, slab, BK) - kc[i];         // elements or rows before the end of K; from the slab's start on where
                                                                  // eight (one) are left, and before the end of K otherwise
-          if (i < kA || TRANS_B) __builtin_memcpy(&to[i], ptr[i] + (left > 8 ? (int64_t)slab * BK : K - 8 - kc[i]), 16);
-          else __builtin_memcpy(&to[i], ptr[i] + (left > 1 ? (int64_t)slab * BK : K - 1 - kc[i]) * ldb, 16);
+          const int k0 = (int)((unsigned)slab * (unsigned)BK);   // (slabs past the last one: any)
+          if (i < kA || TRANS_B) __builtin_memcpy(&to[i], ptr[i] + (left > 8 ? k0 : K - 8 - kc[i]), 16);
+          else __builtin_memcpy(&to[i], ptr[i] + (int64_t)(left > 1 ? k0 : K - 1 - kc[i]) * ldb + (decltype(first)::value ? ahead_of(i) : 0), 16);
         }
       }
     };
-    auto put = [&](const u32x4 (&from)[kCopies], int slab, int stage, auto plain) __attribute__((always_inline)) {
+    auto put = [&](const u32x4 (&from)[kCopies], int slab, int stage, auto plain, auto first) __attribute__((always_inline)) {
       char* to = lds + stage * kStageBytes + threadIdx.x * 16;
 #pragma unroll
       for (int i = 0; i < kCopies; ++i) {
@@ -258,7 +267,7 @@ void gemm_few_kernel(const T* __restrict__ A, const T* __restrict__ B, OutT* C, 
         if constexpr (!decltype(plain)::value) {
           const int left = rest_of(K, slab, BK) - kc[i];
           const u32x4 zero = {0u, 0u, 0u, 0u};
-          v = shift_columns(v, zero, i < kA || TRANS_B ? (left < 8 ? 8 - left : 0) & 7 : by[i]);
+          v = shift_columns(v, zero, i < kA || TRANS_B ? (left < 8 ? 8 - left : 0) & 7 : by[i] - (decltype(first)::value ? ahead_of(i) : 0));
           v = left > 0 ? v : zero;
         }
         *reinterpret_cast<u32x4*>(to + (i < kA ? i * kThreads * 16 : BM * BK * 2 + (i - kA) * kThreads * 16)) = v;
@@ -271,35 +280,44 @@ void gemm_few_kernel(const T* __restrict__ A, const T* __restrict__ B, OutT* C, 
       asm volatile("" ::: "memory");
       HEXMI_FENCE;
     };
-    if (K < 8 || (!TRANS_B && N < 8)) {                          // less than a chunk: by elements
-#pragma unroll 1
-      for (int slab = 0; slab < slabs; ++slab) {
-        __syncthreads();
-#pragma unroll 1
-        for (int e = threadIdx.x; e < (BM + BN) * BK; e += kThreads) {
-          const bool a = e < BM * BK;
-          const int q = a ? e : e - BM * BK;
-          unsigned short v = 0;
-          if (a || TRANS_B) {
-            const int row = q / BK, k = ((q % BK / 8) ^ swz_row<BK>(row)) * 8 + q % 8;
-            const T* base = (a ? A + (int64_t)m0 * lda : B + (int64_t)n0 * ldb) + (int64_t)slab * BK;
-            if (k < rest_of(K, slab, BK) && row < (a ? M - m0 : N - n0)) v = reinterpret_cast<const unsigned short*>(base)[row * (a ? lda : ldb) + k];
-          } else {
-            const int row = q / BN, col = n0 + ((q % BN / 8) ^ swz_col<BN>(row)) * 8 + q % 8;
-            if (row < rest_of(K, slab, BK) && col < N) v = reinterpret_cast<const unsigned short*>(B)[((int64_t)slab * BK + row) * ldb + col];
-          }
-          reinterpret_cast<unsigned short*>(lds)[e] = v;
-        }
-        __syncthreads();
+    if (K < 8) {                                                 // rows of A shorter than a chunk: chunk 0 by elements, zeros for the rest
+      if (K > 0) {
+        typedef unsigned short E;
+        constexpr int kLoadsA = (BM * 8 + kThreads - 1) / kThreads, kLoadsB = (BN * 8 + kThreads - 1) / kThreads;
+        E va[kLoadsA], vb[kLoadsB];
+        const int last_m = M - m0 - 1, last_n = N - n0 - 1;
 #pragma unroll
-        for (int st = 0; st < S::STEPS; ++st) {
-          Step f;
-          read(0, st, f);
-          multiply(f);
+        for (int t = 0; t < kLoadsA; ++t) {
+          const int e = threadIdx.x + t * kThreads, row = e / 8, k = e % 8;
+          va[t] = reinterpret_cast<const E*>(A)[(int64_t)(m0 + (row < last_m ? row : last_m)) * lda + (k < K ? k : K - 1)];
         }
+#pragma unroll
+        for (int t = 0; t < kLoadsB; ++t) {
+          const int e = threadIdx.x + t * kThreads, n = TRANS_B ? e / 8 : e % BN, k = TRANS_B ? e % 8 : e / BN;
+          const int64_t gn = n0 + (n < last_n ? n : last_n), gk = k < K ? k : K - 1;
+          vb[t] = reinterpret_cast<const E*>(B)[TRANS_B ? gn * ldb + gk : gk * ldb + gn];
+        }
+        for (int e = threadIdx.x; e < kStageBytes / 16; e += kThreads) reinterpret_cast<u32x4*>(lds)[e] = u32x4{0u, 0u, 0u, 0u};
+        __syncthreads();
+        E* st = reinterpret_cast<E*>(lds);
+#pragma unroll
+        for (int t = 0; t < kLoadsA; ++t) {
+          const int e = threadIdx.x + t * kThreads, row = e / 8, k = e % 8;
+          if (row < BM && k < K) st[row * BK + swz_row<BK>(row) * 8 + k] = va[t];
+        }
+#pragma unroll
+        for (int t = 0; t < kLoadsB; ++t) {
+          const int e = threadIdx.x + t * kThreads, n = TRANS_B ? e / 8 : e % BN, k = TRANS_B ? e % 8 : e / BN;
+          if (n < BN && k < K)
+            st[BM * BK + (TRANS_B ? n * BK + swz_row<BK>(n) * 8 + k : k * BN + ((n / 8) ^ swz_col<BN>(k)) * 8 + n % 8)] = vb[t];
+        }
+        __syncthreads();
+        Step f;                                                  // (the slab's second step would multiply zeros)
+        read(0, 0, f);
+        multiply(f);
       }
     } else {
-      constexpr std::true_type kPlain{};
+      constexpr std::true_type kPlain{}, kFirst{};
       constexpr std::false_type kAny{};
       // slab j from its stage; slab j + 1 from its set into the other stage, which slab j - 1 has left; the next slab into that set
       auto turn = [&](int j, int stage, u32x4 (&next)[kCopies], auto plain) __attribute__((always_inline)) {
@@ -309,17 +327,17 @@ void gemm_few_kernel(const T* __restrict__ A, const T* __restrict__ B, OutT* C, 
           Step f;
           read(stage, st, f);
           if (st == 0) {
-            put(next, j + 1, stage ^ 1, plain);
-            fetch(j + 1 + kSets, next, plain);
+            put(next, j + 1, stage ^ 1, plain, kAny);
+            fetch(j + 1 + kSets, next, plain, kAny);
             HEXMI_FENCE;
           }
           multiply(f);
         }
       };
-      fetch(0, set[0], kAny);
-      if constexpr (kSets > 1) fetch(1, set[1], kAny);
-      put(set[0], 0, 0, kAny);
-      fetch(kSets, set[0], kAny);
+      fetch(0, set[0], kAny, kFirst);
+      if constexpr (kSets > 1) fetch(1, set[1], kAny, kAny);
+      put(set[0], 0, 0, kAny, kFirst);
+      fetch(kSets, set[0], kAny, kAny);
       int j = 0;
       if (TRANS_B || n0 + BN <= N) {
         const int whole = K / BK;
