@@ -63,17 +63,19 @@ static_assert(rest_of(kAnyMaxK, kAnyMaxK / 256, 256) == kAnyMaxK % 256 && rest_o
 // 16-byte boundaries; otherwise they go by elements.
 // ANY: operand rows at any alignment, any K and N ([K,N] weights with an odd N, views). A copy into LDS needs its 16 bytes on a
 // boundary, a load into registers does not: two slabs are on their way in registers while a third is multiplied from one of two
-// stages. Bound by the latency of a slab's loads as the copies are, so no load waits for a choice: a chunk that reaches past the end of K or
-// of a [K,N] row is read as the last eight elements before it and shifted into place, with zeros behind K, on its way into LDS, in
-// the last slab and the last column of tiles only. Rows of fewer than eight columns are read with the end of the row before (the first of B from
-// its start); fewer than eight of K are one chunk, put together from elements. (By elements throughout, one latency after the other, 65536 x 1
-// x 4096 took 866 us, 65536 x 7 x 768 167 and 4096 x 4096 x 7 36; with 128 x 128 tiles of chunks under branches 203, 57 and 20; here 132, 29 and 13.) Tiles of 128 x 128 have one slab on its way, so that two fit a CU. (128 x 128 tiles that
-// put such chunks together from elements under a branch of every load had their four chunks of a slab one latency after the other, 2 us
-// for 32 of K. [K,N], us, there / here: 128 x 7219 x 6656 299 / 49, 640 x 7031 x 3584 322 / 105, 16 x 4097 x 4096 120 / 19, 50 x 1001 x 768
-// 48 / 6.8, 4000 x 4001 x 2048 160 / 110, 1021 x 50257 x 768 174 / 157; aligned neighbours with copies into LDS take 43, 61, 18, 5, 48 and
-// 102. What alignment itself costs is a tenth to a fifth: rows on the boundaries / off them, [N,K] 128 x 7224 x 6651 37 / 43,
-// [K,N] 44 / 47, 1021 x 50264 x 763 138 / 145. Two slabs on their way
-// in 128 x 128 tiles leave one to a CU: 1021 x 50257 x 768 211, 640 x 7031 x 3584 140.)
+// stages; tiles of 128 x 128 have one slab on its way, so that two fit a CU. Bound by the latency of a slab's loads as the copies are, so
+// no load waits for a choice: a chunk that reaches past the end of K or of a [K,N] row is read as the last eight elements before it and
+// shifted into place, with zeros behind K, on its way into LDS, in the last slab and the last column of tiles only. Rows of fewer than
+// eight columns are read with the end of the row before (the first of B from its start); fewer than eight of K are one chunk, put
+// together from elements. The last turns ask for no slab; the result leaves by up to eight elements of a thread at a time.
+// us on 128 x 128 tiles that put such chunks together from elements under a branch of every load, a slab's one latency after the other /
+// here ([K,N]): 128 x 7219 x 6656 299 / 47, 640 x 7031 x 3584 322 / 74, 16 x 4097 x 4096 120 / 18.5, 50 x 1001 x 768 48 / 5.3, 4000 x
+// 4001 x 2048 160 / 96, 1021 x 50257 x 768 174 / 143; aligned neighbours with copies into LDS take 43, 61, 18, 5, 48 and 102. Few columns
+// or little of K, there / by elements throughout / here: 65536 x 1 x 4096 203 / 866 / 132, 65536 x 7 x 768 57 / 167 / 29, 4096 x 4096 x 7
+// 20 / 36 / 13. Short K on many tiles, there / with slabs of zeros asked for and one element after the other / here: 1021 x 50257 x 64
+// 50 / 73 / 53, 65536 x 257 x 9 21 / 36 / 24, 20000 x 33 x 33 7.7 / 10.5 / 7.0. What alignment itself costs is a tenth to a fifth: rows on
+// the boundaries / off them, [N,K] 128 x 7224 x 6651 37 / 43, [K,N] 44 / 47, 1021 x 50264 x 763 138 / 145. Two slabs on their way in
+// 128 x 128 tiles leave one to a CU: 1021 x 50257 x 768 211, 640 x 7031 x 3584 140.
 template <typename T, typename OutT, typename S, int NS, bool TRANS_B, bool ANY>
 __global__ __launch_bounds__(S::kThreads, S::STEPS == 2 ? 4 : 2)
 void gemm_few_kernel(const T* __restrict__ A, const T* __restrict__ B, OutT* C, int M, int N, int K, int64_t lda, int64_t ldb,
@@ -317,18 +319,23 @@ void gemm_few_kernel(const T* __restrict__ A, const T* __restrict__ B, OutT* C, 
         multiply(f);
       }
     } else {
-      constexpr std::true_type kPlain{}, kFirst{};
+      constexpr std::true_type kPlain{}, kFirst{}, kEnd{};
       constexpr std::false_type kAny{};
-      // slab j from its stage; slab j + 1 from its set into the other stage, which slab j - 1 has left; the next slab into that set
-      auto turn = [&](int j, int stage, u32x4 (&next)[kCopies], auto plain) __attribute__((always_inline)) {
+      // slab j from its stage; slab j + 1 from its set into the other stage, which slab j - 1 has left; the next slab into that set.
+      // kEnd: the last turns, nothing further to ask for
+      auto turn = [&](int j, int stage, u32x4 (&next)[kCopies], auto plain, auto end) __attribute__((always_inline)) {
         meet();
 #pragma unroll
         for (int st = 0; st < S::STEPS; ++st) {
           Step f;
           read(stage, st, f);
           if (st == 0) {
-            put(next, j + 1, stage ^ 1, plain, kAny);
-            fetch(j + 1 + kSets, next, plain, kAny);
+            if constexpr (decltype(end)::value) {
+              if (j + 1 < slabs) put(next, j + 1, stage ^ 1, kAny, kAny);
+            } else {
+              put(next, j + 1, stage ^ 1, plain, kAny);
+              fetch(j + 1 + kSets, next, plain, kAny);
+            }
             HEXMI_FENCE;
           }
           multiply(f);
@@ -337,19 +344,24 @@ void gemm_few_kernel(const T* __restrict__ A, const T* __restrict__ B, OutT* C, 
       fetch(0, set[0], kAny, kFirst);
       if constexpr (kSets > 1) fetch(1, set[1], kAny, kAny);
       put(set[0], 0, 0, kAny, kFirst);
-      fetch(kSets, set[0], kAny, kAny);
       int j = 0;
-      if (TRANS_B || n0 + BN <= N) {
-        const int whole = K / BK;
-        for (; j + 2 + kSets < whole; j += 2) {
-          turn(j, 0, set[kSets - 1], kPlain);
-          turn(j + 1, 1, set[0], kPlain);
+      if (slabs > kSets) {
+        fetch(kSets, set[0], kAny, kAny);
+        if (TRANS_B || n0 + BN <= N) {
+          const int whole = K / BK;
+          for (; j + 2 + kSets < whole; j += 2) {
+            turn(j, 0, set[kSets - 1], kPlain, kAny);
+            turn(j + 1, 1, set[0], kPlain, kAny);
+          }
+        }
+        for (; slabs - j > kSets + 1; j += 2) {                  // (the last slab but one: zeros asked for that no turn takes)
+          turn(j, 0, set[kSets - 1], kAny, kAny);
+          turn(j + 1, 1, set[0], kAny, kAny);
         }
       }
-      for (; j < slabs; j += 2) {                                // (one slab of zeros where their number is odd)
-        turn(j, 0, set[kSets - 1], kAny);
-        turn(j + 1, 1, set[0], kAny);
-      }
+      turn(j, 0, set[kSets - 1], kAny, kEnd);
+      if (j + 1 < slabs) turn(j + 1, 1, set[0], kAny, kEnd);
+      if (kSets > 1 && j + 2 < slabs) turn(j + 2, 0, set[kSets - 1], kAny, kEnd);
     }
   } else {
     HEXMI_FENCE;
@@ -418,16 +430,34 @@ void gemm_few_kernel(const T* __restrict__ A, const T* __restrict__ B, OutT* C, 
       if (m0 + row < M && n0 + col < N) *reinterpret_cast<Run*>(C + (int64_t)(m0 + row) * ldc + n0 + col) = out;
     }
   } else {
-    // (a residual that is the output itself: an element is read and written by one thread)
-    for (int idx = threadIdx.x; idx < BM * BN; idx += kThreads) {
-      const int row = idx / BN, col = idx % BN;
-      if (m0 + row >= M || n0 + col >= N) continue;
-      float v = 0.f;
+    // By elements, up to eight of a thread at a time. (A residual that is the output itself: an element is read and written by one thread.)
+    constexpr int kEach = (BM * BN + kThreads - 1) / kThreads, kAtOnce = kEach % 8 == 0 ? 8 : kEach % 6 == 0 ? 6 : kEach % 4 == 0 ? 4 : kEach;
+    static_assert(kAtOnce <= 8 && (kEach == 1 || kEach * kThreads == BM * BN), "whole groups");
+#pragma unroll 1
+    for (int base = threadIdx.x; base < BM * BN; base += kAtOnce * kThreads) {
+      float v[kAtOnce];
 #pragma unroll
-      for (int h = 0; h < KH; ++h) v += red[(h * BM + row) * kPitch + col];
-      if (bias) v += to_f32<OutT>(bias[n0 + col]);
-      if (resid) v += to_f32<OutT>(resid[(int64_t)(m0 + row) * ldr + n0 + col]);
-      C[(int64_t)(m0 + row) * ldc + n0 + col] = from_f32<OutT>(v);
+      for (int u = 0; u < kAtOnce; ++u) {
+        const int idx = base + u * kThreads;
+        v[u] = 0.f;
+#pragma unroll
+        for (int h = 0; h < KH; ++h) v[u] += red[(h * BM + idx / BN) * kPitch + idx % BN];
+      }
+      auto row_of = [&](int u) { const int row = m0 + (base + u * kThreads) / BN; return row < M ? row : M - 1; };
+      auto col_of = [&](int u) { const int col = n0 + (base + u * kThreads) % BN; return col < N ? col : N - 1; };
+      if (bias) {
+#pragma unroll
+        for (int u = 0; u < kAtOnce; ++u) v[u] += to_f32<OutT>(bias[col_of(u)]);
+      }
+      if (resid) {
+#pragma unroll
+        for (int u = 0; u < kAtOnce; ++u) v[u] += to_f32<OutT>(resid[(int64_t)row_of(u) * ldr + col_of(u)]);
+      }
+#pragma unroll
+      for (int u = 0; u < kAtOnce; ++u) {
+        const int idx = base + u * kThreads, row = m0 + idx / BN, col = n0 + idx % BN;
+        if (row < M && col < N) C[(int64_t)row * ldc + col] = from_f32<OutT>(v[u]);
+      }
     }
   }
 }

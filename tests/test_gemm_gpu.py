@@ -405,7 +405,8 @@ def test_gemm_few_rows_the_weight_stream_leaves(hexmi, dtype, M, N, K):
     (300, 3001, 129), (1000, 1001, 1000), (1900, 1023, 333),                                                    # 64 x 64, 128 x 64
     (2100, 2049, 63), (2049, 2050, 193), (2177, 2191, 256), (70, 33001, 65), (33025, 129, 127),                 # 128 x 128
     (300, 7, 8), (64, 1, 9), (8, 6, 15), (200, 2, 4096), (1000, 3, 511), (9000, 1, 1030), (33000, 4, 130),      # fewer than eight columns,
-    (4096, 5, 64), (16, 300, 2), (300, 300, 1), (3000, 100, 6), (33000, 130, 7), (70000, 1, 5)])                # or of K
+    (4096, 5, 64), (16, 300, 2), (300, 300, 1), (3000, 100, 6), (33000, 130, 7), (70000, 1, 5),                 # or of K
+    (40, 65, 511), (40, 65, 513), (40, 65, 769), (40, 65, 1023), (40, 65, 1025), (33025, 5, 129), (33025, 5, 257)])    # one to five slabs
 def test_gemm_operand_rows_off_the_boundaries(hexmi, dtype, out_dtype, trans_b, M, N, K):
     _against_double(hexmi, dtype, out_dtype, trans_b, M, N, K, False, False, M + N + K)
     _against_double(hexmi, dtype, out_dtype, trans_b, M, N, K, True, True, M + N + K + 1)
