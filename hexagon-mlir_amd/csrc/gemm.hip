@@ -1591,14 +1591,22 @@ int dispatch_gemm(const void* Av, const void* Bv, void* Cv, int64_t M, int64_t N
     if (plan.channels > 0)
       return launch_gemm_skinny<T, OutT>(plan, A, B, C, M, N, K, lda, ldb, ldc, s, bias, resid, ldr);
   }
-  // 16-bit results: the tiles between 128 x 128 and 256 x 256; of output rows off the boundaries those that the paired-slab kernels leave
+  // the output (and bias and residual) in runs of four columns
+  const bool fours = N % 4 == 0 && N >= 4 && ldc % 4 == 0 && aligned_to(C, run) && (!bias || aligned_to(bias, run)) &&
+                     (!resid || (aligned_to(resid, run) && ldr % 4 == 0));
+  // 16-bit results: the tiles between 128 x 128 and 256 x 256; of output rows off the boundaries those that the paired-slab kernels leave,
+  // from the K on where that is ahead of the 32-k slabs of 128 x 128 below, whose rows leave in pieces of 16 bytes: with a residual, or a bias
+  // off the runs of four, at any K; a bias in runs of four from 128 (3000 x 3004, us: K = 40 17 / 21, 120 21 / 20.6, 328 30 / 26; 20000 x 500
+  // K = 200 0.91 times the rate, 328 1.03); neither from 320 (3000 x 3001: K = 40 16.7 / 22.4, 200 0.95, 328 1.09; 2100 x 5003 K = 328 0.93,
+  // 584 1.02; 1021 x 50257 K = 40 56 / 63, 120 1.05).
   if constexpr (std::is_same<T, OutT>::value) {
     const bool aligned = N % 8 == 0 && ldc % 8 == 0 && aligned_to(C, 16) && (!bias || aligned_to(bias, run)) &&
                          (!resid || (aligned_to(resid, run) && ldr % 4 == 0));
-    const bool whole = K % BK2 == 0, odd = TRANS_B && !aligned && (bias || resid || !whole);
+    const int from = resid || (bias && !fours) ? 0 : bias ? 128 : 320;
+    const bool whole = K % BK2 == 0, odd = TRANS_B && !aligned && (bias || resid || !whole) && K >= from;
     if (chunks && (aligned || odd) && lda < (1 << 21) && ldb < (1 << 21) && K <= (1 << 30)) {
       const int now = odd || !whole ? 0 : large ? 256 : two_per_cu(((M + 127) / 128) * ((N + 127) / 128), K) ? 2 : 1;
-      const GemmMidTile mid = plan_gemm_mid(M, N, K, now, resid != nullptr);
+      const GemmMidTile mid = plan_gemm_mid(M, N, K, now, resid != nullptr, odd);
       if (mid.m) return launch_gemm_mid<T, TRANS_B>(mid, A, B, C, M, N, K, lda, ldb, ldc, s, bias, resid, ldr, odd);
     }
   }
@@ -1618,13 +1626,11 @@ int dispatch_gemm(const void* Av, const void* Bv, void* Cv, int64_t M, int64_t N
     return launch_tiled<T, OutT, 2, 2, TRANS_B>(A, B, C, M, N, K, lda, ldb, ldc, s, nullptr, nullptr, 0, 1);
   }
   if (chunks) {
-    const bool runs = N % 4 == 0 && N >= 4 && ldc % 4 == 0 && aligned_to(C, run) && (!bias || aligned_to(bias, run)) &&
-                      (!resid || (aligned_to(resid, run) && ldr % 4 == 0));
     const int64_t tiles_m = (M + 127) / 128, tiles_n = (N + 127) / 128;
     if (tiles_m * tiles_n > 0x7fffffff) return HEXMI_ENOTSUP;
     hipLaunchKernelGGL((gemm_kernel<T, OutT, 2, 2, TRANS_B, true, false, 2, true, true>), dim3((unsigned)(tiles_m * tiles_n)),
                        dim3(256), 0, s, A, B, C, (int)M, (int)N, (int)K, lda, ldb, ldc, (int)tiles_m, (int)tiles_n, nullptr,
-                       bias, resid, ldr, runs ? 1 : 0);
+                       bias, resid, ldr, fours ? 1 : 0);
     return launch_status();
   }
   return launch_gemm_any<T, OutT, TRANS_B>(A, B, C, M, N, K, lda, ldb, ldc, s, bias, resid, ldr);

@@ -335,13 +335,18 @@ static constexpr MidCost kOne = {128, 128, 1, 4.0, 0.445, 0.073, 1.9, 0.0, 3.9},
 // bias or residual, for which the 256 x 256 tiles have no registers. K off whole 64s comes here always. us on 128 x 128 or 256 x 256 tiles /
 // here: 1336 x 6400 x 1600 + bias 53 / 30 (192 x 192), 3787 x 1712 x 2920 + residual 77 / 49, 5712 x 3200 x 1576 + bias 127 / 65, 1291 x 3096 x 2552
 // + bias 57 / 33, 862 x 11144 x 1216 + bias 35 / 29, 2206 x 3896 x 1344 36 / 27, 645 x 12456 x 6560 202 / 135; all 370: 1.11 times the rate,
-// K off whole 64s 1.49. A twentieth's lead is asked for, since the fits are that good: without it one in ten is slower.
-GemmMidTile plan_gemm_mid(int64_t M, int64_t N, int64_t K, int now, bool resid) {
+// K off whole 64s 1.49. A twentieth's lead is asked for, since the fits are that good: without it one in ten is slower. With it, of 200 other
+// products of whole 64s and of 8s 82 of whole 64s came here, at 1.13 times the rate, five of them 5 to 10 % slower than before (1636 x 21440 x
+// 1408 + both 122 / 135, 4480 x 3840 x 320 + bias 26.2 / 27.5).
+// Odd rows of less than 1024 of K: the larger tiles' elements leave with nothing beside them, so two of 128 x 128 to a CU (or one), us on the
+// 32-k slabs of gemm.hip / the tile of the fit / here: 8000 x 10001 x 456 151 / 205 / 143, 3000 x 15003 x 584 114 / 148 / 106, 6000 x 3333 x 584
+// 61 / 66 / 55, 4000 x 2500 x 584 34.5 / 40 / 33.5 (3000 x 3001 x 776 42 / 34 / 39); from 1024 on the fit is ahead.
+GemmMidTile plan_gemm_mid(int64_t M, int64_t N, int64_t K, int now, bool resid, bool odd) {
   const MidCost* best = nullptr;
   double least = now == 0 ? 1e30 : 0.95 * mid_time(now == 256 ? kLarge : now == 2 ? kTwo : kOne, M, N, K, resid);
   for (const MidCost& c : kMidTiles) {
     if (now != 0 && c.m == 128) continue;                    // (gemm.hip's own are the better ones of whole slabs)
-    if (resid && c.m * c.n > 192 * 192) continue;
+    if ((resid && c.m * c.n > 192 * 192) || (odd && K < 1024 && c.m > 128)) continue;
     if (!grid_fits(((M + c.m - 1) / c.m) * ((N + c.n - 1) / c.n), 256)) continue;
     const double t = mid_time(c, M, N, K, resid);
     if (t < least) least = t, best = &c;

@@ -302,7 +302,7 @@ int launch_gemm_any(const T* A, const T* B, OutT* C, int64_t M, int64_t N, int64
 // boundaries too, in whole runs of eight columns, bias and residual on 8-byte ones, or, odd (B as [N,K]), any of them anywhere. now: what takes the call otherwise, 256 x 256 tiles
 // (256), 128 x 128 two (2) or one (1) to a CU, or nothing of that rate (0).
 struct GemmMidTile { int m, n, per_cu; };
-GemmMidTile plan_gemm_mid(int64_t M, int64_t N, int64_t K, int now, bool resid);
+GemmMidTile plan_gemm_mid(int64_t M, int64_t N, int64_t K, int now, bool resid, bool odd);
 template <typename T, bool TRANS_B>
 int launch_gemm_mid(const GemmMidTile& tile, const T* A, const T* B, T* C, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb,
                     int64_t ldc, hipStream_t s, const T* bias, const T* resid, int64_t ldr, bool odd);

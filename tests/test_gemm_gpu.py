@@ -362,7 +362,9 @@ def test_gemm_tiles_between_128_and_256(hexmi, dtype, trans_b, M, N, K, bias, re
 @pytest.mark.parametrize("M,N,K,bias,residual", [
     (1025, 4097, 8, False, False), (2049, 1097, 72, True, True), (482, 4069, 1024, True, True), (2177, 1033, 136, False, True),   # 128 x 128
     (2049, 1095, 1000, True, False), (1345, 6215, 1608, False, True), (1300, 6401, 1600, True, False), (1300, 6401, 1600, False, True),
-    (700, 9001, 1000, False, True), (645, 12457, 704, True, False), (1009, 24001, 328, True, False)])
+    (700, 9001, 1000, False, True), (645, 12457, 704, True, False), (1009, 24001, 328, True, False),
+    (2049, 1097, 312, False, False), (2049, 1097, 328, False, False), (1345, 6215, 1016, False, False), (1345, 6215, 1032, False, False),
+    (2049, 1100, 120, True, False), (2049, 1100, 136, True, False), (2049, 1100, 40, False, True)])    # the lines of K; runs of four
 def test_gemm_tiles_between_128_and_256_odd_rows(hexmi, dtype, M, N, K, bias, residual):
     _against_double(hexmi, dtype, dtype, True, M, N, K, bias, residual, M + N + K)
     # an output one element off in rows three longer, the residual the output itself, nothing written around it
