@@ -529,7 +529,10 @@ void gemm_merge_kernel(const float* __restrict__ sums, OutT* C, int M, int N, in
 //   25.2, 26.8) nor where tiles of 32 columns and more leave three eighths of the CUs without one (3 x 4192 x 3560 9.8, 11.5;
 //   4 x 9527 x 6416 28, 33);
 //   up to sixteen rows, half of a tile of 32 x 64 (weight stream): 16 x 14336 x 4096 22.8, 25.8 / 22.4, 24.9; 10 x 8666 x 10432 41.4, 45.1 /
-//   41.6, 45.2; 13 x 11368 x 1664 11.7, 12.2 / 8.0, 8.8 (16 x 11008 x 4096 18.9, 20.7 / 19.1, 18.0); or tiles of 16 x 16 for fewer than half
+//   41.6, 45.2; 13 x 11368 x 1664 11.7, 12.2 / 8.0, 8.8 (16 x 11008 x 4096 18.9, 20.7 / 19.1, 18.0); up to 24 of the 64 of a tile of 64 x
+//   96 (weights from HBM: 9 x 20000 x 4096 29.4, 37.4; 16 x 24576 x 512 7.8, 8.6; 16 x 16400 x 1408 11.9, 13.7; 17 x 24576 x 4096 38.6,
+//   42.3; 24 x 24576 x 1408 14.7, 16.5; 24 x 17856 x 4096 36.2, 34.6; 32 rows 39.3, 35.7 at 20000 x 4096, 42.5, 46.2 at
+//   24576); or tiles of 16 x 16 for fewer than half
 //   of the CUs: 9 x 1208 x 15232 17.9, 17.9 / 11.2, 13.8; 12 x 1422 x 9408 13.2, 13.2 / 8.5, 9.4;
 //   up to 32 rows, up to sixteen channels per CU, weights of 3 * 2^24 elements and more (weight stream): 16 x 4096 x 14336 25.3, 27.2 / 24.5,
 //   26.1; 17 x 4096 x 12288 23.2, 25.8 / 23.1, 25.8; 32 x 4096 x 12288 29.4, 31.4 / 29.3, 31.2 -- unless its rows stand a power of two
@@ -553,7 +556,8 @@ GemmFewTile plan_gemm_few(bool trans_b, int64_t M, int64_t N, int64_t K) {
     const int64_t count = ((M + t.m - 1) / t.m) * ((N + t.n - 1) / t.n);
     if (count > cus) continue;
     if (dots && M <= 4 && (N * K >= (int64_t)3 << 24 || (t.n > 16 && 8 * count < 5 * cus))) return {0, 0};
-    if (stream && M <= 16 && (t.n == 64 || (t.n == 16 && 2 * count < cus))) return {0, 0};
+    if (stream && M <= 16 && (t.n >= 64 || (t.n == 16 && 2 * count < cus))) return {0, 0};
+    if (stream && M <= 24 && t.n > 64) return {0, 0};
     const bool narrow = stream && M <= 32 && t.m == 16 && N <= 16 * cus;    // a channel group of sixteen per CU at most
     if (narrow && M > 16 && M <= 24 && t.n == 32 && N * K < (int64_t)1 << 25) return {0, 0};
     if (narrow && N * K >= (int64_t)3 << 24 && (K & (K - 1)) != 0) return {0, 0};
