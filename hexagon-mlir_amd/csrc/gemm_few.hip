@@ -508,9 +508,11 @@ void gemm_merge_kernel(const float* __restrict__ sums, OutT* C, int M, int N, in
 // and 1.07 times the rate over 60 and 25 products, none slower. 48 x 32 before 32 x 64, [N,K]: 92 x 3304 x 8832 33 / 27.6, 687 x 400 x 3680 13.2 / 11.6,
 // level or a few hundredths slower below K of about 1000 and against [K,N] weights (1149 x 320 x 2752 10.5 / 11.4). 48 x 64 with two stages of 256 of K loses 10 % to 64 x 64.)
 // (96 x 96 asks for what 128 x 64 does, an eighth more of C to a tile; us on 128 x 128 tiles two to a CU or one / here: 1336 x 1600 x 1600
-// 20.2 / 16.2, 330 x 5672 x 7232 72 / 56, 3209 x 592 x 9064 101 / 71, 165 x 8632 x 1984 19.7 / 15.2, 189 x 9704 x 384 10.2 / 8.1; 1.15 times
-// the rate over 56 products, two of them slower: 77 x 17216 x 3840 27.6 / 28.6, 1510 x 1512 x 6912 48 / 58. 128 x 128 on eight waves: equal
-// to gemm.hip's.)
+// 20.2 / 16.2, 330 x 5672 x 7232 72 / 56, 3209 x 592 x 9064 101 / 71, 165 x 8632 x 1984 19.7 / 15.2, 189 x 9704 x 384 10.2 / 8.1, 1510 x 1512 x
+// 6912 64 / 47 ([K,N] 70 / 58); 1.23 times the rate over 310 products. Not where K is three or four whole slabs of 64, which those tiles ask for
+// at once: 2176 x 1024 x 256 6.2 / 6.8, 640 x 3456 x 256 6.4 / 7.0, 96 x 22848 x 192 6.7 / 7.1; nor, with odd rows, which leave by elements here,
+// up to 512: 544 x 3484 x 192 + residual 12.6 / 13.7, 848 x 2542 x 192 8.1 / 8.8, 320 x 5529 x 448 9.5 / 10.1. Of the others two are slower: 288 x
+// 6656 x 12416 [K,N] 98 / 109, 73 x 22656 x 512 9.2 / 9.8. 128 x 128 on eight waves: equal to gemm.hip's.)
 // The smallest tile of which there is at most one per CU (more tiles than CUs: a second round, at the same intake per CU as a tile of
 // twice the area; over 250 random products of up to 2000 rows no other tile was more than 6 % ahead of this choice but where K < 128),
 // none where even 128 x 64 and 96 x 96 are more. us for 128 x 64 / 64 x 64 / 32 x 64 / 32 x 32 tiles (how many), K = 3072 [K,N]: N = 768, 2000 rows
@@ -552,6 +554,7 @@ GemmFewTile plan_gemm_few(bool trans_b, int64_t M, int64_t N, int64_t K) {
   static constexpr GemmFewTile kTiles[] = {{16, 16}, {16, 32}, {32, 32}, {48, 32}, {32, 64}, {64, 64}, {64, 96}, {96, 64}, {128, 64}, {96, 96}};
   for (const GemmFewTile& t : kTiles) {
     if (t.m == 48 && (K < 1024 || !trans_b)) continue;
+    if (t.m == 96 && t.n == 96 && K % 64 == 0 && (N % 8 == 0 ? K > 128 && K <= 256 : K <= 512)) continue;
     if (t.n == 16 && !trans_b) continue;                         // sixteen columns of a row of B are a quarter of a line
     const int64_t count = ((M + t.m - 1) / t.m) * ((N + t.n - 1) / t.n);
     if (count > cus) continue;
