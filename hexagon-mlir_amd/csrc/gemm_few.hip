@@ -639,15 +639,20 @@ int launch_gemm_few(const GemmFewTile& tile, const T* A, const T* B, OutT* C, in
 // 4096 19.7 / 13.2, 16 x 8192 x 11008 53 / 39, 32 x 2048 x 11008 44 / 15.6, 64 x 4096 x 4096 20.9 / 15.7, 113 x 304 x 11968 22.7 / 11.6, 256 x
 // 1024 x 11008 47 / 24, 512 x 512 x 8192 22.9 / 19.4. Below these lines the second launch costs what the parts give: 16 x 4096 x 2048 7.8 / 8.7,
 // 64 x 768 x 3072 8.3 / 8.8, 11 x 7296 x 3200 15.4 / 16.7, 58 x 1408 x 4352 10.7 / 11.7; 1.22 times the rate over 110 products of K = 3072 on.
-// Tiles of [N,K] weights come in whole lines and are ahead or behind by a tenth at K of about 10000 (64 x 4096 x 4096 13.0 / 14.1,
-// 512 x 512 x 8192 14.4 / 18.9, 64 x 512 x 10240 10.3 / 11.9, 128 x 2048 x 10240 26 / 22; 64 x 4096 x 11008 33 / 26, 256 x 1024 x 11008 26 / 21,
-// 128 x 1024 x 12288 28.9 / 15.8, 32 x 2048 x 11008 17.7 / 15.0, 32 x 4096 x 11008 21.6 / 21.4).
+// Tiles of [N,K] weights come in whole lines (64 x 4096 x 4096 13.0 / 14.1, 512 x 512 x 8192 14.4 / 18.9), and as a whole the product has
+// tiles of 16 x 16 to 32 x 64 on all CUs, whose operands pass from one to the next through L2 while all of them fit: parts are ahead from
+// 19 MiB of operands on, and from K = 12800 on, where the walk is what is long. Rate in parts over that as a whole, 430 products of 33 to 600
+// rows and K = 9216 to 18944, by millions of (M + N) K: up to 8 0.98, to 9 1.00, to 10.5 1.09, to 12 1.24, to 15 1.26, beyond 1.29; with less than
+// 10.5, K of 12800 and more 1.12; K = 8192 0.94 (64 x 4096 x 11008 33 / 26, 128 x 1024 x 12288 28.9 / 15.8, 128 x 2048 x 10240 26 / 22, 40 x 2048 x 10240
+// 20.2 / 15.1; 64 x 512 x 10240 10.3 / 11.9, 453 x 400 x 9344 16.4 / 18.0). Up to 32 rows the whole has few tiles: 8704 1.03, 9728 1.13, 11008 1.16,
+// 12288 1.32; in fewer than eight parts a tenth ahead or level (32 x 4096 x 11008 21.6 / 21.4) for a second launch, so as a whole.
 // [K,N] weights whose rows stand off the boundaries, whole / in parts: 16 x 2027 x 12144 47 / 19, 128 x 1175 x 11904 49 / 24, 3 x 485 x 8704 20.6 / 11.4, 128 x
 // 2250 x 5312 28.9 / 19.9, 15 x 1601 x 4352 13.8 / 11.8, 2 x 405 x 3136 10.9 / 11.3; 1.45 times the rate over 44 (up to 16 rows parts of 256 and
 // more: a slab through registers is a latency; with 512 and more 2 x 1497 x 4512 13.2 / 13.8, with 256 and more at 64 rows 90 x 318 x 11584 13.3 -> 15.5).
 // Up to 16 rows of more than 1024 columns tiles of 128 columns: 16 x 2560 x 11376 23.0 on 64 columns, 20.2; 1 x 1024 x 11376 11.5, 12.6.
 GemmParts plan_gemm_parts(bool trans_b, int64_t M, int64_t N, int64_t K, bool any) {
-  if (trans_b ? K < 11008 || M <= 16 : M <= 32 ? K < 3072 || K < N : K < 4608) return {};
+  if (trans_b ? M <= 16 || K < (M <= 32 ? 9728 : 9216) : M <= 32 ? K < 3072 || K < N : K < 4608) return {};
+  if (trans_b && M > 32 && K < 12800 && (M + N) * K < 19 << 19) return {};
   const GemmFewTile t = M <= 16 ? GemmFewTile{16, N <= 1024 || any ? 64 : 128} : GemmFewTile{M <= 32 ? 32 : 64, 64};
   const int64_t tiles = ((M + t.m - 1) / t.m) * ((N + t.n - 1) / t.n);
   const int64_t parts = std::min(hexmi_num_cus() / std::max<int64_t>(tiles, 1), K / (any && M <= 16 ? 256 : 512));

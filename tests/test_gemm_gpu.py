@@ -271,6 +271,8 @@ def test_gemm_one_round_of_tiles(hexmi, dtype, out_dtype, trans_b, M, N, K):
     (17, 2047, 11008, True, True), (64, 4097, 11008, True, True), (255, 1030, 11016, True, True),
     (16, 4104, 4096, False, False), (16, 11008, 11376, False, False), (64, 768, 4096, False, False), (16, 1024, 11008, True, False),
     (64, 4096, 8192, True, False), (32, 4096, 11008, True, False),
+    (128, 1032, 9216, True, True), (128, 1032, 9208, True, False), (64, 700, 12800, True, True), (64, 700, 12792, True, False),
+    (24, 1000, 9728, True, True), (24, 1000, 9720, True, False),                                             # the lines of [N,K]
     (8, 1001, 4096, False, True), (16, 4097, 4100, False, True), (1, 3, 3075, False, True), (31, 2049, 5001, False, True),   # rows off the
     (128, 531, 9736, False, True), (64, 1024, 4611, False, True), (64, 2047, 11009, True, False)])                          # boundaries
 def test_gemm_parts_of_a_long_k(hexmi, dtype, out_dtype, M, N, K, trans_b, parts):
