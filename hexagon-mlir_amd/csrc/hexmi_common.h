@@ -315,7 +315,7 @@ int gemm_w8a16_any_shape(int64_t M, int64_t N, int64_t K, const f16* A, const in
 
 // W8A16 of 33 rows and more in one round of tiles over the CUs (w8a16_few.hip): the tile, m == 0 for none, and the launch. K % 16 == 0,
 // A and W on 16-byte boundaries; zero_points may be null. tiles: whether the tiles of gemm.hip are a choice.
-GemmFewTile plan_w8a16_few(int64_t M, int64_t N, int64_t K, bool tiles);
+GemmFewTile plan_w8a16_few(int64_t M, int64_t N, int64_t K, bool tiles, bool zero_points);
 int launch_w8a16_few(const GemmFewTile& tile, int64_t M, int64_t N, int64_t K, const f16* A, const int8_t* W, const f16* scales,
                      const int8_t* zero_points, int per_tensor, f16* C, hipStream_t s);
 

@@ -822,7 +822,7 @@ int gemm_w8a16_any(int64_t M, int64_t N, int64_t K, const void* A, const int8_t*
     return launch_status();
   }
   // three rows and more where the tiles of w8a16_few.hip give every CU a share
-  const GemmFewTile few = plan_w8a16_few(M, N, K, tile_kernel);
+  const GemmFewTile few = plan_w8a16_few(M, N, K, tile_kernel, zp != nullptr);
   if (few.m) return launch_w8a16_few(few, M, N, K, a, W, s, zp, pt, c, st);
   // what is left of more than 128 rows that the 128 x 128 tiles do not take (rows too long for those tiles' offsets): the chunked
   // kernel in passes of 128 rows (130 x 1001 x 4194368 22.5 ms; a workgroup per 16 channels in passes of 64 rows took 34.0)
@@ -914,7 +914,7 @@ bool prefer_split(int64_t M, int64_t N, int64_t K, int cus) {
 // CUs 128 x 2048 x 14336 30.2 / 32.5 and 29.0 / 26.8).
 bool prefer_few(int64_t M, int64_t N, int64_t K) {
   if (K % 16 != 0) return false;
-  const GemmFewTile t = plan_w8a16_few(M, N, K, K % 64 == 0 && N % 8 == 0);
+  const GemmFewTile t = plan_w8a16_few(M, N, K, K % 64 == 0 && N % 8 == 0, false);
   return t.m && !(K > 12288 && 4 * ((M + 31) / 32) * ((N + 63) / 64) <= hexmi_num_cus());
 }
 }  // namespace

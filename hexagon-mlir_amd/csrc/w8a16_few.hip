@@ -303,15 +303,28 @@ template <> struct FewShape<64, 192> { typedef Shape<4, 3, 1, 4, 2, 3> S; };
 // (128 x 128 tiles, 1000 x 4096 x 4096: 35.1, gemm.hip's 34.5. 48 x 32, 16 x 48, 32 x 48, 48 x 96, 96 x 64 and 32 x 128 tiles: nowhere ahead of
 // both neighbours by more than 2 %.)
 // The chunked kernel, a workgroup per CU with all rows and up to 48 channels, reads each weight once: it stays ahead where the weights are
-// what counts (16 x 11008 x 4096 11.9, 12.5 on 16 x 48; 16 x 8192 x 4096 9.9, 10.6; 32 x 10064 x 3328 13.0, 13.9; 40 x 11008 x 4096 16.2, 17.1;
-// 80 x 11008 x 4096 20.6, 22.6) -- unless there are more channels than that (40 x 14336 x 992 10.8, 6.9).
+// what counts (us there / on the tile; 4500 products of 3 to 64 rows, N = 720 to 49152 and K = 512 to 14336):
+//   up to sixteen rows against 24 million of them, or 20 from five rows on: 16 x 11008 x 4096 11.9 / 12.5 (16 x 48), 16 x 3072 x 7872 10.2 / 11.0,
+//   16 x 1984 x 12032 11.9 / 13.0 (3 x 1984 x 11008 1.02 times the rate);
+//   up to 32 rows, tiles of 32 x 32 from K = 4096 on and of 32 x 64 from 1600: 32 x 6144 x 11008 23.3 / 26.0, 32 x 6144 x 4096 10.5 / 11.5,
+//   24 x 12288 x 1920 9.0 / 9.7, 24 x 11136 x 2176 10.2 / 11.3 (K = 3072 level, 8192 1.0);
+//   up to 48 rows tiles of 48 x 64 from 1600 on, up to 64 rows of 32 x 96 from 2048: 40 x 11008 x 4096 16.2 / 17.1, 56 x 11136 x 11008 37.3 / 40.5,
+//   64 x 9216 x 12032 with zero points 41 / 45; up to 112 rows of 64 x 96 and more from 2048: 80 x 11008 x 4096 20.6 / 22.6;
+//   with zero points, which every tile takes from its weights and the chunked kernel once a weight: up to sixteen rows tiles of sixteen
+//   columns from K = 8192 on (16 x 1984 x 12032 12.7 / 13.8), up to 32 rows of 64 from 1600 (16 x 11136 x 2176 9.1 / 10.3, 24 x 5120 x 1920
+//   7.2 / 7.8), up to 48 rows of 32 x 64 from 3072 (48 x 8192 x 11008 0.94); K = 2176 on tiles of 16 x 16 stays a twentieth behind
+// -- unless there are more channels than that (40 x 14336 x 992 10.8 / 6.9, 16 x 14336 x 4096 16.9 / 15.0, 16 x 32000 x 5120 1.10, 32 x 32000 x 4096
+// 38 / 32), but for up to sixteen rows where eight ninths and more of the CUs would have a tile of weights whose rows stand whole 4 KiB
+// apart, which then come from the same channels: 8 x 24576 x 4096 21.7 / 25.8, 16 x 32768 x 4096 32.4 / 36.4, 6 x 22016 x 4096 20.5 / 23.0 (24576 x
+// 5120 1.06, 40000 x 4096 1.05).
 // Calls that the tiles of gemm.hip do not take (zero points, K off whole slabs of 64) would go in passes of 128 rows: they come
 // here at any size, with the tile whose rounds cost least (weights: us per 3000 of K measured above; 511 x 10907 x 13056 1238 ->
 // 180, 1000 x 14336 x 992 139 -> 53, 304 x 11008 x 4368 73 -> 60).
-GemmFewTile plan_w8a16_few(int64_t M, int64_t N, int64_t K, bool tiles) {
+GemmFewTile plan_w8a16_few(int64_t M, int64_t N, int64_t K, bool tiles, bool zp) {
   const int64_t cus = hexmi_num_cus();
   if (cus <= 0 || M <= 2 || K > (1 << 22) || M > (1 << 30) || N > (1 << 30)) return {0, 0};
-  const bool chunked = N <= 48 * cus, heavy = N * K >= (24 << 20);       // heavy: the stream of weights is most of the call
+  const bool chunked = N <= 48 * cus, heavy = N * K >= (24 << 20) || (M > 4 && N * K > (20 << 20));    // the stream of
+                                                                 // weights is most of the call
   struct Tile { GemmFewTile tile; int weight; };
   static constexpr Tile kShort[] = {{{16, 16}, 0}, {{16, 32}, 0}, {{16, 64}, 0}, {{32, 32}, 0}};
   static constexpr Tile kLong[] = {{{16, 16}, 0}, {{16, 32}, 0}, {{32, 32}, 0}, {{16, 64}, 0}};
@@ -320,6 +333,8 @@ GemmFewTile plan_w8a16_few(int64_t M, int64_t N, int64_t K, bool tiles) {
   for (const Tile& t : K <= 2048 ? kShort : kLong) {
     if (count(t.tile) > cus) continue;
     if (chunked && heavy && (M <= 16 || (M <= 32 && t.tile.n == 64))) return {0, 0};
+    if (chunked && M <= 32 && t.tile.m == 32 && K > 3072) return {0, 0};
+    if (chunked && zp && ((M <= 16 && t.tile.n == 16 && K >= 8192) || (M <= 32 && t.tile.n == 64 && K > 1536))) return {0, 0};
     return t.tile;
   }
   GemmFewTile best = {0, 0};
@@ -329,7 +344,9 @@ GemmFewTile plan_w8a16_few(int64_t M, int64_t N, int64_t K, bool tiles) {
     if (rounds == 1) {
       const int area = t.tile.m * t.tile.n;
       if (area == 64 * 96 && K > (M <= 192 ? 2048 : 4608)) continue;
-      if (chunked && ((M <= 32 && heavy) || (M <= 48 && area > 32 * 64 && K > 2048) || (M <= 112 && area >= 64 * 96 && K >= 2048))) return {0, 0};
+      if (chunked && ((M <= 32 && K > 1536) || (M <= 48 && (area > 32 * 64 ? K > 1536 : zp && K >= 3072)) ||
+                      (M <= 64 && t.tile.n == 96 && K >= 2048) || (M <= 112 && area >= 64 * 96 && K >= 2048))) return {0, 0};
+      if (M <= 16 && K % 4096 == 0 && 9 * count(t.tile) >= 8 * cus) return {0, 0};
       return t.tile;
     }
     if (!t.weight || tiles || M <= 128 || count(t.tile) > 0x7fffffff) continue;
