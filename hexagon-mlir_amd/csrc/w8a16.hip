@@ -11,6 +11,7 @@
 //
 // Zero points, the asymmetric forms of quant.dcast, f = (float(q) - zero_point) * scale with per-channel or per-tensor parameters:
 // the zero point (an int8, exact in fp16, as is every difference q - zero_point) is subtracted from the widened weights.
+#include "hexmi_calibrate.h"
 #include "hexmi_common.h"
 
 namespace hexmi {
@@ -754,9 +755,59 @@ void w8a16_generic_kernel(const f16* __restrict__ A, const int8_t* __restrict__ 
 using namespace hexmi;
 
 namespace {
-// hexmi_gemm_w8a16 (zp == nullptr, pt == 0) and hexmi_gemm_w8a16_ex: one choice of kernels for both. The decode
+// The chunked kernel's workgroups: channels of one, channel tiles of 16 that hold them, two workgroups to a CU at a time.
+struct MidPlan { int channels, tiles; bool paired; };
+MidPlan plan_mid(int64_t M, int64_t N, int64_t cus) {
+  const int64_t per_cu = (N + cus - 1) / cus;
+  MidPlan plan = {(int)(per_cu < 16 ? 16 : per_cu), 0, false};   // one full tile at least
+  if (per_cu > kMidCh) {
+    // More than a workgroup's 48 channels per CU: equal workgroups in whole rounds over the CUs, not 48 each and
+    // a last round of a few (N = 14336, K = 4096, M = 16: 19.3 us that way). Either one workgroup per CU at a
+    // time, of up to three channel tiles, or, with up to 16 rows, two of up to two tiles each (their LDS fits
+    // twice, so their starts and ends overlap: 14.8 us); whichever copies fewer tile rows, empty ones counted.
+    const int64_t r1 = (per_cu + kMidCh - 1) / kMidCh, c1 = (N + cus * r1 - 1) / (cus * r1);
+    plan.channels = (int)c1;
+    if (M <= 16) {
+      const int64_t r2 = (per_cu + 63) / 64, c2 = (N + cus * 2 * r2 - 1) / (cus * 2 * r2);
+      if (c2 > 16 && r2 * 2 * ((c2 + 15) / 16) <= r1 * ((c1 + 15) / 16)) {
+        plan.channels = (int)c2;
+        plan.paired = true;
+      }
+    }
+  }
+  plan.tiles = (plan.channels + 15) / 16;
+  return plan;
+}
+
+// The kernel of a product: one choice for hexmi_gemm_w8a16 (no zero points, a scale per channel) and hexmi_gemm_w8a16_ex. The decode
 // kernels, the chunked kernel and the tiles of w8a16_few.hip have a zero-point instantiation; the 128 x 128 tile kernel does not, so
 // more than 128 rows with a zero point or a per-tensor scale run on w8a16_few.hip at any size.
+// aligned: A and W on 16-byte boundaries; whole: C on them too, scales on 8-byte ones.
+struct W8Route { int kernel; GemmFewTile few; };
+W8Route route_w8a16(int64_t M, int64_t N, int64_t K, bool zp, bool pt, bool aligned, bool whole) {
+  const bool fits = K % 16 == 0 && aligned;                 // rows of whole 16-byte pieces
+  // two rows over a long K and at least 16 channels per CU go faster through the chunked kernel
+  // (N = 4096, K = 11008: 11.2 against 12.9 us; N = K = 8192: 14.1 against 18.0)
+  const bool chunked_pair = M == 2 && K >= 8192 && K % 64 == 0 && N >= 4096;
+  if (M <= 2 && !chunked_pair && fits && K <= 16384) return {HEXMI_W8A16_DOTS, {0, 0}};
+  // the fast kernels copy 16 bytes of a weight row per lane: K % 16 == 0 and aligned bases; other shapes take the
+  // generic ones, as do rows past the offsets of the others. (K % 64 != 0 runs the chunked kernel or the tiles of w8a16_few.hip.)
+  const bool tile_kernel = !zp && !pt && M > 64 && K % 64 == 0 && N % 8 == 0 && whole;
+  // Enough output for it: 128x128 tiles on the matrix cores, the slabs staged through registers at any alignment
+  // (N = 11008, K = 4040: M = 64 1.43 -> 0.14 ms, M = 1024 22.5 -> 0.23 ms). With few tiles that kernel waits out a
+  // memory latency per slab (about 110 us at K = 4040 whatever the rows), and the elements' kernel, a wave per channel
+  // with lanes striding over k, is ahead while M * N stays small (M = 16: 76 us at N = 4096, 371 at N = 11008).
+  if (!fits || (!tile_kernel && K > (1 << 29))) return {M > 8 && M * N >= 98304 ? HEXMI_W8A16_REGISTERS : HEXMI_W8A16_ELEMENTS, {0, 0}};
+  // three rows and more where the tiles of w8a16_few.hip give every CU a share
+  const GemmFewTile few = plan_w8a16_few(M, N, K, tile_kernel, zp);
+  if (few.m) return {HEXMI_W8A16_TILES, few};
+  // the chunked kernel: any K (a multiple of 16 here). What is left of more than 128 rows that the 128 x 128 tiles do not take (rows too
+  // long for those tiles' offsets) goes through it in passes of 128 rows (130 x 1001 x 4194368 22.5 ms; a workgroup per 16 channels in
+  // passes of 64 rows took 34.0)
+  if (!tile_kernel || (M <= kMidMaxM && K <= (1 << 29))) return {HEXMI_W8A16_CHUNKED, {0, 0}};
+  return {HEXMI_W8A16_LARGE, {0, 0}};
+}
+
 int gemm_w8a16_any(int64_t M, int64_t N, int64_t K, const void* A, const int8_t* W, const void* scales,
                    const int8_t* zp, int pt, void* C, hexmi_stream_t stream) {
   if (M < 0 || N < 0 || K < 0) return HEXMI_EINVAL;
@@ -769,11 +820,9 @@ int gemm_w8a16_any(int64_t M, int64_t N, int64_t K, const void* A, const int8_t*
   f16* c = static_cast<f16*>(C);
   begin_call();
   if (K == 0) return fill_zero_2d(C, M, N, N, 2, st);      // an empty sum
-  // two rows over a long K and at least 16 channels per CU go faster through the chunked kernel further down
-  // (N = 4096, K = 11008: 11.2 against 12.9 us; N = K = 8192: 14.1 against 18.0)
-  const bool chunked_pair = M == 2 && K >= 8192 && K % 64 == 0 && N >= 4096 && aligned_to(A, 16) && aligned_to(W, 16);
-  if (M <= 2 && !chunked_pair && K % 16 == 0 && K <= 16384 && K != 1024 && K != 2048 && K != 4096 && K != 8192 && aligned_to(A, 16) &&
-      aligned_to(W, 16)) {
+  const W8Route route = route_w8a16(M, N, K, zp != nullptr, pt != 0, aligned_to(A, 16) && aligned_to(W, 16),
+                                    aligned_to(C, 16) && aligned_to(scales, 8));
+  if (route.kernel == HEXMI_W8A16_DOTS && K != 1024 && K != 2048 && K != 4096 && K != 8192) {
     // any other row length: the masked form of the same kernel, instantiated per KiB of row
     const unsigned blocks = (unsigned)((N + 15) / 16);
     const int nj = (int)((K + 1023) / 1024);
@@ -791,15 +840,8 @@ int gemm_w8a16_any(int64_t M, int64_t N, int64_t K, const void* A, const int8_t*
 #undef HEXMI_GEMV_ANY
     return launch_status();
   }
-  // the fast kernels copy 16 bytes of a weight row per lane: K % 16 == 0 and aligned bases; other shapes take the
-  // generic one, as do rows past the offsets of the others. (K % 64 != 0 runs the chunked kernel or the tiles of w8a16_few.hip.)
-  const bool tile_kernel = !zp && !pt && M > 64 && K % 64 == 0 && N % 8 == 0 && aligned_to(C, 16) && aligned_to(scales, 8);
-  if (K % 16 != 0 || !aligned_to(A, 16) || !aligned_to(W, 16) || (!tile_kernel && K > (1 << 29))) {
-    // Enough output for it: 128x128 tiles on the matrix cores, the slabs staged through registers at any alignment
-    // (N = 11008, K = 4040: M = 64 1.43 -> 0.14 ms, M = 1024 22.5 -> 0.23 ms). With few tiles that kernel waits out a
-    // memory latency per slab (about 110 us at K = 4040 whatever the rows), and the kernel below, a wave per channel
-    // with lanes striding over k, is ahead while M * N stays small (M = 16: 76 us at N = 4096, 371 at N = 11008).
-    if (M > 8 && M * N >= 98304) return gemm_w8a16_any_shape(M, N, K, a, W, s, zp, pt, c, st);
+  if (route.kernel == HEXMI_W8A16_REGISTERS) return gemm_w8a16_any_shape(M, N, K, a, W, s, zp, pt, c, st);
+  if (route.kernel == HEXMI_W8A16_ELEMENTS) {
     constexpr int MR = 4;
     const int64_t gy = (M + MR - 1) / MR;
     if (gy > 65535) return HEXMI_ENOTSUP;
@@ -807,7 +849,7 @@ int gemm_w8a16_any(int64_t M, int64_t N, int64_t K, const void* A, const int8_t*
                        c, (int)M, (int)N, (int)K, zp, pt);
     return launch_status();
   }
-  if (M <= 2 && !chunked_pair && (K == 1024 || K == 2048 || K == 4096 || K == 8192)) {
+  if (route.kernel == HEXMI_W8A16_DOTS) {
     // one channel per wave, eight waves per workgroup: measured against two and four channels per wave and
     // workgroups of two, four and sixteen waves at N = 11008, K = 4096 (0.60 of the HBM figure against 0.57 for two
     // channels x four waves on the same box)
@@ -821,12 +863,8 @@ int gemm_w8a16_any(int64_t M, int64_t N, int64_t K, const void* A, const int8_t*
 #undef HEXMI_GEMV
     return launch_status();
   }
-  // three rows and more where the tiles of w8a16_few.hip give every CU a share
-  const GemmFewTile few = plan_w8a16_few(M, N, K, tile_kernel, zp != nullptr);
-  if (few.m) return launch_w8a16_few(few, M, N, K, a, W, s, zp, pt, c, st);
-  // what is left of more than 128 rows that the 128 x 128 tiles do not take (rows too long for those tiles' offsets): the chunked
-  // kernel in passes of 128 rows (130 x 1001 x 4194368 22.5 ms; a workgroup per 16 channels in passes of 64 rows took 34.0)
-  if (!tile_kernel && M > kMidMaxM) {
+  if (route.kernel == HEXMI_W8A16_TILES) return launch_w8a16_few(route.few, M, N, K, a, W, s, zp, pt, c, st);
+  if (route.kernel == HEXMI_W8A16_CHUNKED && M > kMidMaxM) {
     int rc = HEXMI_OK;
     for (int64_t m = 0; m < M && rc == HEXMI_OK; m += kMidMaxM) {
       const int64_t rows = M - m < kMidMaxM ? M - m : kMidMaxM;
@@ -834,32 +872,15 @@ int gemm_w8a16_any(int64_t M, int64_t N, int64_t K, const void* A, const int8_t*
     }
     return rc;
   }
-  // the chunked kernel: any K (a multiple of 16 here)
-  if (M <= kMidMaxM && K <= (1 << 29)) {
+  if (route.kernel == HEXMI_W8A16_CHUNKED) {
     const int cus = hexmi_num_cus();
     if (cus <= 0) return HEXMI_ELAUNCH;
-    const int64_t per_cu = (N + cus - 1) / cus;
-    int chan_per_wg = (int)(per_cu < 16 ? 16 : per_cu);     // one full tile at least
-    bool paired = false;
-    if (per_cu > kMidCh) {
-      // More than a workgroup's 48 channels per CU: equal workgroups in whole rounds over the CUs, not 48 each and
-      // a last round of a few (N = 14336, K = 4096, M = 16: 19.3 us that way). Either one workgroup per CU at a
-      // time, of up to three channel tiles, or, with up to 16 rows, two of up to two tiles each (their LDS fits
-      // twice, so their starts and ends overlap: 14.8 us); whichever copies fewer tile rows, empty ones counted.
-      const int64_t r1 = (per_cu + kMidCh - 1) / kMidCh, c1 = (N + cus * r1 - 1) / (cus * r1);
-      chan_per_wg = (int)c1;
-      if (M <= 16) {
-        const int64_t r2 = (per_cu + 63) / 64, c2 = (N + cus * 2 * r2 - 1) / (cus * 2 * r2);
-        if (c2 > 16 && r2 * 2 * ((c2 + 15) / 16) <= r1 * ((c1 + 15) / 16)) {
-          chan_per_wg = (int)c2;
-          paired = true;
-        }
-      }
-    }
+    const MidPlan plan = plan_mid(M, N, cus);
+    const int chan_per_wg = plan.channels, tiles = plan.tiles;
+    const bool paired = plan.paired;
     const int64_t grid64 = (N + chan_per_wg - 1) / chan_per_wg;
     if (grid64 > 0x7fffffff) return HEXMI_ENOTSUP;
     const int grid = (int)grid64;
-    const int tiles = (chan_per_wg + 15) / 16;              // channel tiles of a workgroup that hold channels
 #define HEXMI_MID_T(MB, NT, KC, ZP, TAIL) \
   hipLaunchKernelGGL((w8a16_mid_kernel<MB, NT, KC, ZP, TAIL>), dim3(grid), dim3(1024), 0, st, a, W, s, c, (int)M, (int)N, (int)K, chan_per_wg, paired ? 0 : 1, zp, pt)
   // up to 32 rows the form that takes any K is the only one (its masks and clamps cost nothing there)
@@ -882,6 +903,15 @@ int gemm_w8a16_any(int64_t M, int64_t N, int64_t K, const void* A, const int8_t*
   return gemm_w8a16_tiled(M, N, K, a, W, s, c, st);
 }
 }  // namespace
+
+extern "C" int hexmi_gemm_w8a16_kernel(int64_t M, int64_t N, int64_t K, int zero_points, int per_tensor) {
+  const int cus = hexmi_num_cus();
+  if (M <= 0 || N <= 0 || K <= 0 || M > 0x7fffffff || N > 0x7fffffff - 16 || K > 0x7fffffff || cus <= 0) return 0;
+  const W8Route route = route_w8a16(M, N, K, zero_points != 0, per_tensor != 0, true, true);
+  if (route.kernel != HEXMI_W8A16_CHUNKED) return route.kernel;
+  const MidPlan plan = plan_mid(std::min<int64_t>(M, kMidMaxM), N, cus);
+  return route.kernel + plan.tiles + (plan.paired ? HEXMI_W8A16_PAIRED : 0);
+}
 
 extern "C" int hexmi_gemm_w8a16(int64_t M, int64_t N, int64_t K, const void* A, const int8_t* W, const void* scales,
                                 void* C, hexmi_stream_t stream) {

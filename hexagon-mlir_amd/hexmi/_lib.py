@@ -81,6 +81,7 @@ PROBE_SIGNATURES = {
     "hexmi_issue_slots": (_int, [_int, _int, _int, _i64, _int, _ptr, _ptr]),
     "hexmi_lds_read_pattern": (_int, [_int, _i64, _ptr, _ptr]),
     "hexmi_l2_stream": (_int, [_int, _int, _i64, _i64, _ptr, _ptr, _ptr]),
+    "hexmi_gemm_w8a16_kernel": (_int, [_i64, _i64, _i64, _int, _int]),
 }
 
 _lib = None

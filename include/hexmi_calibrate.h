@@ -22,6 +22,22 @@ extern "C" {
 
 #define HEXMI_CALIBRATE_MAX_ITERS (1 << 20)
 
+/* Which of its kernels hexmi_gemm_w8a16 (and, with zero points or one scale for
+ * the tensor, hexmi_gemm_w8a16_ex) takes a product of these sizes to on the
+ * current device, operands on 16-byte boundaries: what a test that is aimed at
+ * a kernel asks first. HEXMI_W8A16_CHUNKED comes with the channel tiles of a
+ * workgroup (1 to 3) and HEXMI_W8A16_PAIRED added; 0: no device, or sizes that
+ * are refused or empty. */
+#define HEXMI_W8A16_DOTS 1       /* a row or two: a wave per channel */
+#define HEXMI_W8A16_ELEMENTS 2   /* any K and alignment, a wave per channel */
+#define HEXMI_W8A16_REGISTERS 3  /* any K and alignment, tiles of 128 x 128 */
+#define HEXMI_W8A16_TILES 4      /* tiles of 16 x 16 to 64 x 192 */
+#define HEXMI_W8A16_LARGE 5      /* tiles of 128 x 128 and 256 x 256 */
+#define HEXMI_W8A16_CHUNKED 16   /* a workgroup per channel range, all rows */
+#define HEXMI_W8A16_PAIRED 32    /* ... two of them to a compute unit */
+int hexmi_gemm_w8a16_kernel(int64_t M, int64_t N, int64_t K, int zero_points,
+                            int per_tensor);
+
 /* A stream of nothing but MFMAs (operands and accumulators in registers, no
  * memory traffic): what the matrix cores of this GPU sustain for one
  * instruction shape on operands of the caller's choice. It has no counterpart

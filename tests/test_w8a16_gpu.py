@@ -78,11 +78,96 @@ def test_w8a16_parity(hexmi, oracle, M, N, K):
     assert (got.float() - want.float()).abs().max() / math.sqrt(K) <= 2e-2
 
 
+@pytest.fixture(scope="module")
+def channels():
+    """Weights, scales and zero points of more channels than 48 per CU, on the device: products take what they need of them."""
+    g = torch.Generator("cuda").manual_seed(11)
+    return (torch.randint(-127, 128, (62000, 2048), generator=g, dtype=torch.int8, device="cuda"),
+            (0.001 + 0.019 * torch.rand(62000, generator=g, device="cuda")).half(),
+            torch.randint(-128, 128, (62000,), generator=g, dtype=torch.int8, device="cuda"))
+
+
+def _chunked(M, N, K, tiles, paired, zero_points, w, s, z):
+    """The product on the chunked kernel, with that many channel tiles to a workgroup, against 64 bits."""
+    from hexmi import _lib
+    lib = _lib.lib()
+    kernel = lib.hexmi_gemm_w8a16_kernel(M, N, K, int(zero_points), 0)
+    assert kernel == 16 + tiles + (32 if paired else 0), kernel        # HEXMI_W8A16_CHUNKED, _PAIRED: what the case is for
+    a = torch.randn(M, K, generator=torch.Generator("cuda").manual_seed(M + K), device="cuda").half()
+    out = torch.full((M, N), math.nan, dtype=torch.float16, device="cuda")
+    assert lib.hexmi_gemm_w8a16_ex(M, N, K, a.data_ptr(), w.data_ptr(), s.data_ptr(), z.data_ptr() if zero_points else None, 0,
+                                   out.data_ptr(), torch.cuda.current_stream().cuda_stream) == _lib.OK
+    for n in range(0, N, 8192):
+        weights = w[n:n + 8192].double()
+        if zero_points:
+            weights -= z[n:n + len(weights), None].double()
+        want = (a.double() @ weights.t()) * s[n:n + len(weights)].double()
+        assert close16(out[:, n:n + 8192].cpu(), want.half().cpu(), max_ulp=1, atol=2e-4)
+
+
+# The chunked kernel stops copying ahead and lowers its waits by the number of chunks left: every count of chunks up to the depth of its
+# pipeline and beyond, both parities, for every count of row blocks, whole and short last chunks, and K off whole 64s, which it masks.
+# Few chunks reach it where there are more channels than one round of the widest tiles takes.
+@pytest.mark.parametrize("M", [3, 9, 16, 17, 32, 33, 48, 64, 96, 100, 128])
+@pytest.mark.parametrize("K", [16, 48, 64, 128, 192, 256, 272, 320, 384, 512, 640, 768, 1008, 1024, 1280, 1536, 1808, 2048])
+def test_w8a16_chunked_kernel_few_chunks(hexmi, channels, M, K):
+    w, s, z = channels
+    _chunked(M, 49168, K, 3, False, K % 3 == 1, w[:49168, :K].contiguous(), s, z)
+
+
+# ... two workgroups to a CU: one chunk, short last chunks, several rounds, a last workgroup with fewer channels
+@pytest.mark.parametrize("M", [3, 8, 16])
+@pytest.mark.parametrize("N,K", [(62000, 64), (62000, 80), (62000, 256), (61999, 320), (62000, 640), (62000, 832), (62000, 1984), (61990, 2048)])
+def test_w8a16_chunked_kernel_paired(hexmi, channels, M, N, K):
+    w, s, z = channels
+    _chunked(M, N, K, 2, True, M == 8, w[:N, :K].contiguous(), s, z)
+
+
+# ... and up to 48 channels a CU, one, two and three tiles of them, where K leaves the call to it: chunks of 768, 384, 256 or 128, whole and
+# short last ones, K off whole 64s, zero points
+@pytest.mark.parametrize("M,N,K,tiles,zero_points", [
+    (16, 2000, 10752, 1, False), (5, 2000, 10560, 1, False), (16, 2000, 10512, 1, False), (9, 1992, 8192, 1, True), (3, 2000, 12672, 1, False),
+    (16, 5000, 4224, 2, False), (5, 5000, 4240, 2, False), (16, 5001, 4416, 2, True), (3, 5000, 5120, 2, False),
+    (16, 10000, 2112, 3, False), (5, 10000, 2304, 3, False), (16, 10001, 2128, 3, True), (3, 10000, 2624, 3, False), (16, 11008, 4096, 3, False),
+    (17, 5000, 3136, 2, False), (32, 5000, 3456, 2, False), (32, 5001, 3152, 2, True), (20, 5000, 4096, 2, False),
+    (17, 10000, 1600, 3, False), (32, 10000, 1616, 3, True), (32, 10000, 1792, 3, False), (25, 10000, 2368, 3, False),
+    (33, 6000, 3072, 2, True), (48, 6001, 3088, 2, True), (48, 8000, 3200, 2, True),
+    (33, 10000, 1600, 3, False), (48, 10001, 1616, 3, True), (40, 10000, 1792, 3, False),
+    (49, 10000, 2048, 3, False), (64, 10001, 2064, 3, True), (64, 10000, 2112, 3, False), (64, 11008, 2304, 3, False),
+    (65, 10000, 2048, 3, False), (96, 10001, 2064, 3, True), (96, 10000, 2112, 3, False), (80, 10000, 4096, 3, False),
+    (97, 10000, 2048, 3, False), (112, 10001, 2096, 3, True), (112, 10000, 2112, 3, False), (100, 10000, 4096, 3, False)])
+def test_w8a16_chunked_kernel_long_rows(hexmi, M, N, K, tiles, zero_points):
+    g = torch.Generator("cuda").manual_seed(N + K)
+    w = torch.randint(-127, 128, (N, K), generator=g, dtype=torch.int8, device="cuda")
+    s = (0.001 + 0.019 * torch.rand(N, generator=g, device="cuda")).half()
+    z = torch.randint(-128, 128, (N,), generator=g, dtype=torch.int8, device="cuda")
+    _chunked(M, N, K, tiles, False, zero_points, w, s, z)
+
+
+# the lines of plan_w8a16_few on 256 CUs: the kernels to both sides of each (tiles 4, chunked 16 and its channel tiles), and their results
+@pytest.mark.parametrize("M,N,K,zero_points,kernel", [
+    (16, 4096, 5120, False, 4), (16, 4112, 5120, False, 18), (4, 4112, 5120, False, 4), (4, 4096, 6144, False, 17),
+    (32, 4608, 3072, False, 4), (32, 4608, 3088, False, 18), (32, 9216, 1536, False, 4), (32, 9216, 1552, False, 19),
+    (16, 2048, 8176, True, 4), (16, 2048, 8192, True, 17), (16, 2048, 8192, False, 4), (24, 4608, 1536, True, 4), (24, 4608, 1552, True, 18),
+    (48, 6144, 3056, True, 4), (48, 6144, 3072, True, 18), (48, 6144, 3072, False, 4), (48, 9216, 1536, False, 4), (48, 9216, 1552, False, 19),
+    (56, 9216, 2032, False, 4), (56, 9216, 2048, False, 19), (16, 24576, 4096, False, 19), (17, 24576, 4096, False, 4),
+    (16, 24576, 4160, False, 4), (16, 20000, 4096, False, 4), (16, 14336, 4096, False, 4)])
+def test_w8a16_lines_between_tiles_and_the_chunked_kernel(hexmi, M, N, K, zero_points, kernel):
+    from hexmi import _lib
+    assert _lib.lib().hexmi_gemm_w8a16_kernel(M, N, K, int(zero_points), 0) & ~32 == kernel
+    g = torch.Generator("cuda").manual_seed(N + K)
+    w = torch.randint(-127, 128, (N, K), generator=g, dtype=torch.int8, device="cuda")
+    s = (0.001 + 0.019 * torch.rand(N, generator=g, device="cuda")).half()
+    z = torch.randint(-128, 128, (N,), generator=g, dtype=torch.int8, device="cuda") if zero_points else None
+    a = torch.randn(M, K, generator=g, device="cuda").half()
+    want = (a.double() @ (w.double() - (z[:, None].double() if zero_points else 0.0)).t()) * s.double()
+    assert close16(hexmi.w8a16_matmul(a, w, s, zero_points=z).cpu(), want.half().cpu(), max_ulp=1, atol=2e-4)
+
+
 @pytest.mark.parametrize("M", [3, 8, 9, 16, 32, 48, 64, 80, 96, 100, 128])
 @pytest.mark.parametrize("chunks", [1, 2, 3, 4, 5, 6, 7, 8, 9, 12, 13])
-def test_w8a16_every_tail_of_the_chunked_kernel(hexmi, oracle, M, chunks):
-    # the chunked kernel (M <= 128) stops copying ahead and lowers its waits by the number of chunks left: every
-    # count of chunks up to the depth of the pipeline and beyond, both parities, for every count of row blocks
+def test_w8a16_every_count_of_slabs(hexmi, oracle, M, chunks):
+    # a narrow product on the tiles of w8a16_few.hip: fewer slabs of K than stages and more, whole and halves of them
     K = 256 * chunks
     a, w, s = _inputs(M, 100, K, seed=23 + chunks)
     got = hexmi.w8a16_matmul(a.cuda(), w.cuda(), s.cuda()).cpu()
@@ -93,9 +178,8 @@ def test_w8a16_every_tail_of_the_chunked_kernel(hexmi, oracle, M, chunks):
 @pytest.mark.parametrize("M", [3, 9, 16, 17, 32, 48, 64, 96, 128])
 @pytest.mark.parametrize("N", [100, 5000, 10000])
 @pytest.mark.parametrize("K", [64, 192, 320, 448, 704, 768, 832, 1536, 1600, 2368, 4096])
-def test_w8a16_chunked_kernel_takes_any_k(hexmi, oracle, M, N, K):
-    # chunks of 768, 384, 256 or 128 k by the rows and the channel tiles per workgroup (one, two, three at N = 100,
-    # 5000, 10000 on 256 CUs), K any multiple of 64: a last chunk that is short, a single short chunk, whole chunks
+def test_w8a16_inner_dimension_in_sixty_fours(hexmi, oracle, M, N, K):
+    # K any multiple of 64, mostly on tiles: a last slab that is short, a single short slab, whole slabs
     a, w, s = _inputs(M, N, K, seed=K + M)
     got = hexmi.w8a16_matmul(a.cuda(), w.cuda(), s.cuda()).cpu()
     want = torch.from_numpy(oracle.matmul_w8a16(a.numpy(), w.numpy(), s.numpy()))
@@ -107,8 +191,7 @@ def test_w8a16_chunked_kernel_takes_any_k(hexmi, oracle, M, N, K):
 @pytest.mark.parametrize("K", [16, 48, 80, 272, 1008, 1040, 4048])
 @pytest.mark.parametrize("zero_points", [False, True])
 def test_w8a16_inner_dimension_in_sixteens(hexmi, oracle, M, N, K, zero_points):
-    # K a multiple of 16 but not of 64: the chunked kernel masks a lane's sixteen weights past K (its copies are
-    # clamped to the row's end); more than 128 rows run it in passes
+    # K a multiple of 16 but not of 64, mostly on tiles: the chunks of a slab past K are fetched from zeros
     if zero_points and (M in (17, 100, 130) or K in (48, 1040)):
         pytest.skip("zero points: a subset of the shapes")
     a, w, s = _inputs(M, N, K, seed=K + M + 1)
@@ -176,12 +259,10 @@ def test_w8a16_short_last_chunk_ignores_what_lies_behind_the_row(hexmi):
 
 @pytest.mark.parametrize("M,N,K", [(4, 14336, 512), (16, 14336, 4096), (9, 28672, 768), (16, 22016, 1024),
                                    (64, 14336, 1024), (128, 22016, 512), (32, 13824, 5120),
-                                   # up to 16 rows, two workgroups per CU at a time: one chunk, short last chunks,
-                                   # a last workgroup with fewer channels, several rounds
                                    (16, 14336, 256), (3, 13000, 832), (16, 13000, 64), (8, 40000, 640),
                                    (16, 22016, 1984), (5, 52000, 320), (16, 12300, 1280)])
 def test_w8a16_more_than_a_workgroup_of_channels_per_cu(hexmi, oracle, M, N, K):
-    # N beyond 48 channels per CU: equal workgroups in whole rounds, two at a time per CU with up to 16 rows;
+    # N beyond 48 channels per CU: one round of wider tiles, or a workspace's parts of K, or the chunked kernel;
     # the oracle covers every 29th output channel and the first and last 64
     a, w, s = _inputs(M, N, K, seed=N % 97 + M)
     got = hexmi.w8a16_matmul(a.cuda(), w.cuda(), s.cuda()).cpu()
