@@ -673,15 +673,17 @@ int launch_gemm_parts(const GemmParts& plan, const T* A, const T* B, OutT* C, in
                      plan.part)
 #define HEXMI_PARTS(BM, BN)                                                                                                  \
   do {                                                                                                                       \
-    if (!TRANS_B && any) HEXMI_PARTS_AS(BM, BN, 2, !TRANS_B);                                                                 \
-    else HEXMI_PARTS_AS(BM, BN, (FewShape<BM, BN>::NS), false);                                                               \
+    if constexpr (!TRANS_B) {                                                                                                \
+      if (any) { HEXMI_PARTS_AS(BM, BN, 2, true); break; }                                                                     \
+    }                                                                                                                        \
+    HEXMI_PARTS_AS(BM, BN, (FewShape<BM, BN>::NS), false);                                                                    \
   } while (0)
   if (any && (TRANS_B || plan.tile.n > 64)) return HEXMI_ENOTSUP;
-  if (plan.tile.m == 16 && plan.tile.n == 64) HEXMI_PARTS(16, 64);
-  else if (plan.tile.m == 16) HEXMI_PARTS_AS(16, 128, (FewShape<16, 128>::NS), false);
-  else if (plan.tile.m == 32) HEXMI_PARTS(32, 64);
+  if (plan.tile.m == 32) HEXMI_PARTS(32, 64);
   else if (plan.tile.m == 64) HEXMI_PARTS(64, 64);
-  else return HEXMI_ENOTSUP;
+  else if constexpr (TRANS_B) return HEXMI_ENOTSUP;              // (the plan gives [N,K] weights no tiles of sixteen rows)
+  else if (plan.tile.n == 64) HEXMI_PARTS(16, 64);
+  else HEXMI_PARTS_AS(16, 128, (FewShape<16, 128>::NS), false);
 #undef HEXMI_PARTS
 #undef HEXMI_PARTS_AS
   const int rc = launch_status();
