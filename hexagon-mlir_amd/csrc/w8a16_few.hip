@@ -106,8 +106,9 @@ void w8a16_few_kernel(const f16* __restrict__ A, const int8_t* __restrict__ W, c
   const int scale_at = n0 + (int)threadIdx.x < N ? n0 + (int)threadIdx.x : N - 1;
   const f16 scale = scales[pt ? 0 : scale_at];
 
-  // Partial sums of an element over K, one to four of a wave group each: one chain of K / 32 additions would round more than the
-  // chunked kernel's sixteen (up to 16 rows) or four to eight do.
+  // Partial sums of an element over K, one to four of a wave group each: sixteen on tiles of sixteen rows and of 32 x 32, four on the
+  // others. One chain of K / 32 additions would round more than the chunked kernel's sums, one for each 64 k of a chunk: twelve, six or
+  // four by the channel tiles of a workgroup up to 16 rows, six or four up to 32, four up to 64, two beyond.
   constexpr int kParts = TM == 1 ? 16 / KH : KH == 4 ? 1 : 2;
   f32x4 acc[kParts][TM][TN];
 #pragma unroll
