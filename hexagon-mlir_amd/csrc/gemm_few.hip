@@ -76,7 +76,9 @@ static_assert(rest_of(kAnyMaxK, kAnyMaxK / 256, 256) == kAnyMaxK % 256 && rest_o
 // 50 / 73 / 53, 65536 x 257 x 9 21 / 36 / 24, 20000 x 33 x 33 7.7 / 10.5 / 7.0. What alignment itself costs is a tenth to a fifth: rows on
 // the boundaries / off them, [N,K] 128 x 7224 x 6651 37 / 43, [K,N] 44 / 47, 1021 x 50264 x 763 138 / 145. Two slabs on their way in
 // 128 x 128 tiles leave one to a CU: 1021 x 50257 x 768 211, 640 x 7031 x 3584 140.
-template <typename T, typename OutT, typename S, int NS, bool TRANS_B, bool ANY>
+// PARTS: blockIdx.y takes a part of K; a form of its own, since working the part out first cost every small product of [K,N] weights a
+// fortieth (3.10 us where it now takes 3.03).
+template <typename T, typename OutT, typename S, int NS, bool TRANS_B, bool ANY, bool PARTS = false>
 __global__ __launch_bounds__(S::kThreads, S::STEPS == 2 ? 4 : 2)
 void gemm_few_kernel(const T* __restrict__ A, const T* __restrict__ B, OutT* C, int M, int N, int K, int64_t lda, int64_t ldb,
                      int64_t ldc, const OutT* __restrict__ bias, const OutT* resid, int64_t ldr, int tiles_m, int tiles_n,
@@ -94,7 +96,7 @@ void gemm_few_kernel(const T* __restrict__ A, const T* __restrict__ B, OutT* C, 
   int tm, tn;
   tile_of_block<8>(blockIdx.x, tiles_m, tiles_n, tm, tn);
   const int m0 = tm * BM, n0 = tn * BN;
-  {                                                              // blockIdx.y: the part of K, whole slabs, whose sums go to a C of its own
+  if constexpr (PARTS) {                                         // the part of K, whole slabs, whose sums go to a C of its own
     const int k0 = blockIdx.y * part;
     A += k0;
     B += TRANS_B ? (int64_t)k0 : k0 * ldb;
@@ -667,7 +669,7 @@ int launch_gemm_parts(const GemmParts& plan, const T* A, const T* B, OutT* C, in
   const int tiles_m = (int)((M + plan.tile.m - 1) / plan.tile.m), tiles_n = (int)((N + plan.tile.n - 1) / plan.tile.n);
   const int64_t pitch = gemm_parts_pitch(N);
 #define HEXMI_PARTS_AS(BM, BN, NS, ANY)                                                                                            \
-  hipLaunchKernelGGL((gemm_few_kernel<T, float, FewShape<BM, BN>::S, NS, TRANS_B, ANY>),                                             \
+  hipLaunchKernelGGL((gemm_few_kernel<T, float, FewShape<BM, BN>::S, NS, TRANS_B, ANY, true>),                                             \
                      dim3((unsigned)(tiles_m * tiles_n), (unsigned)plan.parts), dim3(FewShape<BM, BN>::S::kThreads), 0, s, A, B, sums, \
                      (int)M, (int)N, (int)K, lda, ldb, pitch, (const float*)nullptr, (const float*)nullptr, (int64_t)0, tiles_m, tiles_n, 1, \
                      plan.part)
