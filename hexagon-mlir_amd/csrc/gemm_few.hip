@@ -530,8 +530,8 @@ void gemm_merge_kernel(const float* __restrict__ sums, OutT* C, int M, int N, in
 //   three and four rows from K = 1024 on (dot products): the tiles ahead at 4 x 4096 x 4096 (9.9, 8.9 / 9.4, 7.9), 4 x 11008 x 4096
 //   (19.5, 19.7 / 19.2, 17.5), 3 x 14336 x 1024 (9.6, 8.2 / 9.2, 7.4), 4 x 4096 x 11008 (21.9, 21.2 / 21.5, 16.7); not with weights of 3 * 2^24
 //   elements and more (3 x 16384 x 4096 25.9, 29.6 / 25.7, 29.5; 4 x 14336 x 4096 24.3, 25.5 / 23.9, 26.0; 3 x 8192 x 8192 26.0, 27.1 /
-//   25.2, 26.8) nor where tiles of 32 columns and more leave three eighths of the CUs without one (3 x 4192 x 3560 9.8, 11.5;
-//   4 x 9527 x 6416 28, 33);
+//   25.2, 26.8), nor on tiles of 64 x 96 (4 x 20056 x 1984 17.4, 18.7; 4 x 22858 x 2048 22.1, 24.2), nor where tiles of 32 columns and more
+//   leave three eighths of the CUs without one (3 x 4192 x 3560 9.8, 11.5; 4 x 9527 x 6416 28, 33);
 //   up to sixteen rows, half of a tile of 32 x 64 (weight stream): 16 x 14336 x 4096 22.8, 25.8 / 22.4, 24.9; 10 x 8666 x 10432 41.4, 45.1 /
 //   41.6, 45.2; 13 x 11368 x 1664 11.7, 12.2 / 8.0, 8.8 (16 x 11008 x 4096 18.9, 20.7 / 19.1, 18.0); up to 24 of the 64 of a tile of 64 x
 //   96 (weights from HBM: 9 x 20000 x 4096 29.4, 37.4; 16 x 24576 x 512 7.8, 8.6; 16 x 16400 x 1408 11.9, 13.7; 17 x 24576 x 4096 38.6,
@@ -560,7 +560,7 @@ GemmFewTile plan_gemm_few(bool trans_b, int64_t M, int64_t N, int64_t K) {
     if (t.n == 16 && !trans_b) continue;                         // sixteen columns of a row of B are a quarter of a line
     const int64_t count = ((M + t.m - 1) / t.m) * ((N + t.n - 1) / t.n);
     if (count > cus) continue;
-    if (dots && M <= 4 && (N * K >= (int64_t)3 << 24 || (t.n > 16 && 8 * count < 5 * cus))) return {0, 0};
+    if (dots && M <= 4 && (N * K >= (int64_t)3 << 24 || t.n > 64 || (t.n > 16 && 8 * count < 5 * cus))) return {0, 0};
     if (stream && M <= 16 && (t.n >= 64 || (t.n == 16 && 2 * count < cus))) return {0, 0};
     if (stream && M <= 24 && t.n > 64) return {0, 0};
     const bool narrow = stream && M <= 32 && t.m == 16 && N <= 16 * cus;    // a channel group of sixteen per CU at most

@@ -139,7 +139,7 @@ def test_gemm_few_rows_every_workgroup_shape(hexmi, dtype, M, N, K):
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("M,N,K", [(3, 4094, 3080), (4, 5200, 2424), (3, 16380, 1032), (3, 4099, 3104), (4, 9001, 1408), (4, 6151, 8192),
                                    (5, 16401, 2056), (8, 50257, 2048), (6, 17001, 2112), (7, 20011, 2048), (16, 9001, 1408), (9, 16380, 1032),
-                                   (20, 3001, 2816), (20, 3001, 2808), (25, 3001, 2816), (24, 4090, 8256),
+                                   (4, 16384, 1984), (4, 16392, 1984), (3, 20001, 2048), (20, 3001, 2816), (20, 3001, 2808), (25, 3001, 2816), (24, 4090, 8256),
                                    (11, 2030, 6400), (30, 4090, 12352), (16, 16401, 544), (24, 20001, 288), (25, 20001, 288)])
 def test_gemm_few_rows_at_the_lines_between_kernels(hexmi, dtype, M, N, K):
     for out_dtype in (dtype, torch.float32):
