@@ -506,8 +506,11 @@ void gemm_merge_kernel(const float* __restrict__ sums, OutT* C, int M, int N, in
 // (Tiles of sixteen rows at any number of rows: 85 x 512 x 9664 16.5 / 11.0, 113 x 304 x 11968 29.9 / 23.8, 72 x 1280 x 1280 6.5 / 6.2, 267 x 272 x 4480
 // 9.9 / 8.3; 1.12 times the rate over 50 products of 65 to 267 rows, none slower.)
 // (64 x 96 and 96 x 64 ask for an eighth less than the tile of 128 x 64 that took their calls and leave fewer CUs idle: 2638 x 512 x 5600 40 /
-// 31, 168 x 6128 x 9520 86 / 68, 1725 x 624 x 9728 64 / 53, 583 x 2144 x 4288 24 / 20, 2751 x 488 x 5312 28.8 / 23.8, 280 x 4992 x 384 6.8 / 6.2; 1.12
-// and 1.07 times the rate over 60 and 25 products, none slower. 48 x 32 before 32 x 64, [N,K]: 92 x 3304 x 8832 33 / 27.6, 687 x 400 x 3680 13.2 / 11.6,
+// 31, 168 x 6128 x 9520 86 / 68, 1725 x 624 x 9728 64 / 53, 583 x 2144 x 4288 24 / 20, 2751 x 488 x 5312 28.8 / 23.8, 280 x 4992 x 384 6.8 / 6.2; 1.08
+// times the rate over 3150 products. Not where the last row of 128 x 64 tiles is half padding, which costs no intake, and the weights are
+// more than the L2s hold of them beside the rest: 160 x 6016 x 6016 36 / 42, 284 x 4992 x 6096 40 / 49, [K,N] 427 x 2432 x 6656 44 / 54;
+// [N,K] weights of 6 to 7 million 1.01 times the rate, 7 to 8 0.93, 12 to 16 0.89, beyond 0.88; [K,N] 7 to 8 1.02, 8 to 9 0.94, 12 to 16 0.88;
+// 1130 products, an even count of 64 rows 1.05 to 1.10 at any. 48 x 32 before 32 x 64, [N,K]: 92 x 3304 x 8832 33 / 27.6, 687 x 400 x 3680 13.2 / 11.6,
 // level or a few hundredths slower below K of about 1000 and against [K,N] weights (1149 x 320 x 2752 10.5 / 11.4). 48 x 64 with two stages of 256 of K loses 10 % to 64 x 64.)
 // (96 x 96 asks for what 128 x 64 does, an eighth more of C to a tile; us on 128 x 128 tiles two to a CU or one / here: 1336 x 1600 x 1600
 // 20.2 / 16.2, 330 x 5672 x 7232 72 / 56, 3209 x 592 x 9064 101 / 71, 165 x 8632 x 1984 19.7 / 15.2, 189 x 9704 x 384 10.2 / 8.1, 1510 x 1512 x
@@ -553,13 +556,15 @@ GemmFewTile plan_gemm_few(bool trans_b, int64_t M, int64_t N, int64_t K) {
   if ((dots || stream) && M <= 64) {
     if (M > 32 ? K <= 128 : N * K < (int64_t)(M > 16 ? 2 : 3) << 22 && !(M >= 5 && M <= 8 && K >= 2048)) return {0, 0};
   }
+  // half of the last row of 128 x 64 tiles is padding, and weights of 14 MiB and more ([K,N]: 16)
+  const bool half = (M + 63) / 64 % 2 && N * K >= (int64_t)(trans_b ? 7 : 8) << 20 && ((M + 127) / 128) * ((N + 63) / 64) <= cus;
   static constexpr GemmFewTile kTiles[] = {{16, 16}, {16, 32}, {32, 32}, {48, 32}, {32, 64}, {64, 64}, {64, 96}, {96, 64}, {128, 64}, {96, 96}};
   for (const GemmFewTile& t : kTiles) {
     if (t.m == 48 && (K < 1024 || !trans_b)) continue;
     if (t.m == 96 && t.n == 96 && K % 64 == 0 && (N % 8 == 0 ? K > 128 && K <= 256 : K <= 512)) continue;
     if (t.n == 16 && !trans_b) continue;                         // sixteen columns of a row of B are a quarter of a line
     const int64_t count = ((M + t.m - 1) / t.m) * ((N + t.n - 1) / t.n);
-    if (count > cus) continue;
+    if (count > cus || (half && t.m * t.n == 64 * 96)) continue;
     if (dots && M <= 4 && (N * K >= (int64_t)3 << 24 || t.n > 64 || (t.n > 16 && 8 * count < 5 * cus))) return {0, 0};
     if (stream && M <= 16 && (t.n >= 64 || (t.n == 16 && 2 * count < cus))) return {0, 0};
     if (stream && M <= 24 && t.n > 64) return {0, 0};

@@ -232,6 +232,7 @@ def _against_double(hexmi, dtype, out_dtype, trans_b, M, N, K, bias, residual, s
     (1921, 1024, 392), (2000, 768, 1032), (129, 8128, 8), (2048, 1024, 128),     # 128 x 64; the last of a round
     (1345, 1536, 264), (1343, 1544, 520), (70, 17752, 72), (193, 8056, 136),     # 96 x 96
     (640, 3456, 128), (640, 3456, 192), (640, 3456, 256), (640, 3456, 320), (544, 3484, 512), (544, 3484, 576),      # ... and not
+    (130, 4096, 1784), (130, 4096, 1792), (130, 4096, 2040), (130, 4096, 2048), (129, 8192, 1032), (282, 5248, 1600),   # 128 x 64 half empty
     (1985, 760, 136), (1983, 776, 520), (65, 12296, 264), (2017, 672, 1288),     # 64 x 96, 96 x 64
     (2305, 264, 1032), (47, 8200, 1160), (145, 2008, 2056), (95, 4088, 1024),    # 48 x 32
     (113, 304, 1000), (197, 408, 264), (511, 256, 72), (65, 1592, 2056)])        # sixteen rows a tile, many rows
