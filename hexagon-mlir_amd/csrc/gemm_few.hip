@@ -653,6 +653,11 @@ int launch_gemm_few(const GemmFewTile& tile, const T* A, const T* B, OutT* C, in
 // 10.5, K of 12800 and more 1.12; K = 8192 0.94 (64 x 4096 x 11008 33 / 26, 128 x 1024 x 12288 28.9 / 15.8, 128 x 2048 x 10240 26 / 22, 40 x 2048 x 10240
 // 20.2 / 15.1; 64 x 512 x 10240 10.3 / 11.9, 453 x 400 x 9344 16.4 / 18.0). Up to 32 rows the whole has few tiles: 8704 1.03, 9728 1.13, 11008 1.16,
 // 12288 1.32; in fewer than eight parts a tenth ahead or level (32 x 4096 x 11008 21.6 / 21.4) for a second launch, so as a whole.
+// [K,N] weights of few columns are read in whole lines as they are, so that only the walk is long: rate in parts over that as a whole, N up
+// to 32 and M up to 16, K = 3072 to 3500 0.87, to 4000 0.91, to 4600 0.98, to 5500 1.05; M to 1024 and K to 5500 0.83 to 0.99, to 7000 1.03 to 1.25; M
+// beyond 2048 0.77 to 0.94 at any K; N to 64 and M beyond 128 1.0 and less up to 5500 (17 x 16 x 3072 5.5 / 7.7, 4862 x 32 x 6080 12.8 / 16.3, 56 x 16 x
+// 4760 7.0 / 8.6; 7000 products). Up to 16 rows of more than 1024 columns K to 3500 0.92, to 4000 0.99, to 4600 1.15 (3 x 1904 x 3184 8.9 / 10.5).
+// Rows of [N,K] products past 1536 whose last tiles are half empty 0.78 to 0.95 (2630 x 76 x 10072 20.1 / 24.0).
 // [K,N] weights whose rows stand off the boundaries, whole / in parts: 16 x 2027 x 12144 47 / 19, 128 x 1175 x 11904 49 / 24, 3 x 485 x 8704 20.6 / 11.4, 128 x
 // 2250 x 5312 28.9 / 19.9, 15 x 1601 x 4352 13.8 / 11.8, 2 x 405 x 3136 10.9 / 11.3; 1.45 times the rate over 44 (up to 16 rows parts of 256 and
 // more: a slab through registers is a latency; with 512 and more 2 x 1497 x 4512 13.2 / 13.8, with 256 and more at 64 rows 90 x 318 x 11584 13.3 -> 15.5).
@@ -660,6 +665,12 @@ int launch_gemm_few(const GemmFewTile& tile, const T* A, const T* B, OutT* C, in
 GemmParts plan_gemm_parts(bool trans_b, int64_t M, int64_t N, int64_t K, bool any) {
   if (trans_b ? M <= 16 || K < (M <= 32 ? 9728 : 9216) : M <= 32 ? K < 3072 || K < N : K < 4608) return {};
   if (trans_b && M > 32 && K < 12800 && (M + N) * K < 19 << 19) return {};
+  if (trans_b && M > 1536 && (N - 1) % 64 < 32) return {};       // the columns of the last tiles half padding and more
+  if (!trans_b && !any) {
+    if (N <= 32 && (M > 2048 || K < (M <= 16 ? 4608 : M <= 1024 ? 5632 : 7168))) return {};
+    if (N <= 64 && K < (M <= 128 ? 4096 : 5632)) return {};
+    if (M <= 16 && N > 1024 && K < 4096) return {};
+  }
   const GemmFewTile t = M <= 16 ? GemmFewTile{16, N <= 1024 || any ? 64 : 128} : GemmFewTile{M <= 32 ? 32 : 64, 64};
   const int64_t tiles = ((M + t.m - 1) / t.m) * ((N + t.n - 1) / t.n);
   const int64_t parts = std::min(hexmi_num_cus() / std::max<int64_t>(tiles, 1), K / (any && M <= 16 ? 256 : 512));

@@ -273,7 +273,12 @@ def test_gemm_one_round_of_tiles(hexmi, dtype, out_dtype, trans_b, M, N, K):
     (16, 4104, 4096, False, False), (16, 11008, 11376, False, False), (64, 768, 4096, False, False), (16, 1024, 11008, True, False),
     (64, 4096, 8192, True, False), (32, 4096, 11008, True, False),
     (128, 1032, 9216, True, True), (128, 1032, 9208, True, False), (64, 700, 12800, True, True), (64, 700, 12792, True, False),
-    (24, 1000, 9728, True, True), (24, 1000, 9720, True, False),                                             # the lines of [N,K]
+    (24, 1000, 9728, True, True), (24, 1000, 9720, True, False), (1536, 96, 9216, True, True), (1537, 96, 9216, True, False),
+    (1537, 97, 9216, True, True),                                                                            # the lines of [N,K]
+    (16, 32, 4608, False, True), (16, 32, 4600, False, False), (17, 24, 5632, False, True), (17, 24, 5624, False, False),
+    (1025, 32, 7168, False, True), (1025, 32, 7160, False, False), (2049, 16, 8192, False, False), (128, 40, 4608, False, True),
+    (16, 64, 4096, False, True), (16, 64, 4088, False, False), (129, 40, 5632, False, True), (129, 40, 5624, False, False),
+    (16, 1032, 4096, False, True), (16, 1032, 4088, False, False), (16, 1024, 3072, False, True),            # ... of [K,N]
     (8, 1001, 4096, False, True), (16, 4097, 4100, False, True), (1, 3, 3075, False, True), (31, 2049, 5001, False, True),   # rows off the
     (128, 531, 9736, False, True), (64, 1024, 4611, False, True), (64, 2047, 11009, True, False)])                          # boundaries
 def test_gemm_parts_of_a_long_k(hexmi, dtype, out_dtype, M, N, K, trans_b, parts):
