@@ -338,6 +338,9 @@ static constexpr MidCost kOne = {128, 128, 1, 4.0, 0.445, 0.073, 1.9, 0.0, 3.9},
 // K off whole 64s 1.49. A twentieth's lead is asked for, since the fits are that good: without it one in ten is slower. With it, of 200 other
 // products of whole 64s and of 8s 82 of whole 64s came here, at 1.13 times the rate, five of them 5 to 10 % slower than before (1636 x 21440 x
 // 1408 + both 122 / 135, 4480 x 3840 x 320 + bias 26.2 / 27.5).
+// The fits begin at K = 256 and say too little below for the tiles of 192 x 128: 339 x 28864 x 64 10.2 / 13.5, 285 x 31872 x 128 10.7 / 13.2, 192 x
+// 12800 x 64 + residual 8.1 / 9.9, beside 256 x 256 tiles also 384 x 30464 x 384 18.3 / 21.2 (all 44 slower but two; up to 64 rows they are ahead
+// of 256 x 256 tiles by a third, in the place of 128 x 128 ones two to a CU from 320 on).
 // Odd rows of less than 1024 of K: the larger tiles' elements leave with nothing beside them, so two of 128 x 128 to a CU (or one), us on the
 // 32-k slabs of gemm.hip / the tile of the fit / here: 8000 x 10001 x 456 151 / 205 / 143, 3000 x 15003 x 584 114 / 148 / 106, 6000 x 3333 x 584
 // 61 / 66 / 55, 4000 x 2500 x 584 34.5 / 40 / 33.5 (3000 x 3001 x 776 42 / 34 / 39); from 1024 on the fit is ahead.
@@ -346,6 +349,7 @@ GemmMidTile plan_gemm_mid(int64_t M, int64_t N, int64_t K, int now, bool resid, 
   double least = now == 0 ? 1e30 : 0.95 * mid_time(now == 256 ? kLarge : now == 2 ? kTwo : kOne, M, N, K, resid);
   for (const MidCost& c : kMidTiles) {
     if (now != 0 && c.m == 128) continue;                    // (gemm.hip's own are the better ones of whole slabs)
+    if (now != 0 && c.m * c.n == 192 * 128 && M > 64 && K <= (now == 256 ? 768 : 128)) continue;
     if ((resid && c.m * c.n > 192 * 192) || (odd && K < 1024 && c.m > 128)) continue;
     if (!grid_fits(((M + c.m - 1) / c.m) * ((N + c.n - 1) / c.n), 256)) continue;
     const double t = mid_time(c, M, N, K, resid);
