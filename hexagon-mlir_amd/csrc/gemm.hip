@@ -1598,13 +1598,16 @@ int dispatch_gemm(const void* Av, const void* Bv, void* Cv, int64_t M, int64_t N
   // from the K on where that is ahead of the 32-k slabs of 128 x 128 below, whose rows leave in pieces of 16 bytes: with a residual, or a bias
   // off the runs of four, at any K; a bias in runs of four from 128 (3000 x 3004, us: K = 40 17 / 21, 120 21 / 20.6, 328 30 / 26; 20000 x 500
   // K = 200 0.91 times the rate, 328 1.03); neither from 320 (3000 x 3001: K = 40 16.7 / 22.4, 200 0.95, 328 1.09; 2100 x 5003 K = 328 0.93,
-  // 584 1.02; 1021 x 50257 K = 40 56 / 63, 120 1.05).
+  // 584 1.02; 1021 x 50257 K = 40 56 / 63, 120 1.05). Not up to sixteen rows against [K,N] weights of more tiles than CUs, K past 256 and off
+  // whole slabs, which are a stream of the weights (3 x 44624 x 432 13.1 / 14.8, 4 x 47848 x 744 19.5 / 22.1, 5 x 39680 x 528 14.8 / 17.0; 1.06 times
+  // the rate over 45; K to 192 0.92).
   if constexpr (std::is_same<T, OutT>::value) {
     const bool aligned = N % 8 == 0 && ldc % 8 == 0 && aligned_to(C, 16) && (!bias || aligned_to(bias, run)) &&
                          (!resid || (aligned_to(resid, run) && ldr % 4 == 0));
     const int from = resid || (bias && !fours) ? 0 : bias ? 128 : 320;
     const bool whole = K % BK2 == 0, odd = TRANS_B && !aligned && (bias || resid || !whole) && K >= from;
-    if (chunks && (aligned || odd) && lda < (1 << 21) && ldb < (1 << 21) && K <= (1 << 30)) {
+    const bool wide = !TRANS_B && M <= 16 && K > 256 && !whole && N > 128 * (int64_t)hexmi_num_cus();
+    if (chunks && (aligned || odd) && !wide && lda < (1 << 21) && ldb < (1 << 21) && K <= (1 << 30)) {
       const int now = odd || !whole ? 0 : large ? 256 : two_per_cu(((M + 127) / 128) * ((N + 127) / 128), K) ? 2 : 1;
       const GemmMidTile mid = plan_gemm_mid(M, N, K, now, resid != nullptr, odd);
       if (mid.m) return launch_gemm_mid<T, TRANS_B>(mid, A, B, C, M, N, K, lda, ldb, ldc, s, bias, resid, ldr, odd);
