@@ -46,7 +46,9 @@ constexpr int kPast = (int)0x80000000u;     // a copy's offset past the end of i
 // leave, and take bias and residual, by elements, 64 columns of a row to an instruction; the residual of the next rows is on its way meanwhile.
 // (us on 128 x 128 tiles of 32-k slabs, bias and residual one load after the other / here: 6177 x 869 x 1344 + residual 61 / 32, 896 x 35335 x 400 +
 // residual 190 / 88, 1021 x 50257 x 768 + bias 239 / 159, 2942 x 3571 x 3984 163 / 118, 4524 x 3741 x 384 + both 133 / 53; 1.83 times the rate over 40.)
-template <typename T, int TM, int TN, int NS, bool TRANS_B, bool EPI, bool ODD = false>
+// PLAIN: the result leaves by plain stores. Those past the caches are for rows in whole lines or half of them; rows 16 or 32 bytes off share
+// a line with the next tile, which memory then puts together twice.
+template <typename T, int TM, int TN, int NS, bool TRANS_B, bool EPI, bool ODD = false, bool PLAIN = false>
 __global__ __launch_bounds__(256)
 void gemm_mid_kernel(const T* __restrict__ A, const T* __restrict__ B, T* C, int M, int N, int K, int64_t lda, int64_t ldb, int64_t ldc,
                      int tiles_m, int tiles_n, const T* __restrict__ bias, const T* resid, int64_t ldr) {
@@ -309,7 +311,10 @@ void gemm_mid_kernel(const T* __restrict__ A, const T* __restrict__ B, T* C, int
     if (64 % CP && (lane >= RPI * CP || row >= TM * 16)) continue;
     const u32x4 v = *reinterpret_cast<const u32x4*>(cs + row * PITCH + ((c ^ swz(row)) * 8));
     const int grow = m0 + wm * TM * 16 + row, gcol = n0 + wn * TN * 16 + c * 8;
-    if (grow < M && gcol < N) __builtin_nontemporal_store(v, reinterpret_cast<u32x4*>(C + (int64_t)grow * ldc + gcol));
+    u32x4* to = reinterpret_cast<u32x4*>(C + (int64_t)grow * ldc + gcol);
+    if (grow < M && gcol < N) {
+      if constexpr (PLAIN) *to = v; else __builtin_nontemporal_store(v, to);
+    }
   }
 }
 
@@ -363,14 +368,19 @@ int launch_gemm_mid(const GemmMidTile& tile, const T* A, const T* B, T* C, int64
                     int64_t ldc, hipStream_t s, const T* bias, const T* resid, int64_t ldr, bool odd) {
   const int64_t tiles_m = (M + tile.m - 1) / tile.m, tiles_n = (N + tile.n - 1) / tile.n;
   if (!grid_fits(tiles_m * tiles_n, 256) || (resid && tile.m * tile.n > 192 * 192)) return HEXMI_ENOTSUP;
-#define HEXMI_MID_AS(TM, TN, NS, EPI, ODD)                                                                                           \
-  hipLaunchKernelGGL((gemm_mid_kernel<T, TM, TN, NS, TRANS_B, EPI, ODD>), dim3((unsigned)(tiles_m * tiles_n)), dim3(256), 0, s, A, B, C, \
-                     (int)M, (int)N, (int)K, lda, ldb, ldc, (int)tiles_m, (int)tiles_n, bias, resid, ldr)
+  // (us past the caches / plain: 4946 x 19608 x 32 + bias 94 / 62, 5925 x 6544 x 16 32 / 24, 1610 x 31888 x 32 45 / 32, 4108 x 8232 x 64 32 / 27, 5437 x 6200
+  // x 256 39 / 34, 1400 x 23656 x 512 56 / 53; 1.20 times the rate over 400. Results of 8 to 32 MiB 0.96 to 1.04 times it, with a residual 0.98, rows
+  // half a line off 0.95.)
+  const bool plain = ldc % 32 != 0 && !resid && M * N >= (16 << 20);
+#define HEXMI_MID_AS(TM, TN, NS, EPI, ODD, PLAIN)                                                                                    \
+  hipLaunchKernelGGL((gemm_mid_kernel<T, TM, TN, NS, TRANS_B, EPI, ODD, PLAIN>), dim3((unsigned)(tiles_m * tiles_n)), dim3(256), 0, s, A, B, \
+                     C, (int)M, (int)N, (int)K, lda, ldb, ldc, (int)tiles_m, (int)tiles_n, bias, resid, ldr)
 #define HEXMI_MID(TM, TN, NS)                                                                                                  \
   do {                                                                                                                         \
-    if (TRANS_B && odd) HEXMI_MID_AS(TM, TN, NS, false, TRANS_B);                                                               \
-    else if (bias || resid) HEXMI_MID_AS(TM, TN, NS, true, false);                                                              \
-    else HEXMI_MID_AS(TM, TN, NS, false, false);                                                                                \
+    if (TRANS_B && odd) HEXMI_MID_AS(TM, TN, NS, false, TRANS_B, false);                                                        \
+    else if (bias || resid) { if (plain) HEXMI_MID_AS(TM, TN, NS, true, false, true); else HEXMI_MID_AS(TM, TN, NS, true, false, false); } \
+    else if (plain) HEXMI_MID_AS(TM, TN, NS, false, false, true);                                                              \
+    else HEXMI_MID_AS(TM, TN, NS, false, false, false);                                                                         \
   } while (0)
   if (odd && !TRANS_B) return HEXMI_ENOTSUP;
   if (tile.m == 128 && tile.per_cu == 2) HEXMI_MID(4, 4, 2);

@@ -348,7 +348,9 @@ def test_gemm_parts_of_a_long_k(hexmi, dtype, out_dtype, M, N, K, trans_b, parts
     (645, 12456, 704, True, False), (1009, 24000, 328, True, False), (3073, 3080, 128, True, False),           # 256 x 192
     (301, 16392, 64, False, False), (339, 28864, 64, False, False), (192, 12800, 64, False, True), (130, 16120, 128, False, True),
     (384, 30464, 768, False, False), (384, 30464, 832, False, False),                                         # ... and not 192 x 128
-    (16, 32776, 264, False, False), (3, 40000, 600, True, True), (17, 32776, 264, False, False), (16, 32776, 256, True, False)])    # few rows
+    (16, 32776, 264, False, False), (3, 40000, 600, True, True), (17, 32776, 264, False, False), (16, 32776, 256, True, False),    # few rows
+    (4088, 4104, 40, False, False), (4089, 4104, 40, True, False), (4088, 4112, 136, True, False), (4088, 4128, 40, False, False),
+    (3001, 8200, 64, False, False), (2100, 8008, 200, False, True)])                                          # 32 MiB and more, rows off the lines
 def test_gemm_tiles_between_128_and_256(hexmi, dtype, trans_b, M, N, K, bias, residual):
     _against_double(hexmi, dtype, dtype, trans_b, M, N, K, bias, residual, M + N + K)
     # a strided output, the residual the output itself, nothing written around it
