@@ -317,7 +317,8 @@ template <> struct FewShape<64, 192> { typedef Shape<4, 3, 1, 4, 2, 3> S; };
 // -- unless there are more channels than that (40 x 14336 x 992 10.8 / 6.9, 16 x 14336 x 4096 16.9 / 15.0, 16 x 32000 x 5120 1.10, 32 x 32000 x 4096
 // 38 / 32), but for up to sixteen rows where eight ninths and more of the CUs would have a tile of weights whose rows stand whole 4 KiB
 // apart, which then come from the same channels: 8 x 24576 x 4096 21.7 / 25.8, 16 x 32768 x 4096 32.4 / 36.4, 6 x 22016 x 4096 20.5 / 23.0 (24576 x
-// 5120 1.06, 40000 x 4096 1.05).
+// 5120 1.06, 40000 x 4096 1.05), and where three quarters and fewer would have one of 64 x 192 and K is past 3000 (14 x 36608 x 4128 34.8 / 46.7, 6 x
+// 34731 x 5264 38 / 49, 3 x 33024 x 4192 32 / 37; 1.13 times the rate over 155, K to 3000 level, more channels 0.95 and less).
 // Calls that the tiles of gemm.hip do not take (zero points, K off whole slabs of 64) would go in passes of 128 rows: they come
 // here at any size, with the tile whose rounds cost least (weights: us per 3000 of K measured above; 511 x 10907 x 13056 1238 ->
 // 180, 1000 x 14336 x 992 139 -> 53, 304 x 11008 x 4368 73 -> 60).
@@ -347,7 +348,8 @@ GemmFewTile plan_w8a16_few(int64_t M, int64_t N, int64_t K, bool tiles, bool zp)
       if (area == 64 * 96 && K > (M <= 192 ? 2048 : 4608)) continue;
       if (chunked && ((M <= 32 && K > 1536) || (M <= 48 && (area > 32 * 64 ? K > 1536 : zp && K >= 3072)) ||
                       (M <= 64 && t.tile.n == 96 && K >= 2048) || (M <= 112 && area >= 64 * 96 && K >= 2048))) return {0, 0};
-      if (M <= 16 && K % 4096 == 0 && 9 * count(t.tile) >= 8 * cus) return {0, 0};
+      if (M <= 16 && ((K % 4096 == 0 && 9 * count(t.tile) >= 8 * cus) || (t.tile.n == 192 && K > 3000 && 4 * count(t.tile) <= 3 * cus)))
+        return {0, 0};
       return t.tile;
     }
     if (!t.weight || tiles || M <= 128 || count(t.tile) > 0x7fffffff) continue;
