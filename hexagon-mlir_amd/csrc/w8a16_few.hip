@@ -310,7 +310,8 @@ template <> struct FewShape<64, 192> { typedef Shape<4, 3, 1, 4, 2, 3> S; };
 //   up to 32 rows, tiles of 32 x 32 from K = 4096 on and of 32 x 64 from 1600: 32 x 6144 x 11008 23.3 / 26.0, 32 x 6144 x 4096 10.5 / 11.5,
 //   24 x 12288 x 1920 9.0 / 9.7, 24 x 11136 x 2176 10.2 / 11.3 (K = 3072 level, 8192 1.0);
 //   up to 48 rows tiles of 48 x 64 from 1600 on, up to 64 rows of 32 x 96 from 2048: 40 x 11008 x 4096 16.2 / 17.1, 56 x 11136 x 11008 37.3 / 40.5,
-//   64 x 9216 x 12032 with zero points 41 / 45; up to 112 rows of 64 x 96 and more from 2048: 80 x 11008 x 4096 20.6 / 22.6;
+//   64 x 9216 x 12032 with zero points 41 / 45; up to 112 rows of 64 x 96 and more from 2048: 80 x 11008 x 4096 20.6 / 22.6; up to 96 of 64 x 96 whose results leave by
+//   elements, or of a second slab that is mostly short (66 x 9866 x 304 5.5 / 6.8, 83 x 11894 x 1088 8.9 / 9.6, 77 x 10264 x 304 6.0 / 6.6; 108 rows 1.05);
 //   with zero points, which every tile takes from its weights and the chunked kernel once a weight: up to sixteen rows tiles of sixteen
 //   columns from K = 8192 on (16 x 1984 x 12032 12.7 / 13.8), up to 32 rows of 64 from 1600 (16 x 11136 x 2176 9.1 / 10.3, 24 x 5120 x 1920
 //   7.2 / 7.8), up to 48 rows of 32 x 64 from 3072 (48 x 8192 x 11008 0.94); K = 2176 on tiles of 16 x 16 stays a twentieth behind
@@ -348,6 +349,7 @@ GemmFewTile plan_w8a16_few(int64_t M, int64_t N, int64_t K, bool tiles, bool zp)
       if (area == 64 * 96 && K > (M <= 192 ? 2048 : 4608)) continue;
       if (chunked && ((M <= 32 && K > 1536) || (M <= 48 && (area > 32 * 64 ? K > 1536 : zp && K >= 3072)) ||
                       (M <= 64 && t.tile.n == 96 && K >= 2048) || (M <= 112 && area >= 64 * 96 && K >= 2048))) return {0, 0};
+      if (chunked && M <= 96 && area == 64 * 96 && (N % 8 != 0 || (K > 256 && K <= 384))) return {0, 0};
       if (M <= 16 && ((K % 4096 == 0 && 9 * count(t.tile) >= 8 * cus) || (t.tile.n == 192 && K > 3000 && 4 * count(t.tile) <= 3 * cus)))
         return {0, 0};
       return t.tile;

@@ -152,7 +152,9 @@ def test_w8a16_chunked_kernel_long_rows(hexmi, M, N, K, tiles, zero_points):
     (48, 6144, 3056, True, 4), (48, 6144, 3072, True, 18), (48, 6144, 3072, False, 4), (48, 9216, 1536, False, 4), (48, 9216, 1552, False, 19),
     (56, 9216, 2032, False, 4), (56, 9216, 2048, False, 19), (16, 24576, 4096, False, 19), (17, 24576, 4096, False, 4),
     (16, 24576, 4160, False, 4), (16, 20000, 4096, False, 4), (16, 14336, 4096, False, 4),
-    (16, 32840, 2992, False, 4), (16, 32840, 3008, False, 19), (5, 36864, 3008, True, 19), (16, 36872, 3008, False, 4), (17, 32840, 3008, False, 4)])
+    (16, 32840, 2992, False, 4), (16, 32840, 3008, False, 19), (5, 36864, 3008, True, 19), (16, 36872, 3008, False, 4), (17, 32840, 3008, False, 4),
+    (80, 9739, 400, False, 19), (80, 9736, 400, False, 4), (80, 9736, 384, False, 19), (80, 9736, 256, True, 4), (80, 9739, 1024, True, 19),
+    (97, 9739, 400, False, 4)])
 def test_w8a16_lines_between_tiles_and_the_chunked_kernel(hexmi, M, N, K, zero_points, kernel):
     from hexmi import _lib
     assert _lib.lib().hexmi_gemm_w8a16_kernel(M, N, K, int(zero_points), 0) & ~32 == kernel
