@@ -265,7 +265,8 @@ def test_gemm_one_round_of_tiles(hexmi, dtype, out_dtype, trans_b, M, N, K):
 @pytest.mark.parametrize("dtype,out_dtype", [(torch.float16, torch.float16), (torch.bfloat16, torch.float32),
                                              (torch.bfloat16, torch.bfloat16)])
 @pytest.mark.parametrize("M,N,K,trans_b,parts", [
-    (1, 8, 3072, False, True), (16, 1024, 4104, False, True), (3, 1000, 11376, False, True),                        # 16 x 64
+    (1, 8, 4608, False, True), (16, 1024, 4104, False, True), (3, 1000, 11376, False, True),                        # 16 x 64
+    (1, 8, 3072, False, False),                                     # (in parts before: 1 x 16 x 3088 7.0 us, as a whole 5.9)
     (1, 1032, 4096, False, True), (16, 4096, 4096, False, True), (15, 8200, 9000, False, True),                     # 16 x 128
     (17, 72, 3080, False, True), (32, 2048, 11008, False, True), (29, 2560, 5128, False, True),                     # 32 x 64
     (33, 56, 4608, False, True), (113, 304, 11968, False, True), (513, 512, 8192, False, True),                     # 64 x 64
