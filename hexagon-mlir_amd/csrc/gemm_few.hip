@@ -507,7 +507,7 @@ void gemm_merge_kernel(const float* __restrict__ sums, OutT* C, int M, int N, in
 // 9.9 / 8.3; 1.12 times the rate over 50 products of 65 to 267 rows, none slower.)
 // (64 x 96 and 96 x 64 ask for an eighth less than the tile of 128 x 64 that took their calls and leave fewer CUs idle: 2638 x 512 x 5600 40 /
 // 31, 168 x 6128 x 9520 86 / 68, 1725 x 624 x 9728 64 / 53, 583 x 2144 x 4288 24 / 20, 2751 x 488 x 5312 28.8 / 23.8, 280 x 4992 x 384 6.8 / 6.2; 1.08
-// times the rate over 3150 products. Not where the last row of 128 x 64 tiles is half padding, which costs no intake, and the weights are
+// and 1.04 times the rate over 2731 and 421 products. Not where the last row of 128 x 64 tiles is half padding, which costs no intake, and the weights are
 // more than the L2s hold of them beside the rest: 160 x 6016 x 6016 36 / 42, 284 x 4992 x 6096 40 / 49, [K,N] 427 x 2432 x 6656 44 / 54;
 // [N,K] weights of 6 to 7 million 1.01 times the rate, 7 to 8 0.93, 12 to 16 0.89, beyond 0.88; [K,N] 7 to 8 1.02, 8 to 9 0.94, 12 to 16 0.88;
 // 1130 products, an even count of 64 rows 1.05 to 1.10 at any. 48 x 32 before 32 x 64, [N,K]: 92 x 3304 x 8832 33 / 27.6, 687 x 400 x 3680 13.2 / 11.6,

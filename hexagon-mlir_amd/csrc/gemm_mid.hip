@@ -344,7 +344,7 @@ static constexpr MidCost kOne = {128, 128, 1, 4.0, 0.445, 0.073, 1.9, 0.0, 3.9},
 // products of whole 64s and of 8s 82 of whole 64s came here, at 1.13 times the rate, five of them 5 to 10 % slower than before (1636 x 21440 x
 // 1408 + both 122 / 135, 4480 x 3840 x 320 + bias 26.2 / 27.5).
 // The fits begin at K = 256 and say too little below for the tiles of 192 x 128: 339 x 28864 x 64 10.2 / 13.5, 285 x 31872 x 128 10.7 / 13.2, 192 x
-// 12800 x 64 + residual 8.1 / 9.9, beside 256 x 256 tiles also 384 x 30464 x 384 18.3 / 21.2 (all 44 slower but two; up to 64 rows they are ahead
+// 12800 x 64 + residual 8.1 / 9.9, beside 256 x 256 tiles also 384 x 30464 x 384 18.3 / 21.2 (33 of 34 slower; up to 64 rows they are ahead
 // of 256 x 256 tiles by a third, in the place of 128 x 128 ones two to a CU from 320 on).
 // Odd rows of less than 1024 of K: the larger tiles' elements leave with nothing beside them, so two of 128 x 128 to a CU (or one), us on the
 // 32-k slabs of gemm.hip / the tile of the fit / here: 8000 x 10001 x 456 151 / 205 / 143, 3000 x 15003 x 584 114 / 148 / 106, 6000 x 3333 x 584
